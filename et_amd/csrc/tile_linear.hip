@@ -31,8 +31,10 @@
 // tile_ffn_fused_kernel (feed-forward block / whole layer tail in one launch,
 // hidden activations in LDS), tile_linear_generic_kernel (raw and dense input).
 #include "tile_plan.h"
+#include "tile_walk.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <cstdlib>
 #include <cstring>
@@ -47,13 +49,18 @@ void set_attn_packed(int v);
 void set_ln_rows(int v);
 void set_tail_pair(int v);
 void set_tail_spin(int v);
+// tile_rows.hip
+bool tile_rows_fits(int K);
+int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *X, int M, int K, double pairs, bool gelu,
+                     bool raw, hipStream_t st);
 int tail_spin();
 
 constexpr int TL_THREADS = 512;
 constexpr int TL_WAVES = 8;
 constexpr int TL_BM = 32;
 constexpr int TL_PAD = 16;       // halves; LDS row stride == 32 (mod 64) bytes: measured conflict-free for ds_read_b128
-constexpr int TL_MAX_PANEL = 992;  // single-panel K limit: 32*(992+16)*2 B < 64 KB
+constexpr int TL_MAX_PANEL = 1024;      // plans: single-panel K limit, two 16-byte pieces per lane and row
+constexpr int TL_MAX_RAW_PANEL = 992;   // generic kernel: 32*(992+16)*2 B < 64 KB
 constexpr int TL_CHUNK = 768;
 constexpr int TL_MAX_LIN = 4;
 
@@ -75,6 +82,7 @@ struct TlProblem {
     int N;
     int nbr; // N / 16
     int ntile = 0; // surviving tiles where known (plans), 0 otherwise
+    int npair = 0; // index of an all-zero pair (plans)
 };
 
 // kernel arguments; per-linear fields as separate arrays that are only ever
@@ -1515,123 +1523,6 @@ __global__ void __launch_bounds__(TL_THREADS) tile_linear_generic_kernel(const T
     tl_epilogue<NB, GELU>(a, x, xs, Yp, N, nbr, acc, b4);
 }
 
-// ---------------------------------------------------------------------------
-// Few rows (a single short sequence).  Such a launch is a chain of memory
-// latencies, not a stream: the kernels above give a wave one (32-row panel,
-// block-row) unit whose tile pairs it requests TL_DEPTH at a time, one round
-// trip to memory per TL_DEPTH pairs and one more per K chunk of the panel
-// (BERT-base FFN2 on 128 rows: 20 us).  Here a workgroup of 16 waves takes a
-// 16-row panel with ALL of its K columns in LDS (16 x 3072 halves = 97 KB) and
-// 16/SPLIT block-rows; the pairs of a block-row are split over SPLIT waves (by
-// K chunk and by pair ranges inside a chunk - with the whole row of X in LDS
-// any partition works), and a wave requests up to TL_SK_D pairs at once, which
-// covers its whole share in the dense BERT-base cases: the panel and all of W
-// arrive in one round trip.  The SPLIT partial sums meet in LDS and are added
-// in a fixed order, so the result does not depend on timing.
-// ---------------------------------------------------------------------------
-constexpr int TL_SK_WAVES = 16;
-constexpr int TL_SK_BM = 16; // rows per panel
-constexpr int TL_SK_D = 12;  // pairs in flight per wave
-
-template <bool GELU, int SPLIT>
-__global__ void __launch_bounds__(TL_SK_WAVES * 64) tile_linear_splitk_kernel(const TlArgs a) {
-    constexpr int BR = TL_SK_WAVES / SPLIT; // block-rows per workgroup
-    extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
-    f16 *xs = reinterpret_cast<f16 *>(tl_smem);
-    const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3); // a panel's workgroups on one XCD
-    if (vid >= a.total)
-        return;
-    const int per_rp = a.ncg * a.nlin;
-    const int rp = vid / per_rp, rest = vid - rp * per_rp;
-    const int lin = rest / a.ncg, grp = rest - lin * a.ncg;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int c16 = lane & 15, g4 = lane >> 4, khalf8 = (g4 & 1) * 8, hi = lane >> 5;
-    const int ldx = a.K + ((a.K & 31) ? 0 : TL_PAD); // row stride == 32 (mod 64) bytes
-    const int m0 = rp * TL_SK_BM;
-    f16 *const Yp = TL_SEL(Y);
-    const int *const cptr = TL_SEL(cptr);
-    const int *const poff = TL_SEL(row_offset);
-    const f16 *const data = TL_SEL(data);
-    const f16 *const bias = TL_SEL(bias);
-    const int N = TL_SEL(N);
-    const int nbr = N >> 4;
-
-    // the panel: wave w fetches row w (DMA, 16 bytes per lane and instruction)
-    if (m0 + wave < a.M) {
-        const f16 *src = a.X + (size_t)(m0 + wave) * a.K;
-        f16 *dstrow = xs + wave * ldx;
-        const int pcpr = a.K >> 3;
-        for (int c0 = 0; c0 < pcpr; c0 += 64)
-            if (c0 + lane < pcpr)
-                load_lds16(src + (c0 + lane) * 8, dstrow + c0 * 8);
-    }
-    const int j = wave % BR, sp = wave / BR; // block-row of the group, split
-    const int bn = grp * BR + j;
-    // this wave's pairs: chunk ck of the plan, part `sub` of `spc` of the block-row's segment there
-    const int spc = SPLIT / a.nchunk; // (nchunk divides SPLIT)
-    const int ck = sp / spc, sub = sp - ck * spc;
-    int qa = 0, qb = 0;
-    f16x4 b4 = f16x4{0, 0, 0, 0};
-    if (bn < nbr) {
-        const int p0 = cptr[ck * nbr + bn] >> 1, p1 = cptr[ck * nbr + bn + 1] >> 1;
-        const int len = p1 - p0;
-        qa = p0 + len * sub / spc;
-        qb = p0 + len * (sub + 1) / spc;
-        b4 = *reinterpret_cast<const f16x4 *>(bias + bn * 16 + g4 * 4);
-    }
-    qa = __builtin_amdgcn_readfirstlane(qa);
-    qb = __builtin_amdgcn_readfirstlane(qb);
-    // Pairs at or beyond qb are replaced by the plan's spare pair (all-zero W,
-    // behind the last real pair): every slot loads and multiplies, nothing
-    // inside a round is conditional.
-    const int qsp = __builtin_amdgcn_readfirstlane(cptr[a.nchunk * nbr] >> 1);
-    const unsigned lane_w = hi * 256 + c16 * 16 + khalf8;
-    f16x8 w[TL_SK_D];
-    int o[TL_SK_D];
-    // (requested while the panel is still arriving: loads return in order, the
-    // wait below covers both)
-#pragma unroll
-    for (int i = 0; i < TL_SK_D; i++)
-        tl_load_pair(data, poff, qa + i < qb ? qa + i : qsp, lane_w, hi, w[i], o[i]);
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
-    __syncthreads();
-
-    // chunk-local column offsets of a multi-chunk plan -> offsets in the full row
-    const char *xlane = reinterpret_cast<const char *>(xs + c16 * ldx + khalf8) + (size_t)ck * a.KC * 2;
-    f32x4 acc0 = f32x4{0.f, 0.f, 0.f, 0.f}, acc1 = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int q = qa;;) {
-#pragma unroll
-        for (int i = 0; i < TL_SK_D; i += 2) { // two accumulators: two independent MFMA chains
-            acc0 = mfma16x16x32(w[i], *reinterpret_cast<const f16x8 *>(xlane + o[i]), acc0);
-            acc1 = mfma16x16x32(w[i + 1], *reinterpret_cast<const f16x8 *>(xlane + o[i + 1]), acc1);
-        }
-        q += TL_SK_D;
-        if (q >= qb)
-            break;
-#pragma unroll
-        for (int i = 0; i < TL_SK_D; i++)
-            tl_load_pair(data, poff, q + i < qb ? q + i : qsp, lane_w, hi, w[i], o[i]);
-    }
-    const f32x4 acc = acc0 + acc1;
-
-    // partial sums -> LDS (behind the panel), summed by the first wave of each block-row
-    f32x4 *red = reinterpret_cast<f32x4 *>(xs + TL_SK_BM * ldx);
-    red[(sp * BR + j) * 64 + lane] = acc;
-    __syncthreads();
-    if (sp == 0 && bn < nbr) {
-        f32x4 t = red[j * 64 + lane];
-#pragma unroll
-        for (int k = 1; k < SPLIT; k++)
-            t += red[(k * BR + j) * 64 + lane];
-        f16x4 ov = __builtin_convertvector(t + __builtin_convertvector(b4, f32x4), f16x4);
-        if (GELU)
-            ov = gelu4(ov);
-        if (m0 + c16 < a.M)
-            *reinterpret_cast<f16x4 *>(Yp + (size_t)(m0 + c16) * N + bn * 16 + g4 * 4) = ov;
-    }
-}
-
 #undef TL_SEL
 
 // ---------------------------------------------------------------------------
@@ -1657,28 +1548,34 @@ static hipError_t allow_lds(size_t lds) {
 }
 
 template <int NB, bool GELU, int MODE>
-static void launch_inst(const TlArgs &a, size_t lds, hipStream_t st) {
+static int launch_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     const dim3 grid(a.per_xcd * 8), block(TL_THREADS);
     if constexpr (MODE == TL_PLAN) {
         // (block-rows per wave beyond 3 never paid off for the plan kernels)
         constexpr int PNB = NB > 3 ? 3 : NB;
-        if (a.nchunk == 1)
-            hipLaunchKernelGGL((tile_linear_resident_kernel<PNB, GELU, TL_WAVES, false>), grid, block, lds, st, a);
-        else
-            hipLaunchKernelGGL((tile_linear_plan_kernel<PNB, GELU, TL_WAVES, false>), grid, block, lds, st, a);
+        if (a.nchunk == 1) {
+            constexpr auto k = &tile_linear_resident_kernel<PNB, GELU, TL_WAVES, false>;
+            ET_HIP(allow_lds<k>(lds));
+            hipLaunchKernelGGL(k, grid, block, lds, st, a);
+        } else {
+            constexpr auto k = &tile_linear_plan_kernel<PNB, GELU, TL_WAVES, false>;
+            ET_HIP(allow_lds<k>(lds));
+            hipLaunchKernelGGL(k, grid, block, lds, st, a);
+        }
     } else {
         hipLaunchKernelGGL((tile_linear_generic_kernel<NB, GELU, MODE>), grid, block, lds, st, a);
     }
+    return launch_status("tile_linear launch");
 }
 
 template <bool GELU, int MODE>
-static void launch_nb(int nb, const TlArgs &a, size_t lds, hipStream_t st) {
+static int launch_nb(int nb, const TlArgs &a, size_t lds, hipStream_t st) {
     switch (nb) {
-    case 1: launch_inst<1, GELU, MODE>(a, lds, st); break;
-    case 2: launch_inst<2, GELU, MODE>(a, lds, st); break;
-    case 3: launch_inst<3, GELU, MODE>(a, lds, st); break;
-    case 4: launch_inst<4, GELU, MODE>(a, lds, st); break;
-    default: launch_inst<6, GELU, MODE>(a, lds, st); break;
+    case 1: return launch_inst<1, GELU, MODE>(a, lds, st);
+    case 2: return launch_inst<2, GELU, MODE>(a, lds, st);
+    case 3: return launch_inst<3, GELU, MODE>(a, lds, st);
+    case 4: return launch_inst<4, GELU, MODE>(a, lds, st);
+    default: return launch_inst<6, GELU, MODE>(a, lds, st);
     }
 }
 
@@ -1870,8 +1767,7 @@ static int g_tile_bm64 = 1; // et_tuning_set("tile_bm64")
 // below, 128 x 128 blocks leave most CUs without work and the tile kernels win)
 static int g_row_gemm_min_rows = 1024;
 
-static int g_tile_splitk_k1 = 0;
-static int g_tile_splitk_rows = -1; // et_tuning_set("tile_splitk_rows"): row count up to which the few-rows kernel runs, -1 automatic
+static int g_tile_rows_most = -1; // et_tuning_set("tile_splitk_rows"): most rows for which a plan runs on whole rows, -1 automatic
 
 template <int NB, bool GELU, int NW = TL_WAVES>
 static int launch_resident64(const TlArgs &a, size_t lds, hipStream_t st) {
@@ -1903,49 +1799,43 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
     a.K = K;
     a.KC = KC;
     a.nchunk = nchunk;
-    // Few rows and K in several chunks: up to 128 rows, up to 256 where at
-    // least three quarters of the tiles survive (each 16-row panel streams W
-    // once more, which a long dense stream repays for longer than a short one).
-    // With K in one chunk the kernels below are as fast.
-    int sk_rows = g_tile_splitk_rows;
-    if (sk_rows < 0) {
-        const long all_tiles = (long)nbr_max * (K / 16);
-        sk_rows = nlin == 1 && 4L * probs[0].ntile >= 3 * all_tiles ? 256 : 128;
-    }
-    if (mode == TL_PLAN && M <= sk_rows && (nchunk == 2 || nchunk == 4 || nchunk == 8 || g_tile_splitk_k1) &&
-        (nchunk == 1 || nchunk == 2 || nchunk == 4 || nchunk == 8) && g_tile_nb == 0) {
-        // few rows: 16-row panels with the whole of K in LDS, a block-row's pairs split over 4 or 8 waves
-        const int split = nchunk == 1 ? 4 : 8;
-        const int br = TL_SK_WAVES / split;
-        const size_t lds_sk = (size_t)TL_SK_BM * (K + ((K & 31) ? 0 : TL_PAD)) * sizeof(f16) +
-                              (size_t)TL_SK_WAVES * 64 * sizeof(f32x4);
-        if (lds_sk <= 160 * 1024) {
-            a.ncg = (nbr_max + br - 1) / br;
-            a.total = ((M + TL_SK_BM - 1) / TL_SK_BM) * a.ncg * nlin;
-            a.ipw = 1;
-            a.per_xcd = (a.total + 7) / 8;
-            const dim3 grid(a.per_xcd * 8), block(TL_SK_WAVES * 64);
-#define TL_SK_LAUNCH(GELU_, SPLIT_)                                                               \
-    {                                                                                             \
-        constexpr auto k = &tile_linear_splitk_kernel<GELU_, SPLIT_>;                                        \
-        ET_HIP(allow_lds<k>(lds_sk));     \
-        hipLaunchKernelGGL(k, grid, block, lds_sk, st, a);                                        \
-    }
-            if (split == 4) {
-                if (gelu) TL_SK_LAUNCH(true, 4) else TL_SK_LAUNCH(false, 4)
-            } else {
-                if (gelu) TL_SK_LAUNCH(true, 8) else TL_SK_LAUNCH(false, 8)
-            }
-#undef TL_SK_LAUNCH
-            return launch_status("tile_linear (few rows) launch");
+    // Whole rows in LDS (tile_rows.hip): plans with K in several chunks, and the caller's own tile_mat.
+    // Plans: the estimated time of both, in microseconds.  Whole rows: W is streamed once per 16 rows, 5.5 us and 16.5
+    // MB per us.  Chunks: a round of workgroups is a chain of a fetch and a stream per chunk, up to 20 % slower when
+    // all slots are taken.  Both fit 20 measured launches (3072 -> 768 and 4096 -> 1024, 0 / 50 / 80 % pruned, 340 to
+    // 8192 rows) within 15 %; the crossovers are 340 .. 600 rows dense, 1000 at 50 % and 2000 .. 4000 at 80 %.
+    // Raw lists: always where K is beyond the generic kernel's panel (it filters every list once per chunk: three to
+    // eight times slower), else while there is no more than one workgroup per CU (16 rows x 16 block-rows each).
+    if (g_tile_nb == 0 && tile_rows_fits(K) && mode != TL_DENSE && (mode != TL_PLAN || nchunk > 1)) {
+        const bool raw = mode != TL_PLAN;
+        const long panels = (M + 15) / 16;
+        double pairs = 0.0, wmb = 0.0; // per block-row; megabytes of W
+        LfLinear l[TL_MAX_LIN];
+        f16 *Ys[TL_MAX_LIN];
+        for (int i = 0; i < nlin; i++) {
+            const double p = raw ? 0.1 * K / 16 : 0.5 * probs[i].ntile / probs[i].nbr; // (raw: the count is on the device)
+            l[i] = LfLinear{probs[i].data, probs[i].cptr, probs[i].row_offset, probs[i].bias, probs[i].nbr,
+                            raw ? 1 : nchunk, raw ? 0 : KC * 2, probs[i].npair};
+            Ys[i] = probs[i].Y;
+            pairs += p / nlin;
+            wmb += p * probs[i].nbr * 1e-3;
         }
+        const int onb = choose_nb((M + TL_BM - 1) / TL_BM, nbr_max, nlin);
+        const double wgs = (double)((M + TL_BM - 1) / TL_BM) * ((nbr_max + TL_WAVES * onb - 1) / (TL_WAVES * onb)) * nlin / g_tile_min_wgs;
+        const double chunked = std::ceil(wgs) * (5.0 + 1.25 * nchunk + 0.11 * pairs * onb) * (1.0 + 0.2 * std::min(wgs, 1.0));
+        const bool take = raw ? nchunk > 1 || panels * ((nbr_max + 15) / 16) <= std::max(et_device_cu_count(), 1)
+                          : g_tile_rows_most >= 0 ? M <= g_tile_rows_most
+                                                  : 5.5 + (double)panels * wmb / 16.5 <= chunked;
+        if (take)
+            return tile_rows_launch(l, Ys, nlin, X, M, K, pairs, gelu, raw, st);
     }
     if (mode == TL_PLAN && nchunk == 1 && g_tile_bm64 && g_tile_nb == 0) {
         // 64-row panels, one workgroup per CU: twice the rows per kilobyte of W
         // streamed.  Needs the panel and one 64-row staging tile per wave in LDS
         // and at least two items per CU.  Twelve waves of two block-rows (where
         // the LDS holds their staging tiles: K <= 784), or eight waves of three
-        // or of two, and d consecutive items of a panel per workgroup: the
+        // or of two (or of one: K 817 .. 1024; 4096 rows, 1024 -> 4096, 50 %: 55 -> 32 us against 32-row panels),
+        // and d consecutive items of a panel per workgroup: the
         // combination with the least estimated time (a round of workgroups costs
         // the panel load, 2/3 of a 24-block-row item, plus its items).  Twelve
         // waves come first and win ties: the same items as eight waves of three,
@@ -1953,14 +1843,16 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         // (Q/K/V of the benchmark: 20 -> 17.5 us).
         const int cus = std::max(et_device_cu_count(), 1);
         const int nrp64 = (M + TL_BM64 - 1) / TL_BM64;
-        static const int cand[3][2] = {{12, 2}, {8, 3}, {8, 2}}; // waves, block-rows per wave
+        static const int cand[4][2] = {{12, 2}, {8, 3}, {8, 2}, {8, 1}}; // waves, block-rows per wave
         double best = 0.0;
         int best_c = -1, best_d = 1, best_ncg = 1;
         size_t best_lds = 0;
-        for (int c = 0; c < 3; c++) {
+        for (int c = 0; c < 4; c++) {
             const int nw = cand[c][0], nb = cand[c][1];
             if (nw == 12 && g_tile_bm64 == 4)
                 continue; // (tuning: eight waves only)
+            if (nb == 1 && best_c >= 0)
+                continue; // (only where no wider form fits the LDS)
             const size_t lds64 = (size_t)TL_BM64 * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16) +
                                  (size_t)nw * TL_BM64 * (16 * nb + 8) * sizeof(f16);
             const int ncg64 = (nbr_max + nw * nb - 1) / (nw * nb);
@@ -1969,7 +1861,9 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
                 continue;
             const int per_rp = ncg64 * nlin;
             for (int d = 1; d <= per_rp; d++) {
-                if (per_rp % d)
+                // (eight block-rows per item: K beyond 816.  More than 16 of them per workgroup and the launch slows
+                // down: 16384 rows, 1024 -> 4096, 80 %: 101 us with 8, 104 with 16, 122 with 32)
+                if (per_rp % d || (nb == 1 && d > 16))
                     continue;
                 const long nwg = items / d, rounds = (nwg + cus - 1) / cus;
                 const double cost = (double)rounds * (2.0 / 3.0 + d * (nw * nb) / 24.0);
@@ -1992,7 +1886,9 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
                             : launch_resident64<2, false, 12>(a, best_lds, st);
             if (best_c == 1)
                 return gelu ? launch_resident64<3, true>(a, best_lds, st) : launch_resident64<3, false>(a, best_lds, st);
-            return gelu ? launch_resident64<2, true>(a, best_lds, st) : launch_resident64<2, false>(a, best_lds, st);
+            if (best_c == 2)
+                return gelu ? launch_resident64<2, true>(a, best_lds, st) : launch_resident64<2, false>(a, best_lds, st);
+            return gelu ? launch_resident64<1, true>(a, best_lds, st) : launch_resident64<1, false>(a, best_lds, st);
         }
     }
     const int nrp = (M + TL_BM - 1) / TL_BM;
@@ -2032,24 +1928,17 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
     const size_t lds = mode == TL_PLAN
                            ? lds_x + (size_t)TL_WAVES * TL_BM * (16 * nb + 8) * sizeof(f16)
                            : std::max(lds_x, lds_y);
-    if (mode == TL_PLAN) {
-        if (gelu) launch_nb<true, TL_PLAN>(nb, a, lds, st);
-        else launch_nb<false, TL_PLAN>(nb, a, lds, st);
-    } else if (mode == TL_RAW) {
-        if (gelu) launch_nb<true, TL_RAW>(nb, a, lds, st);
-        else launch_nb<false, TL_RAW>(nb, a, lds, st);
-    } else if (mode == TL_FILTER) {
-        if (gelu) launch_nb<true, TL_FILTER>(nb, a, lds, st);
-        else launch_nb<false, TL_FILTER>(nb, a, lds, st);
-    } else {
-        if (gelu) launch_nb<true, TL_DENSE>(nb, a, lds, st);
-        else launch_nb<false, TL_DENSE>(nb, a, lds, st);
-    }
-    return launch_status("tile_linear launch");
+    if (mode == TL_PLAN)
+        return gelu ? launch_nb<true, TL_PLAN>(nb, a, lds, st) : launch_nb<false, TL_PLAN>(nb, a, lds, st);
+    if (mode == TL_RAW)
+        return gelu ? launch_nb<true, TL_RAW>(nb, a, lds, st) : launch_nb<false, TL_RAW>(nb, a, lds, st);
+    if (mode == TL_FILTER)
+        return gelu ? launch_nb<true, TL_FILTER>(nb, a, lds, st) : launch_nb<false, TL_FILTER>(nb, a, lds, st);
+    return gelu ? launch_nb<true, TL_DENSE>(nb, a, lds, st) : launch_nb<false, TL_DENSE>(nb, a, lds, st);
 }
 
-static void chunking(int K, int *KC, int *nchunk) {
-    if (K <= TL_MAX_PANEL) {
+static void chunking(int K, int *KC, int *nchunk, int panel = TL_MAX_PANEL) {
+    if (K <= panel) {
         *KC = K;
         *nchunk = 1;
     } else {
@@ -2078,7 +1967,7 @@ static int raw_tile_linear(void *Y, const void *X, const int *row_ptr, const int
     p.N = N;
     p.nbr = N / 16;
     int KC, nchunk;
-    chunking(K, &KC, &nchunk);
+    chunking(K, &KC, &nchunk, TL_MAX_RAW_PANEL);
     return tile_launch(&p, 1, static_cast<const f16 *>(X), M, K, KC, nchunk, gelu,
                        nchunk == 1 ? TL_RAW : TL_FILTER, static_cast<hipStream_t>(stream));
 }
@@ -2088,12 +1977,8 @@ static int raw_tile_linear(void *Y, const void *X, const int *row_ptr, const int
 static int g_tail_pair_min_wgs = 0; // et_tuning_set("tile_tail_pair_min_wgs"): 0 = three quarters of the CUs
 
 extern "C" int et_tuning_set(const char *key, int value) {
-    if (key && !strcmp(key, "tile_splitk_k1")) {
-        et::g_tile_splitk_k1 = value;
-        return ET_OK;
-    }
     if (key && !strcmp(key, "tile_splitk_rows")) {
-        et::g_tile_splitk_rows = value;
+        et::g_tile_rows_most = value;
         return ET_OK;
     }
     if (key && !strcmp(key, "row_gemm_min_rows")) {
@@ -2209,7 +2094,7 @@ static int row_linear(void *out, const void *in, const void *weight, const void 
     p.N = N;
     p.nbr = N / 16;
     int KC, nchunk;
-    chunking(K, &KC, &nchunk);
+    chunking(K, &KC, &nchunk, TL_MAX_RAW_PANEL);
     return tile_launch(&p, 1, static_cast<const f16 *>(in), M, K, KC, nchunk, gelu, TL_DENSE,
                        static_cast<hipStream_t>(stream));
 }
@@ -2268,7 +2153,9 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
     ET_REQUIRE(v == 0, ET_ERR_FORMAT, "et_tile_plan_create: malformed tile_mat (check %d)", v);
     const int nbr = out_feat / 16;
     int KC, nchunk;
-    chunking(in_feat, &KC, &nchunk);
+    // (a linear that narrows its input is a feed-forward block's second one: chunks of 768 hidden columns are what the
+    // fused kernel walks)
+    chunking(in_feat, &KC, &nchunk, out_feat < in_feat ? TL_MAX_RAW_PANEL : TL_MAX_PANEL);
     // Plan layout: tiles ordered by (chunk, block-row, column); every
     // (chunk, block-row) segment padded to an even count with an all-zero
     // tile that reuses the segment's last column (so a pair never straddles
@@ -2330,6 +2217,7 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
     p->ntile = ntile;
     p->KC = KC;
     p->nchunk = nchunk;
+    p->npair = cptr.back() / 2;
     int rc = ET_OK;
     auto up = [&](void **dst, const void *h, size_t bytes) {
         if (rc != ET_OK)
@@ -2391,6 +2279,8 @@ extern "C" int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *co
         pr[i].bias = plans[i]->d_bias;
         pr[i].N = plans[i]->out_feat;
         pr[i].nbr = plans[i]->out_feat / 16;
+        pr[i].ntile = plans[i]->ntile;
+        pr[i].npair = plans[i]->npair;
     }
     ET_REQUIRE(aligned16(X), ET_ERR_ALIGNMENT, "et_tile_plan_run_multi: X not aligned");
     if (M == 0)
@@ -2607,6 +2497,7 @@ extern "C" int et_tile_plan_run(const et_tile_plan *plan, void *Y, const void *X
     pr.N = plan->out_feat;
     pr.nbr = plan->out_feat / 16;
     pr.ntile = plan->ntile;
+    pr.npair = plan->npair;
     return tile_launch(&pr, 1, static_cast<const f16 *>(X), M, plan->in_feat, plan->KC,
                        plan->nchunk, gelu != 0, TL_PLAN, static_cast<hipStream_t>(stream));
 }

@@ -12,6 +12,7 @@ void tail_program_destroy(TailProgram *p);
 
 struct et_tile_plan {
     int in_feat = 0, out_feat = 0, ntile = 0, KC = 0, nchunk = 0;
+    int npair = 0; // pairs of tiles in the plan layout; pair npair is all zero
     et::f16 *d_data = nullptr;
     int *d_cptr = nullptr;
     int *d_row_offset = nullptr;

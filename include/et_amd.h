@@ -449,11 +449,10 @@ int et_device_synchronize(void);
  *                     64-row panels where two such items per CU exist; 2: also
  *                     with fewer items; 4: as 1 with eight waves per workgroup
  *                     only (no twelve-wave form)
- *   "tile_splitk_rows" most rows for which a planned linear with K > 992 runs
- *                     the few-rows kernel (16-row panels, a block-row's tile
- *                     pairs split over several waves); -1 (default): 128, or
- *                     256 where at least 3/4 of the tiles survive; 0: never
- *   "tile_splitk_k1"  1: the few-rows kernel also for K <= 992 (default 0)
+ *   "tile_splitk_rows" most rows for which a planned linear with K > 1024 runs
+ *                     on whole rows in LDS (16-row panels, a block-row's tile
+ *                     pairs split over several waves where there are few); -1
+ *                     (default): by the amount of W streamed; 0: never
  *   "row_gemm_min_rows" rows from which et_row_spmm_add_bias runs the dense
  *                     GEMM kernel (default 1024; 0: never)
  *   "tile_fuse_ffn"   0: et_tile_plan_ffn_fusable answers no (the feed-forward

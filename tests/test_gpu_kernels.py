@@ -1110,3 +1110,30 @@ def test_microbenchmarks_report_plausible_rates():
         check(mbl.et_microbench(7, 0, 0, C.byref(sec), C.byref(units)))
     with pytest.raises(Exception):               # a stride the 16-byte reads cannot take: refused before anything is allocated
         check(mbl.et_microbench(0, 1570, 16, C.byref(sec), C.byref(units)))
+
+
+@pytest.mark.parametrize("M,N,Kd,sp,gelu", [
+    (1, 16, 4848, 0.5, False),      # the widest row that fits the LDS, one block-row: split over all the waves
+    (17, 272, 4848, 0.9, True),     # a panel of one row, 17 block-rows
+    (20, 48, 4864, 0.6, False),     # one tile wider: the kernels that filter / walk chunks
+    (300, 1040, 1040, 0.7, True),   # two chunks, the second 272 columns; ragged column groups
+    (1000, 768, 3072, 0.8, False), (2050, 784, 3072, 0.95, False),   # several block-rows per wave; empty ones
+    (40, 64, 2048, 1.0, True),      # no tile at all
+    (4100, 64, 1024, 0.5, False), (2050, 1040, 1008, 0.8, True),   # single panel beyond 816 columns: 64-row items
+])
+def test_tile_linear_whole_rows(K, M, N, Kd, sp, gelu):
+    """planned and raw (unsorted lists, odd counts) linears on whole rows in LDS, at the edges of that kernel's range"""
+    from et_amd.encoder import Linear_tile
+    r = rng(900 + M + N)
+    lin = make_tile_linear(r, N, Kd, sp, seed=M + Kd, std=0.05, bias_std=0.2)
+    X = randn_h(r, (M, Kd))
+    rows = np.unique(np.concatenate([np.arange(min(M, 40)), r.integers(0, M, 60), np.arange(max(M - 20, 0), M)]))
+    want = orc.tile_linear(X[rows], lin["row_ptr"], lin["row_offset"], lin["data"], lin["bias"], N, gelu=gelu, f64=True)
+    tol = max(np.abs(want.astype(np.float64)).max() * 2.0 ** -10, 1e-3)
+    ro, data = (dev(lin[k]) if lin[k].size else None for k in ("row_offset", "data"))
+    raw = host(K.tile_spmm_add_bias(dev(X), dev(lin["row_ptr"]), ro, data, dev(lin["bias"]), N, gelu=gelu))
+    check_close(raw[rows], want, max_abs=tol, mean_rel=5e-4, what="raw")
+    lt = Linear_tile(Kd, N, M, lin["row_offset"].size, lin["data"], lin["row_ptr"], lin["row_offset"], lin["bias"], gelu)
+    planned = host(lt.run(dev(X)))
+    check_close(planned[rows], want, max_abs=tol, mean_rel=5e-4, what="planned")
+    assert np.array_equal(planned, host(lt.run(dev(X))))
