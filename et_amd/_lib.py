@@ -49,6 +49,11 @@ PROTOTYPES = {
     "et_tile_plan_tail_prepare": (_i, [_vp, _vp, _vp]),
     "et_tile_plan_tail_ws_bytes": (_sz, [_vp, _vp, _vp, _i]),
     "et_tail_ws_bytes_for": (_sz, [_i, _i]),
+    "et_layer_flow_create": (_i, [C.POINTER(_vp)] + [_vp] * 6 + [_i] * 3),
+    "et_layer_flow_destroy": (None, [_vp]),
+    "et_layer_flow_set_packed": (_i, [_vp, _ip]),
+    "et_layer_flow_pays": (_i, [_vp, _i]),
+    "et_layer_flow_run": (_i, [_vp] * 7 + [_vp, _ip, _ip] + [_vp] * 4 + [_f, _vp]),
     "et_wait_status_take": (_i, []),
     "et_wait_status_raise_for_test": (None, []),
     "et_tile_plan_run_multi": (_i, [C.POINTER(_vp), C.POINTER(_vp), _i, _vp, _i, _vp]),

@@ -72,6 +72,18 @@ __device__ __forceinline__ void load_lds16(const void *gsrc, void *lds_base) {
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 
+// Stores whose data other workgroups of the SAME launch read: an agent-scope
+// store goes through the XCD's own L2 to the device's coherence point, and is
+// there once vmcnt has counted it.
+__device__ __forceinline__ void store_agent4(f16 *p, f16x4 v) {
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), __builtin_bit_cast(unsigned long long, v),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_agent8(f16 *p, f16x8 v) {
+    store_agent4(p, f16x4{v[0], v[1], v[2], v[3]});
+    store_agent4(p + 4, f16x4{v[4], v[5], v[6], v[7]});
+}
+
 // ---- wave64 reductions (all lanes receive the result) -----------------------
 // Data-parallel-primitive moves inside a row of 16 lanes (no LDS round trip as
 // with __shfl): quad_perm [1,0,3,2] and [2,3,0,1], row_half_mirror, row_mirror.

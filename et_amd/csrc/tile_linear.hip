@@ -53,6 +53,7 @@ void set_tail_spin(int v);
 bool tile_rows_fits(int K);
 int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *X, int M, int K, double pairs, bool gelu,
                      bool raw, hipStream_t st);
+void set_flow_rows(int v);
 int tail_spin();
 
 constexpr int TL_THREADS = 512;
@@ -1740,7 +1741,10 @@ static int g_tile_ln_min_panels = 96;
 // the layer tail in one launch: from fewer panels than the linear + LayerNorm kernels (measured on
 // BERT-base at 80 %: one launch 42 us for any count below one per CU, step by step 37 / 43 / 54 us
 // at 52 / 80 / 95 panels)
-static int g_tile_tail_min_panels = 72;
+constexpr int TL_TAIL_MIN_PANELS = 72;
+static int g_tile_tail_min_panels = TL_TAIL_MIN_PANELS;
+// the layer tail's choice is forced (a layer then runs its steps as separate launches)
+bool tail_tuned() { return g_tile_tail_min_panels != TL_TAIL_MIN_PANELS || g_tile_fuse_ffn != 2; }
 
 // Block-rows per wave.  Measured on the BERT-base shapes (rows 4096..8192):
 // three block-rows per wave is the best trade between panel re-reads (fewer
@@ -2019,7 +2023,7 @@ extern "C" int et_tuning_set(const char *key, int value) {
     }
     if (key && !strcmp(key, "tile_ln_min_panels")) {
         et::g_tile_ln_min_panels = value > 0 ? value : 96;
-        et::g_tile_tail_min_panels = value > 0 ? value : 72;
+        et::g_tile_tail_min_panels = value > 0 ? value : et::TL_TAIL_MIN_PANELS;
         return ET_OK;
     }
     if (key && !strcmp(key, "tile_fuse_ln")) {
@@ -2028,6 +2032,10 @@ extern "C" int et_tuning_set(const char *key, int value) {
     }
     if (key && !strcmp(key, "tile_min_wgs")) {
         et::g_tile_min_wgs = value;
+        return ET_OK;
+    }
+    if (key && !strcmp(key, "layer_flow_rows")) {
+        et::set_flow_rows(value);
         return ET_OK;
     }
     if (key && !strcmp(key, "ln_rows")) {

@@ -40,6 +40,8 @@ class Encoder_base {
     // activation units (and behind the score buffer of Encoder_length)
     void *tail_ws;
     size_t tail_ws_bytes;
+    // the layer as one launch, for few rows (et_layer_flow_create); null where that does not exist
+    et_layer_flow *flow;
 
     int rows() const { return batch * seq_len; }
     static size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -60,7 +62,7 @@ class Encoder_base {
           ln_gamma{Weight<half>(ln_gamma_1, d_model_), Weight<half>(ln_gamma_2, d_model_)},
           ln_beta{Weight<half>(ln_beta_1, d_model_), Weight<half>(ln_beta_2, d_model_)},
           has_mask(mask_ != nullptr), mask_summary(nullptr), stream(nullptr), log2_scale(1.0f),
-          total_rows(batch_ * seq_len_), tail_ws(nullptr), tail_ws_bytes(0) {
+          total_rows(batch_ * seq_len_), tail_ws(nullptr), tail_ws_bytes(0), flow(nullptr) {
         if (mask_) {
             mask = Weight<half>(mask_, seq_len_ * seq_len_);
             // the mask never changes after construction: let the attention
@@ -75,6 +77,7 @@ class Encoder_base {
         place_tail_ws(units_bytes(d_model, seq_len, batch));
     }
     virtual ~Encoder_base() {
+        et_layer_flow_destroy(flow);
         if (mask_summary) {
             et_attention_mask_summary_attach(mask.get(), seq_len, nullptr);
             et_free(mask_summary);
@@ -117,6 +120,8 @@ class Encoder_base {
         d_lens = Weight<int>(lens.data(), batch);
         d_cu = Weight<int>(cu.data(), batch + 1);
         d_order = Weight<int>(order.data(), batch);
+        if (flow)
+            etChk(et_layer_flow_set_packed(flow, cu.data()));
     }
     int valid_rows() const { return total_rows; }
     // packed sequence i is rows cu[i]..cu[i+1]-1 and is batch entry order[i]
@@ -126,6 +131,19 @@ class Encoder_base {
   protected:
     half *mask_ptr() const { return has_mask ? mask.get() : nullptr; }
     const int *lens_ptr() const { return lens.empty() ? nullptr : d_lens.get(); }
+
+    void create_flow(const Linear_tile &Q, const Linear_tile &K, const Linear_tile &V, const Linear_tile &O,
+                     const Linear_tile &M1, const Linear_tile &M2) {
+        etChk(et_layer_flow_create(&flow, Q.tile_plan(), K.tile_plan(), V.tile_plan(), O.tile_plan(), M1.tile_plan(),
+                                   M2.tile_plan(), seq_len, nheads, batch));
+    }
+    bool flow_pays(int nrows) const { return et_layer_flow_pays(flow, nrows) != 0; }
+    // the whole layer; `cu`: packed sequences, else a padded batch with `lengths` (or null)
+    void run_flow(half *out, half *in, const int *lengths, const int *cu) {
+        etChk(et_layer_flow_run(flow, out, in, buffers[0], buffers[1], buffers[2], buffers[3], mask_ptr(), lengths, cu,
+                                ln_gamma[0].get(), ln_beta[0].get(), ln_gamma[1].get(), ln_beta[1].get(), log2_scale,
+                                stream));
+    }
 
     // steps 6-10 of encoder/encoder.cu:33-44, shared by every encoder kind:
     // O projection, skip-LN with the layer input, FFN1+GELU, FFN2, skip-LN.
@@ -159,8 +177,13 @@ class Encoder_tile : public Encoder_base {
         // the reference asserts this (encoder/encoder.cu:17)
         etRequire(MLP1_linear.is_gelu, "Encoder_tile: MLP1_linear must be the GELU variant");
         Linear_tile::tail_prepare(O_linear, MLP1_linear, MLP2_linear);
+        create_flow(Q_linear, K_linear, V_linear, O_linear, MLP1_linear, MLP2_linear);
     }
     void run(half *out, half *in) override {
+        if (flow_pays(rows())) {
+            run_flow(out, in, lens_ptr(), nullptr);
+            return;
+        }
         const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
         half *outs[3] = {buffers[0], buffers[1], buffers[2]};
         Linear_tile::run_multi(qkv, outs, 3, in, rows(), stream);
@@ -309,6 +332,7 @@ class Encoder_length : public Encoder_base {
         etRequire(MLP1_linear.is_gelu, "Encoder_length: MLP1_linear must be the GELU variant");
         place_tail_ws(units_and_scores_bytes(d_model, seq_len, nheads, batch));
         Linear_tile::tail_prepare(O_linear, MLP1_linear, MLP2_linear);
+        create_flow(Q_linear, K_linear, V_linear, O_linear, MLP1_linear, MLP2_linear);
     }
     static size_t units_and_scores_bytes(int d_model_, int seq_len_, int nheads_, int batch_) {
         return ((size_t)buffer_num * d_model_ * seq_len_ + (size_t)nheads_ * seq_len_ * seq_len_) *
@@ -324,6 +348,10 @@ class Encoder_length : public Encoder_base {
     // cu[i]..cu[i+1]-1; out_p may alias in_p.
     void run_packed(half *out_p, half *in_p) {
         const int n = total_rows;
+        if (flow_pays(n)) {
+            run_flow(out_p, in_p, nullptr, d_cu.get());
+            return;
+        }
         const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
         half *outs[3] = {buffers[0], buffers[1], buffers[2]};
         Linear_tile::run_multi(qkv, outs, 3, in_p, n, stream);
@@ -341,6 +369,11 @@ class Encoder_length : public Encoder_base {
             const int n = total_rows;
             half *in_p = buffers[4];
             etChk(et_pack_rows_ordered(in_p, in, d_cu.get(), d_order.get(), batch, seq_len, d_model, stream));
+            if (flow_pays(n)) {
+                run_flow(in_p, in_p, nullptr, d_cu.get());
+                etChk(et_unpack_rows_ordered(out, in_p, d_cu.get(), d_order.get(), batch, seq_len, d_model, stream));
+                return;
+            }
             const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
             half *outs[3] = {buffers[0], buffers[1], buffers[2]};
             Linear_tile::run_multi(qkv, outs, 3, in_p, n, stream);
@@ -373,6 +406,10 @@ class Encoder_length : public Encoder_base {
                 etChk(et_skip_layernorm(buffers[0], out, ln_gamma[1].get(), ln_beta[1].get(), n, d_model, stream));
             }
             etChk(et_unpack_rows_ordered(out, buffers[0], d_cu.get(), d_order.get(), batch, seq_len, d_model, stream));
+            return;
+        }
+        if (!use_shared_qk && flow_pays(rows())) {
+            run_flow(out, in, nullptr, nullptr);
             return;
         }
         const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};

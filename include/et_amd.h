@@ -306,6 +306,28 @@ size_t et_tile_plan_tail_ws_bytes(const et_tile_plan *out, const et_tile_plan *f
  * 0 while the paired form is switched off (et_tuning_set "tile_tail_pair" 0, the
  * default), so that Encoder_*::buffer_size is then the reference's five units */
 size_t et_tail_ws_bytes_for(int d_model, int rows);
+
+/* ---- a whole layer in one launch, for few rows ------------------------------
+ * Q/K/V, attention, output projection, skip + LayerNorm, feed-forward block, skip + LayerNorm as units of work
+ * of one grid (the steps of encoder/encoder.cu:20-45; what Encoder_tile and Encoder_length run where it pays).
+ * et_layer_flow_create: the six plans of the layer (they must outlive the object), sequences of seq_len rows,
+ * `batch` of them.  *flow is NULL, with ET_OK, where the form does not exist for these sizes.  The object owns
+ * the device scratch of the hand-overs; one run at a time may use it.
+ * et_layer_flow_set_packed: HOST row offsets of the packed sequences (batch + 1), for runs with cu_seqlens.
+ * et_layer_flow_pays: 1 where et_layer_flow_run is the form to take for that many rows.
+ * et_layer_flow_run: out = layer(in), rows of model width, out may alias in; Q, K, V, attn are distinct scratch
+ * of rows x model width.  cu_seqlens (device, as given to et_layer_flow_set_packed) or seq_lens (device) or
+ * neither; mask, log2_scale as in et_OTF_attention.  Kernel launch only: may be captured in a graph. */
+typedef struct et_layer_flow et_layer_flow;
+int et_layer_flow_create(et_layer_flow **flow, const et_tile_plan *q, const et_tile_plan *k, const et_tile_plan *v,
+                         const et_tile_plan *o, const et_tile_plan *m1, const et_tile_plan *m2, int seq_len,
+                         int nheads, int batch);
+void et_layer_flow_destroy(et_layer_flow *flow);
+int et_layer_flow_set_packed(et_layer_flow *flow, const int *cu_seqlens);
+int et_layer_flow_pays(const et_layer_flow *flow, int rows);
+int et_layer_flow_run(et_layer_flow *flow, void *out, const void *in, void *Q, void *K, void *V, void *attn,
+                      const void *mask, const int *seq_lens, const int *cu_seqlens, const void *gamma1,
+                      const void *beta1, const void *gamma2, const void *beta2, float log2_scale, void *stream);
 /* n (<= 4) planned linears with the same in_feat applied to the same X in ONE
  * launch (the Q/K/V projections, encoder/encoder.cu:22-26, which the
  * reference spreads over three streams). */
@@ -453,6 +475,9 @@ int et_device_synchronize(void);
  *                     on whole rows in LDS (16-row panels, a block-row's tile
  *                     pairs split over several waves where there are few); -1
  *                     (default): by the amount of W streamed; 0: never
+ *   "layer_flow_rows" most rows for which an encoder layer runs as one launch
+ *                     (et_layer_flow_pays); -1 (default): by size and density;
+ *                     0: never
  *   "row_gemm_min_rows" rows from which et_row_spmm_add_bias runs the dense
  *                     GEMM kernel (default 1024; 0: never)
  *   "tile_fuse_ffn"   0: et_tile_plan_ffn_fusable answers no (the feed-forward

@@ -546,3 +546,56 @@ def test_cpp_caller_of_the_reference_classes(tmp_path, program):
             want[B * S + b * S + lens[b]:B * S + (b + 1) * S] = 0
     assert got.shape == same.shape and np.array_equal(got, same)
     check_close(got, want, what="C++ caller " + program)
+
+
+@pytest.mark.parametrize("d,H,dff,S,B,sp,lens,use_mask", [
+    (768, 12, 3072, 1, 1, 0.8, None, False),           # one row
+    (768, 12, 3072, 16, 1, 0.8, None, True),           # one whole panel
+    (768, 12, 3072, 17, 3, 0.5, None, True),           # panels that hold rows of two sequences
+    (768, 12, 3072, 96, 1, 0.9, None, False),          # the most rows
+    (1024, 16, 4096, 24, 2, 0.8, [24, 0], False),      # six chunks of the hidden width; an empty sequence
+    (64, 2, 128, 3, 30, 0.6, [3, 1, 2] * 10, True),    # head width 32, many sequences per panel
+    (512, 8, 2048, 40, 2, 0.0, [7, 33], False),        # dense
+])
+def test_layer_in_one_launch(d, H, dff, S, B, sp, lens, use_mask):
+    """few rows: the whole layer as one launch (padded, and packed where lengths are given) against the oracle and
+    against the separate launches; runs repeat bit for bit, also from a captured graph between eager runs"""
+    from et_amd import lib
+    from et_amd.encoder import Encoder_length
+    r = rng(1300 + d + S * B)
+    lins, ln = make_layer(r, d, dff, sp, seed=1400 + S, std=0.03, bias_std=0.05)
+    mask = randn_h(r, (S, S), 0.5) if use_mask else None
+    enc = Encoder_length(d, S, H, workspace(Encoder_length, d, S, H, B), *build_linears(lins, B * S), *ln, mask, B)
+    xs = [randn_h(r, (B * S, d)) for _ in range(3)]
+    for use in ([None, np.array(lens, np.int32)] if lens else [None]):
+        enc.set_seq_lens(use)
+        valid = np.concatenate([np.arange(b * S, b * S + (S if use is None else use[b])) for b in range(B)])
+        got = [host(enc.run(torch.empty_like(dev(x)), dev(x))) for x in xs]
+        for x, g in zip(xs, got):
+            want = orc.encoder_tile_layer(x, lins, ln, mask, S, H, B, use, 1.0)
+            check_close(g[valid], want[valid], what="layer in one launch")
+            assert (np.delete(g, valid, 0) == 0).all()
+        try:
+            lib().et_tuning_set(b"layer_flow_rows", 0)
+            steps = host(enc.run(torch.empty_like(dev(xs[0])), dev(xs[0])))
+        finally:
+            lib().et_tuning_set(b"layer_flow_rows", -1)
+        assert np.abs(steps.astype(np.float32) - got[0].astype(np.float32)).max() <= 2e-2
+        x_static, out_static = torch.empty_like(dev(xs[0])), torch.empty_like(dev(xs[0]))
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            enc.run(out_static, x_static)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            enc.run(out_static, x_static)
+        for k in (1, 0, 2, 0):
+            x_static.copy_(dev(xs[k]))
+            out_static.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(host(out_static), got[k])
+            assert np.array_equal(host(enc.run(torch.empty_like(x_static), dev(xs[k]))), got[k])
+        del graph
