@@ -1845,6 +1845,9 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         // waves come first and win ties: the same items as eight waves of three,
         // with three waves per SIMD instead of two to cover the stream's waits
         // (Q/K/V of the benchmark: 20 -> 17.5 us).
+        double pairs_avg = 0.0; // tile pairs per block-row
+        for (int i = 0; i < nlin; i++)
+            pairs_avg += 0.5 * probs[i].ntile / probs[i].nbr / nlin;
         const int cus = std::max(et_device_cu_count(), 1);
         const int nrp64 = (M + TL_BM64 - 1) / TL_BM64;
         static const int cand[4][2] = {{12, 2}, {8, 3}, {8, 2}, {8, 1}}; // waves, block-rows per wave
@@ -1855,8 +1858,10 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
             const int nw = cand[c][0], nb = cand[c][1];
             if (nw == 12 && g_tile_bm64 == 4)
                 continue; // (tuning: eight waves only)
-            if (nb == 1 && best_c >= 0)
-                continue; // (only where no wider form fits the LDS)
+            // (one block-row per wave: where no wider form fits the LDS, or none has enough items and the lists are
+            // long - 8192 rows, 768 -> 768: dense 19.9 -> 17.5 us, 50 % 13.7 -> 13.5, 80 % 9.9 -> 11.3)
+            if (nb == 1 && (best_c >= 0 || (KC <= 816 && pairs_avg < 8.0)))
+                continue;
             const size_t lds64 = (size_t)TL_BM64 * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16) +
                                  (size_t)nw * TL_BM64 * (16 * nb + 8) * sizeof(f16);
             const int ncg64 = (nbr_max + nw * nb - 1) / (nw * nb);
