@@ -1,27 +1,28 @@
-// Dense GEMM for the row-pruned linear on gfx950:  Y[M x N] = X[M x K] W^T + b
-// (+ GELU), W = the compacted surviving rows [N x K] row-major, fp16 storage,
-// fp32 accumulate.  Replaces the cublasGemmEx call plus add_bias kernel of
-// kernels/linear.cu:5-34.
+// Dense GEMM on gfx950:  Y[M x N] = X[M x K] W^T + b (+ GELU), W [N x K] row-major, fp16 storage, fp32 accumulate: the
+// row-pruned linear on its compacted rows (in place of the cublasGemmEx call plus add_bias kernel of
+// kernels/linear.cu:5-34) and the plans of fully populated tile matrices from some hundred rows on.
 //
-// Both operands are contiguous along K, which is the layout the 16x16x32 MFMA
-// wants for A and for B (8 consecutive k per lane), so neither is transposed.
-// A workgroup of four waves (2 x 2) computes a 128 x 128 block, a wave 64 x 64
-// = 4 x 4 MFMA tiles (16 fragment reads feed 32 MFMAs per K step of 64: the
-// register blocking a streamed tile list cannot have).  The product is issued
-// as W X^T so that a lane ends with four consecutive output features of one
-// row.  K is walked in steps of 64 through two LDS buffers filled by DMA
-// (global_load_lds_dwordx4, no registers) one step ahead.  A DMA instruction
-// writes 64 x 16 bytes to consecutive LDS, the source address is free per
-// lane: the 16-byte pieces of a row are stored XOR-swizzled by (row / 2) % 8,
-// which makes the ds_read_b128 fragment reads conflict-free without padding
-// (rows r and r + 2 would otherwise share their banks).
+// Both operands are contiguous along K, which is the layout the 16x16x32 MFMA wants for A and for B (8 consecutive k
+// per lane), so neither is transposed.  The product is issued as W X^T so that a lane ends with four consecutive output
+// features of one row.  K is walked in steps of 64 through two or three LDS stages filled by DMA
+// (global_load_lds_dwordx4, no registers).  A DMA instruction writes 64 x 16 bytes to consecutive LDS, the source
+// address is free per lane: the 16-byte pieces of a row are stored XOR-swizzled by (row / 2) % 8, which puts the sixteen
+// rows of a fragment read into sixteen different slots of 256 bytes without padding.
+//
+// What bounds it (measured with the DMA, the fragment reads and the MFMAs timed alone, 256 x 256 blocks, per step):
+// DMA 1.0 us, reads 0.5, MFMAs 1.0, all together 1.5 - the requests are issued in one go behind the barrier, and what
+// they miss in the XCD's L2 arrives late.  A second workgroup per CU fills these waits better than a third stage or
+// larger blocks, except where there is no work for a second one.  At K = 768 the twelve steps are a third of the time
+// of a launch; the rest is its start, the first step's latency and the result's way out.
+#include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "common.h"
 
 namespace et {
 
-constexpr int DG_BN = 128, DG_BK = 64; // (the block has 64 WM rows, WM = 2 or 4 waves along M)
+constexpr int DG_BK = 64; // columns per step
 constexpr int DG_MAX_LIN = 3;
 
 struct DgArgs {
@@ -34,36 +35,22 @@ struct DgArgs {
     int nlin, M, K, tiles_m, tiles_n, per_xcd, total;
 };
 
-// LDS position (in 16-byte pieces) of piece kc of row r in a [rows x 64] tile
-__device__ __forceinline__ int dg_piece(int r, int kc) { return r * 8 + (kc ^ ((r >> 1) & 7)); }
+// where a row keeps its 16-byte piece kc of a step
+__device__ __forceinline__ int dg_swizzle(int r, int kc) { return kc ^ ((r >> 1) & 7); }
 
-// one operand tile: ROWS rows x 64 halves = ROWS / 8 DMA instructions, spread
-// over the NW waves; rows beyond `rows_total` re-read the last row (their
-// products are not stored)
-template <int ROWS, int NW>
-__device__ __forceinline__ void dg_fetch(f16 *lds, const f16 *src, int ld, int row0, int rows_total, int k0,
-                                         int K, int wave, int lane) {
-    static_assert((ROWS / 8) % NW == 0, "whole instructions per wave");
-#pragma unroll
-    for (int i = 0; i < ROWS / 8 / NW; i++) {
-        const int inst = wave * (ROWS / 8 / NW) + i;
-        const int p = inst * 64 + lane; // this lane's piece in the tile
-        const int r = p >> 3, slot = p & 7;
-        const int kc = slot ^ ((r >> 1) & 7);
-        const int row = min(row0 + r, rows_total - 1);
-        const int k = min(k0 + kc * 8, K - 8); // (pieces beyond K belong to a K step that is not multiplied)
-        load_lds16(src + (size_t)row * ld + k, lds + inst * 512);
-    }
-}
-
-template <bool GELU, int WM, int STAGES>
-__global__ void __launch_bounds__(WM * 2 * 64) dense_gemm_kernel(const DgArgs a) {
-    constexpr int NW = WM * 2, DG_BM = WM * 64;
+// WM x WN waves of TM x TN MFMA tiles: a block of 16 WM TM rows and 16 WN TN features.  ST stages of 64 columns; a
+// step's second half of fragments is read while the first half multiplies, then the stage is handed back, the step ST
+// later requested into it and the next step's first fragments read while the second half multiplies: fragment reads and
+// the barrier run under MFMAs.
+// Against the kernel this replaced (128 x 128 by four waves, one stage ahead, reads between the MFMAs), us a launch:
+// 8192 rows 768 -> 768 18.5 -> 16.8, 768 -> 3072 53.0 -> 47.6, 3072 -> 768 49.7 -> 43.3, 928 -> 240 15.2 -> 10.2;
+// 16384 rows 1024 -> 4096 176 -> 132 (1040 TFLOP/s); 4096 x 4096 x 4096 151 -> 114 (1200 TFLOP/s).
+template <bool GELU, int WM, int WN, int TM, int TN, int ST>
+__global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(const DgArgs a) {
+    constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char dg_smem[];
     f16 *smem = reinterpret_cast<f16 *>(dg_smem);
-    constexpr int XT = DG_BM * DG_BK, WT = DG_BN * DG_BK; // halves per operand tile
-    constexpr int STAGE = XT + WT;
-    constexpr int PER_WAVE = (DG_BM + DG_BN) / 8 / NW;    // DMA instructions per wave and K step
+    constexpr int XT = BM * DG_BK, STAGE = XT + BN * DG_BK; // halves
     // consecutive ids on one XCD walk the column tiles of one row tile: they
     // share the X tile in that XCD's L2, and W (small) is everywhere
     const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
@@ -83,117 +70,239 @@ __global__ void __launch_bounds__(WM * 2 * 64) dense_gemm_kernel(const DgArgs a)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int c16 = lane & 15, g4 = lane >> 4;
-    const int wm = wave >> 1, wn = wave & 1; // the wave's 64 x 64 part of the block
-    const int m0 = tm * DG_BM, n0 = tn * DG_BN;
+    const int wm = wave / WN, wn = wave % WN;
+    const int m0 = tm * BM, n0 = tn * BN;
     const int nk = (a.K + DG_BK - 1) / DG_BK;
 
-    f32x4 acc[4][4]; // [feature subtile][row subtile]
+    // requests of a stage per wave: 1 KB = eight rows each
+    constexpr int NXI = BM / 8 / NW, NWI = BN / 8 / NW;
+    static_assert(BM / 8 % NW == 0 && BN / 8 % NW == 0, "whole instructions per wave");
+    unsigned xoff[NXI], woff[NWI]; // byte offsets of the lane's pieces in step 0 (rows beyond M, N: the last one's)
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // K step kt lives in stage kt % STAGES (X tile, W tile behind it); STAGES - 1
-    // steps are requested ahead, so a step has the time of STAGES - 2 steps of
-    // MFMAs (plus the other waves') to arrive
-    auto fetch = [&](int kt) {
-        f16 *xn = smem + (kt % STAGES) * STAGE;
-        dg_fetch<DG_BM, NW>(xn, a.X, a.K, m0, a.M, kt * DG_BK, a.K, wave, lane);
-        dg_fetch<DG_BN, NW>(xn + XT, W, a.K, n0, N, kt * DG_BK, a.K, wave, lane);
-    };
-#pragma unroll
-    for (int t = 0; t < STAGES - 1; t++)
-        if (t < nk)
-            fetch(t);
-    for (int kt = 0; kt < nk; kt++) {
-        const f16 *xs = smem + (kt % STAGES) * STAGE;
-        const f16 *ws = xs + XT;
-        // this wave's pieces of step kt have landed (loads return in order: the
-        // younger steps' instructions may still be out)
-        if (STAGES > 2 && kt + STAGES - 1 <= nk)
-            __builtin_amdgcn_s_waitcnt(0x0F70 | ((STAGES - 2) * PER_WAVE));
-        else
-            __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads(); // ... everyone's, and everyone is done with the stage that is refilled now
-        if (kt + STAGES - 1 < nk)
-            fetch(kt + STAGES - 1);
-        const int ksteps = min(2, (a.K - kt * DG_BK) >> 5); // K is a multiple of 32
-        for (int s = 0; s < ksteps; s++) {
-            f16x8 xf[4], wf[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int r = wm * 64 + j * 16 + c16;
-                xf[j] = *reinterpret_cast<const f16x8 *>(xs + dg_piece(r, s * 4 + g4) * 8);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = wn * 64 + i * 16 + c16;
-                wf[i] = *reinterpret_cast<const f16x8 *>(ws + dg_piece(r, s * 4 + g4) * 8);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    acc[i][j] = mfma16x16x32(wf[i], xf[j], acc[i][j]);
-        }
+    for (int i = 0; i < NXI; i++) {
+        const int r = (wave * NXI + i) * 8 + (lane >> 3);
+        const int kc = dg_swizzle(r, lane & 7);
+        xoff[i] = (unsigned)((min(m0 + r, a.M - 1) - m0) * a.K + kc * 8) * 2u;
     }
-    __syncthreads(); // the tile buffers are free: they stage the output block
-
-    // acc[i][j][r] = Y[row = m0 + wm*64 + j*16 + c16][col = n0 + wn*64 + i*16 + g4*4 + r]
-    // -> the wave's 64 x 64 block in LDS ([row][64 halves + 8]), then 16-byte stores
-    constexpr int LDO = 64 + 8;
-    f16 *os = smem + wave * 64 * LDO;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int col = n0 + wn * 64 + i * 16 + g4 * 4;
+    for (int i = 0; i < NWI; i++) {
+        const int r = (wave * NWI + i) * 8 + (lane >> 3);
+        const int kc = dg_swizzle(r, lane & 7);
+        woff[i] = (unsigned)((min(n0 + r, N - 1) - n0) * a.K + kc * 8) * 2u;
+    }
+    const char *const xbase = reinterpret_cast<const char *>(a.X + (size_t)m0 * a.K);
+    const char *const wbase = reinterpret_cast<const char *>(W + (size_t)n0 * a.K);
+    const int tail_cols = a.K - (nk - 1) * DG_BK; // 64, or 32: pieces beyond it re-read the step's first ones
+    auto fetch = [&](int kt, int slot) {
+        f16 *xn = smem + slot * STAGE;
+        const char *xs = xbase + (size_t)kt * (DG_BK * 2), *ws = wbase + (size_t)kt * (DG_BK * 2);
+        const bool tail = kt == nk - 1 && tail_cols < DG_BK;
+        // (the swizzle flips bit 2 of a piece's number with the parity of its eight rows)
+        const unsigned even = tail && (lane & 4) ? 64u : 0u, odd = tail && !(lane & 4) ? 64u : 0u;
+#pragma unroll
+        for (int i = 0; i < NXI; i++) {
+            unsigned o = xoff[i];
+            asm volatile("" : "+v"(o)); // (a 32-bit offset off a uniform base, not a 64-bit pointer kept per piece)
+            load_lds16(xs + (o - (((wave * NXI + i) & 1) ? odd : even)), xn + (wave * NXI + i) * 512);
+        }
+#pragma unroll
+        for (int i = 0; i < NWI; i++) {
+            unsigned o = woff[i];
+            asm volatile("" : "+v"(o));
+            load_lds16(ws + (o - (((wave * NWI + i) & 1) ? odd : even)), xn + XT + (wave * NWI + i) * 512);
+        }
+    };
+    f32x4 acc[TN][TM]; // [feature subtile][row subtile]
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int j = 0; j < TM; j++)
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f16x8 xf[2][TM], wf[2][TN];
+    // LDS byte offsets of the lane's fragment pieces (subtile j is 16 rows further)
+    const int rx = wm * TM * 16 + c16, rw = wn * TN * 16 + c16;
+    const int px[2] = {rx * 128 + dg_swizzle(rx, g4) * 16, rx * 128 + dg_swizzle(rx, 4 + g4) * 16};
+    const int pw[2] = {XT * 2 + rw * 128 + dg_swizzle(rw, g4) * 16, XT * 2 + rw * 128 + dg_swizzle(rw, 4 + g4) * 16};
+    auto read = [&](int slot, auto half) {
+        constexpr int H = decltype(half)::value;
+        const char *s = reinterpret_cast<const char *>(smem) + slot * (STAGE * 2);
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+            wf[H][i] = *reinterpret_cast<const f16x8 *>(s + pw[H] + i * 2048);
+#pragma unroll
+        for (int j = 0; j < TM; j++)
+            xf[H][j] = *reinterpret_cast<const f16x8 *>(s + px[H] + j * 2048);
+    };
+    auto multiply = [&](auto half) {
+        constexpr int H = decltype(half)::value;
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int j = 0; j < TM; j++)
+#pragma unroll
+            for (int i = 0; i < TN; i++)
+                acc[i][j] = mfma16x16x32(wf[H][i], xf[H][j], acc[i][j]);
+        __builtin_amdgcn_s_setprio(0);
+    };
+    typedef std::integral_constant<int, 0> h0;
+    typedef std::integral_constant<int, 1> h1;
+    auto barrier = [] { asm volatile("s_barrier" ::: "memory"); };
+    constexpr int PER = NXI + NWI; // requests of a stage per wave
+    auto landed = [&](int behind) { // all but the youngest `behind` stages have arrived (this wave's part of them)
+        if (behind >= 1 && ST > 2)
+            __builtin_amdgcn_s_waitcnt(0x0070 | (PER & 15) | (PER >> 4 << 14)); // vmcnt(PER) lgkmcnt(0)
+        else
+            __builtin_amdgcn_s_waitcnt(0x0070); // vmcnt(0) lgkmcnt(0)
+    };
+    static_assert(ST == 2 || ST == 3, "stages");
+#pragma unroll
+    for (int t = 0; t < ST - 1; t++)
+        if (t < nk)
+            fetch(t, t);
+    landed(min(ST - 2, nk - 1));
+    barrier();
+    if (ST - 1 < nk)
+        fetch(ST - 1, ST - 1);
+    read(0, h0());
+    int slot = 0;
+    auto turn = [&](int kt) { // stage kt has been read: wait for the next one, request into this one's place
+        landed(min(ST - 2, nk - 2 - kt));
+        barrier();
+        if (kt + ST < nk)
+            fetch(kt + ST, slot);
+        slot = slot == ST - 1 ? 0 : slot + 1;
+    };
+    for (int kt = 0; kt < nk; kt++) {
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the first half's fragments, read a multiplication ago
+        read(slot, h1());
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(h0());
+        if (kt + 1 < nk) {
+            turn(kt);
+            read(slot, h0());
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (kt < nk - 1 || tail_cols == DG_BK)
+            multiply(h1());
+    }
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    barrier(); // the stages are free: they stage the output block
+
+    // acc[i][j][r] = Y[row = m0 + wm*16*TM + j*16 + c16][col = n0 + wn*16*TN + i*16 + g4*4 + r]
+    // -> the wave's rows in LDS, 64 at a time ([row][16 TN halves + 8]), then 16-byte stores
+    constexpr int LDO = 16 * TN + 8, CH = 2 * TN; // 16-byte pieces per row
+    constexpr int TR = TM < 4 ? TM : 4;           // row subtiles per pass
+    static_assert(TM % TR == 0 && (size_t)NW * TR * 16 * LDO <= ST * (size_t)STAGE, "the output staging fits the stages");
+    f16 *os = smem + wave * TR * 16 * LDO;
+    f32x4 bf[TN];
+#pragma unroll
+    for (int i = 0; i < TN; i++) {
+        const int col = n0 + (wn * TN + i) * 16 + g4 * 4;
         f16x4 b4 = f16x4{0, 0, 0, 0};
         if (col < N)
             b4 = *reinterpret_cast<const f16x4 *>(bias + col);
-        const f32x4 bf = __builtin_convertvector(b4, f32x4);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            f16x4 ov = __builtin_convertvector(acc[i][j] + bf, f16x4);
-            if (GELU)
-                ov = gelu4(ov);
-            *reinterpret_cast<f16x4 *>(os + (j * 16 + c16) * LDO + i * 16 + g4 * 4) = ov;
-        }
+        bf[i] = __builtin_convertvector(b4, f32x4);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // (the staging block is the wave's own: LDS operations of one wave execute in order)
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-        const int p = t * 64 + lane; // 64 rows x 8 pieces
-        const int r = p >> 3, pc = p & 7;
-        const int row = m0 + wm * 64 + r, col = n0 + wn * 64 + pc * 8;
-        if (row < a.M && col < N) { // N is a multiple of 16: a piece is inside or outside as a whole
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(os + r * LDO + pc * 8);
-            *reinterpret_cast<u32x4 *>(Y + (size_t)row * N + col) = v;
+    for (int p = 0; p < TM / TR; p++) {
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+            for (int j = 0; j < TR; j++) {
+                f16x4 ov = __builtin_convertvector(acc[i][p * TR + j] + bf[i], f16x4);
+                if (GELU)
+                    ov = gelu4(ov);
+                *reinterpret_cast<f16x4 *>(os + (j * 16 + c16) * LDO + i * 16 + g4 * 4) = ov;
+            }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // (the staging block is the wave's own: LDS operations of one wave execute in order)
+#pragma unroll
+        for (int t = 0; t < TR * 16 * CH / 64; t++) {
+            const int q = t * 64 + lane, r = q / CH, pc = q % CH;
+            const int row = m0 + wm * TM * 16 + p * TR * 16 + r, col = n0 + wn * TN * 16 + pc * 8;
+            if (row < a.M && col < N) // N is a multiple of 16: a piece is inside or outside as a whole
+                *reinterpret_cast<u32x4 *>(Y + (size_t)row * N + col) = *reinterpret_cast<const u32x4 *>(os + r * LDO + pc * 8);
         }
     }
 }
 
-template <bool GELU, int WM, int STAGES>
-static int dg_launch_inst(DgArgs &a, hipStream_t st) {
-    constexpr int BM = WM * 64;
-    constexpr size_t lds = (size_t)STAGES * (BM + DG_BN) * DG_BK * sizeof(f16);
-    static_assert((size_t)WM * 2 * 64 * (64 + 8) * sizeof(f16) <= lds, "the output staging fits the tile buffers");
+// Row-major copy of a fully populated plan's weights: a workgroup per (chunk, block-row), a thread per 16-byte half row
+// of a tile (tiles of a segment are in column order; a segment's padding tile is not read).
+__global__ void __launch_bounds__(256) dense_from_plan_kernel(f16 *W, const f16 *data, const int *cptr, int K, int KC, int nbr) {
+    const int c = blockIdx.x / nbr, bn = blockIdx.x - c * nbr;
+    const int ntile = (min(KC, K - c * KC) + 15) / 16;
+    const f16 *const src = data + (size_t)cptr[blockIdx.x] * 256;
+    f16 *const dst = W + (size_t)bn * 16 * K + c * KC;
+    for (int q = threadIdx.x; q < ntile * 32; q += 256) {
+        const int t = q >> 5, r = (q >> 1) & 15, h = q & 1;
+        *reinterpret_cast<u32x4 *>(dst + (size_t)r * K + t * 16 + h * 8) =
+            *reinterpret_cast<const u32x4 *>(src + t * 256 + r * 16 + h * 8);
+    }
+}
+int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int nchunk, int nbr) {
+    hipLaunchKernelGGL(dense_from_plan_kernel, dim3(nchunk * nbr), dim3(256), 0, nullptr, W, data, cptr, K, KC, nbr);
+    return launch_status("dense_from_plan launch");
+}
+
+template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launch_inst(DgArgs &a, hipStream_t st) {
+    constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
+    constexpr int lds = ST * (BM + BN) * DG_BK * (int)sizeof(f16);
     a.tiles_m = (a.M + BM - 1) / BM;
+    a.tiles_n = 0;
+    for (int i = 0; i < DG_MAX_LIN; i++) {
+        a.tile0[i] = i < a.nlin ? a.tiles_n : 0;
+        if (i < a.nlin)
+            a.tiles_n += (a.N[i] + BN - 1) / BN;
+    }
     a.total = a.tiles_m * a.tiles_n;
     a.per_xcd = (a.total + 7) / 8;
-    constexpr auto k = &dense_gemm_kernel<GELU, WM, STAGES>;
-    if (lds > 64 * 1024) {
-        static bool done = false; // (asked of the driver once per kernel instance)
-        if (!done) {
-            ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds));
-            done = true;
-        }
-    }
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(WM * 2 * 64), lds, st, a);
+    constexpr auto kern = &dense_gemm_kernel<GELU, WM, WN, TM, TN, ST>;
+    if (lds > 64 * 1024)
+        ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(WM * WN * 64), lds, st, a);
     return launch_status("dense_gemm launch");
 }
+
+// The blocks there are and the time of each form in microseconds, without the launch.  A step takes longer with every
+// further workgroup of a CU; the figures are fits to 13 shapes (128 to 32768 rows, 768 to 4096 columns) within 15 %.
+// Small blocks win while they let more CUs take part, large ones where every CU has several.
+enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_FORMS };
+static int g_dense_form = -1; // et_tuning_set("dense_form"): one of the above, -1 chooses
+static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
+    static const int bm[DG_FORMS] = {64, 128, 128, 128, 256}, bn[DG_FORMS] = {128, 128, 128, 192, 256};
+    const long cus = std::max(et_device_cu_count(), 1);
+    long tiles = 0;
+    for (int i = 0; i < nlin; i++)
+        tiles += (Ns[i] + bn[form] - 1) / bn[form];
+    tiles *= (M + bm[form] - 1) / bm[form];
+    const double n = (double)((tiles + cus - 1) / cus); // blocks of the busiest CU
+    double step = 0.0;
+    switch (form) {
+    case DG_64x128: step = n <= 1 ? 0.43 : n <= 2 ? 0.78 : 0.48 * n; break;                // two per CU (72 KB)
+    case DG_128x128: step = n <= 1 ? 0.69 : n <= 2 ? 0.58 * n : 0.65 * n; break;            // two per CU (64 KB)
+    case DG_128x128_DEEP: step = n <= 1 ? 0.57 : 0.83 * n; break;                           // one per CU (96 KB)
+    case DG_128x192: step = n <= 2 ? 0.15 + 0.68 * n : 0.87 * n; break;                     // two per CU (80 KB)
+    case DG_256x256: step = 1.95 * n; break;                                                // one per CU (128 KB)
+    }
+    return 1.6 + step * ((K + DG_BK - 1) / DG_BK);
+}
+static int dg_choose(const int *Ns, int nlin, int M, int K, double *us) {
+    int best = 0;
+    for (int f = 0; f < DG_FORMS; f++) {
+        const double t = dg_estimate(f, Ns, nlin, M, K);
+        if (f == 0 || t < *us) {
+            *us = t;
+            best = f;
+        }
+    }
+    return best;
+}
+double dense_gemm_estimate(const int *Ns, int nlin, int M, int K) {
+    double us = 0.0;
+    dg_choose(Ns, nlin, M, K, &us);
+    return us;
+}
+void set_dense_form(int v) { g_dense_form = v < DG_FORMS ? v : -1; }
 
 // nlin linears over the same X in one launch.  Returns ET_ERR_UNSUPPORTED where
 // the shapes do not fit this kernel (the caller then takes the tile path).
@@ -203,7 +312,6 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
         return ET_ERR_UNSUPPORTED;
     DgArgs a;
     memset(&a, 0, sizeof(a));
-    int tiles_n = 0;
     for (int i = 0; i < DG_MAX_LIN; i++) {
         const int s = i < nlin ? i : 0;
         if (Ns[s] <= 0 || Ns[s] % 16 != 0 || !aligned16(Ys[s]) || !aligned16(Ws[s]) || !aligned16(biases[s]))
@@ -212,23 +320,26 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
         a.W[i] = static_cast<const f16 *>(Ws[s]);
         a.bias[i] = static_cast<const f16 *>(biases[s]);
         a.N[i] = Ns[s];
-        a.tile0[i] = tiles_n;
-        if (i < nlin)
-            tiles_n += (Ns[s] + DG_BN - 1) / DG_BN;
     }
-    a.tile0[DG_MAX_LIN] = tiles_n;
     if (!aligned16(X))
         return ET_ERR_UNSUPPORTED;
     a.X = static_cast<const f16 *>(X);
     a.nlin = nlin;
     a.M = M;
     a.K = K;
-    a.tiles_n = tiles_n;
-    // 128 x 128 blocks, four waves, two stages: 64 KB of LDS, two workgroups per
-    // CU.  (Measured against 256 x 128 blocks of eight waves and against three
-    // stages, both with one workgroup per CU: 10 to 30 % slower - the second
-    // workgroup hides more latency than the deeper ring.)
-    return gelu ? dg_launch_inst<true, 2, 2>(a, st) : dg_launch_inst<false, 2, 2>(a, st);
+    double us;
+    const int form = g_dense_form >= 0 ? g_dense_form : dg_choose(Ns, nlin, M, K, &us);
+    switch (form) {
+#define DG_CASE(form_, ...)                                                                                            \
+    case form_: return gelu ? dg_launch_inst<true, __VA_ARGS__>(a, st) : dg_launch_inst<false, __VA_ARGS__>(a, st);
+        DG_CASE(DG_64x128, 2, 4, 2, 2, 3)
+        DG_CASE(DG_128x128, 2, 4, 4, 2, 2)
+        DG_CASE(DG_128x128_DEEP, 2, 4, 4, 2, 3)
+        DG_CASE(DG_128x192, 2, 4, 4, 3, 2)
+        DG_CASE(DG_256x256, 2, 4, 8, 4, 2)
+#undef DG_CASE
+    }
+    return ET_ERR_UNSUPPORTED;
 }
 
 } // namespace et

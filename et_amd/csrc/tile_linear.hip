@@ -38,6 +38,7 @@
 #include <type_traits>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <numeric>
 #include <vector>
 
@@ -49,6 +50,7 @@ void set_attn_packed(int v);
 void set_ln_rows(int v);
 void set_tail_pair(int v);
 void set_tail_spin(int v);
+void set_dense_form(int v);
 // tile_rows.hip
 bool tile_rows_fits(int K);
 int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *X, int M, int K, double pairs, bool gelu,
@@ -1770,6 +1772,8 @@ static int g_tile_bm64 = 1; // et_tuning_set("tile_bm64")
 // rows from which the row-pruned linear runs the register-blocked GEMM (et_tuning_set("row_gemm_min_rows");
 // below, 128 x 128 blocks leave most CUs without work and the tile kernels win)
 static int g_row_gemm_min_rows = 1024;
+// fully populated plans as dense products: 1 by size, 0 never, 2 always (et_tuning_set("plan_dense"))
+static int g_plan_dense = 1;
 
 static int g_tile_rows_most = -1; // et_tuning_set("tile_splitk_rows"): most rows for which a plan runs on whole rows, -1 automatic
 
@@ -1990,6 +1994,14 @@ extern "C" int et_tuning_set(const char *key, int value) {
         et::g_tile_rows_most = value;
         return ET_OK;
     }
+    if (key && !strcmp(key, "dense_form")) {
+        et::set_dense_form(value);
+        return ET_OK;
+    }
+    if (key && !strcmp(key, "plan_dense")) {
+        et::g_plan_dense = value;
+        return ET_OK;
+    }
     if (key && !strcmp(key, "row_gemm_min_rows")) {
         et::g_row_gemm_min_rows = value;
         return ET_OK;
@@ -2082,6 +2094,41 @@ namespace et {
 // dense_gemm.hip
 int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, const void *const *biases,
                       const int *Ns, int nlin, int M, int K, bool gelu, hipStream_t st);
+double dense_gemm_estimate(const int *Ns, int nlin, int M, int K);
+int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int nchunk, int nbr); // null stream
+
+// Plans of fully populated matrices: the dense product is the shorter launch from some hundred rows on (many outputs)
+// or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by tile; their time on such
+// plans, fitted to 60 measured launches (128 to 16384 rows) within 20 % where the two are close: the larger of a stream
+// and product term and of a term per row, and for K in several chunks the larger slope.
+static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M) {
+    if (!g_plan_dense || n > 3)
+        return false;
+    int Ns[3], N = 0;
+    for (int i = 0; i < n; i++) {
+        if (!plans[i]->d_dense)
+            return false;
+        N += Ns[i] = plans[i]->out_feat;
+    }
+    if (g_plan_dense == 2)
+        return true;
+    const int K = plans[0]->in_feat;
+    const double gflop = 2e-9 * M * N * K;
+    const double tiles = plans[0]->nchunk > 1 ? 8.5 + 1.95 * gflop
+                                              : std::max(2.1 + 0.0009 * N + 1.3 * gflop, 2.0 + 0.0013 * M);
+    return dense_gemm_estimate(Ns, n, M, K) < tiles;
+}
+static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
+                           hipStream_t st) {
+    const void *Ws[3], *biases[3];
+    int Ns[3];
+    for (int i = 0; i < n; i++) {
+        Ws[i] = plans[i]->d_dense;
+        biases[i] = plans[i]->d_bias;
+        Ns[i] = plans[i]->out_feat;
+    }
+    return dense_gemm_launch(Ys, X, Ws, biases, Ns, n, M, plans[0]->in_feat, gelu, st);
+}
 static int row_linear(void *out, const void *in, const void *weight, const void *bias, int M, int N,
                       int K, bool gelu, void *stream) {
     ET_REQUIRE(out && in && weight && bias, ET_ERR_INVALID_ARG, "et_row_spmm_add_bias: null pointer");
@@ -2178,39 +2225,47 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
     for (int bn = 0; bn < nbr; bn++)
         std::stable_sort(order.begin() + row_ptr[bn], order.begin() + row_ptr[bn + 1],
                          [&](int x, int y) { return row_offset[x] < row_offset[y]; });
-    std::vector<int> off, cptr((size_t)nbr * nchunk + 1);
-    std::vector<uint16_t> packed;
-    off.reserve(ntile + (size_t)nbr * nchunk);
-    packed.reserve(((size_t)ntile + (size_t)nbr * nchunk) * 256);
-    const uint16_t *src = static_cast<const uint16_t *>(data);
-    for (int c = 0; c < nchunk; c++) {
-        for (int bn = 0; bn < nbr; bn++) {
-            cptr[(size_t)c * nbr + bn] = (int)off.size();
-            int cnt = 0, last = 0;
-            for (int i = row_ptr[bn]; i < row_ptr[bn + 1]; i++) {
-                const int o = row_offset[order[i]];
-                if (o / KC != c)
-                    continue;
-                off.push_back((o - c * KC) * 2);
-                packed.insert(packed.end(), src + (size_t)order[i] * 256, src + (size_t)order[i] * 256 + 256);
-                last = (o - c * KC) * 2;
-                cnt++;
-            }
-            if (cnt & 1) {
-                off.push_back(last);
-                packed.insert(packed.end(), 256, (uint16_t)0);
-            }
-        }
-    }
-    cptr[(size_t)nbr * nchunk] = (int)off.size();
+    std::vector<int> cptr((size_t)nbr * nchunk + 1, 0);
+    for (int bn = 0; bn < nbr; bn++)
+        for (int i = row_ptr[bn]; i < row_ptr[bn + 1]; i++)
+            cptr[(size_t)(row_offset[i] / KC) * nbr + bn + 1]++;
+    for (size_t i = 0; i < (size_t)nbr * nchunk; i++)
+        cptr[i + 1] = cptr[i] + (cptr[i + 1] + 1) / 2 * 2;
     // spare all-zero pairs behind the last one: the kernels request the first
     // pairs of a wave's stream before they know whether it is empty, and a
     // stream's last stages request up to 2*TL_DEPTH pairs past its end
-    for (int i = 0; i < 2 * TL_DEPTH + 1; i++) {
-        off.push_back(0);
-        off.push_back(0);
-        packed.insert(packed.end(), 512, (uint16_t)0);
+    const size_t total = (size_t)cptr.back() + 2 * (2 * TL_DEPTH + 1);
+    const int bcols = in_feat / 16;
+    bool full = ntile == nbr * bcols && in_feat % 32 == 0; // (the dense product walks K by 32)
+    for (int i = 0; i < ntile && full; i++)
+        full = row_offset[order[i]] == i % bcols * 16;
+    // one device allocation and one transfer: data, column offsets, segment starts, bias (and a full matrix row-major)
+    auto part = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t at_off = part(total * 512), at_cptr = at_off + part(total * 4), at_bias = at_cptr + part(cptr.size() * 4),
+                 at_dense = at_bias + part((size_t)out_feat * 2);
+    std::unique_ptr<unsigned char[]> image(new unsigned char[at_dense]); // (uninitialised: written once, below)
+    int *const off = reinterpret_cast<int *>(image.get() + at_off);
+    const uint16_t *src = static_cast<const uint16_t *>(data);
+    auto zero_tiles = [&](size_t first, size_t n) { memset(image.get() + first * 512, 0, n * 512); };
+    for (int bn = 0; bn < nbr; bn++) {
+        int i = row_ptr[bn];
+        for (int c = 0; c < nchunk; c++) { // (a block-row's tiles are in column order, hence by chunk)
+            const size_t seg = (size_t)c * nbr + bn;
+            int q = cptr[seg];
+            for (; i < row_ptr[bn + 1] && row_offset[order[i]] / KC == c; i++, q++) {
+                off[q] = (row_offset[order[i]] - c * KC) * 2;
+                memcpy(image.get() + (size_t)q * 512, src + (size_t)order[i] * 256, 512);
+            }
+            if (q < cptr[seg + 1]) {
+                off[q] = off[q - 1];
+                zero_tiles(q, 1);
+            }
+        }
     }
+    zero_tiles(cptr.back(), total - cptr.back());
+    memset(off + cptr.back(), 0, (total - cptr.back()) * 4);
+    memcpy(image.get() + at_cptr, cptr.data(), cptr.size() * 4);
+    memcpy(image.get() + at_bias, bias, (size_t)out_feat * 2);
 
     et_tile_plan *p = new et_tile_plan();
     {
@@ -2220,10 +2275,10 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
     // column-sorted host copy (the layer-tail program is built from it)
     p->h_row_ptr.assign(row_ptr, row_ptr + nbr + 1);
     p->h_col.resize(ntile);
-    p->h_data.resize((size_t)ntile * 256);
+    p->h_data.reserve((size_t)ntile * 256);
     for (int i = 0; i < ntile; i++) {
         p->h_col[i] = row_offset[order[i]];
-        memcpy(&p->h_data[(size_t)i * 256], src + (size_t)order[i] * 256, 512);
+        p->h_data.insert(p->h_data.end(), src + (size_t)order[i] * 256, src + (size_t)order[i] * 256 + 256);
     }
     p->in_feat = in_feat;
     p->out_feat = out_feat;
@@ -2231,18 +2286,24 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
     p->KC = KC;
     p->nchunk = nchunk;
     p->npair = cptr.back() / 2;
-    int rc = ET_OK;
-    auto up = [&](void **dst, const void *h, size_t bytes) {
-        if (rc != ET_OK)
-            return;
-        rc = et_malloc(dst, std::max<size_t>(bytes, 16));
-        if (rc == ET_OK && bytes)
-            rc = et_memcpy_h2d(*dst, h, bytes);
-    };
-    up((void **)&p->d_data, packed.data(), packed.size() * 2);
-    up((void **)&p->d_cptr, cptr.data(), cptr.size() * 4);
-    up((void **)&p->d_row_offset, off.data(), off.size() * 4);
-    up((void **)&p->d_bias, bias, (size_t)out_feat * 2);
+    unsigned char *dev = nullptr;
+    int rc = et_malloc((void **)&dev, at_dense + (full ? (size_t)out_feat * in_feat * 2 : 0));
+    p->d_data = reinterpret_cast<f16 *>(dev);
+    if (rc == ET_OK)
+        rc = et_memcpy_h2d(dev, image.get(), at_dense);
+    if (rc == ET_OK) {
+        p->d_row_offset = reinterpret_cast<int *>(dev + at_off);
+        p->d_cptr = reinterpret_cast<int *>(dev + at_cptr);
+        p->d_bias = reinterpret_cast<f16 *>(dev + at_bias);
+    }
+    if (full && rc == ET_OK) {
+        p->d_dense = reinterpret_cast<f16 *>(dev + at_dense);
+        rc = dense_from_plan(p->d_dense, p->d_data, p->d_cptr, in_feat, KC, nchunk, nbr);
+        if (rc == ET_OK && hipStreamSynchronize(nullptr) != hipSuccess) { // (the plan may run on any stream)
+            set_error("et_tile_plan_create: the row-major copy failed");
+            rc = ET_ERR_HIP;
+        }
+    }
     if (rc != ET_OK) {
         et_tile_plan_destroy(p);
         return rc;
@@ -2254,10 +2315,7 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
 extern "C" void et_tile_plan_destroy(et_tile_plan *p) {
     if (!p)
         return;
-    et_free(p->d_data);
-    et_free(p->d_cptr);
-    et_free(p->d_row_offset);
-    et_free(p->d_bias);
+    et_free(p->d_data); // (all of the plan's device memory)
     et::tail_program_destroy(p->tail);
     delete p;
 }
@@ -2298,6 +2356,8 @@ extern "C" int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *co
     ET_REQUIRE(aligned16(X), ET_ERR_ALIGNMENT, "et_tile_plan_run_multi: X not aligned");
     if (M == 0)
         return ET_OK;
+    if (plans_run_dense(plans, n, M))
+        return run_plans_dense(plans, Ys, n, X, M, false, static_cast<hipStream_t>(stream));
     return tile_launch(pr, n, static_cast<const f16 *>(X), M, plans[0]->in_feat, plans[0]->KC,
                        plans[0]->nchunk, false, TL_PLAN, static_cast<hipStream_t>(stream));
 }
@@ -2326,8 +2386,8 @@ extern "C" int et_tile_plan_run_ln(const et_tile_plan *plan, void *Y, const void
     if (M == 0)
         return ET_OK;
     const int nbr = plan->out_feat / 16;
-    if (!et_tile_plan_ln_fusable(plan) || (!ln_fusion_pays(M) && Y != skip)) {
-        // rows too wide for one workgroup, or too few of them: the two kernels, one after the other
+    if (!et_tile_plan_ln_fusable(plan) || ((!ln_fusion_pays(M) || plans_run_dense(&plan, 1, M)) && Y != skip)) {
+        // rows too wide for one workgroup, too few of them, or a dense product: the two kernels, one after the other
         ET_REQUIRE(Y != skip, ET_ERR_INVALID_ARG,
                    "et_tile_plan_run_ln: Y must not alias skip for out_feat=%d", plan->out_feat);
         const int rc = et_tile_plan_run(plan, Y, X, M, 0, stream);
@@ -2360,6 +2420,12 @@ extern "C" int et_tile_plan_ffn_fusable(const et_tile_plan *p1, const et_tile_pl
                : 0;
 }
 
+// Dense feed-forward products against the fused tail, which streams all of W past every 32 or 64 rows: wherever both
+// products are the shorter launch by themselves (768 wide, 3072 rows: 157 -> 99 us a layer; 8192 rows: 206 -> 181).
+static bool ffn_runs_dense(const et_tile_plan *p1, const et_tile_plan *p2, int M) {
+    return et::plans_run_dense(&p1, 1, M) && et::plans_run_dense(&p2, 1, M);
+}
+
 extern "C" int et_tile_plan_run_ffn_ln(const et_tile_plan *p1, const et_tile_plan *p2, void *Y,
                                        const void *X, void *hidden, const void *skip,
                                        const void *gamma, const void *beta, int M, void *stream) {
@@ -2376,7 +2442,7 @@ extern "C" int et_tile_plan_run_ffn_ln(const et_tile_plan *p1, const et_tile_pla
     if (M == 0)
         return ET_OK;
     const bool fusable = et_tile_plan_ffn_fusable(p1, p2) != 0;
-    if (!fusable || (hidden && !ln_fusion_pays(M))) {
+    if (!fusable || (hidden && (!ln_fusion_pays(M) || ffn_runs_dense(p1, p2, M)))) {
         // the three steps one after the other, through the caller's buffer
         ET_REQUIRE(hidden, ET_ERR_UNSUPPORTED,
                    "et_tile_plan_run_ffn_ln: these shapes need the hidden buffer (%d x %d halves)", M,
@@ -2432,7 +2498,7 @@ extern "C" int et_tile_plan_run_tail(const et_tile_plan *pO, const et_tile_plan 
                ET_ERR_ALIGNMENT, "et_tile_plan_run_tail: pointers must be 16-byte aligned");
     if (M == 0)
         return ET_OK;
-    if (!et_tile_plan_tail_fusable(pO, p1, p2) || (mid && !tail_fusion_pays(M))) {
+    if (!et_tile_plan_tail_fusable(pO, p1, p2) || (mid && (!tail_fusion_pays(M) || ffn_runs_dense(p1, p2, M)))) {
         // step by step through the caller's buffers
         ET_REQUIRE(mid, ET_ERR_UNSUPPORTED,
                    "et_tile_plan_run_tail: these shapes need the mid buffer (%d x %d halves)", M, pO->out_feat);
@@ -2501,6 +2567,8 @@ extern "C" int et_tile_plan_run(const et_tile_plan *plan, void *Y, const void *X
     ET_REQUIRE(aligned16(Y) && aligned16(X), ET_ERR_ALIGNMENT, "et_tile_plan_run: Y/X not aligned");
     if (M == 0)
         return ET_OK;
+    if (plans_run_dense(&plan, 1, M))
+        return run_plans_dense(&plan, &Y, 1, X, M, gelu != 0, static_cast<hipStream_t>(stream));
     TlProblem pr;
     pr.Y = static_cast<f16 *>(Y);
     pr.cptr = plan->d_cptr;
@@ -2547,7 +2615,7 @@ extern "C" int et_tile_plan_run_tail_ws(const et_tile_plan *pO, const et_tile_pl
     using namespace et;
     ET_REQUIRE(pO && p1 && p2 && Y && attn && input && gamma1 && beta1 && gamma2 && beta2,
                ET_ERR_INVALID_ARG, "et_tile_plan_run_tail_ws: null pointer");
-    if (ws && M > 0 && tail_pair_applies(pO, p1, p2)) {
+    if (ws && M > 0 && tail_pair_applies(pO, p1, p2) && !(mid && hidden && ffn_runs_dense(p1, p2, M))) {
         const size_t need = tail_pair_ws_bytes(pO, p1, p2, M);
         const int cus = std::max(et_device_cu_count(), 1);
         const int wgs = 2 * ((M + 63) / 64);

@@ -13,10 +13,11 @@ void tail_program_destroy(TailProgram *p);
 struct et_tile_plan {
     int in_feat = 0, out_feat = 0, ntile = 0, KC = 0, nchunk = 0;
     int npair = 0; // pairs of tiles in the plan layout; pair npair is all zero
-    et::f16 *d_data = nullptr;
+    et::f16 *d_data = nullptr; // one allocation, the parts below lie behind the tiles
     int *d_cptr = nullptr;
     int *d_row_offset = nullptr;
     et::f16 *d_bias = nullptr;
+    et::f16 *d_dense = nullptr; // fully populated matrices only: row-major [out_feat x in_feat]
     // Host copy of the caller's tile_mat with every block-row's tiles sorted by
     // column: the layer-tail program (tile_tail.hip) is built from it.
     std::vector<int> h_row_ptr, h_col;

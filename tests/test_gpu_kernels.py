@@ -1137,3 +1137,40 @@ def test_tile_linear_whole_rows(K, M, N, Kd, sp, gelu):
     planned = host(lt.run(dev(X)))
     check_close(planned[rows], want, max_abs=tol, mean_rel=5e-4, what="planned")
     assert np.array_equal(planned, host(lt.run(dev(X))))
+
+
+@pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("M,Ns,Kd,gelu", [
+    (1, (16,), 32, False),               # half a step of 64 columns, one piece of a block
+    (129, (272, 16, 400), 96, False),    # a row into the second block; three linears, none a multiple of a block
+    (300, (208,), 1056, True),           # 16.5 steps; a plan of two chunks with odd counts
+    (515, (768, 384), 64, False),        # a single step
+])
+def test_full_plan_as_dense_product(K, form, M, Ns, Kd, gelu):
+    """plans of fully populated matrices on the dense kernel, every block size at the edges of its blocks, against the
+    oracle and the tile kernels"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile, run_multi
+    r = rng(77 + M + Kd)
+    mats = [make_tile_linear(r, N, Kd, 0.0, seed=M + N, std=0.05, bias_std=0.2) for N in Ns]
+    X = randn_h(r, (M, Kd))
+    lts = [Linear_tile(Kd, N, M, m["row_offset"].size, m["data"], m["row_ptr"], m["row_offset"], m["bias"], gelu)
+           for N, m in zip(Ns, mats)]
+    rows = np.unique(np.concatenate([np.arange(min(M, 20)), r.integers(0, M, 30), np.arange(max(M - 20, 0), M)]))
+
+    def run():
+        return [host(y) for y in (run_multi(lts, dev(X)) if len(lts) > 1 else [lts[0].run(dev(X))])]
+
+    try:
+        lib().et_tuning_set(b"plan_dense", 0)
+        tiles = run()
+        lib().et_tuning_set(b"plan_dense", 2)
+        lib().et_tuning_set(b"dense_form", form)
+        got = run()
+    finally:
+        lib().et_tuning_set(b"plan_dense", 1)
+        lib().et_tuning_set(b"dense_form", -1)
+    for g, t, N, m in zip(got, tiles, Ns, mats):
+        want = orc.tile_linear(X[rows], m["row_ptr"], m["row_offset"], m["data"], m["bias"], N, gelu=gelu, f64=True)
+        check_close(g[rows], want, max_abs=8e-3, mean_rel=5e-4, what=f"dense, N={N}")
+        assert np.abs(g.astype(np.float32) - t.astype(np.float32)).max() <= 2.0 ** -6
