@@ -125,4 +125,28 @@ __device__ __forceinline__ float f16_bits_to_float(uint16_t b) {
     return (float)__builtin_bit_cast(f16, b);
 }
 
+// n / d by one scalar multiplication: exact while n * d < 2^32 (magic 0: d = 1).  A division in front of a kernel's
+// first request costs tens of vector instructions, fetched cold at every launch.
+inline unsigned magic_of(int d) { return d == 1 ? 0u : 0xFFFFFFFFu / (unsigned)d + 1u; }
+__device__ __forceinline__ int div_magic(int n, unsigned magic) { return magic ? (int)__umulhi((unsigned)n, magic) : n; }
+
+// Dynamic LDS above the 64 KB default has to be allowed per kernel.  The call
+// goes to the driver, so it is made only when a kernel needs more than it was
+// last given (one record per kernel instance and device).
+template <auto KERN>
+inline hipError_t allow_lds(size_t lds) {
+    static size_t allowed[16] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16)
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (lds <= allowed[dev])
+        return hipSuccess;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e == hipSuccess)
+        allowed[dev] = lds;
+    return e;
+}
+
 } // namespace et

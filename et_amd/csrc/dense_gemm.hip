@@ -18,7 +18,7 @@
 #include <cstring>
 #include <type_traits>
 
-#include "common.h"
+#include "tile_plan.h"
 
 namespace et {
 
@@ -33,6 +33,8 @@ struct DgArgs {
     int tile0[DG_MAX_LIN + 1]; // first column tile of each linear in the launch's tile list
     const f16 *X;
     int nlin, M, K, tiles_m, tiles_n, per_xcd, total;
+    int div, by_column; // blocks of a row tile (by_column: of a column tile) that consecutive workgroups take
+    unsigned div_magic;
 };
 
 // where a row keeps its 16-byte piece kc of a step
@@ -52,11 +54,12 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(const DgArgs a)
     f16 *smem = reinterpret_cast<f16 *>(dg_smem);
     constexpr int XT = BM * DG_BK, STAGE = XT + BN * DG_BK; // halves
     // consecutive ids on one XCD walk the column tiles of one row tile: they
-    // share the X tile in that XCD's L2, and W (small) is everywhere
+    // share the X tile in that XCD's L2, and W is everywhere - or, where X is the smaller one, the other way round
     const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
     if (vid >= a.total)
         return;
-    const int tm = vid / a.tiles_n, tn_all = vid - tm * a.tiles_n;
+    const int outer = div_magic(vid, a.div_magic), inner = vid - outer * a.div;
+    const int tm = a.by_column ? inner : outer, tn_all = a.by_column ? outer : inner;
     int lin = 0;
 #pragma unroll
     for (int i = 1; i < DG_MAX_LIN; i++)
@@ -249,16 +252,22 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
     constexpr int lds = ST * (BM + BN) * DG_BK * (int)sizeof(f16);
     a.tiles_m = (a.M + BM - 1) / BM;
     a.tiles_n = 0;
+    double n = 0.0;
     for (int i = 0; i < DG_MAX_LIN; i++) {
         a.tile0[i] = i < a.nlin ? a.tiles_n : 0;
-        if (i < a.nlin)
+        if (i < a.nlin) {
             a.tiles_n += (a.N[i] + BN - 1) / BN;
+            n += a.N[i];
+        }
     }
     a.total = a.tiles_m * a.tiles_n;
     a.per_xcd = (a.total + 7) / 8;
+    // (every L2 that has part of the work takes the operand that all of the work shares)
+    a.by_column = tl_order(2.0 * a.M * a.K, 2.0 * a.K * n, a.tiles_m, a.tiles_n, 4.5e6);
+    a.div = a.by_column ? a.tiles_m : a.tiles_n;
+    a.div_magic = magic_of(a.div);
     constexpr auto kern = &dense_gemm_kernel<GELU, WM, WN, TM, TN, ST>;
-    if (lds > 64 * 1024)
-        ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    ET_HIP(allow_lds<kern>(lds));
     hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(WM * WN * 64), lds, st, a);
     return launch_status("dense_gemm launch");
 }

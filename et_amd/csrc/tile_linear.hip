@@ -99,8 +99,11 @@ struct TlArgs {
     const f16 *bias[TL_MAX_LIN];
     int N[TL_MAX_LIN];
     const f16 *X;
-    int nlin, M, K, KC, nchunk, ncg, total, per_xcd;
-    int ipw; // plan kernel: consecutive work items per (persistent) workgroup
+    int nlin, M, K, KC, nchunk, ncg, per_xcd;
+    int ipw;      // resident kernel: consecutive items of a row panel per workgroup
+    int nwg, div; // workgroups; those of a panel (by_group: of a column group)
+    unsigned div_magic, ncg_magic; // magic_of(div), magic_of(ncg)
+    int by_group; // consecutive workgroups walk the panels of one column group (tl_order)
     // fused skip + LayerNorm epilogue (plan kernels with LN = true)
     const f16 *skip, *gamma, *beta;
     const f16 *gamma2, *beta2; // second LayerNorm of the fused layer tail
@@ -122,23 +125,31 @@ __device__ __forceinline__ f16 gelu_h(f16 v) {
     return v * (f16)t;
 }
 
+// A workgroup's first item.  The hardware deals consecutive workgroup ids round robin over the 8 XCDs; consecutive
+// virtual ids run on ONE of them.  They are the column groups of a row panel, which then enters one L2 only while W
+// enters all eight - or, by_group, the panels of a column group: W enters one L2 and the panels all of them.  The
+// launcher takes the order that moves fewer bytes (tl_order).
+__device__ __forceinline__ bool tl_place(const TlArgs &a, int &rp, int &lin, int &cg) {
+    const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+    if (vid >= a.nwg)
+        return false;
+    const int outer = div_magic(vid, a.div_magic), inner = vid - outer * a.div;
+    rp = a.by_group ? inner : outer;
+    const int rest = (a.by_group ? outer : inner) * a.ipw;
+    lin = div_magic(rest, a.ncg_magic);
+    cg = rest - lin * a.ncg;
+    return true;
+}
+
 // what every variant shares: workgroup -> (row panel, linear, column group)
 struct TlCtx {
     int lin, cg, m0, wave, lane, c16, g4, khalf8, hi, ldx, bn_wg, bn0, ld_r, ld_c;
 };
 
 __device__ __forceinline__ bool tl_context(const TlArgs &a, int nb, TlCtx &x) {
-    // Workgroups that share a row panel of X get consecutive ids on ONE XCD
-    // (hardware round-robins consecutive workgroup ids over the 8 XCDs), so
-    // the panel is fetched into that XCD's L2 once.
-    const int pid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-    if (pid >= a.total)
+    int rp;
+    if (!tl_place(a, rp, x.lin, x.cg))
         return false;
-    const int per_rp = a.ncg * a.nlin;
-    const int rp = pid / per_rp;
-    const int rest = pid - rp * per_rp;
-    x.lin = rest / a.ncg;
-    x.cg = rest - x.lin * a.ncg;
     x.m0 = rp * TL_BM;
     x.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     x.lane = threadIdx.x & 63;
@@ -638,15 +649,10 @@ template <int NB, bool GELU, int NW, bool LN>
 __global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(const TlArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
     f16 *xs = reinterpret_cast<f16 *>(tl_smem);
-    // Workgroups with consecutive virtual ids run on ONE XCD (hardware
-    // round-robins consecutive workgroup ids over the 8 XCDs), so the column
-    // groups of a row panel that do not fit one workgroup share that XCD's L2.
-    const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-    const int it0 = vid * a.ipw;
-    const int it1 = min(it0 + a.ipw, a.total);
-    if (it0 >= it1)
-        return;
     TlCtx x;
+    int rp;
+    if (!tl_place(a, rp, x.lin, x.cg))
+        return;
     x.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     x.lane = threadIdx.x & 63;
     x.c16 = x.lane & 15;
@@ -659,7 +665,6 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(const TlArgs 
     const int xrow16 = 16 * x.ldx * 2; // bytes between the two 16-row subtiles
     f16 *const stage0 = xs + TL_BM * x.ldx;
     f16 *const stage = stage0 + x.wave * tl_wave_stage_halves<NB>();
-    const int per_rp = a.ncg * a.nlin;
 
     // X panel staging: global -> LDS directly (global_load_lds_dwordx4: lane L
     // of the issuing wave writes 16 bytes at  base + 16*L, the source address is
@@ -684,75 +689,57 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(const TlArgs 
         }                                                                                         \
     }
 
-    int panel_rp = -1; // row panel currently in LDS (single-chunk problems only)
-    bool lds_used = false;
-    for (int it = it0; it < it1; it++) {
-        const int rp = it / per_rp;
-        const int rest = it - rp * per_rp;
-        const int lin = rest / a.ncg;
-        x.lin = lin;
-        x.cg = rest - lin * a.ncg;
-        x.m0 = rp * TL_BM;
-        x.bn_wg = x.cg * (NW * NB);
-        x.bn0 = x.bn_wg + x.wave * NB;
-        f16 *const Yp = TL_SEL(Y);
-        const int *const cptr = TL_SEL(cptr);
-        const int *const poff = TL_SEL(row_offset); // LDS byte offset per tile (chunk-local column * 2)
-        const f16 *const data = TL_SEL(data);
-        const f16 *const bias = TL_SEL(bias);
-        const int N = TL_SEL(N);
-        const int nbr = N >> 4;
+    const int lin = x.lin;
+    x.m0 = rp * TL_BM;
+    x.bn_wg = x.cg * (NW * NB);
+    x.bn0 = x.bn_wg + x.wave * NB;
+    f16 *const Yp = TL_SEL(Y);
+    const int *const cptr = TL_SEL(cptr);
+    const int *const poff = TL_SEL(row_offset); // LDS byte offset per tile (chunk-local column * 2)
+    const f16 *const data = TL_SEL(data);
+    const f16 *const bias = TL_SEL(bias);
+    const int N = TL_SEL(N);
+    const int nbr = N >> 4;
 
-        f32x4 acc[NB][2];
-        f16x4 b4[NB];
+    f32x4 acc[NB][2];
+    f16x4 b4[NB];
 #pragma unroll
-        for (int j = 0; j < NB; j++) {
-            acc[j][0] = f32x4{0.f, 0.f, 0.f, 0.f};
-            acc[j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-            b4[j] = f16x4{0, 0, 0, 0};
-            if (x.bn0 + j < nbr)
-                b4[j] = *reinterpret_cast<const f16x4 *>(bias + (x.bn0 + j) * 16 + x.g4 * 4);
-        }
-        const unsigned lane_w = hi * 256 + x.c16 * 16 + x.khalf8; // lane's halves inside a 1 KB tile pair
+    for (int j = 0; j < NB; j++) {
+        acc[j][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+        acc[j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        b4[j] = f16x4{0, 0, 0, 0};
+        if (x.bn0 + j < nbr)
+            b4[j] = *reinterpret_cast<const f16x4 *>(bias + (x.bn0 + j) * 16 + x.g4 * 4);
+    }
+    const unsigned lane_w = hi * 256 + x.c16 * 16 + x.khalf8; // lane's halves inside a 1 KB tile pair
 
-        for (int c = 0; c < a.nchunk; c++) {
-            // pair-index boundaries of the wave's block-rows: lane j holds the end
-            // of block-row j (read back with v_readlane)
-            const int bidx = c * nbr + min(x.bn0 + min(lane, NB), nbr);
-            const int bvec = cptr[bidx] >> 1;
+    for (int c = 0; c < a.nchunk; c++) {
+        // pair-index boundaries of the wave's block-rows: lane j holds the end
+        // of block-row j (read back with v_readlane)
+        const int bidx = c * nbr + min(x.bn0 + min(lane, NB), nbr);
+        const int bvec = cptr[bidx] >> 1;
 
-            const bool reload = a.nchunk > 1 || rp != panel_rp; // workgroup-uniform
-            if (reload) {
-                // (The load, its wait and both barriers stay in this one block:
-                // with the wait further down, behind the first weight loads,
-                // the compiler loses track of the DMA and drains every load in
-                // the pipelined loop below instead of counting.)
-                if (lds_used)
-                    __syncthreads(); // every wave is done with the previous panel
-                TL_PANEL_LOAD(c)
-                lds_used = true;
-                __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this wave's part has landed
-                __syncthreads();                    // ... and everyone else's
-            }
-            // the first pairs of the stream
-            const int q0 = __builtin_amdgcn_readfirstlane(bvec);
-            const int qend = __builtin_amdgcn_readlane(bvec, NB);
-            const int qlast = max(qend - 1, q0);
-            f16x8 w[TL_DEPTH];
-            int o[TL_DEPTH];
-            tl_preload(data, poff, lane_w, hi, q0, qlast, w, o);
-            tl_stream<NB>(xlane, xrow16, data, poff, lane_w, hi, q0, qend, qlast, bvec, w, o,
-                          [&](int j, f32x4 c0, f32x4 c1) { tl_flush_acc<NB>(acc, j, c0, c1); });
-        }
-        panel_rp = a.nchunk > 1 ? -1 : rp;
-        tl_epilogue_wave<NB, GELU, !LN>(a, x, stage, Yp, N, nbr, acc, b4);
-        if constexpr (LN) {
-            TlLnOperands<NB, NW, NW> lnop;
-            tl_ln_fetch(lnop, a, x.wave, lane, x.m0, N);
-            __syncthreads(); // every wave's part of the rows is staged
-            tl_ln_rows(lnop, a, stage0, x.wave, lane, x.m0, Yp, N);
-            lds_used = true; // (the next item's panel load starts with a barrier)
-        }
+        if (c > 0)
+            __syncthreads(); // every wave is done with the previous chunk
+        TL_PANEL_LOAD(c)
+        __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this wave's part has landed
+        __syncthreads();                    // ... and everyone else's
+        // the first pairs of the stream
+        const int q0 = __builtin_amdgcn_readfirstlane(bvec);
+        const int qend = __builtin_amdgcn_readlane(bvec, NB);
+        const int qlast = max(qend - 1, q0);
+        f16x8 w[TL_DEPTH];
+        int o[TL_DEPTH];
+        tl_preload(data, poff, lane_w, hi, q0, qlast, w, o);
+        tl_stream<NB>(xlane, xrow16, data, poff, lane_w, hi, q0, qend, qlast, bvec, w, o,
+                      [&](int j, f32x4 c0, f32x4 c1) { tl_flush_acc<NB>(acc, j, c0, c1); });
+    }
+    tl_epilogue_wave<NB, GELU, !LN>(a, x, stage, Yp, N, nbr, acc, b4);
+    if constexpr (LN) {
+        TlLnOperands<NB, NW, NW> lnop;
+        tl_ln_fetch(lnop, a, x.wave, lane, x.m0, N);
+        __syncthreads(); // every wave's part of the rows is staged
+        tl_ln_rows(lnop, a, stage0, x.wave, lane, x.m0, Yp, N);
     }
 #undef TL_PANEL_LOAD
 }
@@ -782,7 +769,8 @@ __device__ __forceinline__ void tl_barrier_lds() {
 }
 
 struct TlItem {
-    int rp, lin, cg, bn0, nbr, N;
+    int lin, cg, bn0, nbr, N;
+    int q0, qend; // the wave's pairs (scalar loads: a wait for them is none for the panel's requests)
     f16 *Y;
     const int *cptr;
     const int *poff;
@@ -812,10 +800,8 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
     static_assert(BM == TL_BM || (BM == 2 * TL_BM && !LN), "64-row panels: without the LayerNorm epilogue");
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
     f16 *xs = reinterpret_cast<f16 *>(tl_smem);
-    const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3); // see tile_linear_plan_kernel
-    const int it0 = vid * a.ipw;
-    const int it1 = min(it0 + a.ipw, a.total);
-    if (it0 >= it1)
+    int rp, lin0, cg0;
+    if (!tl_place(a, rp, lin0, cg0))
         return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -855,14 +841,18 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
                     load_lds16(src + (64 + lane) * 8, dstrow + 512);                              \
             }                                                                                     \
         }                                                                                         \
+    }
+    // behind the panel's requests and those of the first pairs
+#define TL_PANEL_WAIT()                                                                           \
+    {                                                                                             \
         __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0): this wave's part has landed */           \
         __syncthreads();                    /* ... and everyone else's */                         \
     }
     // the first pairs of an item's stream
-#define TL_PRELOAD(t_, bvec_)                                                                     \
+#define TL_PRELOAD(t_)                                                                            \
     {                                                                                             \
-        q0 = __builtin_amdgcn_readfirstlane(bvec_);                                               \
-        qend = __builtin_amdgcn_readlane(bvec_, NB);                                              \
+        q0 = (t_).q0;                                                                             \
+        qend = (t_).qend;                                                                         \
         qlast = max(qend - 1, q0);                                                                \
         wdata = (t_).data;                                                                        \
         wpoff = (t_).poff;                                                                        \
@@ -878,9 +868,8 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
 #define TL_KARG(type_, field_, lin_)                                                              \
     (*(const __attribute__((address_space(4))) type_ *)(ka + offsetof(TlArgs, field_) +           \
                                                          (lin_) * sizeof(type_)))
-    auto tl_item = [&](int rp, int lin, int cg) {
+    auto tl_item = [&](int lin, int cg) {
         TlItem t;
-        t.rp = rp;
         t.lin = lin;
         t.cg = cg;
         t.bn0 = (cg * NW + wave) * NB;
@@ -894,31 +883,33 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
         t.bias = TL_KARG(HPtr, bias, lin);
         t.N = TL_KARG(int, N, lin);
         t.nbr = t.N >> 4;
+        typedef const __attribute__((address_space(4))) int *IConst;
+        const IConst cp = (IConst)t.cptr;
+        t.q0 = cp[min(t.bn0, t.nbr)] >> 1;
+        t.qend = cp[min(t.bn0 + NB, t.nbr)] >> 1;
         return t;
     };
-    // the item after t in (row panel, linear, column group) order
+    // the panel's next item
     auto tl_next = [&](const TlItem &t) {
         const bool cw = t.cg + 1 == a.ncg;
-        const bool lw = cw && t.lin + 1 == a.nlin;
-        return tl_item(t.rp + (lw ? 1 : 0), lw ? 0 : t.lin + (cw ? 1 : 0), cw ? 0 : t.cg + 1);
+        return tl_item(cw ? (t.lin + 1 == a.nlin ? 0 : t.lin + 1) : t.lin, cw ? 0 : t.cg + 1);
     };
-    const int per_rp = a.ncg * a.nlin;
-    const int rp0 = it0 / per_rp, rest0 = it0 - rp0 * per_rp;
-    TlItem cur = tl_item(rp0, rest0 / a.ncg, rest0 % a.ncg);
+    TlItem cur = tl_item(lin0, cg0);
 
     int bvec = TL_BVEC(cur);
     f16x4 b4[NB];
     TL_BIAS(b4, cur)
-    TL_PANEL(cur.rp)
+    TL_PANEL(rp)
     int q0, qend, qlast;
     const f16 *wdata;
     const int *wpoff;
     f16x8 w[TL_DEPTH];
     int o[TL_DEPTH];
-    TL_PRELOAD(cur, bvec)
+    TL_PRELOAD(cur) // (in flight together with the panel)
+    TL_PANEL_WAIT()
 
-    for (int it = it0;; it++) {
-        const bool has_next = it + 1 < it1;
+    for (int it = 0;; it++) {
+        const bool has_next = it + 1 < a.ipw;
         const TlItem nxt = tl_next(cur); // (past the last item: a valid linear, never run)
         const int bvec_n = TL_BVEC(nxt);
         f16x4 b4n[NB];
@@ -958,23 +949,22 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
                                         f32x4{0.f, 0.f, 0.f, 0.f}, b4[k]);
             }
 
-        const bool same_panel = has_next && nxt.rp == cur.rp;
-        if (same_panel)
-            TL_PRELOAD(nxt, bvec_n)
+        if (has_next)
+            TL_PRELOAD(nxt)
 
         if constexpr (LN) {
             // the workgroup holds whole rows: skip connection + LayerNorm here
             TlLnOperands<NB, NW, NW> lnop;
-            tl_ln_fetch(lnop, a, wave, lane, cur.rp * BM, cur.N);
+            tl_ln_fetch(lnop, a, wave, lane, rp * BM, cur.N);
             __syncthreads(); // every wave's part of the rows is staged
-            tl_ln_rows(lnop, a, stage0, wave, lane, cur.rp * BM, cur.Y, cur.N);
-            if (has_next && same_panel)
+            tl_ln_rows(lnop, a, stage0, wave, lane, rp * BM, cur.Y, cur.N);
+            if (has_next)
                 __syncthreads(); // the staging tiles are free again
         } else {
             // staging tile -> Y: 16-byte stores of 32*NB contiguous bytes per row
             const int nvalid = min(NB, cur.nbr - cur.bn0); // the last column group may be partial
             const int cpr = 2 * nvalid;                    // 16-byte chunks per row
-            const int m0 = cur.rp * BM;
+            const int m0 = rp * BM;
             f16 *ybase = cur.Y + (size_t)m0 * cur.N + cur.bn0 * 16;
 #pragma unroll
             for (int t = 0; t < NB * (BM / TL_BM); t++) {
@@ -988,11 +978,6 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
         }
         if (!has_next)
             break;
-        if (!same_panel) {
-            __syncthreads(); // every wave is done with the previous panel
-            TL_PANEL(nxt.rp)
-            TL_PRELOAD(nxt, bvec_n)
-        }
         cur = nxt;
         bvec = bvec_n;
 #pragma unroll
@@ -1001,6 +986,7 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
     }
 #undef TL_PRELOAD
 #undef TL_PANEL
+#undef TL_PANEL_WAIT
 #undef TL_BIAS
 #undef TL_BVEC
 #undef TL_KARG
@@ -1028,7 +1014,7 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_ln_kernel(con
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
     f16 *xs = reinterpret_cast<f16 *>(tl_smem);
     const int rp = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-    if (rp >= a.total)
+    if (rp >= a.nwg)
         return;
     TlCtx x;
     x.lin = 0;
@@ -1196,7 +1182,7 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
     f16 *xs = reinterpret_cast<f16 *>(tl_smem);
     const int rp = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-    if (rp >= a.total)
+    if (rp >= a.nwg)
         return;
     constexpr int NW = TL_FFN_WAVES;
     TlCtx x;
@@ -1531,25 +1517,6 @@ __global__ void __launch_bounds__(TL_THREADS) tile_linear_generic_kernel(const T
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Dynamic LDS above the 64 KB default has to be allowed per kernel.  The call
-// goes to the driver, so it is made only when a kernel needs more than it was
-// last given (one record per kernel instance and device).
-template <auto KERN>
-static hipError_t allow_lds(size_t lds) {
-    static size_t allowed[16] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16)
-        return hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (lds <= allowed[dev])
-        return hipSuccess;
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e == hipSuccess)
-        allowed[dev] = lds;
-    return e;
-}
-
 template <int NB, bool GELU, int MODE>
 static int launch_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     const dim3 grid(a.per_xcd * 8), block(TL_THREADS);
@@ -1666,9 +1633,9 @@ static int tile_launch_ffn(const TlProblem *pO, const TlProblem &p1, const TlPro
     a.KC = KC2;
     a.nchunk = nchunk2;
     a.ncg = 1;
-    a.total = (M + TL_BM - 1) / TL_BM;
-    a.ipw = 1;
-    a.per_xcd = (a.total + 7) / 8;
+    a.nwg = (M + TL_BM - 1) / TL_BM; // (one workgroup per panel: div and ncg are 1)
+    a.ipw = a.div = 1;
+    a.per_xcd = (a.nwg + 7) / 8;
     a.skip = skip;
     a.gamma = gamma;
     a.beta = beta;
@@ -1704,9 +1671,9 @@ static int tile_launch_ln(const TlProblem &p, const f16 *X, int M, int K, int KC
     a.KC = KC;
     a.nchunk = nchunk;
     a.ncg = 1;
-    a.total = (M + TL_BM - 1) / TL_BM;
-    a.ipw = 1;
-    a.per_xcd = (a.total + 7) / 8;
+    a.nwg = (M + TL_BM - 1) / TL_BM; // (one workgroup per panel: div and ncg are 1)
+    a.ipw = a.div = 1;
+    a.per_xcd = (a.nwg + 7) / 8;
     a.skip = skip;
     a.gamma = gamma;
     a.beta = beta;
@@ -1777,6 +1744,90 @@ static int g_plan_dense = 1;
 
 static int g_tile_rows_most = -1; // et_tuning_set("tile_splitk_rows"): most rows for which a plan runs on whole rows, -1 automatic
 
+static int g_tile_order = 1; // et_tuning_set("tile_order"): 0 panels slowest, 2 column groups slowest, 1 fewer bytes
+// Whether consecutive workgroups walk the panels of a column group (see tl_items): X and W in bytes, numbers of panels
+// and of workgroups per panel.  Every L2 that has part of the work takes what all of the work shares, so W times eight
+// is what bounds a launch of few rows: 256 rows, 1024 -> 4096: dense 14.2 -> 6.6 us, 50 % 10.0 -> 5.6; 768 -> 3072
+// dense 9.7 -> 5.9; 128 rows 3072 -> 768 dense 9.8 -> 6.8.  Only up to x_most bytes of X: beyond, the L2s have time
+// enough for W and the launch is up to 10 % slower in this order (1536 rows, 1024 -> 4096, 50 %: 18.7 and 20.9).
+bool tl_order(double x_bytes, double w_bytes, long panels, long groups, double x_most) {
+    if (g_tile_order != 1)
+        return g_tile_order == 2;
+    return x_bytes <= x_most && std::min(groups, 8L) * x_bytes + w_bytes < x_bytes + std::min(panels, 8L) * w_bytes;
+}
+
+// The forms of the single-panel kernel and the choice among them.  An item is a panel of 32 or 64 rows by waves x nb
+// block-rows; a workgroup keeps its panel in LDS and does d consecutive items of it.  Small items put more CUs to work
+// and end a round sooner, large ones fetch a panel less often and stream each kilobyte of W past more rows.  The choice
+// is the least estimated time: per launch, per byte that the L2s take in, per round of workgroups on the busiest CU (a
+// start and the stream's latency for each item), per panel, output, GELU and MFMA of the busiest CU, per byte of the
+// result and per workgroup.  The figures (us) start from non-negative least squares over 12000 launches (512 / 768 / 1024
+// inputs, 512 .. 4096 outputs, one or three linears, 0 .. 90 % pruned, 37 .. 32768 rows; 5 to 6 % off in the mean) and
+// are then moved by up to a factor of two where that brings the choice closer to the fastest form: 0.5 % from it in the
+// mean, 13 % at most (0.6 % where half of the row counts was left out); the rule before, a number of workgroups to aim
+// for, was 6.3 %.  1536 rows 768 -> 3072, 50 %: 13.8 -> 11.7 us; 3500 rows 768 -> 768, 90 %: 7.3 -> 5.8; 2700 rows
+// 768 -> 3072, 80 %: 16.1 -> 12.4.
+struct TlForm {
+    int rows, waves, nb;
+};
+static const TlForm tl_forms[] = {{TL_BM, 8, 1}, {TL_BM, 8, 2}, {TL_BM, 8, 3}, {TL_BM64, 12, 2}, {TL_BM64, 8, 3},
+                                  {TL_BM64, 8, 2}, {TL_BM64, 8, 1}};
+struct TlCost {
+    double launch, traffic, traffic_over, round, item, item_nb, item_stream, panel, out, gelu, mfma, result, wg;
+};
+static const TlCost tl_cost32 = {2.48, 0.0586, 0.0614, 0.0, 0.458, 0.236, 0.0221, 0.173e-4, 0.403e-3, 0.382e-3, 0.171e-3, 0.192e-6, 0.668e-3},
+                    tl_cost64 = {1.92, 0.0693, 0.0209, 0.696, 0.609, 0.381, 0.0884, 0.111e-4, 0.0, 0.534e-3, 0.0, 0.226e-6, 0.681e-3},
+                    tl_cost64x12 = {2.80, 0.0152, 0.0728, 0.379, 0.0, 0.322, 0.113, 0.266e-4, 0.0, 0.841e-3, 0.0, 0.293e-6, 0.0};
+struct TlChoice {
+    const TlForm *form;
+    int d, ncg, by_group;
+    size_t lds;
+    double us;
+};
+static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, int nbr_max, bool gelu) {
+    const int cus = std::max(et_device_cu_count(), 1);
+    double pairs = 0.0, w_mb = 0.0, result = 0.0; // tile pairs per block-row; W and the result of all linears
+    for (int i = 0; i < nlin; i++) {
+        const double p = 0.5 * probs[i].ntile / probs[i].nbr;
+        pairs += p / nlin;
+        w_mb += p * probs[i].nbr * 1024e-6;
+        result += (double)M * probs[i].N;
+    }
+    const double x_mb = 2e-6 * M * K;
+    const int fnb = g_tile_nb >= 1 && g_tile_nb <= 3 ? g_tile_nb : 0;
+    TlChoice best = {};
+    for (const TlForm &f : tl_forms) {
+        if (f.rows == TL_BM ? (fnb ? f.nb != fnb : g_tile_bm64 == 2) : fnb || g_tile_bm64 == 0)
+            continue; // (tuning; a form of either height fits every K of one chunk)
+        const size_t lds = (size_t)f.rows * (K + ((K & 31) ? 0 : TL_PAD)) * sizeof(f16) +
+                           (size_t)f.waves * f.rows * (16 * f.nb + 8) * sizeof(f16);
+        if (lds > 160 * 1024)
+            continue;
+        const TlCost &c = f.rows == TL_BM ? tl_cost32 : f.waves == 8 ? tl_cost64 : tl_cost64x12;
+        const int ncg = (nbr_max + f.waves * f.nb - 1) / (f.waves * f.nb), per_panel = ncg * nlin;
+        const long panels = (M + f.rows - 1) / f.rows;
+        const long slots = f.rows == TL_BM && 2 * lds <= 160 * 1024 ? 2 : 1; // workgroups per CU
+        const double G = std::min(f.waves * f.nb, nbr_max);
+        const double per_item = c.item + f.nb * (c.item_nb + c.item_stream * pairs);
+        const double cu_item = G * f.rows * (c.out + (gelu ? c.gelu : 0.0) + c.mfma * pairs);
+        const double fixed = c.launch + c.result * result;
+        for (int d = 1; d <= per_panel && d <= 16; d++) { // (beyond 16 items a workgroup the tail of the launch shows)
+            if (per_panel % d)
+                continue;
+            const long groups = per_panel / d, nwg = panels * groups;
+            const long on_cu = (nwg + cus - 1) / cus, rounds = (on_cu + slots - 1) / slots;
+            const bool by_group = tl_order(1e6 * x_mb, 1e6 * w_mb, panels, groups, 1.75e6);
+            const double mb = by_group ? std::min(groups, 8L) * x_mb + w_mb : x_mb + std::min(panels, 8L) * w_mb;
+            const double us = fixed + c.traffic * mb + c.traffic_over * std::max(0.0, mb - 12.0) +
+                              (double)rounds * (c.round + d * per_item) +
+                              (double)on_cu * (c.panel * f.rows * K + d * cu_item) + c.wg * (double)nwg;
+            if (!best.form || us < best.us)
+                best = TlChoice{&f, d, ncg, by_group, lds, us};
+        }
+    }
+    return best;
+}
+
 template <int NB, bool GELU, int NW = TL_WAVES>
 static int launch_resident64(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_resident_kernel<NB, GELU, NW, false, TL_BM64>;
@@ -1837,103 +1888,47 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         if (take)
             return tile_rows_launch(l, Ys, nlin, X, M, K, pairs, gelu, raw, st);
     }
-    if (mode == TL_PLAN && nchunk == 1 && g_tile_bm64 && g_tile_nb == 0) {
-        // 64-row panels, one workgroup per CU: twice the rows per kilobyte of W
-        // streamed.  Needs the panel and one 64-row staging tile per wave in LDS
-        // and at least two items per CU.  Twelve waves of two block-rows (where
-        // the LDS holds their staging tiles: K <= 784), or eight waves of three
-        // or of two (or of one: K 817 .. 1024; 4096 rows, 1024 -> 4096, 50 %: 55 -> 32 us against 32-row panels),
-        // and d consecutive items of a panel per workgroup: the
-        // combination with the least estimated time (a round of workgroups costs
-        // the panel load, 2/3 of a 24-block-row item, plus its items).  Twelve
-        // waves come first and win ties: the same items as eight waves of three,
-        // with three waves per SIMD instead of two to cover the stream's waits
-        // (Q/K/V of the benchmark: 20 -> 17.5 us).
-        double pairs_avg = 0.0; // tile pairs per block-row
-        for (int i = 0; i < nlin; i++)
-            pairs_avg += 0.5 * probs[i].ntile / probs[i].nbr / nlin;
-        const int cus = std::max(et_device_cu_count(), 1);
-        const int nrp64 = (M + TL_BM64 - 1) / TL_BM64;
-        static const int cand[4][2] = {{12, 2}, {8, 3}, {8, 2}, {8, 1}}; // waves, block-rows per wave
-        double best = 0.0;
-        int best_c = -1, best_d = 1, best_ncg = 1;
-        size_t best_lds = 0;
-        for (int c = 0; c < 4; c++) {
-            const int nw = cand[c][0], nb = cand[c][1];
-            if (nw == 12 && g_tile_bm64 == 4)
-                continue; // (tuning: eight waves only)
-            // (one block-row per wave: where no wider form fits the LDS, or none has enough items and the lists are
-            // long - 8192 rows, 768 -> 768: dense 19.9 -> 17.5 us, 50 % 13.7 -> 13.5, 80 % 9.9 -> 11.3)
-            if (nb == 1 && (best_c >= 0 || (KC <= 816 && pairs_avg < 8.0)))
-                continue;
-            const size_t lds64 = (size_t)TL_BM64 * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16) +
-                                 (size_t)nw * TL_BM64 * (16 * nb + 8) * sizeof(f16);
-            const int ncg64 = (nbr_max + nw * nb - 1) / (nw * nb);
-            const long items = (long)nrp64 * ncg64 * nlin;
-            if (lds64 > 160 * 1024 || items < (g_tile_bm64 == 2 ? 1L : 2L * cus))
-                continue;
-            const int per_rp = ncg64 * nlin;
-            for (int d = 1; d <= per_rp; d++) {
-                // (eight block-rows per item: K beyond 816.  More than 16 of them per workgroup and the launch slows
-                // down: 16384 rows, 1024 -> 4096, 80 %: 101 us with 8, 104 with 16, 122 with 32)
-                if (per_rp % d || (nb == 1 && d > 16))
-                    continue;
-                const long nwg = items / d, rounds = (nwg + cus - 1) / cus;
-                const double cost = (double)rounds * (2.0 / 3.0 + d * (nw * nb) / 24.0);
-                if (best_c < 0 || cost < best * 0.999) {
-                    best = cost;
-                    best_c = c;
-                    best_d = d;
-                    best_ncg = ncg64;
-                    best_lds = lds64;
-                }
-            }
+    auto place = [&](int bm, int order) { // order: by_group, or -1 to be worked out
+        const int panels = (M + bm - 1) / bm, per_rp = a.ncg * nlin;
+        while (per_rp % a.ipw)
+            a.ipw--; // (a tuning value: the items of a workgroup are one panel's)
+        a.nwg = panels * (per_rp / a.ipw);
+        a.per_xcd = (a.nwg + 7) / 8;
+        if (order < 0) {
+            double w_bytes = 0.0;
+            for (int i = 0; i < nlin; i++)
+                w_bytes += mode == TL_DENSE ? 2.0 * probs[i].N * K : 512.0 * (probs[i].ntile ? probs[i].ntile : 0.2 * probs[i].nbr * K / 16);
+            order = tl_order(2.0 * M * K, w_bytes, panels, per_rp / a.ipw, 1.75e6);
         }
-        if (best_c >= 0) {
-            a.ncg = best_ncg;
-            a.total = nrp64 * best_ncg * nlin;
-            a.ipw = g_tile_ipw > 0 ? g_tile_ipw : best_d;
-            a.per_xcd = ((a.total + a.ipw - 1) / a.ipw + 7) / 8;
-            if (best_c == 0)
-                return gelu ? launch_resident64<2, true, 12>(a, best_lds, st)
-                            : launch_resident64<2, false, 12>(a, best_lds, st);
-            if (best_c == 1)
-                return gelu ? launch_resident64<3, true>(a, best_lds, st) : launch_resident64<3, false>(a, best_lds, st);
-            if (best_c == 2)
-                return gelu ? launch_resident64<2, true>(a, best_lds, st) : launch_resident64<2, false>(a, best_lds, st);
-            return gelu ? launch_resident64<1, true>(a, best_lds, st) : launch_resident64<1, false>(a, best_lds, st);
-        }
-    }
-    const int nrp = (M + TL_BM - 1) / TL_BM;
-    const int nb = choose_nb(nrp, nbr_max, nlin);
-    a.ncg = (nbr_max + TL_WAVES * nb - 1) / (TL_WAVES * nb);
-    a.total = nrp * a.ncg * nlin;
-    a.ipw = 1;
+        a.by_group = order;
+        a.div = a.by_group ? panels : per_rp / a.ipw;
+        a.div_magic = magic_of(a.div);
+        a.ncg_magic = magic_of(a.ncg);
+    };
+    int nb = 0, order = -1;
     if (mode == TL_PLAN && nchunk == 1) {
-        // Persistent workgroups: d items of one row panel per workgroup, d a
-        // divisor of the items per panel.  A workgroup costs one panel fetch
-        // (about 2/3 of an item) plus d items, and the launch runs in
-        // ceil(workgroups / resident slots) rounds; take the cheapest d.
-        const int per_rp = a.ncg * nlin;
-        const long slots = g_tile_min_wgs; // two workgroups per CU
-        double best = 0.0;
-        for (int d = 1; d <= per_rp; d++) {
-            if (per_rp % d)
-                continue;
-            const long nwg = a.total / d;
-            const long rounds = (nwg + slots - 1) / slots;
-            const double cost = (double)rounds * (2.0 / 3.0 + d);
-            if (a.ipw == 1 && d == 1) {
-                best = cost;
-            } else if (cost < best * 0.999) {
-                best = cost;
-                a.ipw = d;
-            }
+        const TlChoice c = choose_resident(probs, nlin, M, K, nbr_max, gelu);
+        a.ncg = c.ncg;
+        a.ipw = g_tile_ipw > 0 ? g_tile_ipw : c.d;
+        if (c.form->rows == TL_BM64) {
+            place(TL_BM64, c.by_group);
+            if (c.form->waves == 12)
+                return gelu ? launch_resident64<2, true, 12>(a, c.lds, st) : launch_resident64<2, false, 12>(a, c.lds, st);
+            if (c.form->nb == 3)
+                return gelu ? launch_resident64<3, true>(a, c.lds, st) : launch_resident64<3, false>(a, c.lds, st);
+            if (c.form->nb == 2)
+                return gelu ? launch_resident64<2, true>(a, c.lds, st) : launch_resident64<2, false>(a, c.lds, st);
+            return gelu ? launch_resident64<1, true>(a, c.lds, st) : launch_resident64<1, false>(a, c.lds, st);
         }
-        if (g_tile_ipw > 0)
-            a.ipw = g_tile_ipw;
+        nb = c.form->nb;
+        order = c.by_group;
+    } else {
+        const int nrp = (M + TL_BM - 1) / TL_BM;
+        nb = choose_nb(nrp, nbr_max, nlin);
+        a.ncg = (nbr_max + TL_WAVES * nb - 1) / (TL_WAVES * nb);
+        a.ipw = 1;
     }
-    a.per_xcd = ((a.total + a.ipw - 1) / a.ipw + 7) / 8;
+    place(TL_BM, order);
     const size_t lds_x = (size_t)TL_BM * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16);
     const size_t lds_y = (size_t)TL_BM * (TL_WAVES * nb * 16 + TL_PAD) * sizeof(f16);
     // plan kernel: panel + one private staging tile per wave; generic kernel:
@@ -2012,6 +2007,10 @@ extern "C" int et_tuning_set(const char *key, int value) {
     }
     if (key && !strcmp(key, "tile_ipw")) {
         et::g_tile_ipw = value;
+        return ET_OK;
+    }
+    if (key && !strcmp(key, "tile_order")) {
+        et::g_tile_order = value;
         return ET_OK;
     }
     if (key && !strcmp(key, "tile_bm64")) {
@@ -2097,26 +2096,32 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
 double dense_gemm_estimate(const int *Ns, int nlin, int M, int K);
 int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int nchunk, int nbr); // null stream
 
-// Plans of fully populated matrices: the dense product is the shorter launch from some hundred rows on (many outputs)
-// or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by tile; their time on such
-// plans, fitted to 60 measured launches (128 to 16384 rows) within 20 % where the two are close: the larger of a stream
-// and product term and of a term per row, and for K in several chunks the larger slope.
-static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M) {
+// Plans of fully populated matrices: the dense product where it is estimated to be the shorter launch, from some hundred
+// rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
+// tile: their time is that of the choice among the single-panel forms, or, for K in several chunks, a line through the
+// whole-rows and chunk kernels at 128 to 16384 rows (within 20 % where the two are close).
+static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
-    int Ns[3], N = 0;
+    TlProblem probs[3];
+    int Ns[3], nbr_max = 0;
+    double N = 0.0;
     for (int i = 0; i < n; i++) {
         if (!plans[i]->d_dense)
             return false;
-        N += Ns[i] = plans[i]->out_feat;
+        Ns[i] = plans[i]->out_feat;
+        N += Ns[i];
+        probs[i].N = Ns[i];
+        probs[i].nbr = Ns[i] / 16;
+        probs[i].ntile = plans[i]->ntile;
+        nbr_max = std::max(nbr_max, probs[i].nbr);
     }
     if (g_plan_dense == 2)
         return true;
     const int K = plans[0]->in_feat;
-    const double gflop = 2e-9 * M * N * K;
-    const double tiles = plans[0]->nchunk > 1 ? 8.5 + 1.95 * gflop
-                                              : std::max(2.1 + 0.0009 * N + 1.3 * gflop, 2.0 + 0.0013 * M);
-    return dense_gemm_estimate(Ns, n, M, K) < tiles;
+    const double tiles = plans[0]->nchunk > 1 ? 10.9 + 1.95e-9 * 2.0 * M * N * K
+                                              : choose_resident(probs, n, M, K, nbr_max, gelu).us;
+    return 2.4 + dense_gemm_estimate(Ns, n, M, K) < tiles;
 }
 static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
                            hipStream_t st) {
@@ -2356,7 +2361,7 @@ extern "C" int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *co
     ET_REQUIRE(aligned16(X), ET_ERR_ALIGNMENT, "et_tile_plan_run_multi: X not aligned");
     if (M == 0)
         return ET_OK;
-    if (plans_run_dense(plans, n, M))
+    if (plans_run_dense(plans, n, M, false))
         return run_plans_dense(plans, Ys, n, X, M, false, static_cast<hipStream_t>(stream));
     return tile_launch(pr, n, static_cast<const f16 *>(X), M, plans[0]->in_feat, plans[0]->KC,
                        plans[0]->nchunk, false, TL_PLAN, static_cast<hipStream_t>(stream));
@@ -2386,7 +2391,7 @@ extern "C" int et_tile_plan_run_ln(const et_tile_plan *plan, void *Y, const void
     if (M == 0)
         return ET_OK;
     const int nbr = plan->out_feat / 16;
-    if (!et_tile_plan_ln_fusable(plan) || ((!ln_fusion_pays(M) || plans_run_dense(&plan, 1, M)) && Y != skip)) {
+    if (!et_tile_plan_ln_fusable(plan) || ((!ln_fusion_pays(M) || plans_run_dense(&plan, 1, M, false)) && Y != skip)) {
         // rows too wide for one workgroup, too few of them, or a dense product: the two kernels, one after the other
         ET_REQUIRE(Y != skip, ET_ERR_INVALID_ARG,
                    "et_tile_plan_run_ln: Y must not alias skip for out_feat=%d", plan->out_feat);
@@ -2423,7 +2428,7 @@ extern "C" int et_tile_plan_ffn_fusable(const et_tile_plan *p1, const et_tile_pl
 // Dense feed-forward products against the fused tail, which streams all of W past every 32 or 64 rows: wherever both
 // products are the shorter launch by themselves (768 wide, 3072 rows: 157 -> 99 us a layer; 8192 rows: 206 -> 181).
 static bool ffn_runs_dense(const et_tile_plan *p1, const et_tile_plan *p2, int M) {
-    return et::plans_run_dense(&p1, 1, M) && et::plans_run_dense(&p2, 1, M);
+    return et::plans_run_dense(&p1, 1, M, true) && et::plans_run_dense(&p2, 1, M, false);
 }
 
 extern "C" int et_tile_plan_run_ffn_ln(const et_tile_plan *p1, const et_tile_plan *p2, void *Y,
@@ -2567,7 +2572,7 @@ extern "C" int et_tile_plan_run(const et_tile_plan *plan, void *Y, const void *X
     ET_REQUIRE(aligned16(Y) && aligned16(X), ET_ERR_ALIGNMENT, "et_tile_plan_run: Y/X not aligned");
     if (M == 0)
         return ET_OK;
-    if (plans_run_dense(&plan, 1, M))
+    if (plans_run_dense(&plan, 1, M, gelu != 0))
         return run_plans_dense(&plan, &Y, 1, X, M, gelu != 0, static_cast<hipStream_t>(stream));
     TlProblem pr;
     pr.Y = static_cast<f16 *>(Y);

@@ -30,6 +30,9 @@ struct et_tile_plan {
 };
 
 namespace et {
+// whether consecutive workgroups of a linear should share a column group of W rather than a row panel of X (tile_linear.hip)
+bool tl_order(double x_bytes, double w_bytes, long panels, long groups, double x_most);
+
 // One int per process in pinned host memory that kernels set when a bounded
 // wait inside a workgroup gives up (device pointer / host pointer, null if the
 // allocation failed).  The launchers of those kernels read it before every

@@ -36,6 +36,8 @@ struct TrArgs {
     f16 *Y[TR_MAX_LIN];
     const f16 *X;
     int nlin, M, K, ldx, ncg, total, per_xcd, nb, ls;
+    int div, by_group; // workgroups of a panel (by_group: of a column group) that consecutive ids take
+    unsigned div_magic, ncg_magic;
 };
 
 // The caller's list: pair i of a block-row is tiles 2i and 2i + 1, 1 KB of
@@ -65,16 +67,16 @@ template <bool GELU, bool RAW>
 __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(const TrArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char tr_smem[];
     f16 *const xs = reinterpret_cast<f16 *>(tr_smem);
-    // (consecutive ids on one XCD: the column groups of a panel share it in that XCD's L2)
+    // (consecutive ids on one XCD: the column groups of a panel, or, by_group, the panels of a column group)
     const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
     if (vid >= a.total)
         return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int c16 = lane & 15, g4 = lane >> 4, khalf8 = (g4 & 1) * 8, hi = lane >> 5;
     const unsigned lane_w2 = (unsigned)(hi * 256 + c16 * 16 + khalf8) * 2, hi4 = hi * 4;
-    const int per = a.ncg * a.nlin;
-    const int panel = vid / per, rest = vid - panel * per;
-    const int lin = rest / a.ncg, cg = rest - lin * a.ncg;
+    const int outer = div_magic(vid, a.div_magic), inner = vid - outer * a.div;
+    const int panel = a.by_group ? inner : outer, rest = a.by_group ? outer : inner;
+    const int lin = div_magic(rest, a.ncg_magic), cg = rest - lin * a.ncg;
     const int m0 = panel * TR_BM;
     LfLinear l = a.l[0];
     f16 *Y = a.Y[0];
@@ -253,21 +255,23 @@ int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *
     tile_rows_plan(M, K, nbr_max, nlin, pairs, std::max(et_device_cu_count(), 1), &a.nb, &a.ls);
     const int per = (TR_WAVES >> a.ls) * a.nb;
     a.ncg = (nbr_max + per - 1) / per;
-    a.total = ((M + TR_BM - 1) / TR_BM) * a.ncg * nlin;
+    const int panels = (M + TR_BM - 1) / TR_BM;
+    a.total = panels * a.ncg * nlin;
     a.per_xcd = (a.total + 7) / 8;
+    a.by_group = tl_order(2.0 * M * K, 1024.0 * pairs * nbr_max * nlin, panels, a.ncg * nlin, 2.5e6);
+    a.div = a.by_group ? panels : a.ncg * nlin;
+    a.div_magic = magic_of(a.div);
+    a.ncg_magic = magic_of(a.ncg);
     const size_t lds = tile_rows_lds(K);
-    auto launch = [&](auto kern, size_t &allowed) -> int {
-        if (lds > 64 * 1024 && lds > allowed) {
-            ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            allowed = lds;
-        }
+    auto launch = [&](auto gelu_c, auto raw_c) -> int {
+        constexpr auto kern = &tile_rows_kernel<decltype(gelu_c)::value, decltype(raw_c)::value>;
+        ET_HIP(allow_lds<kern>(lds));
         hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(TR_WAVES * 64), lds, st, a);
         return launch_status("tile_linear (whole rows) launch");
     };
-    static size_t allowed[4] = {0, 0, 0, 0};
     if (raw)
-        return gelu ? launch(&tile_rows_kernel<true, true>, allowed[0]) : launch(&tile_rows_kernel<false, true>, allowed[1]);
-    return gelu ? launch(&tile_rows_kernel<true, false>, allowed[2]) : launch(&tile_rows_kernel<false, false>, allowed[3]);
+        return gelu ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
+    return gelu ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
 }
 
 } // namespace et

@@ -930,26 +930,10 @@ int tail_pair_prepare(const et_tile_plan *pO, const et_tile_plan *p1, et_tile_pl
     return ET_OK;
 }
 
-template <auto KERN>
-static hipError_t tt_allow_lds(size_t lds) {
-    static size_t allowed[16] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16)
-        return hipFuncSetAttribute(reinterpret_cast<const void *>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)lds);
-    if (lds <= allowed[dev])
-        return hipSuccess;
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e == hipSuccess)
-        allowed[dev] = lds;
-    return e;
-}
-
 template <int D, int MS>
 static int tt_launch(const TtArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_tail_pair_kernel<D, MS>;
-    ET_HIP(tt_allow_lds<k>(lds));
+    ET_HIP(allow_lds<k>(lds));
     hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TT_WAVES * 64), lds, st, a);
     return launch_status("layer tail (pairs) launch");
 }

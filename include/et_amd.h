@@ -458,8 +458,9 @@ int et_device_synchronize(void);
 /* Launch-heuristic overrides for benchmarking sweeps; value 0 restores the
  * automatic choice unless noted.  Keys:
  *   "tile_nb"         block-rows of W per wave in the tile linear (1, 2, 3; the
- *                     raw launchers also take 4 and 6)
- *   "tile_min_wgs"    workgroups the automatic choices aim for (default 512)
+ *                     raw launchers also take 4 and 6), on 32-row panels
+ *   "tile_min_wgs"    workgroups the choices for raw launchers and for K in
+ *                     several chunks aim for (default 512)
  *   "tile_ipw"        work items per persistent workgroup of a planned linear
  *   "tile_fuse_ln"    0: et_tile_plan_run_ln runs the linear and the LayerNorm
  *                     as two launches; 1 (default): fused where the rows fit
@@ -467,10 +468,10 @@ int et_device_synchronize(void);
  *                     fuses (default 96; below, two launches are faster); a
  *                     value > 0 also replaces the 72 panels from which
  *                     et_tile_plan_run_tail runs as one launch
- *   "tile_bm64"       0: planned linears always use 32-row panels; 1 (default):
- *                     64-row panels where two such items per CU exist; 2: also
- *                     with fewer items; 4: as 1 with eight waves per workgroup
- *                     only (no twelve-wave form)
+ *   "tile_order"      consecutive workgroups of a linear share 0: a row panel, 2:
+ *                     a column group, 1 (default): what moves fewer bytes
+ *   "tile_bm64"       panels of a planned linear of one chunk: 0: 32 rows; 2: 64
+ *                     rows; 1 (default): the less estimated time
  *   "tile_splitk_rows" most rows for which a planned linear with K > 1024 runs
  *                     on whole rows in LDS (16-row panels, a block-row's tile
  *                     pairs split over several waves where there are few); -1
@@ -478,6 +479,12 @@ int et_device_synchronize(void);
  *   "layer_flow_rows" most rows for which an encoder layer runs as one launch
  *                     (et_layer_flow_pays); -1 (default): by size and density;
  *                     0: never
+ *   "plan_dense"      plans of fully populated matrices as dense products: 0
+ *                     never, 1 (default) where the estimated time is less, 2
+ *                     always
+ *   "dense_form"      block of the dense kernel: 0 .. 4: 64 x 128, 128 x 128 with
+ *                     two and three stages, 128 x 192, 256 x 256; -1 (default):
+ *                     the least estimated time
  *   "row_gemm_min_rows" rows from which et_row_spmm_add_bias runs the dense
  *                     GEMM kernel (default 1024; 0: never)
  *   "tile_fuse_ffn"   0: et_tile_plan_ffn_fusable answers no (the feed-forward

@@ -1174,3 +1174,34 @@ def test_full_plan_as_dense_product(K, form, M, Ns, Kd, gelu):
         want = orc.tile_linear(X[rows], m["row_ptr"], m["row_offset"], m["data"], m["bias"], N, gelu=gelu, f64=True)
         check_close(g[rows], want, max_abs=8e-3, mean_rel=5e-4, what=f"dense, N={N}")
         assert np.abs(g.astype(np.float32) - t.astype(np.float32)).max() <= 2.0 ** -6
+
+
+@pytest.mark.parametrize("M,Ns,Kd", [
+    (1, (16,), 16), (33, (272, 16, 400), 768), (129, (400, 144), 1024), (200, (48, 784, 48), 512),
+    (50, (336,), 2048),     # K in several chunks: whole rows in LDS
+])
+def test_tile_linear_orders_and_forms(K, M, Ns, Kd):
+    """planned linears with the row panels slowest and with the column groups slowest, on 32- and 64-row panels, one or
+    several items per workgroup: the oracle's values, and the same bits from every one of them"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile, run_multi
+    r = rng(55 + M + Kd)
+    mats = [make_tile_linear(r, N, Kd, 0.6, seed=M + N, std=0.05, bias_std=0.2) for N in Ns]
+    X = randn_h(r, (M, Kd))
+    lts = [Linear_tile(Kd, N, M, m["row_offset"].size, m["data"], m["row_ptr"], m["row_offset"], m["bias"])
+           for N, m in zip(Ns, mats)]
+    want = [orc.tile_linear(X, m["row_ptr"], m["row_offset"], m["data"], m["bias"], N, f64=True) for N, m in zip(Ns, mats)]
+    first = None
+    try:
+        for order, rows, items in ((0, 0, 0), (2, 0, 0), (0, 2, 0), (2, 2, 0), (0, 0, 2), (2, 0, 3), (0, 2, 3), (2, 2, 2)):
+            lib().et_tuning_set(b"tile_order", order)
+            lib().et_tuning_set(b"tile_bm64", rows)
+            lib().et_tuning_set(b"tile_ipw", items)
+            got = [host(y) for y in run_multi(lts, dev(X))]
+            for g, w in zip(got, want):
+                check_close(g, w, max_abs=4e-3, mean_rel=5e-4, what=f"order {order}, rows {rows}, items {items}")
+            first = first or got
+            assert all(np.array_equal(a, b) for a, b in zip(first, got))
+    finally:
+        for key, value in ((b"tile_order", 1), (b"tile_bm64", 1), (b"tile_ipw", 0)):
+            lib().et_tuning_set(key, value)
