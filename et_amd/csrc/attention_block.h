@@ -124,10 +124,12 @@ __device__ __forceinline__ void transpose_pieces_4x4(f16x4 (&p)[4]) {
 // FLOW: the output rows are read by other workgroups of the SAME launch: they
 // are stored past the XCD's own L2 (store_agent8).
 // One workgroup's work: the NW*16*QS query rows of block qb of (sequence b, head h).
+// MASK: there may be a mask.  Without one (and not PLAIN: ragged lengths) nothing of its bookkeeping is compiled in.
 template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
-          bool FLOW = false>
+          bool FLOW = false, bool MASK = !PLAIN>
 __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, const int h, const int qb) {
     static_assert(!PLAIN || ((!PRUNED || VWIN) && !SHAREDQK), "the plain form exists for the DMA-staged kernels only");
+    static_assert(!PLAIN || !MASK, "the plain form has no mask");
     static_assert(HDK == HD || (!PRUNED && !SHAREDQK && HDK % 32 == 0), "narrow Q/K heads: on-the-fly kernel only");
     static_assert(!VWIN || (PRUNED && HD == 64), "the value-window form exists for the pruned kernel with 64-wide heads");
     constexpr int AT_THREADS = NW * 64; // NW waves, each owning 16*QS query rows
@@ -227,23 +229,25 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
     if (q0 < len) {
         // ---- Q fragments (B operand of S^T), scaled in half like the reference
         f16x8 qf[QS][DK];
-        const f16 sc = (f16)a.scale;
+        auto load_q = [&] {
+            const f16 sc = (f16)a.scale;
 #pragma unroll
-        for (int qs = 0; qs < QS; qs++) {
-            const int q = q0 + (wave * QS + qs) * 16 + c16;
+            for (int qs = 0; qs < QS; qs++) {
+                const int q = q0 + (wave * QS + qs) * 16 + c16;
 #pragma unroll
-            for (int s = 0; s < DK; s++) {
-                f16x8 v = zero8;
-                if (!SHAREDQK && q < len) {
-                    const f16 *qrow = a.Q + (size_t)(row0 + q) * a.ldq + qc0;
-                    if (PRUNED && !VWIN)
-                        v = load8_guard(qrow, s * 32 + g4 * 8, nqk);
-                    else
-                        v = *reinterpret_cast<const f16x8 *>(qrow + s * 32 + g4 * 8);
+                for (int s = 0; s < DK; s++) {
+                    f16x8 v = zero8;
+                    if (!SHAREDQK && q < len) {
+                        const f16 *qrow = a.Q + (size_t)(row0 + q) * a.ldq + qc0;
+                        if (PRUNED && !VWIN)
+                            v = load8_guard(qrow, s * 32 + g4 * 8, nqk);
+                        else
+                            v = *reinterpret_cast<const f16x8 *>(qrow + s * 32 + g4 * 8);
+                    }
+                    qf[qs][s] = v * sc;
                 }
-                qf[qs][s] = v * sc;
             }
-        }
+        };
 
         f32x4 ot[DV][QS];
         float m_run[QS];
@@ -251,10 +255,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
         // maximum is raised (after the first tiles: almost never): the start vector of the score
         // products, four copies of -m (zero while the row has no maximum yet), and the amount a
         // tile's maximum has to exceed before the row's is raised (-inf until then, 8 binades after).
-        // Only the plain form keeps them (there they save a dozen vector instructions per tile); with
+        // Only the forms without a mask keep them (there they save a dozen vector instructions per tile); with
         // mask handling they would be ten registers too many for three waves per SIMD, and the masked
         // forms work both out from m_run in every tile.
-        constexpr bool KEEP_START = PLAIN;
+        constexpr bool KEEP_START = !MASK && !SHAREDQK;
         f32x4 neg_m4[QS];
         float raise_over[QS];
         f32x4 l_acc[QS]; // row sums of P, accumulated by the matrix unit (all 16 rows of the tile equal)
@@ -268,8 +272,6 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
             for (int d = 0; d < DV; d++)
                 ot[d][qs] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        const bool mask_vec = a.mask && ((a.seq_len & 3) == 0) &&
-                              ((reinterpret_cast<uintptr_t>(a.mask) & 7u) == 0);
         const bool qk_vec = SHAREDQK && ((a.seq_len & 3) == 0) &&
                             ((reinterpret_cast<uintptr_t>(a.QK) & 7u) == 0);
         const bool qk_vec16 = qk_vec && ((a.seq_len & 7) == 0) && ((reinterpret_cast<uintptr_t>(a.QK) & 15u) == 0);
@@ -384,40 +386,29 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
                           "a tile is a whole number of DMA instructions");
             f16 *ks = smem + buf * (KBUF + VBUF);
             f16 *vs = ks + KBUF;
-            if (PLAIN || kb + AT_KT <= len) { // (wave-uniform; always so in the plain form)
-                const char *kbase = reinterpret_cast<const char *>(a.K + (size_t)(row0 + kb) * a.ldq + qc0);
-                const char *vbase = reinterpret_cast<const char *>(a.V + (size_t)(row0 + kb) * a.ldv + vc0);
+            if (!PLAIN && __builtin_expect(kb + AT_KT > len, 0)) { // the last tile: rows that do not exist re-read the last one
 #pragma unroll
                 for (int j = 0; j < DMA_PW; j++) {
                     const int i = j * AT_WAVES + wave;
-                    if (DMA_NTOT % AT_WAVES != 0 && i >= DMA_NTOT)
-                        break;
                     const bool isv = i >= DMA_NK;
-                    const int ii = isv ? i - DMA_NK : i;
-                    // (kept opaque in place: otherwise the offsets are folded into 64-bit vector
-                    // addresses again, one 64-bit add per instruction and tile)
-                    asm("" : "+v"(dma_off[j]));
-                    load_lds16((isv ? vbase : kbase) + dma_off[j], (isv ? vs : ks) + ii * 512);
+                    const int p = (isv ? i - DMA_NK : i) * 1024 + lane * 16;
+                    const int row = p / (isv ? DMA_ROWBV : DMA_ROWBK);
+                    dma_off[j] -= (unsigned)(max(row - (len - 1 - kb), 0) * (isv ? a.ldv : a.ldq) * 2);
                 }
-                return;
             }
+            const char *kbase = reinterpret_cast<const char *>(a.K + (size_t)(row0 + kb) * a.ldq + qc0);
+            const char *vbase = reinterpret_cast<const char *>(a.V + (size_t)(row0 + kb) * a.ldv + vc0);
 #pragma unroll
-            for (int i0 = 0; i0 < DMA_NTOT; i0 += AT_WAVES) {
-                const int i = i0 + wave;
+            for (int j = 0; j < DMA_PW; j++) {
+                const int i = j * AT_WAVES + wave;
                 if (DMA_NTOT % AT_WAVES != 0 && i >= DMA_NTOT)
                     break;
                 const bool isv = i >= DMA_NK;
                 const int ii = isv ? i - DMA_NK : i;
-                const int p = ii * 1024 + lane * 16;
-                const int rowb = isv ? DMA_ROWBV : DMA_ROWBK;
-                const int row = p / rowb, cb = p - row * rowb;
-                const int rr = min(kb + row, len - 1);
-                int col = cb < (isv ? HD : HDK) * 2 ? (cb >> 1) : 0;
-                if (VWIN && isv)
-                    col = min(cb >> 1, a.ldv - 8 - vc0);
-                const f16 *src = isv ? a.V + (size_t)(row0 + rr) * a.ldv + vc0 + col
-                                     : a.K + (size_t)(row0 + rr) * a.ldq + qc0 + col;
-                load_lds16(src, (isv ? vs : ks) + ii * 512);
+                // (kept opaque in place: otherwise the offsets are folded into 64-bit vector
+                // addresses again, one 64-bit add per instruction and tile)
+                asm("" : "+v"(dma_off[j]));
+                load_lds16((isv ? vbase : kbase) + dma_off[j], (isv ? vs : ks) + ii * 512);
             }
         };
         typedef std::integral_constant<bool, true> yes_t;
@@ -437,105 +428,77 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
                 c = (a.v_col_id ? a.v_col_id[vc0 + tid] : vc0 + tid) - h * HD;
             wcol[tid] = (c >= 0 && c < HD) ? c : -1;
         }
-        if (DMA) {
-            dma_tile(0, 0);
-            __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
-        } else {
-            if (AT_KT <= len)
-                load_tile(0, yes_t{});
-            else
-                load_tile(0, no_t{});
-            store_tile(0);
-        }
-        __syncthreads();
-
         // Does key tile t hold a non-zero mask element for this wave's query
         // rows?  (wave-uniform; all-zero tiles skip the mask loads and adds,
         // which changes no result bit: s + 0 == s.)  The summary words of the
         // first 64 tiles are fetched once, up front; longer sequences do not
         // use the summary.
         unsigned mw0 = 0xFFFFFFFFu, mw1 = 0xFFFFFFFFu;
-        if (a.msum && a.msum_words <= 2) {
-            unsigned w0 = 0, w1 = 0;
+        if (MASK && a.msum && a.msum_words <= 2) {
+            typedef const __attribute__((address_space(4))) unsigned *UConst; // (scalar loads)
+            const UConst ms = (UConst)a.msum;
+            mw0 = mw1 = 0;
 #pragma unroll
             for (int qs = 0; qs < QS; qs++) {
                 const int g = (q0 + (wave * QS + qs) * 16) >> 4;
                 if (g * 16 < a.seq_len) {
-                    w0 |= a.msum[(size_t)g * a.msum_words];
+                    mw0 |= ms[g * a.msum_words];
                     if (a.msum_words > 1)
-                        w1 |= a.msum[(size_t)g * a.msum_words + 1];
+                        mw1 |= ms[g * a.msum_words + 1];
                 }
             }
-            mw0 = __builtin_amdgcn_readfirstlane(w0);
-            mw1 = __builtin_amdgcn_readfirstlane(w1);
         }
         auto tile_has_mask = [&](int t) -> bool {
             return t >= 64 || (((t < 32 ? mw0 : mw1) >> (t & 31)) & 1u);
         };
 
-        // Additive mask values of one tile, in the score layout.  They are
-        // requested one tile ahead (right after the previous tile consumed
+        // Additive mask values of one tile.  They are requested one tile ahead (right after the previous tile consumed
         // its own) so the L2 latency is covered by a whole tile of work.
+        // Whole mask rows of a tile are 128 bytes: a lane (row, g) takes keys 16g .. 16g+15 as two 16-byte loads, so
+        // that the four lanes of a row read each of its lines once; the score layout wants keys 16k + 4g .. +3 for
+        // k = 0..3, i.e. the 4 x 4 transpose of the 8-byte pieces across the row's four lanes, done with row swaps
+        // when the values are consumed.  Four 8-byte loads per lane, the direct form, touch every line four times from
+        // four requests: with twelve waves per CU the lines do not survive in L1 between them, and a dense mask then
+        // costs more L2 traffic than K and V together.
+        // Rows of any length come this way: the loads need no more than the 2-byte alignment of a half, and what they
+        // read behind a row's end belongs to keys that do not exist (their scores become -inf).  Only the last few
+        // elements of the array, where a whole load would pass its end, are fetched one by one.  (Element loads for
+        // every row that is not 8-byte aligned or that ends inside the tile were sixteen dependent round trips: 2 x
+        // 1021 rows, dense mask, 60 us against 23 for 2 x 1024.)
         f16x4 mk[QS][4];
-        // Whole mask rows of a tile are 128 bytes, one cache line.  Where rows are 16-byte aligned a full tile's
-        // values come as two 16-byte loads per lane that together read each of the 16 lines once (lane (row, g)
-        // takes keys 16g .. 16g+15); the score layout wants keys 16k + 4g .. +3 for k = 0..3, i.e. the 4 x 4
-        // transpose of the 8-byte pieces across the row's four lanes, done with row swaps when the values are
-        // consumed (mk_blocked says that it is still due).  Four 8-byte loads per lane, the direct form, touch
-        // every line four times from four requests: with twelve waves per CU the lines do not survive in L1
-        // between them, and a dense mask then costs more L2 traffic than K and V together.
-        const bool mask_vec16 = mask_vec && ((a.seq_len & 7) == 0) && ((reinterpret_cast<uintptr_t>(a.mask) & 15u) == 0);
-        bool mk_blocked = false;
-        auto load_mask = [&](int kb, auto fast_c) {
-            constexpr bool FAST = decltype(fast_c)::value;
-            mk_blocked = FAST && mask_vec16;
-            if (FAST && mask_vec16) {
+        const f16 *mrow[QS]; // the lane's first key
+        if (MASK && a.mask) {
 #pragma unroll
-                for (int qs = 0; qs < QS; qs++) {
-                    const int q = q0 + (wave * QS + qs) * 16 + c16;
-                    const f16 *mrow = a.mask + (size_t)q * a.seq_len + kb + g4 * 16;
-                    const f16x8 l0 = *reinterpret_cast<const f16x8 *>(mrow);
-                    const f16x8 l1 = *reinterpret_cast<const f16x8 *>(mrow + 8);
-                    mk[qs][0] = f16x4{l0[0], l0[1], l0[2], l0[3]};
-                    mk[qs][1] = f16x4{l0[4], l0[5], l0[6], l0[7]};
-                    mk[qs][2] = f16x4{l1[0], l1[1], l1[2], l1[3]};
-                    mk[qs][3] = f16x4{l1[4], l1[5], l1[6], l1[7]};
-                }
-                return;
-            }
+            for (int qs = 0; qs < QS; qs++)
+                mrow[qs] = a.mask + (size_t)min(q0 + (wave * QS + qs) * 16 + c16, a.seq_len - 1) * a.seq_len + g4 * 16;
+        }
+        auto load_mask = [&](int kb) {
 #pragma unroll
             for (int qs = 0; qs < QS; qs++) {
-                const int q = q0 + (wave * QS + qs) * 16 + c16;
-#pragma unroll
-                for (int ksub = 0; ksub < 4; ksub++) {
-                    const int key = kb + ksub * 16 + g4 * 4;
-                    const f16 *mrow = a.mask + (size_t)q * a.seq_len + key;
-                    f16x4 v = f16x4{0, 0, 0, 0};
-                    if (FAST) {
-                        v = *reinterpret_cast<const f16x4 *>(mrow);
-                    } else if (q < len) {
-                        if (mask_vec && key + 3 < len) {
-                            v = *reinterpret_cast<const f16x4 *>(mrow);
-                        } else {
-#pragma unroll
-                            for (int r = 0; r < 4; r++)
-                                if (key + r < len)
-                                    v[r] = mrow[r];
-                        }
-                    }
-                    mk[qs][ksub] = v;
+                f16x8 l[2];
+                const f16 *m = mrow[qs] + kb;
+                if (kb + AT_KT <= a.seq_len) { // (wave-uniform)
+                    l[0] = *reinterpret_cast<const f16x8_u *>(m);
+                    l[1] = *reinterpret_cast<const f16x8_u *>(m + 8);
+                } else {
+                    const int left = (int)min(a.mask + (size_t)a.seq_len * a.seq_len - m, (ptrdiff_t)16);
+                    l[0] = load8_guard(m, 0, left);
+                    l[1] = load8_guard(m, 8, left);
                 }
+                mk[qs][0] = f16x4{l[0][0], l[0][1], l[0][2], l[0][3]};
+                mk[qs][1] = f16x4{l[0][4], l[0][5], l[0][6], l[0][7]};
+                mk[qs][2] = f16x4{l[1][0], l[1][1], l[1][2], l[1][3]};
+                mk[qs][3] = f16x4{l[1][4], l[1][5], l[1][6], l[1][7]};
             }
         };
-        const bool vec_ok = (!a.mask || mask_vec) && (!SHAREDQK || qk_vec);
-        auto fast_tile = [&](int kb) { return kb + AT_KT <= len && wave_rows_ok && vec_ok; };
-        bool has_mask_cur = !PLAIN && !wave_idle && a.mask && tile_has_mask(0);
-        if (has_mask_cur) {
-            if (fast_tile(0))
-                load_mask(0, yes_t{});
-            else
-                load_mask(0, no_t{});
-        }
+        // (query rows at or beyond len have no Q, and whatever they sum up is never stored; only stored scores are read)
+        auto fast_tile = [&](int kb) { return kb + AT_KT <= len && (!SHAREDQK || (wave_rows_ok && qk_vec)); };
+        bool has_mask_cur = false;
+        auto mask_ahead = [&] { // the first tile's
+            has_mask_cur = MASK && !wave_idle && a.mask && tile_has_mask(0);
+            if (has_mask_cur)
+                load_mask(0);
+        };
 
         // One key tile.  FAST: all 64 keys and all of the wave's query rows are
         // valid and the vector paths apply, so the body has no per-lane
@@ -633,7 +596,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
             // more than 8 binades (P then stays <= 256, exact enough in half),
             // so after the first tiles the accumulator rescale is skipped.
             f16x8 pf[QS][2];
-            if (MASKED && mk_blocked) { // the line-wise loads hold key blocks per lane: into the score layout
+            if (MASKED) { // the loads hold key blocks per lane: into the score layout
 #pragma unroll
                 for (int qs = 0; qs < QS; qs++)
                     transpose_pieces_4x4(mk[qs]);
@@ -654,14 +617,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
                             // form takes the half operand directly, no conversion)
                             st[ksub][qs][r] = __builtin_fmaf((float)mk[qs][ksub][r], one, st[ksub][qs][r]);
             }
-            if (!PLAIN && a.mask) { // next tile's mask
+            if (MASK && a.mask) { // next tile's mask
                 has_mask_next = kb + AT_KT < len && tile_has_mask((kb + AT_KT) / AT_KT);
-                if (has_mask_next) {
-                    if (fast_tile(kb + AT_KT))
-                        load_mask(kb + AT_KT, yes_t{});
-                    else
-                        load_mask(kb + AT_KT, no_t{});
-                }
+                if (has_mask_next)
+                    load_mask(kb + AT_KT);
             }
             // the lane's part of each row maximum (of s - m_ref); the row's other three
             // parts only matter when some row of the wave has to raise its maximum
@@ -687,11 +646,12 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
                 // does this tile add anything to the row?  Not if every score is 160 binades or more under a
                 // maximum the row already has: every exp2 is then exactly zero in fp32 (so is P, and the sums
                 // and the output do not change).
-                live = live || m_run[qs] == -INFINITY || !(mx * ls < -160.0f);
+                if (MASK)
+                    live = live || m_run[qs] == -INFINITY || !(mx * ls < -160.0f);
             }
             // A tile that is dead for every row of the wave - the keys behind a padding mask - ends here: no
             // exponentials, no second product (wave-uniform; same bits as going through with P = 0).
-            if (!PLAIN && __builtin_amdgcn_ballot_w64(live) == 0)
+            if (MASK && __builtin_amdgcn_ballot_w64(live) == 0)
                 return;
 #pragma unroll
             for (int qs = 0; qs < QS; qs++) {
@@ -800,7 +760,35 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
             __builtin_amdgcn_s_setprio(0);
         };
 
-        for (int t = 0; t < nt; t++) {
+        // Everything the first tiles need is requested before anything is waited for: K and V of the first tile, Q, the
+        // first mask values, K and V of the second tile (whose wait is the first tile's end).
+        if (DMA) {
+            dma_tile(0, 0);
+            load_q();
+            mask_ahead();
+            if (nt > 1) {
+                dma_tile(AT_KT, 1);
+                constexpr int BEHIND = DMA_NTOT / AT_WAVES; // at least so many requests of this wave are the second tile's
+                __builtin_amdgcn_s_waitcnt(0x0F70 | (BEHIND & 15) | (BEHIND >> 4 << 14)); // vmcnt(BEHIND)
+            } else {
+                __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+            }
+        } else {
+            if (AT_KT <= len)
+                load_tile(0, yes_t{});
+            else
+                load_tile(0, no_t{});
+            load_q();
+            mask_ahead();
+            store_tile(0);
+        }
+        __syncthreads();
+
+        // Without a mask: the full tiles in a loop of their own, the last one behind it (the bounds as a branch inside
+        // the loop cost 0.15 us a tile: 2 x 1024 rows with lengths 15.9 us, without 13.4).
+        constexpr bool PEEL = DMA && !MASK && !SHAREDQK && !PLAIN;
+        const int nloop = PEEL ? len / AT_KT : nt;
+        for (int t = 0; t < nloop; t++) {
             const int kb = t * AT_KT;
             const f16 *ks = smem + (t & 1) * (KBUF + VBUF);
             const f16 *vt = ks + KBUF;
@@ -810,8 +798,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
             // consumed: by DMA straight away, or through registers that are
             // stored after the tile body
             if (more) {
-                if (DMA)
+                if (DMA && t > 0) // (the second tile is on its way)
                     dma_tile(kb + AT_KT, (t + 1) & 1);
+                else if (DMA)
+                    ;
                 else if (kb + 2 * AT_KT <= len)
                     load_tile(kb + AT_KT, yes_t{});
                 else
@@ -819,6 +809,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
             }
             if constexpr (PLAIN)
                 tile_body(kb, ks, vt, true, false);
+            else if (PEEL) {
+                if (!wave_idle)
+                    tile_body(kb, ks, vt, true, false);
+            }
             else if (!wave_idle)
                 tile_body(kb, ks, vt, fast_tile(kb), has_mask_cur);
             has_mask_cur = has_mask_next;
@@ -828,6 +822,12 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
                 else
                     store_tile((t + 1) & 1);
             }
+            __syncthreads();
+        }
+        if (PEEL && nloop < nt) {
+            const f16 *ks = smem + (nloop & 1) * (KBUF + VBUF);
+            if (!wave_idle)
+                tile_body(nloop * AT_KT, ks, ks + KBUF, false, false);
             __syncthreads();
         }
 

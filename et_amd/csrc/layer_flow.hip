@@ -263,7 +263,7 @@ __device__ __forceinline__ void lf_panel(const LfArgs &a, const f16 *X, f16 *xs,
     }
 }
 
-template <int HD>
+template <int HD, bool MASK>
 __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lf_smem[];
     unsigned *const bc = reinterpret_cast<unsigned *>(lf_smem + a.misc);
@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
         const int row1 = a.at.cu_seqlens ? a.at.cu_seqlens[b + 1] : row0 + a.at.seq_len;
         const int p0 = row0 / LF_BM, p1 = (row1 - 1) / LF_BM;
         lf_wait(a, wave, c_qkv + p0, p1 - p0 + 1, (unsigned)a.g_qkv);
-        attention_block<HD, 1, LF_WAVES, false, false, false, HD, false, true>(a.at, b, h, qb);
+        attention_block<HD, 1, LF_WAVES, false, false, false, HD, false, true, MASK>(a.at, b, h, qb);
         (void)lf_signal(a, c_at + ib);
     } else {
         // ---- second feed-forward linear; whoever completes a panel runs its LayerNorm
@@ -635,9 +635,8 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
     hipStream_t st = static_cast<hipStream_t>(stream);
     static_assert(attn_lds_bytes<64, 1, LF_WAVES, false>() + 64 <= 64 * 1024 && LF_BM * (1024 + 16) * 2 + 64 <= 64 * 1024,
                   "no opt-in for dynamic LDS needed");
-    if (wide)
-        hipLaunchKernelGGL(layer_flow_kernel<64>, dim3(total), dim3(LF_WAVES * 64), lds, st, a);
-    else
-        hipLaunchKernelGGL(layer_flow_kernel<32>, dim3(total), dim3(LF_WAVES * 64), lds, st, a);
+    const auto kern = wide ? (a.at.mask ? layer_flow_kernel<64, true> : layer_flow_kernel<64, false>)
+                           : (a.at.mask ? layer_flow_kernel<32, true> : layer_flow_kernel<32, false>);
+    hipLaunchKernelGGL(kern, dim3(total), dim3(LF_WAVES * 64), lds, st, a);
     return launch_status("layer in one launch");
 }

@@ -1205,3 +1205,25 @@ def test_tile_linear_orders_and_forms(K, M, Ns, Kd):
     finally:
         for key, value in ((b"tile_order", 1), (b"tile_bm64", 1), (b"tile_ipw", 0)):
             lib().et_tuning_set(key, value)
+
+
+@pytest.mark.parametrize("S,B,hd", [(1, 2, 64), (15, 1, 32), (63, 3, 64), (65, 2, 128), (127, 2, 64), (129, 24, 64),
+                                    (191, 1, 64), (250, 5, 64)])
+def test_otf_attention_ragged_rows(K, S, B, hd):
+    """sequence lengths around the tiles' edges: without a mask (full tiles and the last one apart), with lengths, and
+    with a mask whose rows start at any 2-byte address, its last element next to other data"""
+    r = rng(610 + S)
+    H = 12 if S == 129 else 4
+    d = H * hd
+    Q, Kk, V = (randn_h(r, (B * S, d)) for _ in range(3))
+    mask = randn_h(r, (S, S))
+    lens = r.integers(1, S + 1, size=B).astype(np.int32)
+    buf = np.full(S * S + 2, np.nan, np.float16)
+    buf[1:-1] = mask.ravel()
+    md = dev(buf)[1:-1].view(S, S)
+    pick = np.unique([0, B // 2, B - 1])
+    for m, ml, n in ((None, None, None), (None, None, lens), (mask, md, None), (mask, md, lens)):
+        got = host(K.OTF_attention(dev(Q), dev(Kk), dev(V), ml, S, H, B, None if n is None else dev(n), LOG2E))
+        rows = np.concatenate([np.arange(b * S, (b + 1) * S) for b in pick])
+        want = orc.otf_attention(Q[rows], Kk[rows], V[rows], m, S, H, pick.size, None if n is None else n[pick], LOG2E, f64=True)
+        check_close(got[rows], want, max_abs=5e-3, mean_rel=1e-3, what=f"mask {m is not None}, lens {n is not None}")
