@@ -26,7 +26,7 @@
 //
 // Kernels in this file: tile_linear_resident_kernel (K in one panel: persistent
 // workgroups, 32- or 64-row panels, optional LayerNorm epilogue),
-// tile_linear_plan_kernel (K in chunks), tile_linear_chunked_ln_kernel (K in
+// tile_linear_plan_kernel (K in chunks), tile_linear_chunked_kernel (K in
 // chunks + LayerNorm, double-buffered panels with a fetching wave),
 // tile_ffn_fused_kernel (feed-forward block / whole layer tail in one launch,
 // hidden activations in LDS), tile_linear_generic_kernel (raw and dense input).
@@ -53,6 +53,7 @@ void set_tail_spin(int v);
 void set_dense_form(int v);
 // tile_rows.hip
 bool tile_rows_fits(int K);
+double tile_rows_estimate(int M, int K, int nbr_max, int nlin, double pairs, double w_mb);
 int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *X, int M, int K, double pairs, bool gelu,
                      bool raw, hipStream_t st);
 void set_flow_rows(int v);
@@ -993,13 +994,14 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
 }
 
 // ---------------------------------------------------------------------------
-// Chunked fused kernel: linear + skip + LayerNorm for K beyond one LDS panel
-// (FFN2 of BERT-base, K = 3072, N = 768).  One workgroup per row panel holds
-// whole rows: twelve computing waves of NB block-rows each and a thirteenth
-// wave that does nothing but fetch.  K is walked in chunks through two LDS
-// panel buffers; the fetching wave requests chunk c+1 (global -> LDS DMA) as
+// Chunked kernel with fetching waves: K beyond one LDS panel (second
+// feed-forward linear, K = 3072, N = 768).  Twelve computing waves of NB
+// block-rows each and four waves that do nothing but fetch (one alone takes
+// 2.5 us a chunk); LN: the workgroup holds whole rows (one per row panel), and
+// skip connection and LayerNorm follow.  K is walked in chunks through two LDS
+// panel buffers; the fetching waves request chunk c+1 (global -> LDS DMA) as
 // soon as the computing waves have left chunk c-1, so the fetch runs under
-// chunk c's MFMAs.  It has to be a wave of its own: loads return in order
+// chunk c's MFMAs.  They have to be waves of their own: loads return in order
 // within a wave, so a panel request in a computing wave's queue would hold
 // back every weight pair requested after it.  One LDS-only barrier per chunk
 // hands over both "chunk c has landed" and "buffer (c+1)&1 is free".  The
@@ -1007,18 +1009,17 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
 // restarted per chunk with the first pairs requested before the barrier.
 // ---------------------------------------------------------------------------
 constexpr int TL_CWAVES = 12;
-constexpr int TL_CTHREADS = (TL_CWAVES + 1) * 64;
+constexpr int TL_FWAVES = 4; // fetching waves, eight panel rows each
+constexpr int TL_CTHREADS = (TL_CWAVES + TL_FWAVES) * 64;
 
-template <int NB>
-__global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_ln_kernel(const TlArgs a) {
+template <int NB, bool GELU, bool LN>
+__global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_kernel(const TlArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
     f16 *xs = reinterpret_cast<f16 *>(tl_smem);
-    const int rp = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-    if (rp >= a.nwg)
-        return;
     TlCtx x;
-    x.lin = 0;
-    x.cg = 0;
+    int rp;
+    if (!tl_place(a, rp, x.lin, x.cg))
+        return;
     x.m0 = rp * TL_BM;
     x.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     x.lane = threadIdx.x & 63;
@@ -1027,25 +1028,27 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_ln_kernel(con
     x.khalf8 = (x.g4 & 1) * 8;
     x.hi = x.lane >> 5;
     x.ldx = a.KC + ((a.KC & 31) ? 0 : TL_PAD);
-    x.bn_wg = 0;
-    x.bn0 = x.wave * NB;
+    const int lin = x.lin;
+    x.bn_wg = x.cg * (TL_CWAVES * NB);
+    x.bn0 = x.bn_wg + x.wave * NB;
     x.ld_r = x.ld_c = 0;
     const int lane = x.lane;
     const int pbuf = TL_BM * x.ldx; // halves per panel buffer
     f16 *const stage0 = xs + 2 * pbuf;
-    f16 *const Yp = a.Y[0];
-    const int N = a.N[0];
+    f16 *const Yp = TL_SEL(Y);
+    const int N = TL_SEL(N);
     const int nbr = N >> 4;
 
-    if (x.wave == TL_CWAVES) {
-        // ---- the fetching wave ----
+    if (x.wave >= TL_CWAVES) {
+        // ---- the fetching waves ----
+        const int row0 = (x.wave - TL_CWAVES) * (TL_BM / TL_FWAVES);
 #define TL_FETCH(c_)                                                                              \
     {                                                                                             \
         const int pk0 = (c_) * a.KC;                                                              \
         const int pcpr = min(a.KC, a.K - pk0) >> 3; /* 16-byte pieces per row, <= 124 */          \
         f16 *dst = xs + ((c_) & 1) * pbuf;                                                        \
-        const int nrow = min(TL_BM, a.M - x.m0);                                                  \
-        for (int row = 0; row < nrow; row++) {                                                    \
+        const int row1 = min(row0 + TL_BM / TL_FWAVES, a.M - x.m0);                               \
+        for (int row = row0; row < row1; row++) {                                                 \
             const f16 *src = a.X + (size_t)(x.m0 + row) * a.K + pk0;                              \
             if (lane < pcpr)                                                                      \
                 load_lds16(src + lane * 8, dst + row * x.ldx);                                    \
@@ -1067,8 +1070,9 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_ln_kernel(con
 #undef TL_FETCH
     } else {
         // ---- the computing waves ----
-        const int *const cptr = a.cptr[0];
+        const int *const cptr = TL_SEL(cptr);
         const int hi = x.hi;
+        const f16 *const bias = TL_SEL(bias);
         f32x4 acc[NB][2];
         f16x4 b4[NB];
 #pragma unroll
@@ -1077,11 +1081,11 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_ln_kernel(con
             acc[j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
             b4[j] = f16x4{0, 0, 0, 0};
             if (x.bn0 + j < nbr)
-                b4[j] = *reinterpret_cast<const f16x4 *>(a.bias[0] + (x.bn0 + j) * 16 + x.g4 * 4);
+                b4[j] = *reinterpret_cast<const f16x4 *>(bias + (x.bn0 + j) * 16 + x.g4 * 4);
         }
         const int xrow16 = 16 * x.ldx * 2; // bytes between the two 16-row subtiles
-        const f16 *const data = a.data[0];
-        const int *const poff = a.row_offset[0];
+        const f16 *const data = TL_SEL(data);
+        const int *const poff = TL_SEL(row_offset);
         const unsigned lane_w = hi * 256 + x.c16 * 16 + x.khalf8; // lane's halves inside a 1 KB tile pair
         // pair-index boundaries of the wave's block-rows in the current chunk
         // (see tile_linear_plan_kernel); the next chunk's are requested a chunk ahead
@@ -1106,12 +1110,14 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_ln_kernel(con
             bvec = bvec_n;
         }
         f16 *stage = stage0 + x.wave * tl_wave_stage_halves<NB>();
-        tl_epilogue_wave<NB, false, false>(a, x, stage, Yp, N, nbr, acc, b4);
+        tl_epilogue_wave<NB, GELU, !LN>(a, x, stage, Yp, N, nbr, acc, b4);
     }
-    TlLnOperands<NB, TL_CWAVES, TL_CWAVES + 1> lnop;
-    tl_ln_fetch(lnop, a, x.wave, lane, x.m0, N);
-    __syncthreads(); // every computing wave's part of the rows is staged
-    tl_ln_rows(lnop, a, stage0, x.wave, lane, x.m0, Yp, N);
+    if constexpr (LN) {
+        TlLnOperands<NB, TL_CWAVES, TL_CWAVES + TL_FWAVES> lnop;
+        tl_ln_fetch(lnop, a, x.wave, lane, x.m0, N);
+        __syncthreads(); // every computing wave's part of the rows is staged
+        tl_ln_rows(lnop, a, stage0, x.wave, lane, x.m0, Yp, N);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1576,13 +1582,22 @@ static int ln_block_rows(int nbr) {
 
 template <int NB>
 static int launch_chunked_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
-    constexpr auto k = &tile_linear_chunked_ln_kernel<NB>;
+    constexpr auto k = &tile_linear_chunked_kernel<NB, false, true>;
     ET_HIP(allow_lds<k>(lds));
     hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, a);
     return launch_status("tile_linear+LayerNorm (chunked) launch");
 }
 
+template <int NB, bool GELU>
+static int launch_chunked_inst(const TlArgs &a, size_t lds, hipStream_t st) {
+    constexpr auto k = &tile_linear_chunked_kernel<NB, GELU, false>;
+    ET_HIP(allow_lds<k>(lds));
+    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, a);
+    return launch_status("tile_linear (chunked) launch");
+}
+
 static int g_tile_ln_chunked = 1;
+static int g_tile_chunked = -1; // et_tuning_set("tile_chunked")
 static int g_tile_fuse_ffn = 2; // et_tuning_set("tile_fuse_ffn"): 1 feed-forward block, 2 whole layer tail
 
 // LDS bytes of the fused feed-forward kernel: X panel, two hidden buffers (the
@@ -1706,14 +1721,9 @@ static int g_tile_nb = 0;
 static int g_tile_min_wgs = 512;
 static int g_tile_ipw = 0;
 static int g_tile_fuse_ln = 1;
-static int g_tile_ln_min_panels = 96;
-// the layer tail in one launch: from fewer panels than the linear + LayerNorm kernels (measured on
-// BERT-base at 80 %: one launch 42 us for any count below one per CU, step by step 37 / 43 / 54 us
-// at 52 / 80 / 95 panels)
-constexpr int TL_TAIL_MIN_PANELS = 72;
-static int g_tile_tail_min_panels = TL_TAIL_MIN_PANELS;
+static int g_tile_min_panels = 0; // fewest panels of the fused linear + LayerNorm and layer tail kernels, 0 = automatic
 // the layer tail's choice is forced (a layer then runs its steps as separate launches)
-bool tail_tuned() { return g_tile_tail_min_panels != TL_TAIL_MIN_PANELS || g_tile_fuse_ffn != 2; }
+bool tail_tuned() { return g_tile_min_panels != 0 || g_tile_fuse_ffn != 2; }
 
 // Block-rows per wave.  Measured on the BERT-base shapes (rows 4096..8192):
 // three block-rows per wave is the best trade between panel re-reads (fewer
@@ -1754,6 +1764,10 @@ bool tl_order(double x_bytes, double w_bytes, long panels, long groups, double x
     if (g_tile_order != 1)
         return g_tile_order == 2;
     return x_bytes <= x_most && std::min(groups, 8L) * x_bytes + w_bytes < x_bytes + std::min(panels, 8L) * w_bytes;
+}
+double tl_traffic_mb(double x_mb, double w_mb, long panels, long groups, double x_most) {
+    return tl_order(x_mb, w_mb, panels, groups, x_most) ? std::min(groups, 8L) * x_mb + w_mb
+                                                        : x_mb + std::min(panels, 8L) * w_mb;
 }
 
 // The forms of the single-panel kernel and the choice among them.  An item is a panel of 32 or 64 rows by waves x nb
@@ -1816,14 +1830,71 @@ static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, 
                 continue;
             const long groups = per_panel / d, nwg = panels * groups;
             const long on_cu = (nwg + cus - 1) / cus, rounds = (on_cu + slots - 1) / slots;
-            const bool by_group = tl_order(1e6 * x_mb, 1e6 * w_mb, panels, groups, 1.75e6);
-            const double mb = by_group ? std::min(groups, 8L) * x_mb + w_mb : x_mb + std::min(panels, 8L) * w_mb;
+            const double mb = tl_traffic_mb(x_mb, w_mb, panels, groups, 1.75);
+            const bool by_group = tl_order(x_mb, w_mb, panels, groups, 1.75);
             const double us = fixed + c.traffic * mb + c.traffic_over * std::max(0.0, mb - 12.0) +
                               (double)rounds * (c.round + d * per_item) +
                               (double)on_cu * (c.panel * f.rows * K + d * cu_item) + c.wg * (double)nwg;
             if (!best.form || us < best.us)
                 best = TlChoice{&f, d, ncg, by_group, lds, us};
         }
+    }
+    return best;
+}
+
+// Plans with K in several chunks: the kernel with the least estimated time (us).  Whole rows (tile_rows.hip) stream W
+// once per 16 rows and have no chain of chunks: few rows.  The plan kernel fetches, waits and multiplies chunk by
+// chunk, two workgroups of 8 nb block-rows per CU.  The kernel with fetching waves takes in the next chunk meanwhile, one
+// workgroup of 12 nb block-rows per CU: where its workgroups just fit one round it is up to a third shorter (3300 rows
+// 3072 -> 768, 80 %: 18.9 -> 13.4 us; 1536 rows, 50 %: 16.7 -> 14.1; 2300 rows 4096 -> 1024, 50 %: 48.8 -> 26.6).
+// Terms: launch, rounds of workgroups and their chunks, the stream of a wave's pairs, the work of the busiest CU, and
+// the megabytes that the L2s take in; fitted like the single-panel forms to 1600 launches (2048 -> 512, 3072 -> 768,
+// 4096 -> 1024, 0 to 90 % pruned, 48 to 16384 rows): 5 to 6 % off in the mean, the choice 0.2 % behind the fastest
+// kernel, 9 % at most (the rule before: 10.9 %).
+enum { TL_BY_ROWS = -1, TL_BY_PLAN = 0 }; // or 1 .. 4: fetching waves, that many block-rows per computing wave
+static double estimate_plan_kernel(int M, double pairs, double x_mb, double w_mb, int nchunk, int nbr_max, int nlin, long cus) {
+    const long panels = (M + TL_BM - 1) / TL_BM;
+    const int nb = choose_nb((int)panels, nbr_max, nlin), ncg = (nbr_max + TL_WAVES * nb - 1) / (TL_WAVES * nb) * nlin;
+    const long wgs = panels * ncg, rounds = (wgs + 2 * cus - 1) / (2 * cus), on_cu = (wgs + cus - 1) / cus;
+    return 1.367 + rounds * (0.9615 * nchunk + 0.0867 * nb * pairs) +
+           on_cu * (0.4349 * nchunk + 0.01745 * nb * pairs + 0.6037 * nb) + 0.0673 * tl_traffic_mb(x_mb, w_mb, panels, ncg, 1.75);
+}
+static double estimate_chunked(int M, double pairs, double x_mb, double w_mb, int nchunk, int nbr_max, int nlin, int nb, long cus) {
+    const long panels = (M + TL_BM - 1) / TL_BM;
+    const int ncg = (nbr_max + TL_CWAVES * nb - 1) / (TL_CWAVES * nb) * nlin;
+    const long wgs = panels * ncg;
+    const double rounds = (double)((wgs + cus - 1) / cus), fill = std::min(1.0, (double)wgs / cus);
+    return 1.775 + rounds * (1.997 + (0.378 + 0.233 * nb) * nchunk + (0.0397 + 0.0140 * fill) * nb * pairs +
+                             0.00429 * std::min(TL_CWAVES * nb, nbr_max) * pairs) +
+           0.0980 * tl_traffic_mb(x_mb, w_mb, panels, ncg, 1.75);
+}
+static int choose_chunked(const TlProblem *probs, int nlin, int M, int K, int nchunk, int nbr_max, double *us) {
+    const long cus = std::max(et_device_cu_count(), 1);
+    double pairs = 0.0, w_mb = 0.0;
+    for (int i = 0; i < nlin; i++) {
+        const double p = 0.5 * probs[i].ntile / probs[i].nbr;
+        pairs += p / nlin;
+        w_mb += p * probs[i].nbr * 1024e-6;
+    }
+    const double x_mb = 2e-6 * M * K;
+    int best = TL_BY_PLAN;
+    *us = estimate_plan_kernel(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, cus);
+    auto take = [&](int which, double t) {
+        if (t < *us) {
+            *us = t;
+            best = which;
+        }
+    };
+    if (g_tile_chunked < 0)
+        for (int nb = 1; nb <= 4; nb++)
+            take(nb, estimate_chunked(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, nb, cus));
+    if (g_tile_chunked > 0)
+        best = g_tile_chunked;
+    if (tile_rows_fits(K)) {
+        if (g_tile_rows_most >= 0)
+            best = M <= g_tile_rows_most ? TL_BY_ROWS : best;
+        else if (g_tile_chunked <= 0)
+            take(TL_BY_ROWS, tile_rows_estimate(M, K, nbr_max, nlin, pairs, w_mb));
     }
     return best;
 }
@@ -1858,17 +1929,21 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
     a.K = K;
     a.KC = KC;
     a.nchunk = nchunk;
-    // Whole rows in LDS (tile_rows.hip): plans with K in several chunks, and the caller's own tile_mat.
-    // Plans: the estimated time of both, in microseconds.  Whole rows: W is streamed once per 16 rows, 5.5 us and 16.5
-    // MB per us.  Chunks: a round of workgroups is a chain of a fetch and a stream per chunk, up to 20 % slower when
-    // all slots are taken.  Both fit 20 measured launches (3072 -> 768 and 4096 -> 1024, 0 / 50 / 80 % pruned, 340 to
-    // 8192 rows) within 15 %; the crossovers are 340 .. 600 rows dense, 1000 at 50 % and 2000 .. 4000 at 80 %.
-    // Raw lists: always where K is beyond the generic kernel's panel (it filters every list once per chunk: three to
-    // eight times slower), else while there is no more than one workgroup per CU (16 rows x 16 block-rows each).
-    if (g_tile_nb == 0 && tile_rows_fits(K) && mode != TL_DENSE && (mode != TL_PLAN || nchunk > 1)) {
-        const bool raw = mode != TL_PLAN;
+    // Whole rows in LDS (tile_rows.hip).  Plans: see choose_chunked.  Raw lists: always where K is beyond the generic
+    // kernel's panel (it filters every list once per chunk: three to eight times slower), else while there is no more
+    // than one workgroup per CU (16 rows x 16 block-rows each).
+    int which = TL_BY_PLAN;
+    if (mode == TL_PLAN && nchunk > 1) {
+        double us;
+        which = g_tile_nb == 0 ? choose_chunked(probs, nlin, M, K, nchunk, nbr_max, &us) : TL_BY_PLAN;
+    } else if (g_tile_nb == 0 && tile_rows_fits(K) && (mode == TL_RAW || mode == TL_FILTER)) {
         const long panels = (M + 15) / 16;
-        double pairs = 0.0, wmb = 0.0; // per block-row; megabytes of W
+        if (nchunk > 1 || panels * ((nbr_max + 15) / 16) <= std::max(et_device_cu_count(), 1))
+            which = TL_BY_ROWS;
+    }
+    if (which == TL_BY_ROWS) {
+        const bool raw = mode != TL_PLAN;
+        double pairs = 0.0; // per block-row
         LfLinear l[TL_MAX_LIN];
         f16 *Ys[TL_MAX_LIN];
         for (int i = 0; i < nlin; i++) {
@@ -1877,16 +1952,8 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
                             raw ? 1 : nchunk, raw ? 0 : KC * 2, probs[i].npair};
             Ys[i] = probs[i].Y;
             pairs += p / nlin;
-            wmb += p * probs[i].nbr * 1e-3;
         }
-        const int onb = choose_nb((M + TL_BM - 1) / TL_BM, nbr_max, nlin);
-        const double wgs = (double)((M + TL_BM - 1) / TL_BM) * ((nbr_max + TL_WAVES * onb - 1) / (TL_WAVES * onb)) * nlin / g_tile_min_wgs;
-        const double chunked = std::ceil(wgs) * (5.0 + 1.25 * nchunk + 0.11 * pairs * onb) * (1.0 + 0.2 * std::min(wgs, 1.0));
-        const bool take = raw ? nchunk > 1 || panels * ((nbr_max + 15) / 16) <= std::max(et_device_cu_count(), 1)
-                          : g_tile_rows_most >= 0 ? M <= g_tile_rows_most
-                                                  : 5.5 + (double)panels * wmb / 16.5 <= chunked;
-        if (take)
-            return tile_rows_launch(l, Ys, nlin, X, M, K, pairs, gelu, raw, st);
+        return tile_rows_launch(l, Ys, nlin, X, M, K, pairs, gelu, raw, st);
     }
     auto place = [&](int bm, int order) { // order: by_group, or -1 to be worked out
         const int panels = (M + bm - 1) / bm, per_rp = a.ncg * nlin;
@@ -1924,6 +1991,20 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         order = c.by_group;
     } else {
         const int nrp = (M + TL_BM - 1) / TL_BM;
+        if (which > 0) {
+            const int cnb = which;
+            a.ncg = (nbr_max + TL_CWAVES * cnb - 1) / (TL_CWAVES * cnb);
+            a.ipw = 1;
+            place(TL_BM, -1);
+            const size_t lds = 2 * (size_t)TL_BM * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16) +
+                               (size_t)TL_CWAVES * TL_BM * (16 * cnb + 8) * sizeof(f16);
+            switch (cnb) {
+            case 1: return gelu ? launch_chunked_inst<1, true>(a, lds, st) : launch_chunked_inst<1, false>(a, lds, st);
+            case 2: return gelu ? launch_chunked_inst<2, true>(a, lds, st) : launch_chunked_inst<2, false>(a, lds, st);
+            case 3: return gelu ? launch_chunked_inst<3, true>(a, lds, st) : launch_chunked_inst<3, false>(a, lds, st);
+            default: return gelu ? launch_chunked_inst<4, true>(a, lds, st) : launch_chunked_inst<4, false>(a, lds, st);
+            }
+        }
         nb = choose_nb(nrp, nbr_max, nlin);
         a.ncg = (nbr_max + TL_WAVES * nb - 1) / (TL_WAVES * nb);
         a.ipw = 1;
@@ -2009,6 +2090,10 @@ extern "C" int et_tuning_set(const char *key, int value) {
         et::g_tile_ipw = value;
         return ET_OK;
     }
+    if (key && !strcmp(key, "tile_chunked")) {
+        et::g_tile_chunked = value;
+        return ET_OK;
+    }
     if (key && !strcmp(key, "tile_order")) {
         et::g_tile_order = value;
         return ET_OK;
@@ -2038,8 +2123,7 @@ extern "C" int et_tuning_set(const char *key, int value) {
         return ET_OK;
     }
     if (key && !strcmp(key, "tile_ln_min_panels")) {
-        et::g_tile_ln_min_panels = value > 0 ? value : 96;
-        et::g_tile_tail_min_panels = value > 0 ? value : et::TL_TAIL_MIN_PANELS;
+        et::g_tile_min_panels = value > 0 ? value : 0;
         return ET_OK;
     }
     if (key && !strcmp(key, "tile_fuse_ln")) {
@@ -2098,19 +2182,16 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 
 // Plans of fully populated matrices: the dense product where it is estimated to be the shorter launch, from some hundred
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
-// tile: their time is that of the choice among the single-panel forms, or, for K in several chunks, a line through the
-// whole-rows and chunk kernels at 128 to 16384 rows (within 20 % where the two are close).
+// tile: their time is that of the choice among their forms.
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
     TlProblem probs[3];
     int Ns[3], nbr_max = 0;
-    double N = 0.0;
     for (int i = 0; i < n; i++) {
         if (!plans[i]->d_dense)
             return false;
         Ns[i] = plans[i]->out_feat;
-        N += Ns[i];
         probs[i].N = Ns[i];
         probs[i].nbr = Ns[i] / 16;
         probs[i].ntile = plans[i]->ntile;
@@ -2119,8 +2200,11 @@ static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool
     if (g_plan_dense == 2)
         return true;
     const int K = plans[0]->in_feat;
-    const double tiles = plans[0]->nchunk > 1 ? 10.9 + 1.95e-9 * 2.0 * M * N * K
-                                              : choose_resident(probs, n, M, K, nbr_max, gelu).us;
+    double tiles;
+    if (plans[0]->nchunk > 1)
+        (void)choose_chunked(probs, n, M, K, plans[0]->nchunk, nbr_max, &tiles);
+    else
+        tiles = choose_resident(probs, n, M, K, nbr_max, gelu).us;
     return 2.4 + dense_gemm_estimate(Ns, n, M, K) < tiles;
 }
 static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
@@ -2374,10 +2458,26 @@ extern "C" int et_tile_plan_ln_fusable(const et_tile_plan *plan) {
                : 0;
 }
 
-// The fused kernels run one workgroup per 32-row panel; with few rows that
-// leaves most CUs idle and the two-launch form (more, smaller workgroups) wins.
-static bool ln_fusion_pays(int M) { return M >= 32 * et::g_tile_ln_min_panels; }
-static bool tail_fusion_pays(int M) { return M >= 32 * et::g_tile_tail_min_panels; }
+// The fused kernels run one workgroup per 32-row panel and CU, in rounds; with few panels, or few in a second round, most
+// CUs idle and the separate launches (more, smaller workgroups) win.  Whole layers 1024 wide, fused / separate, us:
+// 50 %: 4096 rows 144 / 124, 5120 173 / 170, 6144 185 / 199, 10240 360 / 319, 12288 392 / 372; 80 %: 4096 100 / 92,
+// 6144 129 / 141, 10240 235 / 226, 12288 264 / 262, 16384 327 / 345.
+static bool ln_fusion_pays(int M) {
+    const int panels = (M + et::TL_BM - 1) / et::TL_BM, cus = std::max(et_device_cu_count(), 1);
+    if (et::g_tile_min_panels)
+        return panels >= et::g_tile_min_panels;
+    const int rounds = (panels + cus - 1) / cus;
+    return panels >= (rounds == 1 ? 0.6 : 0.76) * cus * rounds;
+}
+// Fewest panels for which the layer tail runs as one launch: its round takes the time of streaming the three linears
+// past a panel, whatever the number of panels.  Whole layers, one launch / steps, us: 768 wide 50 %: 3072 rows 92 / 78,
+// 4096 93 / 85, 5120 98 / 107; 80 %: 2560 rows 59 / 56, 3072 64 / 62, 3584 64 / 65; 90 %: 2560 52 / 52, 3072 56 / 57;
+// 512 wide, 50 %: 3072 57 / 55, 3584 57 / 58.
+static int tail_min_panels(const et_tile_plan *pO, const et_tile_plan *p1, const et_tile_plan *p2) {
+    if (et::g_tile_min_panels)
+        return et::g_tile_min_panels;
+    return 70 + (int)(14.0 * 512e-6 * ((double)pO->ntile + p1->ntile + p2->ntile));
+}
 
 extern "C" int et_tile_plan_run_ln(const et_tile_plan *plan, void *Y, const void *X,
                                    const void *skip, const void *gamma, const void *beta, int M,
@@ -2503,7 +2603,7 @@ extern "C" int et_tile_plan_run_tail(const et_tile_plan *pO, const et_tile_plan 
                ET_ERR_ALIGNMENT, "et_tile_plan_run_tail: pointers must be 16-byte aligned");
     if (M == 0)
         return ET_OK;
-    if (!et_tile_plan_tail_fusable(pO, p1, p2) || (mid && (!tail_fusion_pays(M) || ffn_runs_dense(p1, p2, M)))) {
+    if (!et_tile_plan_tail_fusable(pO, p1, p2) || (mid && ((M + TL_BM - 1) / TL_BM < tail_min_panels(pO, p1, p2) || ffn_runs_dense(p1, p2, M)))) {
         // step by step through the caller's buffers
         ET_REQUIRE(mid, ET_ERR_UNSUPPORTED,
                    "et_tile_plan_run_tail: these shapes need the mid buffer (%d x %d halves)", M, pO->out_feat);
@@ -2520,7 +2620,7 @@ extern "C" int et_tile_plan_run_tail(const et_tile_plan *pO, const et_tile_plan 
     if (mid && hidden) {
         const int cus = std::max(et_device_cu_count(), 1);
         const int panels = (M + TL_BM - 1) / TL_BM, full = panels / cus * cus, rem = panels - full;
-        if (full > 0 && rem > 0 && rem < g_tile_tail_min_panels) {
+        if (full > 0 && rem > 0 && rem < tail_min_panels(pO, p1, p2)) {
             const int M1 = full * TL_BM;
             int rc = et_tile_plan_run_tail(pO, p1, p2, Y, attn, input, nullptr, nullptr, gamma1, beta1, gamma2,
                                            beta2, M1, stream);

@@ -32,6 +32,8 @@ struct et_tile_plan {
 namespace et {
 // whether consecutive workgroups of a linear should share a column group of W rather than a row panel of X (tile_linear.hip)
 bool tl_order(double x_bytes, double w_bytes, long panels, long groups, double x_most);
+// megabytes that the L2s take in, in that order
+double tl_traffic_mb(double x_mb, double w_mb, long panels, long groups, double x_most);
 
 // One int per process in pinned host memory that kernels set when a bounded
 // wait inside a workgroup gives up (device pointer / host pointer, null if the

@@ -12,8 +12,8 @@
 // the pairs stream through registers instead of one tile after the other
 // (1000 rows, 3072 -> 768, 80 %: 34 us before).
 // What it costs: W is streamed once per 16 rows (L2 to CU, ~130 GB/s per CU),
-// so with many rows and dense lists the 32- and 64-row kernels win; the
-// launcher in tile_linear.hip chooses by the amount of W that would be streamed.
+// so with many rows and dense lists the 32-row kernels win; the launcher in
+// tile_linear.hip chooses by estimated time.
 //
 // Few rows: the pairs of a block-row are split over 2^ls waves so that a wave's
 // share arrives in one or two round trips; the partial sums meet in LDS and are
@@ -231,6 +231,19 @@ static void tile_rows_plan(int M, int K, int nbr_max, int nlin, double pairs, in
                 *ls = s;
             }
         }
+}
+
+// the launch's time in microseconds; traffic: megabytes that the L2s take in.  Fit to 312 launches (2048 -> 512, 3072 ->
+// 768 and 4096 -> 1024, 0 to 90 % pruned, 48 to 16384 rows), 4.5 % off in the mean.
+double tile_rows_estimate(int M, int K, int nbr_max, int nlin, double pairs, double w_mb) {
+    const int cus = std::max(et_device_cu_count(), 1), panels = (M + TR_BM - 1) / TR_BM;
+    int nb = 1, ls = 0;
+    tile_rows_plan(M, K, nbr_max, nlin, pairs, cus, &nb, &ls);
+    const int group = (TR_WAVES >> ls) * nb, ncg = (nbr_max + group - 1) / group * nlin;
+    const long wgs = (long)panels * ncg;
+    const double rounds = (double)((wgs + cus - 1) / cus);
+    return 1.75 + 0.0514 * tl_traffic_mb(2e-6 * M * K, w_mb, panels, ncg, 2.5) +
+           rounds * (0.4525 + 43.3e-5 * K + 1.093e-2 * group * pairs + 1.4 * nb + 0.0825 * std::min(1.0, (double)wgs / cus));
 }
 
 bool tile_rows_fits(int K) { return K % 16 == 0 && tile_rows_lds(K) <= 160 * 1024; }

@@ -465,9 +465,8 @@ int et_device_synchronize(void);
  *   "tile_fuse_ln"    0: et_tile_plan_run_ln runs the linear and the LayerNorm
  *                     as two launches; 1 (default): fused where the rows fit
  *   "tile_ln_min_panels" fewest 32-row panels for which et_tile_plan_run_ln
- *                     fuses (default 96; below, two launches are faster); a
- *                     value > 0 also replaces the 72 panels from which
- *                     et_tile_plan_run_tail runs as one launch
+ *                     fuses and et_tile_plan_run_tail runs as one launch; 0
+ *                     (default): by size and density
  *   "tile_order"      consecutive workgroups of a linear share 0: a row panel, 2:
  *                     a column group, 1 (default): what moves fewer bytes
  *   "tile_bm64"       panels of a planned linear of one chunk: 0: 32 rows; 2: 64
@@ -475,7 +474,10 @@ int et_device_synchronize(void);
  *   "tile_splitk_rows" most rows for which a planned linear with K > 1024 runs
  *                     on whole rows in LDS (16-row panels, a block-row's tile
  *                     pairs split over several waves where there are few); -1
- *                     (default): by the amount of W streamed; 0: never
+ *                     (default): by estimated time; 0: never
+ *   "tile_chunked"    a planned linear with K > 1024 on the kernel with fetching
+ *                     waves: 1 .. 4 block-rows per computing wave; 0: never; -1
+ *                     (default): by estimated time
  *   "layer_flow_rows" most rows for which an encoder layer runs as one launch
  *                     (et_layer_flow_pays); -1 (default): by size and density;
  *                     0: never

@@ -1227,3 +1227,32 @@ def test_otf_attention_ragged_rows(K, S, B, hd):
         rows = np.concatenate([np.arange(b * S, (b + 1) * S) for b in pick])
         want = orc.otf_attention(Q[rows], Kk[rows], V[rows], m, S, H, pick.size, None if n is None else n[pick], LOG2E, f64=True)
         check_close(got[rows], want, max_abs=5e-3, mean_rel=1e-3, what=f"mask {m is not None}, lens {n is not None}")
+
+
+@pytest.mark.parametrize("nb", [1, 2, 3, 4])
+@pytest.mark.parametrize("M,N,Kd,gelu", [
+    (1, 16, 1040, True),        # one row, one block-row, a second chunk of 272 columns
+    (33, 784, 1552, False),     # a row into the second panel; a block-row into the next group; three chunks
+    (95, 400, 3072, True),      # four full chunks, the last panel one row short
+])
+def test_tile_linear_fetching_waves(K, nb, M, N, Kd, gelu):
+    """planned linears with K in several chunks on the kernel with fetching waves: the oracle, and the bits of the kernel
+    that fetches chunk by chunk"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile
+    r = rng(88 + M + N)
+    lin = make_tile_linear(r, N, Kd, 0.7, seed=M + Kd, std=0.05, bias_std=0.2)
+    X = randn_h(r, (M, Kd))
+    lt = Linear_tile(Kd, N, M, lin["row_offset"].size, lin["data"], lin["row_ptr"], lin["row_offset"], lin["bias"], gelu)
+    try:
+        lib().et_tuning_set(b"tile_splitk_rows", 0)
+        lib().et_tuning_set(b"tile_chunked", 0)
+        chunks = host(lt.run(dev(X)))
+        lib().et_tuning_set(b"tile_chunked", nb)
+        got = host(lt.run(dev(X)))
+    finally:
+        lib().et_tuning_set(b"tile_splitk_rows", -1)
+        lib().et_tuning_set(b"tile_chunked", -1)
+    want = orc.tile_linear(X, lin["row_ptr"], lin["row_offset"], lin["data"], lin["bias"], N, gelu=gelu, f64=True)
+    check_close(got, want, max_abs=4e-3, mean_rel=5e-4, what="fetching waves")
+    assert np.array_equal(got, chunks)
