@@ -2036,6 +2036,27 @@ static void chunking(int K, int *KC, int *nchunk, int panel = TL_MAX_PANEL) {
     }
 }
 
+// Columns of a plan's chunks.  A linear that narrows its input is a feed-forward block's second one: chunks of 768 hidden
+// columns are what the fused kernel walks, so only linears that do not get a single panel beyond 992 columns.
+static void plan_chunking(int in_feat, int out_feat, int *KC, int *nchunk) {
+    chunking(in_feat, KC, nchunk, out_feat < in_feat ? TL_MAX_RAW_PANEL : TL_MAX_PANEL);
+}
+// Which launch each of n plans over one input goes into.  The kernels of this file walk all linears of a launch in the
+// same column chunks, and from 993 to 1024 columns a plan's chunks depend on its width: plans of another geometry get a
+// launch of their own.  Returns the number of launches.
+static int join_launches(const int *KC, const int *nchunk, int n, int *launch) {
+    int launches = 0;
+    for (int i = 0; i < n; i++) {
+        launch[i] = -1;
+        for (int j = 0; j < i && launch[i] < 0; j++)
+            if (KC[j] == KC[i] && nchunk[j] == nchunk[i])
+                launch[i] = launch[j];
+        if (launch[i] < 0)
+            launch[i] = launches++;
+    }
+    return launches;
+}
+
 static int raw_tile_linear(void *Y, const void *X, const int *row_ptr, const int *row_offset,
                            const void *data, int M, int N, int K, const void *bias,
                            bool gelu, void *stream, const char *who) {
@@ -2186,25 +2207,36 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
-    TlProblem probs[3];
-    int Ns[3], nbr_max = 0;
+    int Ns[3], KC[3], nchunk[3], launch[3];
     for (int i = 0; i < n; i++) {
         if (!plans[i]->d_dense)
             return false;
         Ns[i] = plans[i]->out_feat;
-        probs[i].N = Ns[i];
-        probs[i].nbr = Ns[i] / 16;
-        probs[i].ntile = plans[i]->ntile;
-        nbr_max = std::max(nbr_max, probs[i].nbr);
+        KC[i] = plans[i]->KC;
+        nchunk[i] = plans[i]->nchunk;
     }
     if (g_plan_dense == 2)
         return true;
-    const int K = plans[0]->in_feat;
-    double tiles;
-    if (plans[0]->nchunk > 1)
-        (void)choose_chunked(probs, n, M, K, plans[0]->nchunk, nbr_max, &tiles);
-    else
-        tiles = choose_resident(probs, n, M, K, nbr_max, gelu).us;
+    const int K = plans[0]->in_feat, launches = join_launches(KC, nchunk, n, launch);
+    double tiles = 0.0;
+    for (int l = 0; l < launches; l++) {
+        TlProblem probs[3];
+        int m = 0, chunks = 0, nbr_max = 0;
+        for (int i = 0; i < n; i++)
+            if (launch[i] == l) {
+                probs[m].N = Ns[i];
+                probs[m].nbr = Ns[i] / 16;
+                probs[m].ntile = plans[i]->ntile;
+                chunks = nchunk[i];
+                nbr_max = std::max(nbr_max, probs[m++].nbr);
+            }
+        double us;
+        if (chunks > 1)
+            (void)choose_chunked(probs, m, M, K, chunks, nbr_max, &us);
+        else
+            us = choose_resident(probs, m, M, K, nbr_max, gelu).us;
+        tiles += us;
+    }
     return 2.4 + dense_gemm_estimate(Ns, n, M, K) < tiles;
 }
 static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
@@ -2302,9 +2334,7 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
     ET_REQUIRE(v == 0, ET_ERR_FORMAT, "et_tile_plan_create: malformed tile_mat (check %d)", v);
     const int nbr = out_feat / 16;
     int KC, nchunk;
-    // (a linear that narrows its input is a feed-forward block's second one: chunks of 768 hidden columns are what the
-    // fused kernel walks)
-    chunking(in_feat, &KC, &nchunk, out_feat < in_feat ? TL_MAX_RAW_PANEL : TL_MAX_PANEL);
+    plan_chunking(in_feat, out_feat, &KC, &nchunk);
     // Plan layout: tiles ordered by (chunk, block-row, column); every
     // (chunk, block-row) segment padded to an even count with an all-zero
     // tile that reuses the segment's last column (so a pair never straddles
@@ -2427,6 +2457,7 @@ extern "C" int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *co
     ET_REQUIRE(n >= 1 && n <= TL_MAX_LIN, ET_ERR_INVALID_ARG, "et_tile_plan_run_multi: n=%d", n);
     ET_REQUIRE(M >= 0, ET_ERR_INVALID_ARG, "et_tile_plan_run_multi: M=%d", M);
     TlProblem pr[TL_MAX_LIN];
+    int KC[TL_MAX_LIN], nchunk[TL_MAX_LIN], launch[TL_MAX_LIN];
     for (int i = 0; i < n; i++) {
         ET_REQUIRE(plans[i] && Ys[i], ET_ERR_INVALID_ARG, "et_tile_plan_run_multi: null entry %d", i);
         ET_REQUIRE(plans[i]->in_feat == plans[0]->in_feat, ET_ERR_INVALID_ARG,
@@ -2441,14 +2472,40 @@ extern "C" int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *co
         pr[i].nbr = plans[i]->out_feat / 16;
         pr[i].ntile = plans[i]->ntile;
         pr[i].npair = plans[i]->npair;
+        KC[i] = plans[i]->KC;
+        nchunk[i] = plans[i]->nchunk;
     }
     ET_REQUIRE(aligned16(X), ET_ERR_ALIGNMENT, "et_tile_plan_run_multi: X not aligned");
     if (M == 0)
         return ET_OK;
     if (plans_run_dense(plans, n, M, false))
         return run_plans_dense(plans, Ys, n, X, M, false, static_cast<hipStream_t>(stream));
-    return tile_launch(pr, n, static_cast<const f16 *>(X), M, plans[0]->in_feat, plans[0]->KC,
-                       plans[0]->nchunk, false, TL_PLAN, static_cast<hipStream_t>(stream));
+    const int launches = join_launches(KC, nchunk, n, launch);
+    for (int l = 0; l < launches; l++) {
+        TlProblem joined[TL_MAX_LIN];
+        int m = 0, last = 0;
+        for (int i = 0; i < n; i++)
+            if (launch[i] == l) {
+                joined[m++] = pr[i];
+                last = i;
+            }
+        const int rc = tile_launch(joined, m, static_cast<const f16 *>(X), M, plans[0]->in_feat, KC[last], nchunk[last],
+                                   false, TL_PLAN, static_cast<hipStream_t>(stream));
+        if (rc != ET_OK)
+            return rc;
+    }
+    return ET_OK;
+}
+
+extern "C" int et_tile_plan_launches(int in_feat, const int *out_feat, int n, int *launch, int *nchunk, int *chunk_cols) {
+    using namespace et;
+    ET_REQUIRE(out_feat && launch && nchunk && chunk_cols, ET_ERR_INVALID_ARG, "et_tile_plan_launches: null pointer");
+    ET_REQUIRE(in_feat > 0 && n >= 1 && n <= TL_MAX_LIN, ET_ERR_INVALID_ARG, "et_tile_plan_launches: in_feat=%d n=%d",
+               in_feat, n);
+    for (int i = 0; i < n; i++)
+        plan_chunking(in_feat, out_feat[i], &chunk_cols[i], &nchunk[i]);
+    join_launches(chunk_cols, nchunk, n, launch);
+    return ET_OK;
 }
 
 extern "C" int et_tile_plan_ln_fusable(const et_tile_plan *plan) {

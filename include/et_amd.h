@@ -330,9 +330,17 @@ int et_layer_flow_run(et_layer_flow *flow, void *out, const void *in, void *Q, v
                       const void *beta1, const void *gamma2, const void *beta2, float log2_scale, void *stream);
 /* n (<= 4) planned linears with the same in_feat applied to the same X in ONE
  * launch (the Q/K/V projections, encoder/encoder.cu:22-26, which the
- * reference spreads over three streams). */
+ * reference spreads over three streams) - or in one per column geometry where
+ * their plans are laid out in different chunks (et_tile_plan_launches). */
 int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *const *Ys,
                            int n, const void *X, int M, void *stream);
+/* Host only: for plans of in_feat x out_feat[i], the column chunks each is laid
+ * out in (as et_tile_plan_query reports them) and the launch of
+ * et_tile_plan_run_multi it goes into on the tile kernels, from 0.  Plans of
+ * one launch have the same chunks: between 993 and 1024 inputs those of a
+ * linear that narrows its input are others than those of one that does not. */
+int et_tile_plan_launches(int in_feat, const int *out_feat, int n, int *launch,
+                          int *nchunk, int *chunk_cols);
 /* device pointers of the plan's buffers, for tests (sorted order) */
 int et_tile_plan_query(const et_tile_plan *plan, int *in_feat, int *out_feat,
                        int *ntile, int *nchunk, int *chunk_cols);

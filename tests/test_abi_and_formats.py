@@ -316,3 +316,26 @@ def test_encoder_workspace_grows_only_while_the_paired_tail_is_switched_on():
         lib.et_tuning_set(b"tile_tail_pair", 0)
     assert Encoder_tile.buffer_size(d, S, H, B) == (units + 255) // 256 * 256
 
+
+
+@pytest.mark.parametrize("in_feat,out_feat,launch", [
+    (768, (768, 768, 230 // 16 * 16), (0, 0, 0)),
+    (992, (992, 16, 1024, 992), (0, 0, 0, 0)),
+    (1008, (1008, 1008, 304), (0, 0, 1)),         # Encoder_prune: a row-pruned V
+    (1008, (16, 1008, 992, 4096), (0, 1, 0, 1)),
+    (1024, (1024, 1024, 320), (0, 0, 1)),
+    (1024, (512, 512, 1024), (0, 0, 1)),          # Encoder_attnaware: row-pruned Q and K
+    (1040, (1040, 16, 2080), (0, 0, 0)),
+    (4096, (1024, 4096), (0, 0)),
+])
+def test_plans_of_one_launch_share_their_column_chunks(in_feat, out_feat, launch):
+    """the kernels walk all linears of a launch in the same chunks: linears whose plans are laid out in others (between
+    993 and 1024 inputs those depend on the output width) must not be joined with them"""
+    n = len(out_feat)
+    arr = lambda: (C.c_int * n)()
+    got, nchunk, cols = arr(), arr(), arr()
+    assert _lib.lib().et_tile_plan_launches(in_feat, (C.c_int * n)(*out_feat), n, got, nchunk, cols) == 0
+    assert tuple(got) == launch
+    for i in range(n):
+        assert (nchunk[i] - 1) * cols[i] < in_feat <= nchunk[i] * cols[i]
+        assert all((nchunk[i], cols[i]) == (nchunk[j], cols[j]) for j in range(n) if launch[j] == launch[i])

@@ -225,9 +225,18 @@ def test_encoder_tile_layer_vs_torch_fp32_layer():
 
 
 def test_encoder_prune_layer():
+    prune_case(768, 12, 3072, 128, 2)
+
+
+@pytest.mark.parametrize("S,B", [(37, 1), (128, 2), (300, 7)])
+def test_encoder_prune_layer_1024_wide(S, B):
+    """V's plan has two column chunks there, Q's and K's one"""
+    prune_case(1024, 16, 4096, S, B)
+
+
+def prune_case(d, H, dff, S, B):
     from et_amd.encoder import Encoder_prune, Linear_row
     r = rng(600)
-    d, H, dff, S, B = 768, 12, 3072, 128, 2
     lins, ln = make_layer(r, d, dff, 0.8, seed=910)
     x = randn_h(r, (B * S, d))
     mask = randn_h(r, (S, S), 0.5)
@@ -242,7 +251,7 @@ def test_encoder_prune_layer():
     want = orc.skip_layernorm(tl(5, tl(4, h1, True)), h1, ln[2], ln[3])
     L = build_linears(lins, B * S)
     L[2] = Linear_row(d, d, B * S, Wv, v_id, v_id.size, bv, H)
-    assert L[2].nrow == 240 and L[2].row_id_size == 230
+    assert d != 768 or (L[2].nrow == 240 and L[2].row_id_size == 230)
     enc = Encoder_prune(d, S, H, workspace(Encoder_prune, d, S, H, B), *L, *ln, mask, B)
     xd = dev(x)
     got = host(enc.run(torch.empty_like(xd), xd))
@@ -265,10 +274,15 @@ def test_encoder_attnaware_layer_config4_full_size():
     attnaware_case(S=256, B=32, balanced=True, sample=[0, 17, 31])
 
 
-def attnaware_case(S, B, balanced, sample):
+@pytest.mark.parametrize("S,B,balanced,sample", [(37, 1, True, [0]), (64, 2, False, [0, 1]), (250, 8, True, [5])])
+def test_encoder_attnaware_layer_1024_wide(S, B, balanced, sample):
+    """Q's and K's plans have two column chunks there, V's one"""
+    attnaware_case(S, B, balanced, sample, d=1024, H=16, dff=4096)
+
+
+def attnaware_case(S, B, balanced, sample, d=768, H=12, dff=3072):
     from et_amd.encoder import Encoder_attnaware, Linear_row, Linear_tile
     r = rng(650)
-    d, H, dff = 768, 12, 3072
     hd = d // H
     x_all = randn_h(r, (B * S, d))
     rows = np.concatenate([np.arange(b * S, (b + 1) * S) for b in sample])
@@ -331,7 +345,7 @@ def attnaware_case(S, B, balanced, sample):
     Lo = Linear_row(d, d, T, W["o"][o_id], o_id, o_id.size, bsz["o"][o_id], H)
     L1 = Linear_row(d, dff, T, W["m1"][m1_id], m1_id, m1_id.size, bsz["m1"][m1_id], H, is_gelu=True)
     L2 = Linear_row(pad16(m1_id.size), d, T, W2c, m2_id, m2_id.size, bsz["m2"][m2_id], H)
-    assert (Lq.nrow, Lo.nrow, L1.nrow, L2.nrow) == (384, 240, 928, 240)
+    assert (Lq.nrow, Lo.nrow, L1.nrow, L2.nrow) == ((384, 240, 928, 240) if d == 768 else (512, 320, 1232, 320))
     enc = Encoder_attnaware(d, S, H, workspace(Encoder_attnaware, d, S, H, B), Lq, Lk, Lv, Lo, L1, L2, *ln, mask, B)
     xd = dev(x_all)
     got = host(enc.run(torch.empty_like(xd), xd))[rows]

@@ -1139,6 +1139,24 @@ def test_tile_linear_whole_rows(K, M, N, Kd, sp, gelu):
     assert np.array_equal(planned, host(lt.run(dev(X))))
 
 
+@pytest.mark.parametrize("M", [1, 33, 700, 5700])
+@pytest.mark.parametrize("Kd,Ns,sp", [
+    (1024, (1024, 1024, 320), 0.8), (1024, (512, 512, 1024), 0.0), (1008, (16, 1008, 992, 1040), 0.5),
+])
+def test_tile_linear_multi_of_different_column_chunks(K, M, Kd, Ns, sp):
+    """between 993 and 1024 inputs the plan of a linear that narrows its input has other column chunks than one that
+    does not: both kinds over the same rows, narrow ones first, last and in turn"""
+    from et_amd.encoder import Linear_tile, run_multi
+    r = rng(34 + M + Kd)
+    lins = [make_tile_linear(r, N, Kd, sp, seed=70 + j, std=0.05, bias_std=0.1) for j, N in enumerate(Ns)]
+    X = randn_h(r, (M, Kd))
+    lts = [Linear_tile(Kd, l["N"], M, l["row_offset"].size, l["data"], l["row_ptr"], l["row_offset"], l["bias"]) for l in lins]
+    rows = np.unique(np.concatenate([np.arange(min(M, 40)), r.integers(0, M, 40), np.arange(max(M - 40, 0), M)]))
+    for l, o in zip(lins, run_multi(lts, dev(X))):
+        want = orc.tile_linear(X[rows], l["row_ptr"], l["row_offset"], l["data"], l["bias"], l["N"], f64=True)
+        check_close(host(o)[rows], want, max_abs=4e-3, mean_rel=5e-4, what=f"multi, {Kd} -> {l['N']}")
+
+
 @pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("M,Ns,Kd,gelu", [
     (1, (16,), 32, False),               # half a step of 64 columns, one piece of a block
