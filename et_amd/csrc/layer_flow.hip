@@ -26,8 +26,12 @@
 // buffer is written once per launch and read only after the counter says so -
 // no cache can hold an older copy of a line from this launch, and those of
 // earlier launches were dropped when this one started.  Plain loads are then
-// correct; the buffers must not be reused inside the launch, which is why the
-// layer has scratch of its own beside the encoder's workspace.
+// correct; the buffers must not be reused inside the launch.  Nor may a line
+// hold rows of two panels: the line would be pulled into an L2 with one panel's
+// rows, before the other's are stored, and read there again later.  So every
+// buffer that is handed over lies in the object's own scratch, from whole lines
+// on, and rows are whole lines (d and dff multiples of 64); the caller's
+// workspace units need only be 16-byte aligned and are not used.
 //
 // Counters (one 128-byte line each): a workgroup that finishes a unit adds one
 // to its row panel's counter of that step.  The workgroup that completes the
@@ -63,7 +67,7 @@ constexpr int LF_SHARE = 12;   // ... that a wave's share of a block-row should 
 constexpr int LF_CS = 32;      // counter stride in words: a line each
 
 struct LfArgs {
-    AttnArgs at; // Q, K, V, out: the workspace units the steps hand over
+    AttnArgs at; // Q, K, V, out: scratch that the steps hand over
     LfLinear q, k, v, o, m1, m2;
     const f16 *in;
     f16 *out;
@@ -409,7 +413,7 @@ static int flow_rows_limit() { return g_flow_rows < 0 ? LF_MOST_ROWS : std::min(
 struct et_layer_flow {
     const et_tile_plan *p[6] = {};
     int d = 0, dff = 0, seq_len = 0, nheads = 0, batch = 0;
-    et::f16 *scratch = nullptr; // oraw, ln1, fraw: rows x d; hid: rows x dff
+    et::f16 *scratch = nullptr; // Q, K, V, attention, oraw, ln1, fraw: rows x d; hid: rows x dff
     unsigned *ctr = nullptr;
     int nctr_max = 0;
     int *d_blk[2] = {nullptr, nullptr}; // padded batch, packed sequences
@@ -488,7 +492,7 @@ extern "C" int et_layer_flow_create(et_layer_flow **flow, const et_tile_plan *q,
     const int npanel = (int)((rows + LF_BM - 1) / LF_BM);
     const int nblk = batch * ((seq_len + LF_QB - 1) / LF_QB);
     f->nctr_max = 2 + 4 * npanel + nblk;
-    const size_t act = (size_t)rows * (3 * (size_t)d + dff) * sizeof(f16);
+    const size_t act = (size_t)rows * (7 * (size_t)d + dff) * sizeof(f16);
     const size_t ctr = (size_t)f->nctr_max * LF_CS * sizeof(unsigned);
     const size_t tab = ((size_t)2 * nblk + 2 * npanel) * sizeof(int);
     // one allocation: activations, counters, the two block tables
@@ -564,10 +568,15 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
     a.status = wait_status_device();
     ET_REQUIRE(a.status, ET_ERR_HIP, "layer in one launch: no wait-status word");
     a.spin = tail_spin();
-    a.at.out = static_cast<f16 *>(attn);
-    a.at.Q = static_cast<const f16 *>(Q);
-    a.at.K = static_cast<const f16 *>(K);
-    a.at.V = static_cast<const f16 *>(V);
+    const size_t unit = (size_t)f->seq_len * f->batch * f->d;
+    a.at.Q = f->scratch;
+    a.at.K = f->scratch + unit;
+    a.at.V = f->scratch + 2 * unit;
+    a.at.out = f->scratch + 3 * unit;
+    a.oraw = f->scratch + 4 * unit;
+    a.ln1 = f->scratch + 5 * unit;
+    a.fraw = f->scratch + 6 * unit;
+    a.hid = f->scratch + 7 * unit;
     a.at.mask = static_cast<const f16 *>(mask);
     a.at.seq_lens = cu_seqlens ? nullptr : seq_lens;
     a.at.cu_seqlens = cu_seqlens;
@@ -592,11 +601,6 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
     }
     a.in = static_cast<const f16 *>(in);
     a.out = static_cast<f16 *>(out);
-    const size_t unit = (size_t)f->seq_len * f->batch * f->d;
-    a.oraw = f->scratch;
-    a.ln1 = f->scratch + unit;
-    a.fraw = f->scratch + 2 * unit;
-    a.hid = f->scratch + 3 * unit;
     a.gamma1 = static_cast<const f16 *>(gamma1);
     a.beta1 = static_cast<const f16 *>(beta1);
     a.gamma2 = static_cast<const f16 *>(gamma2);

@@ -315,8 +315,9 @@ size_t et_tail_ws_bytes_for(int d_model, int rows);
  * the device scratch of the hand-overs; one run at a time may use it.
  * et_layer_flow_set_packed: HOST row offsets of the packed sequences (batch + 1), for runs with cu_seqlens.
  * et_layer_flow_pays: 1 where et_layer_flow_run is the form to take for that many rows.
- * et_layer_flow_run: out = layer(in), rows of model width, out may alias in; Q, K, V, attn are distinct scratch
- * of rows x model width.  cu_seqlens (device, as given to et_layer_flow_set_packed) or seq_lens (device) or
+ * et_layer_flow_run: out = layer(in), rows of model width, out may alias in; Q, K, V, attn are the caller's
+ * workspace units (rows x model width, 16-byte aligned): they stay as they are, the hand-overs need whole cache
+ * lines and lie in the object's scratch.  cu_seqlens (device, as given to et_layer_flow_set_packed) or seq_lens (device) or
  * neither; mask, log2_scale as in et_OTF_attention.  Kernel launch only: may be captured in a graph. */
 typedef struct et_layer_flow et_layer_flow;
 int et_layer_flow_create(et_layer_flow **flow, const et_tile_plan *q, const et_tile_plan *k, const et_tile_plan *v,

@@ -613,3 +613,31 @@ def test_layer_in_one_launch(d, H, dff, S, B, sp, lens, use_mask):
             assert np.array_equal(host(out_static), got[k])
             assert np.array_equal(host(enc.run(torch.empty_like(x_static), dev(xs[k]))), got[k])
         del graph
+
+
+@pytest.mark.parametrize("S,B,off", [(32, 2, 8), (16, 3, 24), (48, 2, 56), (37, 2, 64)])
+def test_layer_in_one_launch_workspace_alignment(S, B, off):
+    """a workspace `off` halves behind a 256-byte boundary, several sequences that end on a panel: the rows handed over
+    inside the launch lie in lines of their own, not in the workspace, which stays as it was"""
+    from et_amd import lib
+    from et_amd.encoder import Encoder_length
+    r = rng(1500 + S + off)
+    d, H, dff = 256, 4, 1024
+    lins, ln = make_layer(r, d, dff, 0.5, seed=1600 + S, std=0.03, bias_std=0.05)
+    x = randn_h(r, (B * S, d))
+    whole = torch.full((Encoder_length.buffer_size(d, S, H, B) // 2 + 128,), 7.0, dtype=torch.float16, device="cuda")
+    assert whole.data_ptr() % 256 == 0
+    enc = Encoder_length(d, S, H, whole[off:], *build_linears(lins, B * S), *ln, None, B)
+    want = orc.encoder_tile_layer(x, lins, ln, None, S, H, B, None, 1.0)
+    first = host(enc.run(torch.empty_like(dev(x)), dev(x)))
+    check_close(first, want, what=f"layer in one launch, workspace at +{2 * off} bytes")
+    for _ in range(20):
+        assert np.array_equal(host(enc.run(torch.empty_like(dev(x)), dev(x))), first)
+    assert (host(whole) == 7.0).all()
+    try:
+        lib().et_tuning_set(b"layer_flow_rows", 0)
+        steps = host(enc.run(torch.empty_like(dev(x)), dev(x)))
+    finally:
+        lib().et_tuning_set(b"layer_flow_rows", -1)
+    check_close(steps, want, what="separate launches")
+    assert (host(whole) != 7.0).any()
