@@ -36,7 +36,12 @@
 // Counters (one 128-byte line each): a workgroup that finishes a unit adds one
 // to its row panel's counter of that step.  The workgroup that completes the
 // last step of a panel runs its final LayerNorm; the one that does so for the
-// last panel sets every counter back to zero (nobody else is waiting then).
+// last panel ends the launch's books.  There are two sets of counters, taken in
+// turn: the launch that uses one leaves the other at zero for its successor.
+// Its own set it must leave alone - after a wait that gave up, units of earlier
+// steps may still be running and add to it.  The word that the tickets come from
+// also says whose turn it is (its top bit); it can be set back at that point,
+// since the units that complete the last panel have the highest tickets.
 //
 // Units.  Linears: 16 rows x (16 / split) block-rows of 16 output features; the
 // pairs of surviving tiles of a block-row are split over `split` waves, so that
@@ -73,14 +78,14 @@ struct LfArgs {
     f16 *out;
     f16 *oraw, *ln1, *hid, *fraw; // output projection, first LayerNorm, hidden activations, second linear
     const f16 *gamma1, *beta1, *gamma2, *beta2;
-    unsigned *ctr;
+    unsigned *ctr;  // tickets and the set in turn, then the two sets of nctr counters
     const int *blk; // attention blocks: [2i] sequence, [2i+1] query block; then per panel first and last block
     int M, d, dff, npanel, nblk;
     int u_at, u_o, u_f1, u_f2;             // first unit of each step (Q/K/V: 0)
     int g_qkv, g_o, g_f1, g_f2;            // units per panel
     int gl_q, gl_k;                        // ... of the query and key linears
     int s_qkv, s_o, s_f1, s_f2;            // log2 of the split
-    int nctr;                              // counters in use
+    int nctr;                              // counters in a set
     int misc;                              // LDS byte offset of the broadcast words
     int spin;
     int *status;
@@ -88,12 +93,12 @@ struct LfArgs {
 
 // ---- hand-over --------------------------------------------------------------
 // wave 0: lanes 0..n-1 wait until counter first + lane has reached target
-__device__ __forceinline__ void lf_poll(const LfArgs &a, int first, int n, unsigned target) {
+__device__ __forceinline__ void lf_poll(const LfArgs &a, const unsigned *ctr, int first, int n, unsigned target) {
     const int lane = threadIdx.x & 63;
     for (int i0 = 0; i0 < n; i0 += 64) {
         const int i = min(i0 + lane, n - 1);
         for (int s = 0;; s++) {
-            const unsigned c = __hip_atomic_load(a.ctr + (size_t)(first + i) * LF_CS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned c = __hip_atomic_load(ctr + (size_t)(first + i) * LF_CS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (__builtin_amdgcn_ballot_w64(c < target) == 0)
                 break;
             if (s >= a.spin) {
@@ -111,19 +116,19 @@ __device__ __forceinline__ void lf_barrier() {
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
-__device__ __forceinline__ void lf_wait(const LfArgs &a, int wave, int first, int n, unsigned target) {
+__device__ __forceinline__ void lf_wait(const LfArgs &a, const unsigned *ctr, int wave, int first, int n, unsigned target) {
     asm volatile("" ::: "memory");
     if (wave == 0)
-        lf_poll(a, first, n, target);
+        lf_poll(a, ctr, first, n, target);
     lf_barrier();
 }
 // every store of the workgroup is acknowledged, then one is added to the counter; thread 0 gets the old value
-__device__ __forceinline__ unsigned lf_signal(const LfArgs &a, int c) {
+__device__ __forceinline__ unsigned lf_signal(unsigned *ctr, int c) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lf_barrier();
     unsigned old = 0;
     if (threadIdx.x == 0)
-        old = __hip_atomic_fetch_add(a.ctr + (size_t)c * LF_CS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        old = __hip_atomic_fetch_add(ctr + (size_t)c * LF_CS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return old;
 }
 
@@ -274,14 +279,15 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
     if (threadIdx.x == 0)
         bc[0] = __hip_atomic_fetch_add(a.ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     lf_barrier();
-    const int unit = __builtin_amdgcn_readfirstlane((int)bc[0]);
+    const unsigned ticket = __builtin_amdgcn_readfirstlane(bc[0]);
+    const int unit = (int)(ticket & 0x7FFFFFFFu), set = (int)(ticket >> 31);
+    unsigned *const ctr = a.ctr + (size_t)(1 + set * a.nctr) * LF_CS;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int c16 = lane & 15, khalf8 = ((lane >> 4) & 1) * 8;
     const unsigned lane_w2 = (unsigned)((lane >> 5) * 256 + c16 * 16 + khalf8) * 2, hi4 = (lane >> 5) * 4;
-    // counters: 0 tickets, 1 finished panels, then per panel Q/K/V, O, first and second feed-forward linear, then
-    // per attention block
-    const int c_qkv = 2, c_o = c_qkv + a.npanel, c_f1 = c_o + a.npanel, c_f2 = c_f1 + a.npanel, c_at = c_f2 + a.npanel;
+    // counters: finished panels, then per panel Q/K/V, O, first and second feed-forward linear, then per attention block
+    const int c_qkv = 1, c_o = c_qkv + a.npanel, c_f1 = c_o + a.npanel, c_f2 = c_f1 + a.npanel, c_at = c_f2 + a.npanel;
     f16 *const xs = reinterpret_cast<f16 *>(lf_smem);
     f32x4 *const red = reinterpret_cast<f32x4 *>(lf_smem);
     const int ldx = a.d + 16;
@@ -329,11 +335,11 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
         } else if (step == 1) {
             // the attention blocks that hold this panel's rows
             const int b0 = a.blk[2 * a.nblk + 2 * panel], b1 = a.blk[2 * a.nblk + 2 * panel + 1];
-            lf_wait(a, wave, c_at + b0, b1 - b0 + 1, (unsigned)a.at.nhead);
+            lf_wait(a, ctr, wave, c_at + b0, b1 - b0 + 1, (unsigned)a.at.nhead);
             lf_panel(a, a.at.out, xs, ldx, m0, wave, lane);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         } else {
-            lf_wait(a, wave, c_o + panel, 1, (unsigned)a.g_o);
+            lf_wait(a, ctr, wave, c_o + panel, 1, (unsigned)a.g_o);
             lf_layernorm(a, a.oraw, a.in, a.gamma1, a.beta1, m0 + wave, lane, [&](int piece, f16x8 v) {
                 *reinterpret_cast<f16x8 *>(xs + wave * ldx + piece * 8) = v;
                 if (grp0 == 0 && m0 + wave < a.M) // the skip operand of the second LayerNorm
@@ -347,7 +353,7 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
             lf_finish<true>(a, acc, red, l, bias, Y, l.nbr * 16, bn, j, sub, ls, m0, lane);
         else
             lf_finish<false>(a, acc, red, l, bias, Y, l.nbr * 16, bn, j, sub, ls, m0, lane);
-        (void)lf_signal(a, (step == 0 ? c_qkv : step == 1 ? c_o : c_f1) + panel);
+        (void)lf_signal(ctr, (step == 0 ? c_qkv : step == 1 ? c_o : c_f1) + panel);
     } else if (unit < a.u_o) {
         // ---- attention: block of query rows of one head
         const int rel = unit - a.u_at;
@@ -356,9 +362,9 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
         const int row0 = a.at.cu_seqlens ? a.at.cu_seqlens[b] : b * a.at.seq_len;
         const int row1 = a.at.cu_seqlens ? a.at.cu_seqlens[b + 1] : row0 + a.at.seq_len;
         const int p0 = row0 / LF_BM, p1 = (row1 - 1) / LF_BM;
-        lf_wait(a, wave, c_qkv + p0, p1 - p0 + 1, (unsigned)a.g_qkv);
+        lf_wait(a, ctr, wave, c_qkv + p0, p1 - p0 + 1, (unsigned)a.g_qkv);
         attention_block<HD, 1, LF_WAVES, false, false, false, HD, false, true, MASK>(a.at, b, h, qb);
-        (void)lf_signal(a, c_at + ib);
+        (void)lf_signal(ctr, c_at + ib);
     } else {
         // ---- second feed-forward linear; whoever completes a panel runs its LayerNorm
         const int rel = unit - a.u_f2;
@@ -370,12 +376,12 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
         const f16x4 bias = lf_bias(a.m2, bn, lane);
         LfPairs<LF_D> p;
         const int n = lf_request(p, a.m2, w, lane_w2, hi4);
-        lf_wait(a, wave, c_f1 + panel, 1, (unsigned)a.g_f1);
+        lf_wait(a, ctr, wave, c_f1 + panel, 1, (unsigned)a.g_f1);
         const char *xr = reinterpret_cast<const char *>(a.hid + (size_t)min(m0 + c16, a.M - 1) * a.dff + khalf8);
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
         lf_multiply_direct(acc, p, n, a.m2, w, xr, lane_w2, hi4);
         lf_finish<false>(a, acc, red, a.m2, bias, a.fraw, a.d, bn, j, sub, ls, m0, lane);
-        const unsigned old = lf_signal(a, c_f2 + panel);
+        const unsigned old = lf_signal(ctr, c_f2 + panel);
         if (threadIdx.x == 0)
             bc[1] = old;
         lf_barrier();
@@ -383,15 +389,19 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
             return;
         // every unit of every earlier step of this panel is done; if this is the last panel, of the launch
         if (threadIdx.x == 0)
-            bc[2] = __hip_atomic_fetch_add(a.ctr + LF_CS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bc[2] = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         lf_layernorm(a, a.fraw, a.ln1, a.gamma2, a.beta2, m0 + wave, lane, [&](int piece, f16x8 v) {
             if (m0 + wave < a.M)
                 *reinterpret_cast<f16x8 *>(a.out + (size_t)(m0 + wave) * a.d + piece * 8) = v;
         });
         lf_barrier();
-        if ((int)bc[2] == a.npanel - 1)
+        if ((int)bc[2] == a.npanel - 1) {
+            unsigned *const other = a.ctr + (size_t)(1 + (set ^ 1) * a.nctr) * LF_CS;
             for (int i = threadIdx.x; i < a.nctr; i += LF_WAVES * 64)
-                __hip_atomic_store(a.ctr + (size_t)i * LF_CS, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(other + (size_t)i * LF_CS, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (threadIdx.x == 0)
+                __hip_atomic_store(a.ctr, (unsigned)(set ^ 1) << 31, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
@@ -415,7 +425,7 @@ struct et_layer_flow {
     int d = 0, dff = 0, seq_len = 0, nheads = 0, batch = 0;
     et::f16 *scratch = nullptr; // Q, K, V, attention, oraw, ln1, fraw: rows x d; hid: rows x dff
     unsigned *ctr = nullptr;
-    int nctr_max = 0;
+    int nctr = 0; // counters in a set: enough for the padded batch and for any lengths
     int *d_blk[2] = {nullptr, nullptr}; // padded batch, packed sequences
     double mbytes = 0.0; // of surviving tiles in the six linears
     int nblk[2] = {0, 0}, rows[2] = {0, 0};
@@ -491,9 +501,9 @@ extern "C" int et_layer_flow_create(et_layer_flow **flow, const et_tile_plan *q,
     f->batch = batch;
     const int npanel = (int)((rows + LF_BM - 1) / LF_BM);
     const int nblk = batch * ((seq_len + LF_QB - 1) / LF_QB);
-    f->nctr_max = 2 + 4 * npanel + nblk;
+    f->nctr = 1 + 4 * npanel + nblk;
     const size_t act = (size_t)rows * (7 * (size_t)d + dff) * sizeof(f16);
-    const size_t ctr = (size_t)f->nctr_max * LF_CS * sizeof(unsigned);
+    const size_t ctr = (size_t)(1 + 2 * f->nctr) * LF_CS * sizeof(unsigned);
     const size_t tab = ((size_t)2 * nblk + 2 * npanel) * sizeof(int);
     // one allocation: activations, counters, the two block tables
     char *base = nullptr;
@@ -611,7 +621,7 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
     a.dff = f->dff;
     a.npanel = (a.M + LF_BM - 1) / LF_BM;
     a.nblk = f->nblk[which];
-    a.nctr = 2 + 4 * a.npanel + a.nblk;
+    a.nctr = f->nctr;
     a.s_qkv = std::max(std::max(flow_split(f->p[0], LF_SHARE), flow_split(f->p[1], LF_SHARE)), flow_split(f->p[2], LF_SHARE));
     a.s_o = flow_split(f->p[3], LF_SHARE);
     a.s_f1 = flow_split(f->p[4], LF_SHARE);

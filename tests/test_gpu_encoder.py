@@ -641,3 +641,47 @@ def test_layer_in_one_launch_workspace_alignment(S, B, off):
         lib().et_tuning_set(b"layer_flow_rows", -1)
     check_close(steps, want, what="separate launches")
     assert (host(whole) != 7.0).any()
+
+
+@pytest.mark.parametrize("S,B,lens", [(37, 1, None), (48, 2, None), (24, 4, [24, 3, 17, 9])])
+def test_layer_in_one_launch_after_a_wait_that_gave_up(S, B, lens):
+    """waits that give up at once (poll limit 0): the launch ends, the next call reports it once, and every run from then
+    on is right, eager and replayed - also after two such launches in a row"""
+    from et_amd import EtError, lib
+    from et_amd.encoder import Encoder_length
+    r = rng(1700 + S)
+    d, H, dff = 768, 12, 3072
+    lins, ln = make_layer(r, d, dff, 0.8, seed=1800 + S, std=0.03, bias_std=0.05)
+    x = dev(randn_h(r, (B * S, d)))
+    enc = Encoder_length(d, S, H, workspace(Encoder_length, d, S, H, B), *build_linears(lins, B * S), *ln, None, B)
+    enc.set_seq_lens(None if lens is None else np.array(lens, np.int32))
+    run = lambda: host(enc.run(torch.empty_like(x), x))
+    good = run()
+    out = torch.empty_like(x)
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        enc.run(out, x)
+    try:
+        for launches in (1, 2, 1):
+            lib().et_tuning_set(b"tile_wait_spin", 0)
+            for _ in range(launches):
+                print("zero-poll launch", flush=True)
+                run()
+                if lib().et_wait_status_take() == 0:
+                    pytest.skip("no wait was ever in vain")
+            lib().et_wait_status_raise_for_test()
+            lib().et_tuning_set(b"tile_wait_spin", -1)
+            with pytest.raises(EtError) as e:
+                run()
+            assert "gave up a bounded wait" in str(e.value)
+            for _ in range(5):
+                assert np.array_equal(run(), good)
+                out.zero_()
+                graph.replay()
+                assert np.array_equal(host(out), good)
+            assert lib().et_wait_status_take() == 0
+    finally:
+        lib().et_tuning_set(b"tile_wait_spin", -1)
+        lib().et_wait_status_take()
+    del graph
