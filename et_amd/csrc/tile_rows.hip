@@ -124,9 +124,9 @@ __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(const TrArgs a
             if constexpr (RAW) {
                 tr_load_raw<I>(p, l, rw, lane_w2, hi);
             } else {
-                int q;
-                lf_next(w, q, p.co[I]);
-                p.o[I] = *reinterpret_cast<const int *>(reinterpret_cast<const char *>(l.poff) + (size_t)q * 8 + hi4);
+                int q, qcol;
+                lf_next(w, q, qcol, p.co[I]);
+                p.o[I] = *reinterpret_cast<const int *>(reinterpret_cast<const char *>(l.poff) + (size_t)qcol * 8 + hi4);
                 p.w[I] = *reinterpret_cast<const f16x8 *>(reinterpret_cast<const char *>(l.data) + (size_t)q * 1024 + lane_w2);
             }
         };

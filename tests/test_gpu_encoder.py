@@ -685,3 +685,27 @@ def test_layer_in_one_launch_after_a_wait_that_gave_up(S, B, lens):
         lib().et_tuning_set(b"tile_wait_spin", -1)
         lib().et_wait_status_take()
     del graph
+
+
+@pytest.mark.parametrize("sp", [0.5, 0.85])
+def test_layer_in_one_launch_infinite_activation_without_a_tile(sp):
+    """an infinite activation in a tile column that Q, K and V have no tile in stays with its own row (the skip
+    connection): the other rows are what they are with a finite one"""
+    from et_amd.encoder import Encoder_length
+    r = rng(2000)
+    d, H, dff, S, B = 768, 12, 3072, 24, 2
+    lins, ln = make_layer(r, d, dff, sp, seed=2100, std=0.03, bias_std=0.05)
+    for l in lins[:3]:
+        keep = l["row_offset"] != 0
+        rows = np.repeat(np.arange(d // 16), np.diff(l["row_ptr"]))[keep]
+        l["row_ptr"] = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=d // 16))]).astype(np.int32)
+        l["data"] = l["data"].reshape(-1, 256)[keep].copy()
+        l["row_offset"] = l["row_offset"][keep].copy()
+    x = randn_h(r, (B * S, d))
+    xi = x.copy()
+    xi[5, 3] = np.inf
+    enc = Encoder_length(d, S, H, workspace(Encoder_length, d, S, H, B), *build_linears(lins, B * S), *ln, None, B)
+    fin, inf = (host(enc.run(torch.empty_like(dev(v)), dev(v))) for v in (x, xi))
+    check_close(fin, orc.encoder_tile_layer(x, lins, ln, None, S, H, B, None, 1.0), what="finite")
+    others = np.arange(B * S) != 5
+    assert np.array_equal(inf[others], fin[others]) and not np.isfinite(inf[5]).any()

@@ -1274,3 +1274,40 @@ def test_tile_linear_fetching_waves(K, nb, M, N, Kd, gelu):
     want = orc.tile_linear(X, lin["row_ptr"], lin["row_offset"], lin["data"], lin["bias"], N, gelu=gelu, f64=True)
     check_close(got, want, max_abs=4e-3, mean_rel=5e-4, what="fetching waves")
     assert np.array_equal(got, chunks)
+
+
+@pytest.mark.parametrize("form", ["planned", "raw"])
+@pytest.mark.parametrize("M,N,Kd", [
+    (5, 160, 2048),       # a block-row's pairs split over many waves
+    (100, 768, 3072),     # ... over some
+    (3000, 272, 1536),    # several block-rows per wave
+])
+def test_tile_linear_whole_rows_infinite_activations(K, form, M, N, Kd):
+    """infinite activations in the first and in a later tile column: block-rows without a tile there are what they are
+    with finite ones, whatever an odd list is filled up with"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile
+    r = rng(1900 + M)
+    lin = make_tile_linear(r, N, Kd, 0.85, seed=M + N, std=0.05, bias_std=0.2)
+    rp, ro = lin["row_ptr"], lin["row_offset"]
+    col = Kd // 2 // 16 * 16
+    hit = np.array([np.isin([0, col], ro[rp[b]:rp[b + 1]]).any() for b in range(N // 16)])
+    assert hit.any() and not hit.all()
+    assert len({(rp[b + 1] - rp[b]) % 4 for b in range(N // 16)}) > 1
+    X = randn_h(r, (M, Kd))
+    Xi = X.copy()
+    Xi[:, [3, col + 7]] = np.inf
+
+    def run(x):
+        if form == "raw":
+            return host(K.tile_spmm_add_bias(dev(x), dev(rp), dev(ro), dev(lin["data"]), dev(lin["bias"]), N))
+        return host(Linear_tile(Kd, N, M, ro.size, lin["data"], rp, ro, lin["bias"]).run(dev(x)))
+
+    try:
+        lib().et_tuning_set(b"tile_splitk_rows", 1 << 20)
+        fin, inf = (run(x).reshape(M, N // 16, 16) for x in (X, Xi))
+    finally:
+        lib().et_tuning_set(b"tile_splitk_rows", -1)
+    assert np.isfinite(fin).all()
+    assert np.array_equal(inf[:, ~hit], fin[:, ~hit])
+    assert not np.isfinite(inf[:, hit]).any()
