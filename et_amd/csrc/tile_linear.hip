@@ -1753,6 +1753,7 @@ static int g_row_gemm_min_rows = 1024;
 static int g_plan_dense = 1;
 
 static int g_tile_rows_most = -1; // et_tuning_set("tile_splitk_rows"): most rows for which a plan runs on whole rows, -1 automatic
+static int g_tile_splitk_k1 = 0;  // et_tuning_set("tile_splitk_k1"): also plans of one chunk, up to that many rows (automatic: 128)
 
 static int g_tile_order = 1; // et_tuning_set("tile_order"): 0 panels slowest, 2 column groups slowest, 1 fewer bytes
 // Whether consecutive workgroups walk the panels of a column group (see tl_items): X and W in bytes, numbers of panels
@@ -1813,6 +1814,8 @@ static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, 
     for (const TlForm &f : tl_forms) {
         if (f.rows == TL_BM ? (fnb ? f.nb != fnb : g_tile_bm64 == 2) : fnb || g_tile_bm64 == 0)
             continue; // (tuning; a form of either height fits every K of one chunk)
+        if (f.waves == 12 && g_tile_bm64 == 4)
+            continue;
         const size_t lds = (size_t)f.rows * (K + ((K & 31) ? 0 : TL_PAD)) * sizeof(f16) +
                            (size_t)f.waves * f.rows * (16 * f.nb + 8) * sizeof(f16);
         if (lds > 160 * 1024)
@@ -1936,6 +1939,8 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
     if (mode == TL_PLAN && nchunk > 1) {
         double us;
         which = g_tile_nb == 0 ? choose_chunked(probs, nlin, M, K, nchunk, nbr_max, &us) : TL_BY_PLAN;
+    } else if (mode == TL_PLAN && g_tile_splitk_k1 && tile_rows_fits(K) && M <= (g_tile_rows_most < 0 ? 128 : g_tile_rows_most)) {
+        which = TL_BY_ROWS;
     } else if (g_tile_nb == 0 && tile_rows_fits(K) && (mode == TL_RAW || mode == TL_FILTER)) {
         const long panels = (M + 15) / 16;
         if (nchunk > 1 || panels * ((nbr_max + 15) / 16) <= std::max(et_device_cu_count(), 1))
@@ -1973,7 +1978,7 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         a.ncg_magic = magic_of(a.ncg);
     };
     int nb = 0, order = -1;
-    if (mode == TL_PLAN && nchunk == 1) {
+    if (mode == TL_PLAN && nchunk == 1) { // (on whole rows: returned above)
         const TlChoice c = choose_resident(probs, nlin, M, K, nbr_max, gelu);
         a.ncg = c.ncg;
         a.ipw = g_tile_ipw > 0 ? g_tile_ipw : c.d;
@@ -2089,6 +2094,10 @@ static int g_tail_pair_min_wgs = 0; // et_tuning_set("tile_tail_pair_min_wgs"): 
 extern "C" int et_tuning_set(const char *key, int value) {
     if (key && !strcmp(key, "tile_splitk_rows")) {
         et::g_tile_rows_most = value;
+        return ET_OK;
+    }
+    if (key && !strcmp(key, "tile_splitk_k1")) {
+        et::g_tile_splitk_k1 = value;
         return ET_OK;
     }
     if (key && !strcmp(key, "dense_form")) {

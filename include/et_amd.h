@@ -479,11 +479,14 @@ int et_device_synchronize(void);
  *   "tile_order"      consecutive workgroups of a linear share 0: a row panel, 2:
  *                     a column group, 1 (default): what moves fewer bytes
  *   "tile_bm64"       panels of a planned linear of one chunk: 0: 32 rows; 2: 64
- *                     rows; 1 (default): the less estimated time
+ *                     rows; 1 (default): the less estimated time; 4: as 1
+ *                     without the twelve-wave form
  *   "tile_splitk_rows" most rows for which a planned linear with K > 1024 runs
  *                     on whole rows in LDS (16-row panels, a block-row's tile
  *                     pairs split over several waves where there are few); -1
  *                     (default): by estimated time; 0: never
+ *   "tile_splitk_k1"  1: whole rows also for K of one chunk, up to
+ *                     "tile_splitk_rows" rows (-1: 128); 0 (default)
  *   "tile_chunked"    a planned linear with K > 1024 on the kernel with fetching
  *                     waves: 1 .. 4 block-rows per computing wave; 0: never; -1
  *                     (default): by estimated time
@@ -524,8 +527,6 @@ int et_device_synchronize(void);
  *                     up sets a status word, the launch's result is wrong, and
  *                     the next launch of that kind returns ET_ERR_HIP once.  0
  *                     makes every wait give up at once (for testing the report)
- *   "tile_tail_min_panels"  row panels below which the layer tail runs step
- *                     by step when the caller gave it buffers (default 72)
  * Not thread-safe; results never depend on these beyond fp32 summation
  * order. */
 int et_tuning_set(const char *key, int value);

@@ -339,3 +339,15 @@ def test_plans_of_one_launch_share_their_column_chunks(in_feat, out_feat, launch
     for i in range(n):
         assert (nchunk[i] - 1) * cols[i] < in_feat <= nchunk[i] * cols[i]
         assert all((nchunk[i], cols[i]) == (nchunk[j], cols[j]) for j in range(n) if launch[j] == launch[i])
+
+
+def test_every_documented_tuning_key_is_known():
+    """the keys that the header lists, and only those, are taken"""
+    text = open(os.path.join(ROOT, "include", "et_amd.h")).read()
+    doc = text[text.index("Launch-heuristic overrides"):text.index("int et_tuning_set")]
+    keys = re.findall(r'^ \*   "([a-z0-9_]+)"', doc, flags=re.M)
+    assert len(keys) >= 20 and len(set(keys)) == len(keys)
+    src = open(os.path.join(ROOT, "et_amd", "csrc", "tile_linear.hip")).read()
+    known = set(re.findall(r'strcmp\(key, "([a-z0-9_]+)"\)', src))
+    assert set(keys) == known
+    assert _lib.lib().et_tuning_set(b"no_such_key", 1) < 0

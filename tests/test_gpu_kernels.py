@@ -1225,6 +1225,27 @@ def test_tile_linear_orders_and_forms(K, M, Ns, Kd):
             lib().et_tuning_set(key, value)
 
 
+@pytest.mark.parametrize("M,Ns,Kd", [(1, (16,), 16), (33, (272, 400), 768), (128, (1040,), 1024)])
+def test_tile_linear_forms_behind_tuning_keys(K, M, Ns, Kd):
+    """whole rows for K of one chunk and the choice without the twelve-wave form: the oracle's values"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile, run_multi
+    r = rng(57 + M + Kd)
+    mats = [make_tile_linear(r, N, Kd, 0.6, seed=M + N, std=0.05, bias_std=0.2) for N in Ns]
+    X = randn_h(r, (M, Kd))
+    lts = [Linear_tile(Kd, N, M, m["row_offset"].size, m["data"], m["row_ptr"], m["row_offset"], m["bias"])
+           for N, m in zip(Ns, mats)]
+    for key, value, off in ((b"tile_splitk_k1", 1, 0), (b"tile_bm64", 4, 1)):
+        try:
+            assert lib().et_tuning_set(key, value) == 0
+            got = [host(y) for y in run_multi(lts, dev(X))]
+        finally:
+            lib().et_tuning_set(key, off)
+        for g, N, m in zip(got, Ns, mats):
+            want = orc.tile_linear(X, m["row_ptr"], m["row_offset"], m["data"], m["bias"], N, f64=True)
+            check_close(g, want, max_abs=4e-3, mean_rel=5e-4, what=f"{key}, N={N}")
+
+
 @pytest.mark.parametrize("S,B,hd", [(1, 2, 64), (15, 1, 32), (63, 3, 64), (65, 2, 128), (127, 2, 64), (129, 24, 64),
                                     (191, 1, 64), (250, 5, 64)])
 def test_otf_attention_ragged_rows(K, S, B, hd):
