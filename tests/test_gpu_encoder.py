@@ -139,7 +139,7 @@ def test_encoder_tile_layer_config3_full_size_with_a_mask(kind):
 
 
 @pytest.mark.parametrize("d,H,dff,S,B,sp", [
-    (1024, 16, 4096, 128, 8, 0.8),    # BERT-large widths: K = 1024 needs two panel chunks everywhere
+    (1024, 16, 4096, 128, 8, 0.8),    # BERT-large widths: K = 1024 in one chunk, 4096 in six
     (1024, 16, 4096, 64, 1, 0.5),     # ... and on few rows
     (512, 8, 2048, 96, 40, 0.7),      # 3840 rows of 512: the one-launch tail on another width
     (384, 12, 1536, 50, 3, 0.6),      # head_dim 32
@@ -161,7 +161,7 @@ def test_encoder_tile_layer_other_widths(d, H, dff, S, B, sp):
 
 @pytest.mark.parametrize("S,B", [(128, 2), (200, 3)])
 def test_encoder_tile_layer_fused_tail_forced(S, B):
-    """the one-launch layer tail (normally used from 96 row panels up) inside Encoder_tile, forced on small shapes"""
+    """the one-launch layer tail (normally used for more row panels) inside Encoder_tile, forced on small shapes"""
     from et_amd import lib
     from et_amd.encoder import Encoder_tile
     r = rng(620 + S)
@@ -571,15 +571,19 @@ def test_cpp_caller_of_the_reference_classes(tmp_path, program):
     (64, 2, 128, 3, 30, 0.6, [3, 1, 2] * 10, True),    # head width 32, many sequences per panel
     (512, 8, 2048, 40, 2, 0.0, [7, 33], False),        # dense
 ])
-def test_layer_in_one_launch(d, H, dff, S, B, sp, lens, use_mask):
+def test_layer_in_one_launch(request, d, H, dff, S, B, sp, lens, use_mask):
     """few rows: the whole layer as one launch (padded, and packed where lengths are given) against the oracle and
     against the separate launches; runs repeat bit for bit, also from a captured graph between eager runs"""
     from et_amd import lib
     from et_amd.encoder import Encoder_length
+    # (dense weights would have 80 rows run as separate launches)
+    request.addfinalizer(lambda: lib().et_tuning_set(b"layer_flow_rows", -1))
+    lib().et_tuning_set(b"layer_flow_rows", 96)
     r = rng(1300 + d + S * B)
     lins, ln = make_layer(r, d, dff, sp, seed=1400 + S, std=0.03, bias_std=0.05)
     mask = randn_h(r, (S, S), 0.5) if use_mask else None
-    enc = Encoder_length(d, S, H, workspace(Encoder_length, d, S, H, B), *build_linears(lins, B * S), *ln, mask, B)
+    work = workspace(Encoder_length, d, S, H, B).fill_(7.0)
+    enc = Encoder_length(d, S, H, work, *build_linears(lins, B * S), *ln, mask, B)
     xs = [randn_h(r, (B * S, d)) for _ in range(3)]
     for use in ([None, np.array(lens, np.int32)] if lens else [None]):
         enc.set_seq_lens(use)
@@ -589,11 +593,14 @@ def test_layer_in_one_launch(d, H, dff, S, B, sp, lens, use_mask):
             want = orc.encoder_tile_layer(x, lins, ln, mask, S, H, B, use, 1.0)
             check_close(g[valid], want[valid], what="layer in one launch")
             assert (np.delete(g, valid, 0) == 0).all()
+        if use is None:                 # (it is that form: the separate launches write the workspace)
+            assert (host(work) == 7.0).all()
         try:
             lib().et_tuning_set(b"layer_flow_rows", 0)
             steps = host(enc.run(torch.empty_like(dev(xs[0])), dev(xs[0])))
         finally:
-            lib().et_tuning_set(b"layer_flow_rows", -1)
+            lib().et_tuning_set(b"layer_flow_rows", 96)
+        assert (host(work) != 7.0).any()
         assert np.abs(steps.astype(np.float32) - got[0].astype(np.float32)).max() <= 2e-2
         x_static, out_static = torch.empty_like(dev(xs[0])), torch.empty_like(dev(xs[0]))
         side = torch.cuda.Stream()

@@ -90,8 +90,8 @@ TILE_CASES = [
     (48, 64, 96, 0.95, False),        # mostly empty block-rows
     (32, 32, 32, 1.0, True),          # no tile at all: Y = gelu(bias)
     (1, 128, 1024, 0.3, False),       # single row, odd tile counts
-    (257, 1040, 1008, 0.6, True),     # ragged everything, largest single-panel K
-    (40, 48, 1024, 0.5, False),       # smallest K that needs two chunks
+    (257, 1040, 1008, 0.6, True),     # ragged everything, one chunk of 1008 columns
+    (40, 48, 1024, 0.5, False),       # narrower than its input: two chunks
 ]
 
 
@@ -166,9 +166,21 @@ def test_tile_linear_fused_skip_layernorm(K, M, N, Kd, sp):
     want = orc.skip_layernorm(y, skip, g, b)
     want64 = orc.skip_layernorm(y, skip, g, b, f64=True)
     lt = Linear_tile(Kd, N, M, lin["row_offset"].size, lin["data"], lin["row_ptr"], lin["row_offset"], lin["bias"], False)
-    got = host(lt.run_ln(dev(X), dev(skip), dev(g), dev(b)))
-    check_close(got, want64, what="fused linear+LN vs f64")
-    check_close(got, want, what="fused linear+LN vs f32")
+    from et_amd import lib
+    got = host(lt.run_ln(dev(X), dev(skip), dev(g), dev(b)))     # so few panels: the two launches
+    try:
+        lib().et_tuning_set(b"tile_ln_min_panels", 1)            # the fused kernel wherever the rows fit one workgroup
+        lib().et_tuning_set(b"plan_dense", 0)
+        fused = host(lt.run_ln(dev(X), dev(skip), dev(g), dev(b)))
+        lib().et_tuning_set(b"tile_ln_chunked", 0)               # ... K in chunks through one panel buffer
+        single = host(lt.run_ln(dev(X), dev(skip), dev(g), dev(b)))
+    finally:
+        lib().et_tuning_set(b"tile_ln_min_panels", 0)
+        lib().et_tuning_set(b"plan_dense", 1)
+        lib().et_tuning_set(b"tile_ln_chunked", 1)
+    for res, name in ((got, "two launches"), (fused, "fused"), (single, "fused, one panel buffer")):
+        check_close(res, want64, what=f"linear+LN vs f64, {name}")
+        check_close(res, want, what=f"linear+LN vs f32, {name}")
     # against the two separate launches of this library: same linear, same
     # LayerNorm arithmetic, only the summation order of the row statistics differs
     two = lt.run(dev(X))
@@ -180,13 +192,10 @@ def test_tile_linear_fused_skip_layernorm(K, M, N, Kd, sp):
         sk = dev(skip)
         lt.run_ln(dev(X), sk, dev(g), dev(b), out=sk)
         inplace = host(sk)
-        if M > 256:
-            assert np.array_equal(inplace, got)
-        else:
-            # few rows: the call above ran the few-rows linear (a block-row's products summed in four
-            # parts) and the LayerNorm kernel, the in-place call the fused kernel - other summation order
-            assert np.abs(inplace.astype(np.float32) - got.astype(np.float32)).max() <= 2.0 ** -7
-            assert (inplace != got).mean() < 0.02
+        assert np.array_equal(inplace, fused)
+        # the two launches add a block-row's products in other parts
+        assert np.abs(inplace.astype(np.float32) - got.astype(np.float32)).max() <= 2.0 ** -7
+        assert (inplace != got).mean() < 0.02
 
 
 FFN_CASES = [
@@ -458,7 +467,7 @@ def test_tile_linear_multi_qkv_one_launch(K):
 @pytest.mark.parametrize("M", [200, 5700])
 def test_tile_linear_multi_unequal_widths(K, M):
     """Q and K narrower than V (attention-aware pruning): linears of different widths in one launch,
-    with column groups that exist for the widest one only (M = 5700 takes the 64-row kernel)"""
+    with column groups that exist for the widest one only"""
     from et_amd.encoder import Linear_tile, run_multi
     r = rng(33 + M)
     d = 768
@@ -466,26 +475,36 @@ def test_tile_linear_multi_unequal_widths(K, M):
     lins = [make_tile_linear(r, n, d, sp, seed=60 + j, std=0.05, bias_std=0.1) for j, (n, sp) in enumerate(zip(widths, (0.0, 0.5, 0.5)))]
     X = randn_h(r, (M, d))
     lts = [Linear_tile(d, l["N"], M, l["row_offset"].size, l["data"], l["row_ptr"], l["row_offset"], l["bias"]) for l in lins]
-    outs = [host(o) for o in run_multi(lts, dev(X))]
     rows = np.unique(np.concatenate([np.arange(0, 70), r.integers(0, M, 130), np.arange(M - 70, M)]))
-    for l, lt, o in zip(lins, lts, outs):
-        assert o.shape == (M, l["N"])
-        want = orc.tile_linear(X[rows], l["row_ptr"], l["row_offset"], l["data"], l["bias"], l["N"], f64=True)
-        check_close(o[rows], want, max_abs=2e-3, mean_rel=5e-4, what="multi, unequal widths")
-        assert np.array_equal(o, host(lt.run(dev(X))))   # the same linear launched alone
+    from et_amd import lib
+    try:
+        for height in (1, 0, 2):         # by estimated time, 32-row and 64-row panels
+            lib().et_tuning_set(b"tile_bm64", height)
+            outs = [host(o) for o in run_multi(lts, dev(X))]
+            for l, lt, o in zip(lins, lts, outs):
+                assert o.shape == (M, l["N"])
+                want = orc.tile_linear(X[rows], l["row_ptr"], l["row_offset"], l["data"], l["bias"], l["N"], f64=True)
+                check_close(o[rows], want, max_abs=2e-3, mean_rel=5e-4, what=f"multi, unequal widths, tile_bm64 {height}")
+                lib().et_tuning_set(b"plan_dense", 0)
+                assert np.array_equal(o, host(lt.run(dev(X))))   # the same linear launched alone
+                lib().et_tuning_set(b"plan_dense", 1)
+    finally:
+        lib().et_tuning_set(b"tile_bm64", 1)
+        lib().et_tuning_set(b"plan_dense", 1)
 
 
 @pytest.mark.parametrize("M,N,Kd,sp,gelu", [
     (128, 768, 3072, 0.0, False),   # BERT-base FFN2 on one sequence of 128, dense: four chunks, eight waves per block-row
     (128, 768, 3072, 0.8, False),
     (1, 768, 3072, 0.5, False), (17, 768, 3072, 0.8, True), (100, 256, 1536, 0.5, True),   # two chunks
-    (200, 768, 3072, 0.0, True),    # above 128 rows: dense plans only
-    (256, 768, 3072, 0.0, False), (64, 768, 6144, 0.8, False),   # eight chunks
+    (200, 768, 3072, 0.0, True),
+    (256, 768, 3072, 0.0, False), (64, 768, 4608, 0.8, False),   # six chunks
     (120, 48, 1040, 0.3, False),    # ragged second chunk (272 columns), three block-rows
 ])
 def test_tile_linear_few_rows_kernel(K, M, N, Kd, sp, gelu):
-    """K in several chunks and few rows: 16-row panels, a block-row's pairs split over several waves.
-    Against the oracle and against the kernels that take over from 257 rows (forced by the tuning key)."""
+    """K in several chunks and few rows: whole rows in LDS, a block-row's pairs split over several waves, against the
+    oracle and against the kernels that walk the chunks (both forced, a full plan's dense product switched off); and
+    whatever the estimated time chooses"""
     from et_amd import lib
     from et_amd.encoder import Linear_tile
     r = rng(34 + M + Kd)
@@ -495,12 +514,17 @@ def test_tile_linear_few_rows_kernel(K, M, N, Kd, sp, gelu):
     want = orc.tile_linear(X, lin["row_ptr"], lin["row_offset"], lin["data"], lin["bias"], N, f64=True)
     if gelu:
         want = orc.gelu(want)
-    got = host(lt.run(dev(X)))
+    auto = host(lt.run(dev(X)))
     try:
+        lib().et_tuning_set(b"plan_dense", 0)
+        lib().et_tuning_set(b"tile_splitk_rows", M)
+        got = host(lt.run(dev(X)))
         lib().et_tuning_set(b"tile_splitk_rows", 0)
         other = host(lt.run(dev(X)))
     finally:
         lib().et_tuning_set(b"tile_splitk_rows", -1)
+        lib().et_tuning_set(b"plan_dense", 1)
+    check_close(auto, want, max_abs=4e-3, mean_rel=5e-4, what="automatic choice")
     check_close(got, want, max_abs=4e-3, mean_rel=5e-4, what="few-rows kernel")
     check_close(other, want, max_abs=4e-3, mean_rel=5e-4, what="general kernel, few rows")
     assert np.abs(got.astype(np.float32) - other.astype(np.float32)).max() <= 2.0 ** -7
@@ -571,8 +595,8 @@ def test_tile_linear_full_size_config2_rows_sample(K, sp, ntile):
     normal = np.abs(got) >= 2.0 ** -13
     assert np.array_equal(got2[normal], (got * np.float16(2))[normal])
     assert np.abs(got2.astype(np.float64) - 2 * got.astype(np.float64))[~normal].max() <= 2.0 ** -23
-    # the planned form of the same linear (Linear_tile::run: the 64-row resident kernel that the encoders
-    # and the benchmark run at this size), its index arrays from the product's own generator and packer
+    # the planned form of the same linear (Linear_tile::run: what the encoders run at this size, the tile kernel and at
+    # 0 % the dense product), its index arrays from the product's own generator and packer
     from et_amd import formats
     from et_amd.encoder import Linear_tile
     rp, ro = formats.gen_sparse_tile_mat(N, Kd, sp, 2024)
@@ -1119,7 +1143,8 @@ def test_microbenchmarks_report_plausible_rates():
     (300, 1040, 1040, 0.7, True),   # two chunks, the second 272 columns; ragged column groups
     (1000, 768, 3072, 0.8, False), (2050, 784, 3072, 0.95, False),   # several block-rows per wave; empty ones
     (40, 64, 2048, 1.0, True),      # no tile at all
-    (4100, 64, 1024, 0.5, False), (2050, 1040, 1008, 0.8, True),   # single panel beyond 816 columns: 64-row items
+    (4100, 64, 1024, 0.5, False),   # narrower than its input: two chunks
+    (4100, 1024, 1024, 0.9, False), (2050, 1040, 1008, 0.8, True),   # one chunk beyond 816 columns: 64-row panels too
 ])
 def test_tile_linear_whole_rows(K, M, N, Kd, sp, gelu):
     """planned and raw (unsorted lists, odd counts) linears on whole rows in LDS, at the edges of that kernel's range"""
@@ -1137,6 +1162,16 @@ def test_tile_linear_whole_rows(K, M, N, Kd, sp, gelu):
     planned = host(lt.run(dev(X)))
     check_close(planned[rows], want, max_abs=tol, mean_rel=5e-4, what="planned")
     assert np.array_equal(planned, host(lt.run(dev(X))))
+    from et_amd import lib
+    for keys in (((b"tile_splitk_rows", M, -1), (b"tile_splitk_k1", 1, 0)), ((b"tile_bm64", 2, 1), (b"tile_splitk_rows", 0, -1))):
+        try:
+            for key, value, _ in keys:
+                lib().et_tuning_set(key, value)
+            forced = host(lt.run(dev(X)))
+        finally:
+            for key, _, off in keys:
+                lib().et_tuning_set(key, off)
+        check_close(forced[rows], want, max_abs=tol, mean_rel=5e-4, what=f"planned, {keys[0][0]}")
 
 
 @pytest.mark.parametrize("M", [1, 33, 700, 5700])
