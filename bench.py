@@ -36,7 +36,7 @@ D, H, DFF = 768, 12, 3072
 # WRITE_SIZE, scaled by the 64 MiB copy kernel launched below).  The summary records a fingerprint of the kernel
 # sources it was measured on; when the sources have changed since, `traffic` is null rather than a stale figure.
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "encoder_layer_b16_s512_hbm_traffic.txt")
-KERNEL_SOURCES = ("tile_linear.hip", "tile_tail.hip", "tile_plan.h", "attention.hip", "skip_layernorm.hip", "common.h")
+KERNEL_SOURCES = tuple(sorted(f for f in os.listdir(os.path.join(ROOT, "et_amd", "csrc")) if f.endswith((".hip", ".h"))))
 TRAFFIC_KERNELS = {  # bench line -> kernel instance in the profile summary (the default workload's launches)
     "tile_linear qkv (3 x 768->768, one launch)": "et::tile_linear_resident_kernel<2, false, 12, false, 64>",
     "attention (on-the-fly)": "et::attention_kernel<64, 2, 4, false, false, true, 64, false>",

@@ -34,6 +34,24 @@ def test_traffic_is_read_per_kernel_instance_and_dropped_when_stale(tmp_path, mo
     assert bench.measured_traffic_mib() == {}
 
 
+def test_fingerprint_covers_every_kernel_source():
+    """a change in any file that the library's kernels are built from makes the profile summaries stale"""
+    import re
+    import bench
+    from et_amd import build
+    csrc = os.path.join(ROOT, "et_amd", "csrc")
+    want = {f for f in build.SOURCES if f.endswith(".hip")}
+    for f in sorted(want):
+        todo = [f]
+        while todo:
+            for inc in re.findall(r'^#include "([^"/]+)"', open(os.path.join(csrc, todo.pop())).read(), flags=re.M):
+                if inc not in want:
+                    want.add(inc)
+                    todo.append(inc)
+    assert "attention_block.h" in want and "layer_flow.hip" in want
+    assert want <= set(bench.KERNEL_SOURCES)
+
+
 def test_more_than_one_gpu_is_refused():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0
