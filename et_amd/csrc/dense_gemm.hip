@@ -308,6 +308,8 @@ static int dg_choose(const int *Ns, int nlin, int M, int K, double *us) {
 }
 double dense_gemm_estimate(const int *Ns, int nlin, int M, int K) {
     double us = 0.0;
+    if (g_dense_form >= 0)
+        return dg_estimate(g_dense_form, Ns, nlin, M, K);
     dg_choose(Ns, nlin, M, K, &us);
     return us;
 }

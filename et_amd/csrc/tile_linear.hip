@@ -1720,6 +1720,7 @@ static int tile_launch_ln(const TlProblem &p, const f16 *X, int M, int K, int KC
 static int g_tile_nb = 0;
 static int g_tile_min_wgs = 512;
 static int g_tile_ipw = 0;
+static int g_tile_form = -1; // et_tuning_set("tile_form"): index in tl_forms
 static int g_tile_fuse_ln = 1;
 static int g_tile_min_panels = 0; // fewest panels of the fused linear + LayerNorm and layer tail kernels, 0 = automatic
 // the layer tail's choice is forced (a layer then runs its steps as separate launches)
@@ -1811,13 +1812,20 @@ static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, 
     const double x_mb = 2e-6 * M * K;
     const int fnb = g_tile_nb >= 1 && g_tile_nb <= 3 ? g_tile_nb : 0;
     TlChoice best = {};
+    auto lds_of = [&](const TlForm &f) {
+        return (size_t)f.rows * (K + ((K & 31) ? 0 : TL_PAD)) * sizeof(f16) +
+               (size_t)f.waves * f.rows * (16 * f.nb + 8) * sizeof(f16);
+    };
+    const TlForm *only = nullptr; // (tuning)
+    if (g_tile_form >= 0 && g_tile_form < (int)(sizeof(tl_forms) / sizeof(tl_forms[0])) &&
+        lds_of(tl_forms[g_tile_form]) <= 160 * 1024)
+        only = &tl_forms[g_tile_form];
     for (const TlForm &f : tl_forms) {
-        if (f.rows == TL_BM ? (fnb ? f.nb != fnb : g_tile_bm64 == 2) : fnb || g_tile_bm64 == 0)
+        if (only ? &f != only
+                 : (f.rows == TL_BM ? (fnb ? f.nb != fnb : g_tile_bm64 == 2) : fnb || g_tile_bm64 == 0) ||
+                       (f.waves == 12 && g_tile_bm64 == 4))
             continue; // (tuning; a form of either height fits every K of one chunk)
-        if (f.waves == 12 && g_tile_bm64 == 4)
-            continue;
-        const size_t lds = (size_t)f.rows * (K + ((K & 31) ? 0 : TL_PAD)) * sizeof(f16) +
-                           (size_t)f.waves * f.rows * (16 * f.nb + 8) * sizeof(f16);
+        const size_t lds = lds_of(f);
         if (lds > 160 * 1024)
             continue;
         const TlCost &c = f.rows == TL_BM ? tl_cost32 : f.waves == 8 ? tl_cost64 : tl_cost64x12;
@@ -1828,7 +1836,16 @@ static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, 
         const double per_item = c.item + f.nb * (c.item_nb + c.item_stream * pairs);
         const double cu_item = G * f.rows * (c.out + (gelu ? c.gelu : 0.0) + c.mfma * pairs);
         const double fixed = c.launch + c.result * result;
-        for (int d = 1; d <= per_panel && d <= 16; d++) { // (beyond 16 items a workgroup the tail of the launch shows)
+        // (beyond 16 items a workgroup the tail of the launch shows; a tuning value counts down to a whole number of
+        // workgroups per panel)
+        int first = 1, last = std::min(per_panel, 16);
+        if (g_tile_ipw > 0) {
+            first = std::min(g_tile_ipw, per_panel);
+            while (per_panel % first)
+                first--;
+            last = first;
+        }
+        for (int d = first; d <= last; d++) {
             if (per_panel % d)
                 continue;
             const long groups = per_panel / d, nwg = panels * groups;
@@ -1880,9 +1897,22 @@ static int choose_chunked(const TlProblem *probs, int nlin, int M, int K, int nc
         w_mb += p * probs[i].nbr * 1024e-6;
     }
     const double x_mb = 2e-6 * M * K;
+    auto estimate = [&](int which) {
+        return which == TL_BY_ROWS   ? tile_rows_estimate(M, K, nbr_max, nlin, pairs, w_mb)
+               : which == TL_BY_PLAN ? estimate_plan_kernel(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, cus)
+                                     : estimate_chunked(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, which, cus);
+    };
+    const bool rows_fit = tile_rows_fits(K);
     int best = TL_BY_PLAN;
-    *us = estimate_plan_kernel(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, cus);
-    auto take = [&](int which, double t) {
+    if (rows_fit && g_tile_rows_most >= 0 && M <= g_tile_rows_most)
+        best = TL_BY_ROWS; // (tuning)
+    else if (g_tile_chunked > 0)
+        best = std::min(g_tile_chunked, 4);
+    *us = estimate(best);
+    if (best != TL_BY_PLAN)
+        return best;
+    auto take = [&](int which) {
+        const double t = estimate(which);
         if (t < *us) {
             *us = t;
             best = which;
@@ -1890,16 +1920,35 @@ static int choose_chunked(const TlProblem *probs, int nlin, int M, int K, int nc
     };
     if (g_tile_chunked < 0)
         for (int nb = 1; nb <= 4; nb++)
-            take(nb, estimate_chunked(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, nb, cus));
-    if (g_tile_chunked > 0)
-        best = g_tile_chunked;
-    if (tile_rows_fits(K)) {
-        if (g_tile_rows_most >= 0)
-            best = M <= g_tile_rows_most ? TL_BY_ROWS : best;
-        else if (g_tile_chunked <= 0)
-            take(TL_BY_ROWS, tile_rows_estimate(M, K, nbr_max, nlin, pairs, w_mb));
-    }
+            take(nb);
+    if (rows_fit && g_tile_rows_most < 0)
+        take(TL_BY_ROWS);
     return best;
+}
+
+// the tile kernels' estimated time for planned linears over one input, launches of their own added up (join_launches)
+static double tiles_estimate(const int *out_feat, const int *ntile, const int *nchunk, const int *launch, int launches, int n,
+                             int M, int K, bool gelu) {
+    double sum = 0.0;
+    for (int l = 0; l < launches; l++) {
+        TlProblem probs[TL_MAX_LIN];
+        int m = 0, chunks = 0, nbr_max = 0;
+        for (int i = 0; i < n; i++)
+            if (launch[i] == l) {
+                probs[m].N = out_feat[i];
+                probs[m].nbr = out_feat[i] / 16;
+                probs[m].ntile = ntile[i];
+                chunks = nchunk[i];
+                nbr_max = std::max(nbr_max, probs[m++].nbr);
+            }
+        double us;
+        if (chunks > 1)
+            (void)choose_chunked(probs, m, M, K, chunks, nbr_max, &us);
+        else
+            us = choose_resident(probs, m, M, K, nbr_max, gelu).us;
+        sum += us;
+    }
+    return sum;
 }
 
 template <int NB, bool GELU, int NW = TL_WAVES>
@@ -1981,7 +2030,7 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
     if (mode == TL_PLAN && nchunk == 1) { // (on whole rows: returned above)
         const TlChoice c = choose_resident(probs, nlin, M, K, nbr_max, gelu);
         a.ncg = c.ncg;
-        a.ipw = g_tile_ipw > 0 ? g_tile_ipw : c.d;
+        a.ipw = c.d;
         if (c.form->rows == TL_BM64) {
             place(TL_BM64, c.by_group);
             if (c.form->waves == 12)
@@ -2100,6 +2149,10 @@ extern "C" int et_tuning_set(const char *key, int value) {
         et::g_tile_splitk_k1 = value;
         return ET_OK;
     }
+    if (key && !strcmp(key, "tile_form")) {
+        et::g_tile_form = value;
+        return ET_OK;
+    }
     if (key && !strcmp(key, "dense_form")) {
         et::set_dense_form(value);
         return ET_OK;
@@ -2216,36 +2269,19 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
-    int Ns[3], KC[3], nchunk[3], launch[3];
+    int Ns[3], ntile[3], KC[3], nchunk[3], launch[3];
     for (int i = 0; i < n; i++) {
         if (!plans[i]->d_dense)
             return false;
         Ns[i] = plans[i]->out_feat;
+        ntile[i] = plans[i]->ntile;
         KC[i] = plans[i]->KC;
         nchunk[i] = plans[i]->nchunk;
     }
     if (g_plan_dense == 2)
         return true;
     const int K = plans[0]->in_feat, launches = join_launches(KC, nchunk, n, launch);
-    double tiles = 0.0;
-    for (int l = 0; l < launches; l++) {
-        TlProblem probs[3];
-        int m = 0, chunks = 0, nbr_max = 0;
-        for (int i = 0; i < n; i++)
-            if (launch[i] == l) {
-                probs[m].N = Ns[i];
-                probs[m].nbr = Ns[i] / 16;
-                probs[m].ntile = plans[i]->ntile;
-                chunks = nchunk[i];
-                nbr_max = std::max(nbr_max, probs[m++].nbr);
-            }
-        double us;
-        if (chunks > 1)
-            (void)choose_chunked(probs, m, M, K, chunks, nbr_max, &us);
-        else
-            us = choose_resident(probs, m, M, K, nbr_max, gelu).us;
-        tiles += us;
-    }
+    const double tiles = tiles_estimate(Ns, ntile, nchunk, launch, launches, n, M, K, gelu);
     return 2.4 + dense_gemm_estimate(Ns, n, M, K) < tiles;
 }
 static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
@@ -2503,6 +2539,24 @@ extern "C" int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *co
         if (rc != ET_OK)
             return rc;
     }
+    return ET_OK;
+}
+
+extern "C" int et_tile_plan_estimate(int in_feat, const int *out_feat, const int *ntile, int n, int M, int gelu,
+                                     double *tiles_us, double *dense_us) {
+    using namespace et;
+    ET_REQUIRE(out_feat && ntile && tiles_us && dense_us, ET_ERR_INVALID_ARG, "et_tile_plan_estimate: null pointer");
+    ET_REQUIRE(in_feat > 0 && in_feat % 16 == 0 && M > 0 && n >= 1 && n <= TL_MAX_LIN, ET_ERR_INVALID_ARG,
+               "et_tile_plan_estimate: in_feat=%d M=%d n=%d", in_feat, M, n);
+    int KC[TL_MAX_LIN], nchunk[TL_MAX_LIN], launch[TL_MAX_LIN];
+    for (int i = 0; i < n; i++) {
+        ET_REQUIRE(out_feat[i] > 0 && out_feat[i] % 16 == 0 && ntile[i] >= 0, ET_ERR_INVALID_ARG,
+                   "et_tile_plan_estimate: out_feat=%d ntile=%d", out_feat[i], ntile[i]);
+        plan_chunking(in_feat, out_feat[i], &KC[i], &nchunk[i]);
+    }
+    const int launches = join_launches(KC, nchunk, n, launch);
+    *tiles_us = tiles_estimate(out_feat, ntile, nchunk, launch, launches, n, M, in_feat, gelu != 0);
+    *dense_us = dense_gemm_estimate(out_feat, n, M, in_feat);
     return ET_OK;
 }
 

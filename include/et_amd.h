@@ -342,7 +342,12 @@ int et_tile_plan_run_multi(const et_tile_plan *const *plans, void *const *Ys,
  * linear that narrows its input are others than those of one that does not. */
 int et_tile_plan_launches(int in_feat, const int *out_feat, int n, int *launch,
                           int *nchunk, int *chunk_cols);
-/* device pointers of the plan's buffers, for tests (sorted order) */
+/* Host only: the estimated microseconds by which the form of a launch is chosen, for linears of in_feat x out_feat[i] with
+ * ntile[i] tiles over M rows - on the tile kernels, and as a dense product (what plans of full matrices may take).
+ * Follows the tuning keys: a forced form's own estimate. */
+int et_tile_plan_estimate(int in_feat, const int *out_feat, const int *ntile, int n, int M, int gelu,
+                          double *tiles_us, double *dense_us);
+/* a plan's sizes and its column chunks */
 int et_tile_plan_query(const et_tile_plan *plan, int *in_feat, int *out_feat,
                        int *ntile, int *nchunk, int *chunk_cols);
 
@@ -478,6 +483,10 @@ int et_device_synchronize(void);
  *                     (default): by size and density
  *   "tile_order"      consecutive workgroups of a linear share 0: a row panel, 2:
  *                     a column group, 1 (default): what moves fewer bytes
+ *   "tile_form"       form of a planned linear of one chunk: 0 .. 2: 32 rows, eight
+ *                     waves of 1 .. 3 block-rows; 3: 64 rows, twelve waves of 2; 4
+ *                     .. 6: 64 rows, eight waves of 3, 2, 1; -1 (default) and where
+ *                     the form does not fit the LDS: by estimated time
  *   "tile_bm64"       panels of a planned linear of one chunk: 0: 32 rows; 2: 64
  *                     rows; 1 (default): the less estimated time; 4: as 1
  *                     without the twelve-wave form

@@ -1,0 +1,78 @@
+"""The program that keeps the linear forms' times and fits (CPU part): its terms are the library's."""
+import ctypes as C
+import os
+import re
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "et_amd", "bench"))
+
+import linear_forms as lf  # noqa: E402
+from et_amd import lib  # noqa: E402
+
+
+def library_estimate(line, **keys):
+    L, n = lib(), len(line["outputs"])
+    K = line["inputs"]
+    tiles = [int((K // 16) * (v // 16) * (1.0 - line["sparsity"])) for v in line["outputs"]]
+    t, g = C.c_double(), C.c_double()
+    try:
+        for k, v in keys.items():
+            assert L.et_tuning_set(k.encode(), v[0]) == 0
+        assert L.et_tile_plan_estimate(K, (C.c_int * n)(*line["outputs"]), (C.c_int * n)(*tiles), n, line["rows"],
+                                       line["gelu"], C.byref(t), C.byref(g)) == 0
+    finally:
+        for k, v in keys.items():
+            L.et_tuning_set(k.encode(), v[1])
+    return t.value
+
+
+def panel_costs():
+    src = open(os.path.join(ROOT, "et_amd", "csrc", "tile_linear.hip")).read()
+    return {name: [float(v) for v in re.search(key + r" = \{([^}]*)\}", src).group(1).split(",")]
+            for name, key in (("32 rows", "tl_cost32"), ("64 rows", "tl_cost64"), ("64 rows, 12 waves", "tl_cost64x12"))}
+
+
+@pytest.mark.parametrize("rows", [37, 700, 9000])
+@pytest.mark.parametrize("K,Ns,gelu", lf.PANEL)
+def test_panel_terms_add_up_to_the_estimate(K, Ns, gelu, rows):
+    costs, cus = panel_costs(), max(lib().et_device_cu_count(), 1)
+    for k, (height, waves, nb) in enumerate(lf.FORMS):
+        if height * (K + 16) * 2 + waves * height * (16 * nb + 8) * 2 > 160 * 1024:
+            continue
+        per = lf.up(max(Ns) // 16, waves * nb) * len(Ns)
+        for d in {1, per if per <= 16 else 1}:
+            line = dict(inputs=K, outputs=Ns, gelu=gelu, sparsity=0.8, rows=rows, form=f"panel{k}", d=d)
+            name, terms = lf.features(line, cus)
+            want = library_estimate(line, tile_form=(k, -1), tile_ipw=(d, 0))
+            assert len(terms) == len(lf.TERMS[name])
+            assert sum(c * v for c, v in zip(costs[name], terms)) == pytest.approx(want, rel=1e-9)
+
+
+@pytest.mark.parametrize("rows", [37, 700, 9000])
+@pytest.mark.parametrize("K,Ns,gelu", lf.CHUNKS)
+def test_chunk_terms_follow_the_estimate(K, Ns, gelu, rows):
+    """the constants stand in the library's formulas: the terms have to span the same differences"""
+    cus = max(lib().et_device_cu_count(), 1)
+    for form, keys, const in (
+            ("chunk", dict(tile_chunked=(0, -1), tile_splitk_rows=(0, -1)),
+             (1.367, 0.9615, 0.0867, 0.4349, 0.01745, 0.6037, 0.0673)),
+            ("fetch1", dict(tile_chunked=(1, -1), tile_splitk_rows=(0, -1)),
+             (1.775, 1.997, 0.378, 0.233, 0.0397, 0.0140, 0.00429, 0.0980)),
+            ("fetch4", dict(tile_chunked=(4, -1), tile_splitk_rows=(0, -1)),
+             (1.775, 1.997, 0.378, 0.233, 0.0397, 0.0140, 0.00429, 0.0980)),
+            ("rows", dict(tile_splitk_rows=(1 << 20, -1)), (1.75, 0.0514, 0.4525, 43.3e-5, 1.093e-2, 1.4, 0.0825))):
+        line = dict(inputs=K, outputs=Ns, gelu=gelu, sparsity=0.5, rows=rows, form=form, d=0)
+        name, terms = lf.features(line, cus)
+        assert len(terms) == len(lf.TERMS[name]) == len(const)
+        assert sum(c * v for c, v in zip(const, terms)) == pytest.approx(library_estimate(line, **keys), rel=1e-6), form
+
+
+def test_times_are_read_back(tmp_path):
+    p = tmp_path / "times.txt"
+    p.write_text("A heading.\n\n768 768+768 1 0.8 100 panel3 2 7.25 6.90\n768 768+768 1 0.8 100 auto 0 7.10 6.90\n")
+    a, b = lf.read(p)
+    assert a["outputs"] == (768, 768) and a["form"] == "panel3" and a["d"] == 2 and a["us"] == 7.25 and a["est"] == 6.9
+    assert lf.shape_of(a) == lf.shape_of(b)
