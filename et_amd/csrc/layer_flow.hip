@@ -48,8 +48,8 @@
 // a wave has its whole share of W in registers before it waits, and the partial
 // sums meet in LDS in a fixed order.  The projections and the first feed-forward
 // linear hold the 16-row panel in LDS; the second feed-forward linear (hidden
-// width: too wide for a panel) reads its operand from memory, one block-row per
-// workgroup and only the surviving tiles' columns.  The first LayerNorm is
+// width: too wide for a panel) reads its operand from memory, only the surviving
+// tiles' columns, two block-rows per workgroup with eight waves each.  The first LayerNorm is
 // recomputed by every workgroup of the first feed-forward linear that needs the
 // rows (one hand-over less).  Attention: attention_block, 256 query rows per
 // unit and head.
@@ -173,9 +173,8 @@ __device__ __forceinline__ void lf_multiply_direct(f32x4 &acc, LfPairs<LF_D> &p,
 
 // Sums of the split waves meet in LDS (`red`, free for everyone once the barrier
 // in front is passed) and are added in the order of the split; bias, GELU, half,
-// 8-byte stores of four consecutive features.  The rows of subtile ms of a
-// block-row are finished by the block-row's wave ms (split >= 2) or by the one
-// wave (split 1).
+// 8-byte stores of four consecutive features: by the first of the waves that
+// share the block-row.
 __device__ __forceinline__ f16x4 lf_bias(const LfLinear &l, int bn, int lane) {
     return *reinterpret_cast<const f16x4 *>(l.bias + min(bn, l.nbr - 1) * 16 + (lane >> 4) * 4);
 }
@@ -206,9 +205,8 @@ __device__ __forceinline__ void lf_finish(const LfArgs &a, f32x4 acc, f32x4 *red
     lf_put<GELU>(a, acc, bias, Y, N, bn, m0 + c16, g4);
 }
 
-// one row is spread over the wave in 16-byte pieces (the math and the order of summation of skip_layernorm.hip)
-// LayerNorm(y + skip) of one row, spread over the wave in 16-byte pieces.  Every load is requested before the first
-// value is used.  put(piece, values).
+// LayerNorm(y + skip) of one row, spread over the wave in 16-byte pieces (the math and the order of summation of
+// skip_layernorm.hip).  Every load is requested before the first value is used.  put(piece, values).
 template <class Put>
 __device__ __forceinline__ void lf_layernorm(const LfArgs &a, const f16 *Y, const f16 *S, const f16 *gamma,
                                              const f16 *beta, int row, int lane, Put &&put) {

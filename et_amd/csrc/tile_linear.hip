@@ -27,9 +27,11 @@
 // Kernels in this file: tile_linear_resident_kernel (K in one panel: persistent
 // workgroups, 32- or 64-row panels, optional LayerNorm epilogue),
 // tile_linear_plan_kernel (K in chunks), tile_linear_chunked_kernel (K in
-// chunks + LayerNorm, double-buffered panels with a fetching wave),
-// tile_ffn_fused_kernel (feed-forward block / whole layer tail in one launch,
-// hidden activations in LDS), tile_linear_generic_kernel (raw and dense input).
+// chunks, double-buffered panels with fetching waves, optional LayerNorm
+// epilogue), tile_ffn_fused_kernel (feed-forward block / whole layer tail in one
+// launch, hidden activations in LDS), tile_linear_generic_kernel (raw and dense
+// input).  Whole rows in LDS (tile_rows.hip) and the dense product
+// (dense_gemm.hip) are launched from here where they are the shorter launch.
 #include "tile_plan.h"
 #include "tile_walk.h"
 
@@ -623,17 +625,14 @@ __device__ __forceinline__ void tl_ln_rows_at(const TlLnOperands<NB, NW, NLW> &o
 }
 
 // ---------------------------------------------------------------------------
-// Plan kernel (the fast path).
+// Plan kernel: K in chunks, one panel buffer.
 //
-// Work items are (row panel, linear, column group) triples, numbered with the
-// row panel slowest.  A workgroup is persistent over `ipw` consecutive items:
-// as long as the row panel does not change (and K fits one chunk) the X panel
-// stays in LDS, so it is fetched once for several column groups, and because
-// every wave stages its output through a private LDS tile the waves never
-// meet at a barrier between items - one wave's stores overlap the others'
-// MFMAs and the next item's weight loads.
+// A workgroup does one (row panel, linear, column group): it fetches a chunk of
+// the panel, waits, multiplies and goes on to the next chunk; every wave stages
+// its output through a private LDS tile, so one wave's stores overlap the
+// others' MFMAs.
 //
-// Within an item a wave owns NB CONSECUTIVE block-rows, and the plan stores
+// A wave owns NB CONSECUTIVE block-rows, and the plan stores
 // tiles in (chunk, block-row) order with even segments, so the wave's work for
 // a chunk is ONE contiguous stream of tile pairs: 1 KB of W per pair at an
 // address that is linear in the pair index, plus one int per half-wave giving
@@ -676,7 +675,7 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(const TlArgs 
 #define TL_PANEL_LOAD(c_)                                                                         \
     {                                                                                             \
         const int pk0 = (c_) * a.KC;                                                              \
-        const int pcpr = min(a.KC, a.K - pk0) >> 3; /* 16-byte chunks per row, <= 124 */          \
+        const int pcpr = min(a.KC, a.K - pk0) >> 3; /* 16-byte chunks per row, <= 96 */           \
         _Pragma("unroll") for (int rr = 0; rr < TL_BM / NW; rr++) {                               \
             const int row = x.wave * (TL_BM / NW) + rr;                                           \
             if (x.m0 + row < a.M) {                                                               \
@@ -1045,7 +1044,7 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_kernel(const 
 #define TL_FETCH(c_)                                                                              \
     {                                                                                             \
         const int pk0 = (c_) * a.KC;                                                              \
-        const int pcpr = min(a.KC, a.K - pk0) >> 3; /* 16-byte pieces per row, <= 124 */          \
+        const int pcpr = min(a.KC, a.K - pk0) >> 3; /* 16-byte pieces per row, <= 96 */           \
         f16 *dst = xs + ((c_) & 1) * pbuf;                                                        \
         const int row1 = min(row0 + TL_BM / TL_FWAVES, a.M - x.m0);                               \
         for (int row = row0; row < row1; row++) {                                                 \
@@ -1694,7 +1693,7 @@ static int tile_launch_ln(const TlProblem &p, const f16 *X, int M, int K, int KC
     a.beta = beta;
     const size_t lds_x = (size_t)TL_BM * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16);
     // K in chunks and rows narrow enough for twelve waves of <= 4 block-rows:
-    // the double-buffered kernel with a fetching wave
+    // the double-buffered kernel with fetching waves
     const int cnb = (p.nbr + TL_CWAVES - 1) / TL_CWAVES;
     if (nchunk > 1 && cnb <= 4 && g_tile_ln_chunked) {
         const size_t lds = 2 * lds_x + (size_t)TL_CWAVES * TL_BM * (16 * cnb + 8) * sizeof(f16);
@@ -1757,7 +1756,7 @@ static int g_tile_rows_most = -1; // et_tuning_set("tile_splitk_rows"): most row
 static int g_tile_splitk_k1 = 0;  // et_tuning_set("tile_splitk_k1"): also plans of one chunk, up to that many rows (automatic: 128)
 
 static int g_tile_order = 1; // et_tuning_set("tile_order"): 0 panels slowest, 2 column groups slowest, 1 fewer bytes
-// Whether consecutive workgroups walk the panels of a column group (see tl_items): X and W in bytes, numbers of panels
+// Whether consecutive workgroups walk the panels of a column group (tl_place): X and W in bytes, numbers of panels
 // and of workgroups per panel.  Every L2 that has part of the work takes what all of the work shares, so W times eight
 // is what bounds a launch of few rows: 256 rows, 1024 -> 4096: dense 14.2 -> 6.6 us, 50 % 10.0 -> 5.6; 768 -> 3072
 // dense 9.7 -> 5.9; 128 rows 3072 -> 768 dense 9.8 -> 6.8.  Only up to x_most bytes of X: beyond, the L2s have time
@@ -1781,7 +1780,9 @@ double tl_traffic_mb(double x_mb, double w_mb, long panels, long groups, double 
 // inputs, 512 .. 4096 outputs, one or three linears, 0 .. 90 % pruned, 37 .. 32768 rows; 5 to 6 % off in the mean) and
 // are then moved by up to a factor of two where that brings the choice closer to the fastest form: 0.5 % from it in the
 // mean, 13 % at most (0.6 % where half of the row counts was left out); the rule before, a number of workgroups to aim
-// for, was 6.3 %.  1536 rows 768 -> 3072, 50 %: 13.8 -> 11.7 us; 3500 rows 768 -> 768, 90 %: 7.3 -> 5.8; 2700 rows
+// for, was 6.3 %.  bench/linear_forms.py times the forms and fits the terms anew: on its 320 linears (launches of a graph)
+// the estimates are 4 to 7 % off and all choices of this file together 1.3 % behind the fastest form, 20 % at most (2048
+// -> 512 dense, 1343 rows: 12.7 against 10.6 us).  1536 rows 768 -> 3072, 50 %: 13.8 -> 11.7 us; 3500 rows 768 -> 768, 90 %: 7.3 -> 5.8; 2700 rows
 // 768 -> 3072, 80 %: 16.1 -> 12.4.
 struct TlForm {
     int rows, waves, nb;
@@ -1870,7 +1871,8 @@ static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, 
 // Terms: launch, rounds of workgroups and their chunks, the stream of a wave's pairs, the work of the busiest CU, and
 // the megabytes that the L2s take in; fitted like the single-panel forms to 1600 launches (2048 -> 512, 3072 -> 768,
 // 4096 -> 1024, 0 to 90 % pruned, 48 to 16384 rows): 5 to 6 % off in the mean, the choice 0.2 % behind the fastest
-// kernel, 9 % at most (the rule before: 10.9 %).
+// kernel, 9 % at most (the rule before: 10.9 %).  The 576 launches that bench/linear_forms.py times in graphs: 14, 6 and
+// 9 % off.
 enum { TL_BY_ROWS = -1, TL_BY_PLAN = 0 }; // or 1 .. 4: fetching waves, that many block-rows per computing wave
 static double estimate_plan_kernel(int M, double pairs, double x_mb, double w_mb, int nchunk, int nbr_max, int nlin, long cus) {
     const long panels = (M + TL_BM - 1) / TL_BM;
@@ -2001,7 +2003,10 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         LfLinear l[TL_MAX_LIN];
         f16 *Ys[TL_MAX_LIN];
         for (int i = 0; i < nlin; i++) {
-            const double p = raw ? 0.1 * K / 16 : 0.5 * probs[i].ntile / probs[i].nbr; // (raw: the count is on the device)
+            // (a raw list's length is on the device: 80 % pruned is assumed.  That only decides the split; with the true
+            // density the launch takes the same time within 2 % from 16 to 4096 rows and 0 to 90 %, but for dense lists
+            // over 3072 columns at 200 rows, 11.6 against 8.7 us, and 2000 rows, 48.5 against 44.1)
+            const double p = raw ? 0.1 * K / 16 : 0.5 * probs[i].ntile / probs[i].nbr;
             l[i] = LfLinear{probs[i].data, probs[i].cptr, probs[i].row_offset, probs[i].bias, probs[i].nbr,
                             raw ? 1 : nchunk, raw ? 0 : KC * 2, probs[i].npair};
             Ys[i] = probs[i].Y;
@@ -2265,7 +2270,10 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 
 // Plans of fully populated matrices: the dense product where it is estimated to be the shorter launch, from some hundred
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
-// tile: their time is that of the choice among their forms.
+// tile: their time is that of the choice among their forms.  The 2.4 us stand for the launch,
+// which dense_gemm_estimate leaves out.  Over 80 full plans (bench/linear_forms.py, launches of a graph) the choice is then
+// 0.7 % behind the faster side in the mean and 15 % at most; 0.9 and 32 % with nothing on top, 0.4 and 15 % with 1.2 us,
+// 1.2 and 21 % with 3.6.
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
@@ -2593,6 +2601,11 @@ static bool ln_fusion_pays(int M) {
 // past a panel, whatever the number of panels.  Whole layers, one launch / steps, us: 768 wide 50 %: 3072 rows 92 / 78,
 // 4096 93 / 85, 5120 98 / 107; 80 %: 2560 rows 59 / 56, 3072 64 / 62, 3584 64 / 65; 90 %: 2560 52 / 52, 3072 56 / 57;
 // 512 wide, 50 %: 3072 57 / 55, 3584 57 / 58.
+// The same line decides for the panels of a last round behind full ones (et_tile_plan_run_tail), where the steps' launches
+// come on top of the fused one.  Tail behind 256 full panels, last round fused / by steps, us: 768 wide 50 % (line 144): 80
+// panels 150 / 127, 128 143 / 141, 144 145 / 155; 80 % (99): 52 87 / 79, 80 87 / 85, 96 87 / 88, 112 87 / 92; 90 % (84): 64
+// 73 / 70, 80 73 / 74, 96 73 / 77; 512 wide 50 % (103): 96 79 / 78, 112 79 / 80; 80 % (83): 52 54 / 54, 80 54 / 58 - the
+// furthest that it is off.  Behind 512 full panels the same.
 static int tail_min_panels(const et_tile_plan *pO, const et_tile_plan *p1, const et_tile_plan *p2) {
     if (et::g_tile_min_panels)
         return et::g_tile_min_panels;

@@ -46,10 +46,7 @@ struct TrArgs {
 struct TrRawWalk {
     int t, end;
 };
-struct TrSlots {
-    f16x8 w[LF_D];
-    int o[LF_D], co[LF_D]; // co: RAW: tiles in the slot, else byte offset of the column chunk
-};
+typedef LfPairs<LF_D> TrSlots; // co: RAW: tiles in the slot, else byte offset of the column chunk
 
 template <int I>
 __device__ __forceinline__ void tr_load_raw(TrSlots &p, const LfLinear &l, TrRawWalk &w, unsigned lane_w2, int hi) {
@@ -121,14 +118,10 @@ __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(const TrArgs a
         auto pairs_left = [&] { return RAW ? (rw.end - rw.t + 1) >> 1 : w.left; };
         auto load = [&](auto ic) {
             constexpr int I = decltype(ic)::value;
-            if constexpr (RAW) {
+            if constexpr (RAW)
                 tr_load_raw<I>(p, l, rw, lane_w2, hi);
-            } else {
-                int q, qcol;
-                lf_next(w, q, qcol, p.co[I]);
-                p.o[I] = *reinterpret_cast<const int *>(reinterpret_cast<const char *>(l.poff) + (size_t)qcol * 8 + hi4);
-                p.w[I] = *reinterpret_cast<const f16x8 *>(reinterpret_cast<const char *>(l.data) + (size_t)q * 1024 + lane_w2);
-            }
+            else
+                lf_load<LF_D, I>(p, l, w, lane_w2, hi4);
         };
         n = min(pairs_left(), LF_D);
         // two pairs at a time; a group is requested as a whole where its first pair exists (wave-uniform)
@@ -234,7 +227,8 @@ static void tile_rows_plan(int M, int K, int nbr_max, int nlin, double pairs, in
 }
 
 // the launch's time in microseconds; traffic: megabytes that the L2s take in.  Fit to 312 launches (2048 -> 512, 3072 ->
-// 768 and 4096 -> 1024, 0 to 90 % pruned, 48 to 16384 rows), 4.5 % off in the mean.
+// 768 and 4096 -> 1024, 0 to 90 % pruned, 48 to 16384 rows), 4.5 % off in the mean; 9 % on the 96 launches of a graph that
+// bench/linear_forms.py times.
 double tile_rows_estimate(int M, int K, int nbr_max, int nlin, double pairs, double w_mb) {
     const int cus = std::max(et_device_cu_count(), 1), panels = (M + TR_BM - 1) / TR_BM;
     int nb = 1, ls = 0;

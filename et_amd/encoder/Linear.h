@@ -124,8 +124,10 @@ class Linear_row {
     Weight<half> bias;
     bool is_gelu;    // added: GELU on the compact output (a row-pruned FFN1)
     // the compact rows as a fully populated tile_mat: the planned tile kernels
-    // (panel in LDS, pipelined weight stream) then serve the dense product too;
-    // null when in_feat is not a multiple of 16
+    // (panel in LDS, pipelined weight stream) then serve the dense product too.
+    // The rows are on the device up to three times: `weight`, the plan's tiles and,
+    // where in_feat is a multiple of 32, the plan's row-major copy.  Null when
+    // in_feat is not a multiple of 16
     et_tile_plan *plan;
     // kept rows per head where every head keeps the same number and no padding
     // row exists (head h is then columns h*w .. of the compact output), else 0

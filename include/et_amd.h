@@ -213,7 +213,8 @@ int et_qk_scores(void *QK, const void *Q, const void *K, int seq_len,
  * The plan keeps device copies of the weight in a kernel-friendly order
  * (tiles of a block-row sorted by column so K can be walked in LDS-sized
  * chunks); results equal et_tile_spmm_add_bias on the same tile_mat up to
- * fp32 summation order.
+ * fp32 summation order.  A plan whose every tile survives (in_feat a multiple
+ * of 32) holds W once more, row-major, for the dense product: twice in all.
  * ---------------------------------------------------------------------- */
 typedef struct et_tile_plan et_tile_plan;
 
@@ -243,7 +244,8 @@ int et_tile_plan_ln_fusable(const et_tile_plan *plan);
  * The hidden activations are rounded to half exactly as the reference stores
  * them, but stay in LDS: a workgroup walks the hidden dimension in chunks and
  * feeds every chunk straight into the second linear.  Needs
- * et_tile_plan_ffn_fusable(first, second): in_feat of the first <= 992, hidden
+ * et_tile_plan_ffn_fusable(first, second): the panel and two hidden chunks
+ * within 160 KB of LDS (in_feat of the first <= 976 with chunks of 768), hidden
  * chunks and out_feat of the second <= 768 columns.  `hidden` is a device
  * buffer of M x hidden-width halves for the cases where the fused kernel does
  * not apply or does not pay (few rows): then the launches run one after the
@@ -479,7 +481,8 @@ int et_device_synchronize(void);
  *   "tile_fuse_ln"    0: et_tile_plan_run_ln runs the linear and the LayerNorm
  *                     as two launches; 1 (default): fused where the rows fit
  *   "tile_ln_min_panels" fewest 32-row panels for which et_tile_plan_run_ln
- *                     fuses and et_tile_plan_run_tail runs as one launch; 0
+ *                     fuses and et_tile_plan_run_tail runs as one launch (its
+ *                     last round too, behind rounds of a panel per CU); 0
  *                     (default): by size and density
  *   "tile_order"      consecutive workgroups of a linear share 0: a row panel, 2:
  *                     a column group, 1 (default): what moves fewer bytes
@@ -490,14 +493,14 @@ int et_device_synchronize(void);
  *   "tile_bm64"       panels of a planned linear of one chunk: 0: 32 rows; 2: 64
  *                     rows; 1 (default): the less estimated time; 4: as 1
  *                     without the twelve-wave form
- *   "tile_splitk_rows" most rows for which a planned linear with K > 1024 runs
- *                     on whole rows in LDS (16-row panels, a block-row's tile
+ *   "tile_splitk_rows" most rows for which a planned linear with K in several
+ *                     chunks (et_tile_plan_launches) runs on whole rows in LDS (16-row panels, a block-row's tile
  *                     pairs split over several waves where there are few); -1
  *                     (default): by estimated time; 0: never
  *   "tile_splitk_k1"  1: whole rows also for K of one chunk, up to
  *                     "tile_splitk_rows" rows (-1: 128); 0 (default)
- *   "tile_chunked"    a planned linear with K > 1024 on the kernel with fetching
- *                     waves: 1 .. 4 block-rows per computing wave; 0: never; -1
+ *   "tile_chunked"    a planned linear with K in several chunks on the kernel with
+ *                     fetching waves: 1 .. 4 block-rows per computing wave; 0: never; -1
  *                     (default): by estimated time
  *   "layer_flow_rows" most rows for which an encoder layer runs as one launch
  *                     (et_layer_flow_pays); -1 (default): by size and density;
@@ -513,8 +516,8 @@ int et_device_synchronize(void);
  *   "tile_fuse_ffn"   0: et_tile_plan_ffn_fusable answers no (the feed-forward
  *                     block runs as separate launches); 1: the block is fused
  *                     but et_tile_plan_tail_fusable answers no; 2 (default)
- *   "tile_ln_chunked" 0: fused LayerNorm with K > 992 uses the single-buffer
- *                     kernel; 1 (default): the double-buffered one
+ *   "tile_ln_chunked" 0: fused LayerNorm with K in several chunks uses the
+ *                     single-buffer kernel; 1 (default): the double-buffered one
  *   "ln_rows"         rows per wave of et_skip_layernorm (1, 2, 4)
  *   "attn_variant"    0: 4 waves x 32 query rows, 1: 8 waves x 16 rows,
  *                     2: 4 waves x 16 rows; -1 automatic
@@ -540,7 +543,8 @@ int et_device_synchronize(void);
  * order. */
 int et_tuning_set(const char *key, int value);
 /* The fused layer-tail kernels order their waves with bounded waits on LDS
- * counters.  A wave that gives up (it never should) sets one status word per
+ * counters, the one-launch layer its workgroups with bounded waits on counters
+ * in memory.  A wave that gives up (it never should) sets one status word per
  * process and goes on, so the kernel ends - with a wrong result - instead of
  * hanging the GPU; the next launch of such a kernel returns ET_ERR_HIP once and
  * clears the word.  et_wait_status_take does the same check on demand (ET_OK or
