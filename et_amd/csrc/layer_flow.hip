@@ -427,6 +427,7 @@ struct et_layer_flow {
     int *d_blk[2] = {nullptr, nullptr}; // padded batch, packed sequences
     double mbytes = 0.0; // of surviving tiles in the six linears
     int nblk[2] = {0, 0}, rows[2] = {0, 0};
+    bool packed = false; // et_layer_flow_set_packed has been called
 };
 
 namespace et {
@@ -541,8 +542,16 @@ extern "C" void et_layer_flow_destroy(et_layer_flow *f) {
 }
 
 extern "C" int et_layer_flow_set_packed(et_layer_flow *f, const int *cu) {
+    using namespace et;
     ET_REQUIRE(f && cu, ET_ERR_INVALID_ARG, "et_layer_flow_set_packed: null pointer");
-    return et::flow_tables(f, 1, cu, f->batch);
+    // (scratch, counters and tables are sized for the padded batch)
+    ET_REQUIRE(cu[0] == 0, ET_ERR_INVALID_ARG, "et_layer_flow_set_packed: the first row is %d", cu[0]);
+    for (int b = 0; b < f->batch; b++)
+        ET_REQUIRE(cu[b + 1] >= cu[b] && cu[b + 1] - cu[b] <= f->seq_len, ET_ERR_INVALID_ARG,
+                   "et_layer_flow_set_packed: sequence %d has %d rows of at most %d", b, cu[b + 1] - cu[b], f->seq_len);
+    const int rc = flow_tables(f, 1, cu, f->batch);
+    f->packed = rc == ET_OK;
+    return rc;
 }
 
 extern "C" int et_layer_flow_pays(const et_layer_flow *f, int rows) {
@@ -563,6 +572,7 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
                    aligned16(gamma1) && aligned16(beta1) && aligned16(gamma2) && aligned16(beta2),
                ET_ERR_ALIGNMENT, "et_layer_flow_run: pointers must be 16-byte aligned");
     const int which = cu_seqlens ? 1 : 0;
+    ET_REQUIRE(!which || f->packed, ET_ERR_INVALID_ARG, "et_layer_flow_run: cu_seqlens without et_layer_flow_set_packed");
     LfArgs a;
     memset(&a, 0, sizeof(a));
     a.M = f->rows[which];

@@ -315,7 +315,8 @@ size_t et_tail_ws_bytes_for(int d_model, int rows);
  * et_layer_flow_create: the six plans of the layer (they must outlive the object), sequences of seq_len rows,
  * `batch` of them.  *flow is NULL, with ET_OK, where the form does not exist for these sizes.  The object owns
  * the device scratch of the hand-overs; one run at a time may use it.
- * et_layer_flow_set_packed: HOST row offsets of the packed sequences (batch + 1), for runs with cu_seqlens.
+ * et_layer_flow_set_packed: HOST row offsets of the packed sequences (batch + 1, each sequence of 0 to seq_len rows), for
+ * runs with cu_seqlens; they need it.
  * et_layer_flow_pays: 1 where et_layer_flow_run is the form to take for that many rows.
  * et_layer_flow_run: out = layer(in), rows of model width, out may alias in; Q, K, V, attn are the caller's
  * workspace units (rows x model width, 16-byte aligned): they stay as they are, the hand-overs need whole cache

@@ -716,3 +716,41 @@ def test_layer_in_one_launch_infinite_activation_without_a_tile(sp):
     check_close(fin, orc.encoder_tile_layer(x, lins, ln, None, S, H, B, None, 1.0), what="finite")
     others = np.arange(B * S) != 5
     assert np.array_equal(inf[others], fin[others]) and not np.isfinite(inf[5]).any()
+
+
+def test_layer_flow_refuses_what_it_has_no_room_for():
+    """row offsets beyond the object's capacity, and a packed run without any, are errors in front of the launch"""
+    import ctypes as C
+    from et_amd import lib
+    from et_amd._lib import EtError, check
+    L, d, H, dff, S, B = lib(), 64, 2, 128, 10, 3
+    lins, ln = make_layer(rng(2200), d, dff, 0.5, seed=2300)
+    p = lambda a: np.ascontiguousarray(a).ctypes.data_as(C.c_void_p)
+    ip = lambda a: np.ascontiguousarray(a, np.int32).ctypes.data_as(C.POINTER(C.c_int))
+    plans = []
+    flow = C.c_void_p()
+    try:
+        for l in lins:
+            plans.append(C.c_void_p())
+            check(L.et_tile_plan_create(C.byref(plans[-1]), l["K"], l["N"], l["row_offset"].size, p(l["data"]), ip(l["row_ptr"]),
+                                        ip(l["row_offset"]), p(l["bias"])))
+        check(L.et_layer_flow_create(C.byref(flow), *plans, S, H, B))
+        assert flow.value
+        x = dev(np.zeros((7, B * S, d), np.float16))
+        vec = dev(np.ones(d, np.float16))
+        cu = dev(np.array([0, 10, 12, 30], np.int32))
+        ptr = lambda t: C.c_void_p(t.data_ptr())
+        cup = C.cast(cu.data_ptr(), C.POINTER(C.c_int))
+        run = lambda: check(L.et_layer_flow_run(flow, *[ptr(x[i]) for i in range(6)], None, None, cup, *[ptr(vec)] * 4, 1.0, None))
+        with pytest.raises(EtError):
+            run()
+        for bad in ([0, 10, 20, 31], [0, 11, 12, 13], [1, 2, 3, 4], [0, 5, 4, 9]):
+            with pytest.raises(EtError):
+                check(L.et_layer_flow_set_packed(flow, ip(bad)))
+            with pytest.raises(EtError):
+                run()
+        check(L.et_layer_flow_set_packed(flow, ip([0, 10, 12, 22])))
+    finally:
+        L.et_layer_flow_destroy(flow)
+        for q in plans:
+            L.et_tile_plan_destroy(q)
