@@ -120,7 +120,7 @@ def main():
     ap.add_argument("--seq", type=int, default=512)
     ap.add_argument("--sparsity", type=float, default=0.8)
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
-    ap.add_argument("--extras", action="store_true", help="also time the other BASELINE configurations")
+    ap.add_argument("--extras", action="store_true", help="also time the other workloads")
     ap.add_argument("--one-stream", action="store_true",
                     help="skip the two-batches-in-flight figure (for profiler runs: launches that overlap on two "
                          "streams would mix into the per-kernel averages)")
@@ -331,7 +331,7 @@ def main():
         "latency_us": round(ms_per_step * 1e3, 1), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f16 storage, f32 accumulate", "data": "synthetic",
         "config": {"workload": f"BERT-base encoder layer, {int(args.sparsity * 100)}% tile-pruned linears (16x16), "
-                               f"on-the-fly attention, batch {B} x seq {S}, all full length (BASELINE config 3)",
+                               f"on-the-fly attention, batch {B} x seq {S}, all full length",
                    "batch": B, "seq_len": S, "d_model": D, "heads": H, "d_ff": DFF, "sparsity": args.sparsity,
                    "softmax_base": 2, "mask": "additive zeros"},
         "layer_GFLOP_surviving": round(layer_flops, 2),
@@ -411,7 +411,7 @@ def event_time(torch, fn, reps=100, warm=10):
 
 def second_targets(torch, K, dev, enc, out, x, B, S, mask_h, lins, ln, two_streams=True):
     """Figures that belong in the default line next to the headline: the stand-alone skip + LayerNorm on
-    operands beyond the 256 MB last-level cache (an HBM figure, not a cache figure)
+    operands beyond the 256 MB last-level cache (an HBM figure, not a cache figure), the dense layer of one short sequence
     (dense layer, batch 1 x seq 128) and the headline layer with a padding mask instead of the all-zero one."""
     from et_amd.encoder import Encoder_tile, Linear_tile
     from et_amd.synthetic import randn_h, rng
@@ -502,7 +502,7 @@ def second_targets(torch, K, dev, enc, out, x, B, S, mask_h, lins, ln, two_strea
 
 
 def run_extras(torch, orc, K, dev):
-    """Other BASELINE configurations, timed with HIP events (reported, not the headline)."""
+    """Other workloads, timed with HIP events (reported, not the headline)."""
     from et_amd.encoder import Encoder_tile, Linear_tile
     from et_amd.synthetic import randn_h, rng
     out = {}

@@ -63,7 +63,7 @@ def test_encoder_tile_layer(S, B, sp, ls, use_mask):
 
 
 def test_encoder_tile_layer_config3_full_size():
-    """BASELINE config 3 at its size (batch 16 x seq 512, 80 % tiles, zero additive mask - the benchmark's
+    """The benchmark's layer at its size (batch 16 x seq 512, 80 % tiles, zero additive mask, the default
     workload): sequences do not interact, so the oracle runs two of them as a batch of their own and the
     full launch must agree on their rows; in place gives the same bits."""
     from et_amd.encoder import Encoder_tile
@@ -260,7 +260,7 @@ def prune_case(d, H, dff, S, B):
 
 @pytest.mark.parametrize("balanced", [True, False])
 def test_encoder_attnaware_layer_config4_wiring(balanced):
-    """Q/K keep 32 of 64 columns per head (same set), O/FFN1/FFN2 row-pruned at 70 %.
+    """Attention-aware pruning through the layer: Q/K keep 32 of 64 columns per head (same set), O/FFN1/FFN2 row-pruned at 70 %.
     Oracle = its own ops chained step by step; invariant = the same layer with DENSE linears whose pruned
     rows are zero (and, for FFN2, the dropped hidden units' columns).  balanced = False moves 12 kept
     columns from head 0 to head 1 (20 and 44 columns): the ragged pruned-attention kernel instead of the
@@ -269,7 +269,7 @@ def test_encoder_attnaware_layer_config4_wiring(balanced):
 
 
 def test_encoder_attnaware_layer_config4_full_size():
-    """the same layer at BASELINE config 4's size (batch 32 x seq 256).  Sequences do not interact, so the
+    """the same layer at the benchmark's size (batch 32 x seq 256).  Sequences do not interact, so the
     oracle runs three of them as a batch of their own and the full launch must agree on their rows."""
     attnaware_case(S=256, B=32, balanced=True, sample=[0, 17, 31])
 
@@ -422,7 +422,7 @@ def test_encoder_stack_variable_length():
 
 
 def test_encoder_stack_config5_full_size():
-    """BASELINE config 5 at its size: 12 BERT-base layers, 80 % tile-pruned, batch 64, lengths drawn from
+    """The benchmark's stack at its size: 12 BERT-base layers, 80 % tile-pruned, batch 64, lengths drawn from
     32..512 and padded to 512.  Sequences do not interact, so the oracle runs three of them (the shortest,
     a middle one, the longest) one at a time through the 12 layers; the packed run must agree on their
     valid rows and leave their padding rows zero, and the padded run on the shortest one's 512 rows.
