@@ -15,7 +15,7 @@ def test_traffic_is_read_per_kernel_instance_and_dropped_when_stale(tmp_path, mo
     lines = [
         "et::tile_linear_resident_kernel<2, false, 12, false, 64>   n= 95  fetch avg     17.95 MiB  write avg     36.01 MiB   (fetch min/max 17.95/17.96)",
         "et::tile_linear_resident_kernel<1, false, 8, false, 32>    n=220  fetch avg      9.56 MiB  write avg      0.38 MiB   (fetch min/max 5.02/14.10)",
-        "et::attention_kernel<64, 2, 4, false, false, true, 64, false>  n= 35  fetch avg     36.08 MiB  write avg     12.00 MiB   (fetch min/max 36.08/36.08)",
+        "et::attention_kernel<64, 2, 4, false, false, true, 64, false, false>  n= 35  fetch avg     36.08 MiB  write avg     12.00 MiB   (fetch min/max 36.08/36.08)",
         "et::tile_ffn_fused_kernel<3, true>   n= 95  fetch avg     43.45 MiB  write avg     14.00 MiB   (fetch min/max 43.45/43.45)",
     ]
     p = tmp_path / "traffic.txt"
