@@ -36,6 +36,7 @@
 #include "tile_walk.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <type_traits>
 #include <cstdlib>
@@ -2441,7 +2442,7 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
 
     et_tile_plan *p = new et_tile_plan();
     {
-        static unsigned long long next_uid = 0;
+        static std::atomic<unsigned long long> next_uid{0}; // (plans are created from any thread)
         p->uid = ++next_uid;
     }
     // column-sorted host copy (the layer-tail program is built from it)
