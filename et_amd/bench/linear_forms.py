@@ -247,6 +247,14 @@ def report(lines):
             worst.sort(reverse=True)
             print(f"{choice}: {len(behind)} linears, {100 * sum(behind) / len(behind):.1f} % behind the fastest form measured "
                   f"in the mean; furthest: " + "; ".join(f"{s} {g:.1f} against {b:.1f} us" for _, g, b, s in worst[:3]))
+    blocks = {}
+    for l in lines:
+        if l["form"].startswith("dense"):
+            blocks.setdefault(shape_of(l), []).append(l)
+    if blocks:
+        behind = [min(ls, key=lambda l: l["est"])["us"] / min(l["us"] for l in ls) - 1 for ls in blocks.values()]
+        print(f"dense blocks: {len(behind)} full plans, {100 * sum(behind) / len(behind):.1f} % behind the fastest block in the "
+              f"mean, {100 * max(behind):.0f} % at most")
     both = {}
     for l in lines:
         if l["form"] == "auto+dense":

@@ -200,8 +200,8 @@ static void attn_launch_one(const AttnArgs &a, hipStream_t st) {
 // packed sequences: as many workgroups (4 waves x 16 query rows) as the chip holds at once, or fewer
 template <int HD, bool MASK>
 static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
-    // (32 query rows per wave need 207 registers here, two waves per SIMD: 63 us against 48 us on a batch of
-    // 64 sequences of 32..512 rows)
+    // (32 query rows per wave needed 207 registers here, two waves per SIMD: 63 us against 48 us on a batch of
+    // 64 sequences of 32..512 rows - with the mask's bookkeeping; not tried without)
     constexpr size_t lds = attn_lds_bytes<HD, 1, 4, false>();
     auto kern = attention_packed_kernel<HD, 1, 4, MASK>;
     if (lds > 64 * 1024) {
