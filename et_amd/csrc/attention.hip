@@ -197,13 +197,23 @@ static void attn_launch_one(const AttnArgs &a, hipStream_t st) {
     hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, a);
 }
 
-// packed sequences: as many workgroups (4 waves x 16 query rows) as the chip holds at once, or fewer
-template <int HD, bool MASK>
+// Blocks of 128 query rows for packed sequences without a mask: K and V are read from LDS once per 32 queries of a wave
+// instead of 16, but a short last block wastes more and fewer blocks balance worse.  The lengths are on the device; the
+// line is two rounds of the workgroups that the chip holds by the blocks of the LONGEST sequence.  12 heads, lengths
+// uniform up to the second figure, blocks of 64 / 128 rows, us: 64 x 512 36.6 / 32.6, 200 x 300 55.4 / 50.8, 64 x 256
+// 17.3 / 16.7, 40 x 512 27.3 / 27.4 (beyond the line); 64 x 128 9.1 / 9.1, 20 x 300 9.7 / 10.2, 16 x 512 13.1 / 14.9.
+static bool packed_by_128(const AttnArgs &a) {
+    return (long)((a.seq_len + 127) / 128) * a.nhead * a.batch >= 2 * 3 * (long)std::max(et_device_cu_count(), 1);
+}
+
+// packed sequences: as many workgroups (4 waves x 16 QS query rows) as the chip holds at once, or fewer
+template <int HD, bool MASK, int QS = 1>
 static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
-    // (32 query rows per wave needed 207 registers here, two waves per SIMD: 63 us against 48 us on a batch of
-    // 64 sequences of 32..512 rows - with the mask's bookkeeping; not tried without)
-    constexpr size_t lds = attn_lds_bytes<HD, 1, 4, false>();
-    auto kern = attention_packed_kernel<HD, 1, 4, MASK>;
+    // (32 query rows per wave with the mask's bookkeeping needed 207 registers, two waves per SIMD: 63 us against 48 us on
+    // a batch of 64 sequences of 32..512 rows; without it 154 and three)
+    static_assert(QS == 1 || !MASK, "two subtiles a wave: without a mask");
+    constexpr size_t lds = attn_lds_bytes<HD, QS, 4, false>();
+    auto kern = attention_packed_kernel<HD, QS, 4, MASK>;
     if (lds > 64 * 1024) {
         static bool done = false;
         if (!done) {
@@ -212,7 +222,7 @@ static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
             done = true;
         }
     }
-    const long resident = (long)std::max(et_device_cu_count(), 1) * (HD <= 64 ? 4 : 2);
+    const long resident = (long)std::max(et_device_cu_count(), 1) * (QS == 2 ? 3 : HD <= 64 ? 4 : 2);
     const long wgs = std::min<long>(resident, a.total);
     hipLaunchKernelGGL(kern, dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256), lds, st, a);
 }
@@ -426,11 +436,12 @@ static int attention_dispatch(AttnArgs a, int d_model, bool pruned, bool sharedq
         a.qk_width = qk_width;
     }
     // packed sequences: the grid the chip holds, every workgroup walks its share of the query blocks that exist
+    // (variant 2 counts the blocks of 64)
     if (a.cu_seqlens && !pruned && !sharedqk && variant == 2 && a.batch <= 64 * AT_PX && g_attn_packed) {
         if (hd == 32)
             no_mask ? attn_launch_packed<32, false>(a, st) : attn_launch_packed<32, true>(a, st);
         else if (hd == 64)
-            no_mask ? attn_launch_packed<64, false>(a, st) : attn_launch_packed<64, true>(a, st);
+            no_mask ? (packed_by_128(a) ? attn_launch_packed<64, false, 2>(a, st) : attn_launch_packed<64, false>(a, st)) : attn_launch_packed<64, true>(a, st);
         else
             no_mask ? attn_launch_packed<128, false>(a, st) : attn_launch_packed<128, true>(a, st);
         return launch_status(who);

@@ -859,6 +859,38 @@ def test_otf_attention_varlen_walks_existing_blocks(K, S, H, d, lens):
     check_close(walked, want[sel], max_abs=5e-3, mean_rel=1e-3, what="varlen attention, walked blocks")
 
 
+@pytest.mark.parametrize("S,H,lens,walked_by", [
+    (80, 16, [80 - (i % 81) for i in range(96)], 128),          # 1536 possible blocks of 128: just over the line; empty ones
+    (300, 8, [300, 257, 256, 255, 129, 128, 127, 65, 64, 63, 33, 1, 0] * 5, 128),  # block and tile edges
+    (80, 16, [80 - (i % 81) for i in range(95)], 64),           # just under it
+])
+def test_otf_attention_varlen_blocks_of_128_rows(K, S, H, lens, walked_by):
+    """packed sequences without a mask, either side of the line between blocks of 64 and 128 query rows: every block
+    size gives the bits of one workgroup per possible block, which the oracle pins"""
+    from et_amd._lib import lib
+    if lib().et_device_cu_count() != 256:
+        pytest.skip("the line counts the workgroups of 256 compute units")
+    r = rng(70 + S + len(lens))
+    lens = np.array(sorted(lens, reverse=True), np.int32)
+    assert ((S + 127) // 128 * H * lens.size >= 1536) == (walked_by == 128)
+    B, d = lens.size, H * 64
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(cu[-1])
+    Q, Kk, V = (randn_h(r, (T, d)) for _ in range(3))
+    args = (dev(Q), dev(Kk), dev(V), None, dev(cu), S, H, 1.0)
+    walked = host(K.OTF_attention_varlen(*args))
+    try:
+        lib().et_tuning_set(b"attn_packed", 0)
+        grid = host(K.OTF_attention_varlen(*args))
+    finally:
+        lib().et_tuning_set(b"attn_packed", 1)
+    assert np.array_equal(walked, grid)
+    for b in (0, B // 2, int(np.count_nonzero(lens)) - 1):
+        rows = slice(int(cu[b]), int(cu[b + 1]))
+        want = orc.otf_attention(Q[rows], Kk[rows], V[rows], None, int(lens[b]), H, 1, None, 1.0, f64=True)
+        check_close(walked[rows], want, max_abs=5e-3, mean_rel=1e-3, what="varlen attention, 128-row blocks")
+
+
 @pytest.mark.parametrize("S,keep,value", [(512, 300, -30000.0), (512, 64, -65504.0), (256, 200, -1000.0), (192, 1, -30000.0)])
 def test_otf_attention_padding_mask_with_dead_tiles(K, S, keep, value):
     """a padding mask that blanks the keys from `keep` on: key tiles that lie wholly behind it add nothing (every
