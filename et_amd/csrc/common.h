@@ -70,6 +70,21 @@ __device__ __forceinline__ void load_lds16(const void *gsrc, void *lds_base) {
         (__attribute__((address_space(3))) void *)lds_base, 16, 0, 0);
 }
 
+// The same from a wave-uniform base and a byte offset per lane, for loops that keep requests in flight while they use
+// other parts of the LDS and wait for them by themselves (s_waitcnt vmcnt).  The compiler tracks requests of the builtin
+// above and waits for ALL of them in front of LDS stores and barriers; this form it does not see.
+__device__ __forceinline__ void load_lds16_untracked(const void *base, unsigned lane_offset, void *lds_base) {
+    const unsigned dst = (unsigned)(size_t)(__attribute__((address_space(3))) char *)lds_base;
+    const unsigned long long at = (unsigned long long)base;
+    const unsigned long long src = (unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(at >> 32)) << 32 |
+                                   (unsigned)__builtin_amdgcn_readfirstlane((unsigned)at);
+    unsigned keep; // (M0 is the compiler's)
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(lane_offset), "s"(src)
+                 : "memory");
+}
+
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 
 // Stores whose data other workgroups of the SAME launch read: an agent-scope

@@ -60,6 +60,7 @@ double tile_rows_estimate(int M, int K, int nbr_max, int nlin, double pairs, dou
 int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *X, int M, int K, double pairs, bool gelu,
                      bool raw, hipStream_t st);
 void set_flow_rows(int v);
+void set_qkv_attention(int v);
 int tail_spin();
 
 constexpr int TL_THREADS = 512;
@@ -2227,6 +2228,10 @@ extern "C" int et_tuning_set(const char *key, int value) {
         et::set_flow_rows(value);
         return ET_OK;
     }
+    if (key && !strcmp(key, "qkv_attention")) {
+        et::set_qkv_attention(value);
+        return ET_OK;
+    }
     if (key && !strcmp(key, "ln_rows")) {
         et::set_ln_rows(value);
         return ET_OK;
@@ -2459,6 +2464,8 @@ extern "C" int et_tile_plan_create(et_tile_plan **plan, int in_feat, int out_fea
     p->KC = KC;
     p->nchunk = nchunk;
     p->npair = cptr.back() / 2;
+    for (size_t i = 0; i + 1 < cptr.size(); i++)
+        p->most_pairs = std::max(p->most_pairs, (cptr[i + 1] - cptr[i]) / 2);
     unsigned char *dev = nullptr;
     int rc = et_malloc((void **)&dev, at_dense + (full ? (size_t)out_feat * in_feat * 2 : 0));
     p->d_data = reinterpret_cast<f16 *>(dev);

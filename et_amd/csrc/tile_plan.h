@@ -13,6 +13,7 @@ void tail_program_destroy(TailProgram *p);
 struct et_tile_plan {
     int in_feat = 0, out_feat = 0, ntile = 0, KC = 0, nchunk = 0;
     int npair = 0; // pairs of tiles in the plan layout; pair npair is all zero
+    int most_pairs = 0; // of a (column chunk, block-row)
     et::f16 *d_data = nullptr; // one allocation, the parts below lie behind the tiles
     int *d_cptr = nullptr;
     int *d_row_offset = nullptr;

@@ -36,6 +36,7 @@ class Encoder_base {
     Weight<int> d_cu;    // row offsets of the packed sequences
     Weight<int> d_order; // packed position -> batch index
     int total_rows; // sum of lengths when set, else batch*seq_len
+    int longest;    // the longest sequence's rows
     // scratch of the layer tail's paired form (et_tile_plan_run_tail_ws), behind the
     // activation units (and behind the score buffer of Encoder_length)
     void *tail_ws;
@@ -62,7 +63,7 @@ class Encoder_base {
           ln_gamma{Weight<half>(ln_gamma_1, d_model_), Weight<half>(ln_gamma_2, d_model_)},
           ln_beta{Weight<half>(ln_beta_1, d_model_), Weight<half>(ln_beta_2, d_model_)},
           has_mask(mask_ != nullptr), mask_summary(nullptr), stream(nullptr), log2_scale(1.0f),
-          total_rows(batch_ * seq_len_), tail_ws(nullptr), tail_ws_bytes(0), flow(nullptr) {
+          total_rows(batch_ * seq_len_), longest(seq_len_), tail_ws(nullptr), tail_ws_bytes(0), flow(nullptr) {
         if (mask_) {
             mask = Weight<half>(mask_, seq_len_ * seq_len_);
             // the mask never changes after construction: let the attention
@@ -103,6 +104,7 @@ class Encoder_base {
                       "set_seq_lens: every length must lie in [0, seq_len]");
         lens.clear();
         total_rows = batch * seq_len;
+        longest = seq_len;
         if (!host_lens)
             return;
         lens.assign(host_lens, host_lens + batch);
@@ -117,6 +119,7 @@ class Encoder_base {
         for (int i = 0; i < batch; i++)
             cu[i + 1] = cu[i] + lens[order[i]];
         total_rows = cu[batch];
+        longest = batch > 0 ? lens[order[0]] : 0;
         d_lens = Weight<int>(lens.data(), batch);
         d_cu = Weight<int>(cu.data(), batch + 1);
         d_order = Weight<int>(order.data(), batch);
@@ -143,6 +146,27 @@ class Encoder_base {
         etChk(et_layer_flow_run(flow, out, in, buffers[0], buffers[1], buffers[2], buffers[3], mask_ptr(), lengths, cu,
                                 ln_gamma[0].get(), ln_beta[0].get(), ln_gamma[1].get(), ln_beta[1].get(), log2_scale,
                                 stream));
+    }
+
+    // Steps 1-5 (encoder/encoder.cu:22-32): attention of `in`'s rows into unit 3.  `cu`: packed sequences, else a padded
+    // batch with `lengths` (or null).  Short sequences: one launch without units 0..2.
+    void attend(half *in, const Linear_tile &Q, const Linear_tile &K, const Linear_tile &V, int nrows,
+                const int *lengths, const int *cu) {
+        const int most = cu ? longest : seq_len;
+        if (et_qkv_attention_pays(Q.tile_plan(), K.tile_plan(), V.tile_plan(), most, d_model, nheads, batch)) {
+            etChk(et_qkv_attention(buffers[3], in, Q.tile_plan(), K.tile_plan(), V.tile_plan(), mask_ptr(), lengths, cu,
+                                   most, seq_len, d_model, nheads, batch, log2_scale, stream));
+            return;
+        }
+        const Linear_tile *qkv[3] = {&Q, &K, &V};
+        half *outs[3] = {buffers[0], buffers[1], buffers[2]};
+        Linear_tile::run_multi(qkv, outs, 3, in, nrows, stream);
+        if (cu)
+            etChk(et_OTF_attention_varlen(buffers[3], buffers[0], buffers[1], buffers[2], mask_ptr(), cu, seq_len, d_model,
+                                          nheads, batch, log2_scale, stream));
+        else
+            etChk(et_OTF_attention(buffers[3], buffers[0], buffers[1], buffers[2], mask_ptr(), seq_len, d_model, nheads,
+                                   batch, lengths, log2_scale, stream));
     }
 
     // steps 6-10 of encoder/encoder.cu:33-44, shared by every encoder kind:
@@ -184,11 +208,7 @@ class Encoder_tile : public Encoder_base {
             run_flow(out, in, lens_ptr(), nullptr);
             return;
         }
-        const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
-        half *outs[3] = {buffers[0], buffers[1], buffers[2]};
-        Linear_tile::run_multi(qkv, outs, 3, in, rows(), stream);
-        etChk(et_OTF_attention(buffers[3], buffers[0], buffers[1], buffers[2], mask_ptr(), seq_len,
-                               d_model, nheads, batch, lens_ptr(), log2_scale, stream));
+        attend(in, Q_linear, K_linear, V_linear, rows(), lens_ptr(), nullptr);
         tail(out, in, buffers[3], O_linear, MLP1_linear, MLP2_linear, rows());
     }
 };
@@ -352,11 +372,7 @@ class Encoder_length : public Encoder_base {
             run_flow(out_p, in_p, nullptr, d_cu.get());
             return;
         }
-        const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
-        half *outs[3] = {buffers[0], buffers[1], buffers[2]};
-        Linear_tile::run_multi(qkv, outs, 3, in_p, n, stream);
-        etChk(et_OTF_attention_varlen(buffers[3], buffers[0], buffers[1], buffers[2], mask_ptr(),
-                                      d_cu.get(), seq_len, d_model, nheads, batch, log2_scale, stream));
+        attend(in_p, Q_linear, K_linear, V_linear, n, nullptr, d_cu.get());
         tail(out_p, in_p, buffers[3], O_linear, MLP1_linear, MLP2_linear, n);
     }
 
@@ -374,11 +390,7 @@ class Encoder_length : public Encoder_base {
                 etChk(et_unpack_rows_ordered(out, in_p, d_cu.get(), d_order.get(), batch, seq_len, d_model, stream));
                 return;
             }
-            const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
-            half *outs[3] = {buffers[0], buffers[1], buffers[2]};
-            Linear_tile::run_multi(qkv, outs, 3, in_p, n, stream);
-            etChk(et_OTF_attention_varlen(buffers[3], buffers[0], buffers[1], buffers[2], mask_ptr(),
-                                          d_cu.get(), seq_len, d_model, nheads, batch, log2_scale, stream));
+            attend(in_p, Q_linear, K_linear, V_linear, n, nullptr, d_cu.get());
             if (Linear_tile::tail_fusable(O_linear, MLP1_linear, MLP2_linear)) {
                 // steps 6-10 in one launch, straight into unit 0.  (With few rows
                 // they run one after the other, in place in unit 0 with the hidden
@@ -412,16 +424,15 @@ class Encoder_length : public Encoder_base {
             run_flow(out, in, nullptr, nullptr);
             return;
         }
-        const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
-        half *outs[3] = {buffers[0], buffers[1], buffers[2]};
-        Linear_tile::run_multi(qkv, outs, 3, in, rows(), stream);
         if (use_shared_qk) {
+            const Linear_tile *qkv[3] = {&Q_linear, &K_linear, &V_linear};
+            half *outs[3] = {buffers[0], buffers[1], buffers[2]};
+            Linear_tile::run_multi(qkv, outs, 3, in, rows(), stream);
             etChk(et_qk_scores(QK_buf, buffers[0], buffers[1], seq_len, d_model, nheads, batch, stream));
             etChk(et_sharedQK_attention(buffers[3], QK_buf, buffers[2], mask_ptr(), seq_len, d_model,
                                         nheads, batch, nullptr, log2_scale, stream));
         } else {
-            etChk(et_OTF_attention(buffers[3], buffers[0], buffers[1], buffers[2], mask_ptr(), seq_len,
-                                   d_model, nheads, batch, nullptr, log2_scale, stream));
+            attend(in, Q_linear, K_linear, V_linear, rows(), nullptr, nullptr);
         }
         tail(out, in, buffers[3], O_linear, MLP1_linear, MLP2_linear, rows());
     }

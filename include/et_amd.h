@@ -332,6 +332,18 @@ int et_layer_flow_pays(const et_layer_flow *flow, int rows);
 int et_layer_flow_run(et_layer_flow *flow, void *out, const void *in, void *Q, void *K, void *V, void *attn,
                       const void *mask, const int *seq_lens, const int *cu_seqlens, const void *gamma1,
                       const void *beta1, const void *gamma2, const void *beta2, float log2_scale, void *stream);
+/* ---- projections and attention of a head in one launch ------------------------
+ * out = attention(X Wq^T, X Wk^T, X Wv^T) (steps 1-5 of a layer, encoder/encoder.cu:22-32) for heads of 64 columns and
+ * sequences of at most 128 rows; Q, K and V are not written anywhere.  Plans of d_model x d_model in one column chunk
+ * (d_model up to 1024).  Sequences: cu_seqlens (device row offsets of batch + 1, packed rows, each sequence of at most
+ * max_len rows) or a padded batch of seq_len rows each (max_len == seq_len) with optional seq_lens (device).  mask,
+ * log2_scale as in et_OTF_attention.  out must not overlap X.
+ * et_qkv_attention_pays: 1 where the form exists and is the one to take (et_tuning_set "qkv_attention"). */
+int et_qkv_attention_pays(const et_tile_plan *q, const et_tile_plan *k, const et_tile_plan *v, int max_len,
+                          int d_model, int nheads, int batch);
+int et_qkv_attention(void *out, const void *X, const et_tile_plan *q, const et_tile_plan *k, const et_tile_plan *v,
+                     const void *mask, const int *seq_lens, const int *cu_seqlens, int max_len, int seq_len,
+                     int d_model, int nheads, int batch, float log2_scale, void *stream);
 /* n (<= 4) planned linears with the same in_feat applied to the same X in ONE
  * launch (the Q/K/V projections, encoder/encoder.cu:22-26, which the
  * reference spreads over three streams) - or in one per column geometry where
@@ -506,6 +518,8 @@ int et_device_synchronize(void);
  *   "layer_flow_rows" most rows for which an encoder layer runs as one launch
  *                     (et_layer_flow_pays); -1 (default): by size and density;
  *                     0: never
+ *   "qkv_attention"   projections and attention of a head in one launch: 0 never, 1
+ *                     wherever the form exists, -1 (default) where it pays
  *   "plan_dense"      plans of fully populated matrices as dense products: 0
  *                     never, 1 (default) where the estimated time is less, 2
  *                     always

@@ -622,6 +622,84 @@ def test_layer_in_one_launch(request, d, H, dff, S, B, sp, lens, use_mask):
         del graph
 
 
+@pytest.mark.parametrize("d,S,B,sp,lens,use_mask,ls", [
+    (64, 1, 1, 0.5, None, False, 1.0),                      # one row, one head
+    (768, 16, 3, 0.8, None, True, 1.0),                     # whole panels; mask rows of whole loads
+    (768, 37, 2, 0.8, [37, 5], True, LOG2E),                # odd panels and mask rows; padding rows
+    (768, 64, 9, 0.8, None, False, 1.0),                    # the sequences of an XCD in turn, one of them over
+    (512, 65, 2, 0.5, [65, 0], False, LOG2E),               # one row in the last panel; an empty sequence
+    (768, 128, 2, 0.8, [128, 97], True, 1.0),               # the most rows: five panels of eight in the ring
+    (1024, 113, 3, 0.9, [96, 113, 48], False, LOG2E),       # three panels in the ring, refilled
+    (320, 50, 2, 0.0, None, True, 1.0),                     # dense lists of ten pairs
+])
+def test_projections_and_attention_of_a_head_in_one_launch(d, S, B, sp, lens, use_mask, ls):
+    """et_qkv_attention on a padded batch, with lengths and packed, against the oracle's linears and attention"""
+    import ctypes as C
+    from et_amd import lib
+    from et_amd._lib import check
+    r = rng(2100 + d + S + B)
+    H = d // 64
+    lins = [make_tile_linear(r, d, d, sp, seed=2200 + S + j, std=0.04, bias_std=0.05) for j in range(3)]
+    x = randn_h(r, (B * S, d))
+    mask = randn_h(r, (S, S), 0.5) if use_mask else None
+    q, k, v = (orc.tile_linear(x, l["row_ptr"], l["row_offset"], l["data"], l["bias"], d) for l in lins)
+    L = lib()
+    plans = []
+    try:
+        for l in lins:
+            plans.append(C.c_void_p())
+            check(L.et_tile_plan_create(C.byref(plans[-1]), d, d, l["row_offset"].size, l["data"].ctypes.data,
+                                        l["row_ptr"].ctypes.data, l["row_offset"].ctypes.data, l["bias"].ctypes.data))
+        md = dev(mask) if use_mask else None
+        mp = md.data_ptr() if use_mask else None
+        for n in ([None, np.array(lens, np.int32)] if lens else [None]):
+            want = orc.otf_attention(q, k, v, mask, S, H, B, n, ls)
+            nd = None if n is None else dev(n)
+            out = torch.full((B * S, d), 9.0, dtype=torch.float16, device="cuda")
+            check(L.et_qkv_attention(out.data_ptr(), dev(x).data_ptr(), *plans, mp, None if n is None else nd.data_ptr(), None,
+                                     S, S, d, H, B, ls, torch.cuda.current_stream().cuda_stream))
+            got = host(out)
+            valid = np.concatenate([np.arange(b * S, b * S + (S if n is None else n[b])) for b in range(B)])
+            check_close(got[valid], want[valid], max_abs=5e-3, mean_rel=1e-3, what="projections and attention")
+            assert (np.delete(got, valid, 0) == 0).all()
+            if n is not None:
+                cu = dev(np.concatenate([[0], np.cumsum(n)]).astype(np.int32))
+                xp = dev(x[valid])
+                out = torch.full_like(xp, 9.0)
+                check(L.et_qkv_attention(out.data_ptr(), xp.data_ptr(), *plans, mp, None, cu.data_ptr(), int(n.max()), S, d, H,
+                                         B, ls, torch.cuda.current_stream().cuda_stream))
+                assert np.array_equal(host(out), got[valid])
+    finally:
+        for p in plans:
+            L.et_tile_plan_destroy(p)
+
+
+def test_projections_and_attention_refuse_what_they_do_not_take():
+    import ctypes as C
+    from et_amd import lib
+    from et_amd._lib import check
+    L, r = lib(), rng(2300)
+    mats = {n: make_tile_linear(r, n, n, 0.5, seed=n) for n in (128, 1536)}
+    mats["dense"] = make_tile_linear(r, 768, 768, 0.0, seed=3)  # lists beyond a wave's registers
+    plans = {}
+    try:
+        for n, l in mats.items():
+            plans[n] = C.c_void_p()
+            check(L.et_tile_plan_create(C.byref(plans[n]), l["K"], l["N"], l["row_offset"].size, l["data"].ctypes.data,
+                                        l["row_ptr"].ctypes.data, l["row_offset"].ctypes.data, l["bias"].ctypes.data))
+        x = torch.zeros((129, 1536), dtype=torch.float16, device="cuda")
+
+        def run(name, d, H, most, S, cu=None):
+            p = plans[name]
+            return L.et_qkv_attention(x.data_ptr(), x.data_ptr(), p, p, p, None, None, cu, most, S, d, H, 1, 1.0, None)
+        for args in ((128, 128, 4, 32, 32), (128, 128, 2, 129, 129), (1536, 1536, 24, 32, 32), ("dense", 768, 12, 32, 32),
+                     (128, 128, 2, 16, 32), (128, 128, 2, 0, 0)):
+            assert run(*args) < 0, args
+    finally:
+        for p in plans.values():
+            L.et_tile_plan_destroy(p)
+
+
 @pytest.mark.parametrize("S,B,off", [(32, 2, 8), (16, 3, 24), (48, 2, 56), (37, 2, 64)])
 def test_layer_in_one_launch_workspace_alignment(S, B, off):
     """a workspace `off` halves behind a 256-byte boundary, several sequences that end on a panel: the rows handed over
