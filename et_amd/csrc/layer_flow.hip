@@ -51,10 +51,18 @@
 // width: too wide for a panel) reads its operand from memory, only the surviving
 // tiles' columns, two block-rows per workgroup with eight waves each.  The first LayerNorm is
 // recomputed by every workgroup of the first feed-forward linear that needs the
-// rows (one hand-over less).  Attention: attention_block, 256 query rows per
-// unit and head.
-#include "attention_block.h"
-#include "tile_plan.h"
+// rows (one hand-over less), and by those of the second one for its skip operand
+// while they wait, where every unit has a CU of its own (0.2 to 0.7 us less than
+// having the first linear's store it; with more units 1.2 us more).  Attention: attention_block, 256 query rows per
+// unit and head.  Where the lists are short enough for a wave's registers, heads
+// are 64 wide and sequences at most 128 rows, a unit is a head's projections AND
+// attention (qkv_block.h): a hand-over less.  80 % pruned, 768 wide: 16 rows
+// 24.5 -> 18.9 us, 37 25.1 -> 21.1, 64 25.0 -> 22.8, 96 28.1 -> 24.9.  Where the
+// 21 us of 37 rows go: launch and ticket 3, projections and attention 5.8 (a CU
+// reads 1 KB of X from LDS per product), then per step 1.2 to 2.5 of work (rows
+// from memory 0.9, LayerNorm of 16 rows 0.9), 0.7 for the stores to be
+// acknowledged and 0.4 until the counter is seen.
+#include "qkv_block.h"
 #include "tile_walk.h"
 
 #include <algorithm>
@@ -70,9 +78,11 @@ constexpr int LF_BM = 16;      // rows per panel: a wave each in the LayerNorms
 constexpr int LF_QB = 256;     // query rows per attention unit
 constexpr int LF_SHARE = 12;   // ... that a wave's share of a block-row should not exceed
 constexpr int LF_CS = 32;      // counter stride in words: a line each
+constexpr int LF_HEAD_PAIRS = 12; // tile pairs of a block-row in a unit of projections and attention (sixteen waves: 128 registers)
 
 struct LfArgs {
     AttnArgs at; // Q, K, V, out: scratch that the steps hand over
+    QaArgs qa;   // FUSED: projections and attention of a head
     LfLinear q, k, v, o, m1, m2;
     const f16 *in;
     f16 *out;
@@ -81,6 +91,8 @@ struct LfArgs {
     unsigned *ctr;  // tickets and the set in turn, then the two sets of nctr counters
     const int *blk; // attention blocks: [2i] sequence, [2i+1] query block; then per panel first and last block
     int M, d, dff, npanel, nblk;
+    float inv_d;
+    int again; // the second feed-forward linear's units compute the first LayerNorm's rows once more
     int u_at, u_o, u_f1, u_f2;             // first unit of each step (Q/K/V: 0)
     int g_qkv, g_o, g_f1, g_f2;            // units per panel
     int gl_q, gl_k;                        // ... of the query and key linears
@@ -206,55 +218,63 @@ __device__ __forceinline__ void lf_finish(const LfArgs &a, f32x4 acc, f32x4 *red
 }
 
 // LayerNorm(y + skip) of one row, spread over the wave in 16-byte pieces (the math and the order of summation of
-// skip_layernorm.hip).  Every load is requested before the first value is used.  put(piece, values).
-template <class Put>
-__device__ __forceinline__ void lf_layernorm(const LfArgs &a, const f16 *Y, const f16 *S, const f16 *gamma,
-                                             const f16 *beta, int row, int lane, Put &&put) {
+// skip_layernorm.hip); a lane's pieces lie at lane and lane + 64, what is behind the row is not used.
+struct LfPieces {
+    f16x8 p[2];
+};
+__device__ __forceinline__ LfPieces lf_pieces(const LfArgs &a, const f16 *row, int lane) {
+    const int npiece = a.d >> 3;
+    LfPieces v;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+        v.p[i] = *reinterpret_cast<const f16x8 *>(row + min(lane + 64 * i, npiece - 1) * 8);
+    return v;
+}
+__device__ __forceinline__ const f16 *lf_row(const LfArgs &a, const f16 *rows, int row) {
+    return rows + (size_t)min(row, a.M - 1) * a.d;
+}
+__device__ __forceinline__ LfPieces lf_layernorm(const LfArgs &a, LfPieces y, const LfPieces &skip, const LfPieces &gamma,
+                                                 const LfPieces &beta, int lane) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     const int npiece = a.d >> 3;
-    const float inv_n = 1.0f / (float)a.d;
-    const size_t at = (size_t)min(row, a.M - 1) * a.d;
-    f16x8 x[2], s[2], g[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int pc = min(lane + 64 * i, npiece - 1) * 8;
-        x[i] = *reinterpret_cast<const f16x8 *>(Y + at + pc);
-        s[i] = *reinterpret_cast<const f16x8 *>(S + at + pc);
-        g[i] = *reinterpret_cast<const f16x8 *>(gamma + pc);
-        b[i] = *reinterpret_cast<const f16x8 *>(beta + pc);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    // (a half times 1.0 plus a float is one instruction; the multiplier is opaque, or it is a conversion and an addition)
+    float one = 1.0f;
+    asm("" : "+s"(one));
     float sum = 0.f, var = 0.f;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        x[i] += s[i]; // half add, one rounding
+        y.p[i] += skip.p[i]; // half add, one rounding
         if (lane + 64 * i >= npiece)
-            x[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            y.p[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int j = 0; j < 8; j += 2)
-            sum = __builtin_amdgcn_fdot2(h2{x[i][j], x[i][j + 1]}, h2{(f16)1, (f16)1}, sum, false);
+            sum = __builtin_amdgcn_fdot2(h2{y.p[i][j], y.p[i][j + 1]}, h2{(f16)1, (f16)1}, sum, false);
     }
-    const float mean = wave_sum(sum) * inv_n;
+    const float mean = wave_sum(sum) * a.inv_d;
 #pragma unroll
     for (int i = 0; i < 2; i++)
         if (lane + 64 * i < npiece) {
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const float d = (float)x[i][j] - mean;
+                const float d = __builtin_fmaf((float)y.p[i][j], one, -mean);
                 var += d * d;
             }
         }
-    const float rstd = rsqrtf(wave_sum(var) * inv_n + 1e-6f);
+    const float rstd = __builtin_amdgcn_rsqf(wave_sum(var) * a.inv_d + 1e-6f); // (never a denormal)
     const float shift = -mean * rstd;
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        f16x8 o;
+    for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 8; j++)
-            o[j] = (f16)(__builtin_fmaf((float)x[i][j], rstd, shift) * (float)g[i][j] + (float)b[i][j]);
-        if (lane + 64 * i < npiece)
-            put(lane + 64 * i, o);
-    }
+            y.p[i][j] = (f16)(__builtin_fmaf((float)y.p[i][j], rstd, shift) * (float)gamma.p[i][j] + (float)beta.p[i][j]);
+    return y;
+}
+
+__device__ __forceinline__ void lf_put_row(const LfArgs &a, f16 *row, const LfPieces &v, int lane) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+        if (lane + 64 * i < a.d >> 3)
+            *reinterpret_cast<f16x8 *>(row + (lane + 64 * i) * 8) = v.p[i];
 }
 
 // rows of X -> panel, DMA; rows at or beyond M stay unwritten (they only feed rows that are never stored)
@@ -270,7 +290,7 @@ __device__ __forceinline__ void lf_panel(const LfArgs &a, const f16 *X, f16 *xs,
     }
 }
 
-template <int HD, bool MASK>
+template <int HD, bool MASK, bool FUSED>
 __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lf_smem[];
     unsigned *const bc = reinterpret_cast<unsigned *>(lf_smem + a.misc);
@@ -291,9 +311,9 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
     const int ldx = a.d + 16;
     const char *const xlane = reinterpret_cast<const char *>(xs + c16 * ldx + khalf8);
 
-    if (unit < a.u_at || (unit >= a.u_o && unit < a.u_f2)) {
+    if ((!FUSED && unit < a.u_at) || (unit >= a.u_o && unit < a.u_f2)) {
         // ---- a linear on a panel in LDS: Q/K/V, output projection, first feed-forward linear
-        const int step = unit < a.u_at ? 0 : unit < a.u_f1 ? 1 : 2;
+        const int step = !FUSED && unit < a.u_at ? 0 : unit < a.u_f1 ? 1 : 2;
         const int rel = unit - (step == 0 ? 0 : step == 1 ? a.u_o : a.u_f1);
         const int per = step == 0 ? a.g_qkv : step == 1 ? a.g_o : a.g_f1;
         const int ls = step == 0 ? a.s_qkv : step == 1 ? a.s_o : a.s_f1;
@@ -337,12 +357,17 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
             lf_panel(a, a.at.out, xs, ldx, m0, wave, lane);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         } else {
+            const LfPieces skip = lf_pieces(a, lf_row(a, a.in, m0 + wave), lane), gamma = lf_pieces(a, a.gamma1, lane),
+                           beta = lf_pieces(a, a.beta1, lane);
             lf_wait(a, ctr, wave, c_o + panel, 1, (unsigned)a.g_o);
-            lf_layernorm(a, a.oraw, a.in, a.gamma1, a.beta1, m0 + wave, lane, [&](int piece, f16x8 v) {
-                *reinterpret_cast<f16x8 *>(xs + wave * ldx + piece * 8) = v;
-                if (grp0 == 0 && m0 + wave < a.M) // the skip operand of the second LayerNorm
-                    store_agent8(a.ln1 + (size_t)(m0 + wave) * a.d + piece * 8, v);
-            });
+            const LfPieces v = lf_layernorm(a, lf_pieces(a, lf_row(a, a.oraw, m0 + wave), lane), skip, gamma, beta, lane);
+            lf_put_row(a, xs + wave * ldx, v, lane);
+            // (the skip operand of the second LayerNorm)
+            if (!a.again && grp0 == 0 && m0 + wave < a.M)
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    if (lane + 64 * i < a.d >> 3)
+                        store_agent8(a.ln1 + (size_t)(m0 + wave) * a.d + (lane + 64 * i) * 8, v.p[i]);
         }
         lf_barrier();
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -357,11 +382,15 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
         const int rel = unit - a.u_at;
         const int ib = rel / a.at.nhead, h = rel - ib * a.at.nhead;
         const int b = a.blk[2 * ib], qb = a.blk[2 * ib + 1];
-        const int row0 = a.at.cu_seqlens ? a.at.cu_seqlens[b] : b * a.at.seq_len;
-        const int row1 = a.at.cu_seqlens ? a.at.cu_seqlens[b + 1] : row0 + a.at.seq_len;
-        const int p0 = row0 / LF_BM, p1 = (row1 - 1) / LF_BM;
-        lf_wait(a, ctr, wave, c_qkv + p0, p1 - p0 + 1, (unsigned)a.g_qkv);
-        attention_block<HD, 1, LF_WAVES, false, false, false, HD, false, true, MASK>(a.at, b, h, qb);
+        if constexpr (FUSED) { // ... and its projections
+            qkv_attention_block<LF_WAVES, LF_HEAD_PAIRS, MASK, true>(a.qa, b, h);
+        } else {
+            const int row0 = a.at.cu_seqlens ? a.at.cu_seqlens[b] : b * a.at.seq_len;
+            const int row1 = a.at.cu_seqlens ? a.at.cu_seqlens[b + 1] : row0 + a.at.seq_len;
+            const int p0 = row0 / LF_BM, p1 = (row1 - 1) / LF_BM;
+            lf_wait(a, ctr, wave, c_qkv + p0, p1 - p0 + 1, (unsigned)a.g_qkv);
+            attention_block<HD, 1, LF_WAVES, false, false, false, HD, false, true, MASK>(a.at, b, h, qb);
+        }
         (void)lf_signal(ctr, c_at + ib);
     } else {
         // ---- second feed-forward linear; whoever completes a panel runs its LayerNorm
@@ -374,6 +403,16 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
         const f16x4 bias = lf_bias(a.m2, bn, lane);
         LfPairs<LF_D> p;
         const int n = lf_request(p, a.m2, w, lane_w2, hi4);
+        // The skip operand of the second LayerNorm is the first one's rows, which the linear before stores - and is held up
+        // by it.  Where every unit has a CU of its own from the start, this one computes them again while it waits.
+        f16 *const midrow = xs + LF_WAVES * 64 * 8 + wave * a.d; // (behind the partial sums)
+        if (a.again) {
+            const LfPieces skip = lf_pieces(a, lf_row(a, a.in, m0 + wave), lane), gamma = lf_pieces(a, a.gamma1, lane),
+                           beta = lf_pieces(a, a.beta1, lane);
+            lf_wait(a, ctr, wave, c_o + panel, 1, (unsigned)a.g_o);
+            const LfPieces v = lf_layernorm(a, lf_pieces(a, lf_row(a, a.oraw, m0 + wave), lane), skip, gamma, beta, lane);
+            lf_put_row(a, midrow, v, lane);
+        }
         lf_wait(a, ctr, wave, c_f1 + panel, 1, (unsigned)a.g_f1);
         const char *xr = reinterpret_cast<const char *>(a.hid + (size_t)min(m0 + c16, a.M - 1) * a.dff + khalf8);
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -388,10 +427,14 @@ __global__ void __launch_bounds__(LF_WAVES * 64, 4) layer_flow_kernel(const LfAr
         // every unit of every earlier step of this panel is done; if this is the last panel, of the launch
         if (threadIdx.x == 0)
             bc[2] = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        lf_layernorm(a, a.fraw, a.ln1, a.gamma2, a.beta2, m0 + wave, lane, [&](int piece, f16x8 v) {
+        {
+            const LfPieces y = lf_pieces(a, lf_row(a, a.fraw, m0 + wave), lane),
+                           skip = lf_pieces(a, a.again ? midrow : lf_row(a, a.ln1, m0 + wave), lane),
+                           gamma = lf_pieces(a, a.gamma2, lane), beta = lf_pieces(a, a.beta2, lane);
+            const LfPieces v = lf_layernorm(a, y, skip, gamma, beta, lane);
             if (m0 + wave < a.M)
-                *reinterpret_cast<f16x8 *>(a.out + (size_t)(m0 + wave) * a.d + piece * 8) = v;
-        });
+                lf_put_row(a, a.out + (size_t)(m0 + wave) * a.d, v, lane);
+        }
         lf_barrier();
         if ((int)bc[2] == a.npanel - 1) {
             unsigned *const other = a.ctr + (size_t)(1 + (set ^ 1) * a.nctr) * LF_CS;
@@ -408,14 +451,19 @@ static int g_flow_rows = -1; // et_tuning_set("layer_flow_rows"): rows up to whi
 void set_flow_rows(int v) { g_flow_rows = v; }
 bool tail_tuned();
 
-// Automatic choice: up to 96 rows, and up to 30 MB of W in all (every 16-row panel streams the layer's tiles once).
-// One launch against seven, us, rows 37 / 64 / 96 / 128: 768 wide, 80 % pruned 25.2 / 25.5 / 29.7 / 33.3 against
-// 30.3 / 30.2 / 30.9 / 30.6; 50 % 27.9 / 31.2 / 33.0 against 32.2 / 32.4 / 34.0; dense 34.5 / 38.8 against
-// 35.1 / 35.4; 512 wide, 80 % 22.4 / 22.9 / 25.0 / 27.8 against 30.
+// Automatic choice.  With projections and attention as one unit: while there is about one unit per CU - then all of them
+// request their weights at once; a second round of units costs what a launch does.  One launch against the separate ones
+// (five to seven), us, 80 % pruned, sequences x rows (units): 768 wide 1 x 16 (51) 18.9 / 23.8, 1 x 37 (129) 21.1 / 25.0, 1 x 64
+// (168) 22.8 / 26.1, 1 x 96 (246) 24.9 / 28.4, 3 x 32 (270) 24.7 / 24.6, 1 x 112 (285) 30.9 / 29.5, 8 x 16 (408) 24.9 / 24.1; 512
+// wide 2 x 64 (224) 20.0 / 24.5, 1 x 128 (216) 23.9 / 29.0, 8 x 16 (272) 21.0 / 24.3; 1024 wide 1 x 64 (224) 24.5 / 27.6, 6 x 10
+// (304) 25.9 / 24.9.  Else up to 96 rows, and up to 30 MB of W in all (every 16-row panel streams the layer's tiles once),
+// where the separate launches do not have projections and attention in one either: 768 wide, 50 % pruned 1 x 37 27.4 / 29.5,
+// 1 x 64 29.9 / 29.4; with them 2 x 32 29.5 / 27.0.
 constexpr int LF_MOST_ROWS = 96;
 constexpr double LF_MOST_MB = 30.0;
+constexpr int LF_MOST_ROOM = 160; // rows of a layer that an object is made for: what fits the units of a narrow one
 constexpr int LF_MAX_ROWS = 2048; // (forced by the tuning key)
-static int flow_rows_limit() { return g_flow_rows < 0 ? LF_MOST_ROWS : std::min(g_flow_rows, LF_MAX_ROWS); }
+static int flow_rows_limit() { return g_flow_rows < 0 ? LF_MOST_ROOM : std::min(g_flow_rows, LF_MAX_ROWS); }
 } // namespace et
 
 struct et_layer_flow {
@@ -428,6 +476,11 @@ struct et_layer_flow {
     double mbytes = 0.0; // of surviving tiles in the six linears
     int nblk[2] = {0, 0}, rows[2] = {0, 0};
     bool packed = false; // et_layer_flow_set_packed has been called
+    bool fused = false;  // a head's projections and attention are one unit
+    int s_qkv = 0, s_o = 0, s_f1 = 0, s_f2 = 0;                   // log2 of the splits
+    int gl_q = 0, gl_k = 0, g_qkv = 0, g_o = 0, g_f1 = 0, g_f2 = 0; // units per panel (fused: none of Q/K/V)
+    int units(int which) const { return npanel(which) * (g_qkv + g_o + g_f1 + g_f2) + nblk[which] * nheads; }
+    int npanel(int which) const { return (rows[which] + et::LF_BM - 1) / et::LF_BM; }
 };
 
 namespace et {
@@ -493,6 +546,23 @@ extern "C" int et_layer_flow_create(et_layer_flow **flow, const et_tile_plan *q,
         f->p[i] = ps[i];
         f->mbytes += ps[i]->ntile * 512e-6;
     }
+    f->fused = qa_shapes(q, k, v, seq_len, d, nheads, LF_HEAD_PAIRS);
+    auto groups = [](const et_tile_plan *p, int s) {
+        const int br = LF_WAVES >> s;
+        return (p->out_feat / 16 + br - 1) / br;
+    };
+    if (!f->fused) {
+        f->s_qkv = std::max(std::max(flow_split(q, LF_SHARE), flow_split(k, LF_SHARE)), flow_split(v, LF_SHARE));
+        f->gl_q = groups(q, f->s_qkv);
+        f->gl_k = groups(k, f->s_qkv);
+        f->g_qkv = f->gl_q + f->gl_k + groups(v, f->s_qkv);
+    }
+    f->s_o = flow_split(o, LF_SHARE);
+    f->s_f1 = flow_split(m1, LF_SHARE);
+    f->s_f2 = 3;
+    f->g_o = groups(o, f->s_o);
+    f->g_f1 = groups(m1, f->s_f1);
+    f->g_f2 = groups(m2, f->s_f2);
     f->d = d;
     f->dff = dff;
     f->seq_len = seq_len;
@@ -558,7 +628,13 @@ extern "C" int et_layer_flow_pays(const et_layer_flow *f, int rows) {
     using namespace et;
     if (!f || rows <= 0 || rows > flow_rows_limit() || tail_pair_enabled() || tail_tuned())
         return 0;
-    return g_flow_rows >= 0 || (rows + LF_BM - 1) / LF_BM * f->mbytes <= LF_MOST_MB ? 1 : 0;
+    if (g_flow_rows >= 0)
+        return 1;
+    const int which = f->packed && rows == f->rows[1] ? 1 : 0, cus = std::max(et_device_cu_count(), 1);
+    if (f->fused)
+        return rows <= f->rows[which] && f->units(which) <= cus + cus / 16;
+    return rows <= LF_MOST_ROWS && (rows + LF_BM - 1) / LF_BM * f->mbytes <= LF_MOST_MB &&
+           !et_qkv_attention_pays(f->p[0], f->p[1], f->p[2], f->seq_len, f->d, f->nheads, f->batch);
 }
 
 extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, void *Q, void *K, void *V, void *attn,
@@ -626,39 +702,61 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
     a.ctr = f->ctr;
     a.blk = f->d_blk[which];
     a.d = f->d;
+    a.inv_d = 1.0f / (float)f->d;
     a.dff = f->dff;
-    a.npanel = (a.M + LF_BM - 1) / LF_BM;
+    a.npanel = f->npanel(which);
     a.nblk = f->nblk[which];
     a.nctr = f->nctr;
-    a.s_qkv = std::max(std::max(flow_split(f->p[0], LF_SHARE), flow_split(f->p[1], LF_SHARE)), flow_split(f->p[2], LF_SHARE));
-    a.s_o = flow_split(f->p[3], LF_SHARE);
-    a.s_f1 = flow_split(f->p[4], LF_SHARE);
-    a.s_f2 = 3;
-    auto groups = [](const et_tile_plan *p, int s) {
-        const int br = LF_WAVES >> s;
-        return (p->out_feat / 16 + br - 1) / br;
-    };
-    a.gl_q = groups(f->p[0], a.s_qkv);
-    a.gl_k = groups(f->p[1], a.s_qkv);
-    a.g_qkv = a.gl_q + a.gl_k + groups(f->p[2], a.s_qkv);
-    a.g_o = groups(f->p[3], a.s_o);
-    a.g_f1 = groups(f->p[4], a.s_f1);
-    a.g_f2 = groups(f->p[5], a.s_f2);
+    a.s_qkv = f->s_qkv;
+    a.s_o = f->s_o;
+    a.s_f1 = f->s_f1;
+    a.s_f2 = f->s_f2;
+    a.gl_q = f->gl_q;
+    a.gl_k = f->gl_k;
+    a.g_qkv = f->g_qkv;
+    a.g_o = f->g_o;
+    a.g_f1 = f->g_f1;
+    a.g_f2 = f->g_f2;
+    const bool fused = f->fused;
     a.u_at = a.npanel * a.g_qkv;
     a.u_o = a.u_at + a.nblk * f->nheads;
     a.u_f1 = a.u_o + a.npanel * a.g_o;
     a.u_f2 = a.u_f1 + a.npanel * a.g_f1;
     const int total = a.u_f2 + a.npanel * a.g_f2;
+    a.again = total <= std::max(et_device_cu_count(), 1);
     const bool wide = f->d / f->nheads == 64;
     const size_t lds_at = wide ? attn_lds_bytes<64, 1, LF_WAVES, false>() : attn_lds_bytes<32, 1, LF_WAVES, false>();
     const size_t lds_x = (size_t)LF_BM * (f->d + 16) * sizeof(f16);
-    a.misc = (int)std::max(std::max(lds_at, lds_x), (size_t)LF_WAVES * 64 * sizeof(f32x4));
+    size_t lds_head = 0;
+    if (fused) {
+        qa_operands(a.qa, f->p[0], f->p[1], f->p[2], f->seq_len, f->d, 160 * 1024 - 64);
+        a.qa.X = a.in;
+        a.qa.mask = a.at.mask;
+        a.qa.out = a.at.out;
+        a.qa.seq_lens = a.at.seq_lens;
+        a.qa.cu_seqlens = a.at.cu_seqlens;
+        a.qa.seq_len = f->seq_len;
+        a.qa.nhead = f->nheads;
+        a.qa.batch = f->batch;
+        a.qa.log2_scale = log2_scale;
+        a.qa.scale = a.at.scale;
+        lds_head = qa_lds(a.qa.ring, f->d, f->seq_len);
+    }
+    a.misc = (int)std::max(std::max(fused ? lds_head : lds_at, lds_x), (size_t)LF_WAVES * 64 * sizeof(f32x4) + (size_t)LF_BM * f->d * sizeof(f16));
     const size_t lds = a.misc + 64;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    static_assert(attn_lds_bytes<64, 1, LF_WAVES, false>() + 64 <= 64 * 1024 && LF_BM * (1024 + 16) * 2 + 64 <= 64 * 1024,
-                  "no opt-in for dynamic LDS needed");
-    const auto kern = wide ? (a.at.mask ? layer_flow_kernel<64, true> : layer_flow_kernel<64, false>)
-                           : (a.at.mask ? layer_flow_kernel<32, true> : layer_flow_kernel<32, false>);
-    hipLaunchKernelGGL(kern, dim3(total), dim3(LF_WAVES * 64), lds, st, a);
-    return launch_status("layer in one launch");
+    auto launch = [&](auto hd_c, auto mask_c, auto fused_c) -> int {
+        constexpr auto kern = &layer_flow_kernel<decltype(hd_c)::value, decltype(mask_c)::value, decltype(fused_c)::value>;
+        if (lds > 64 * 1024) // (the default limit)
+            ET_HIP(allow_lds<kern>(lds));
+        hipLaunchKernelGGL(kern, dim3(total), dim3(LF_WAVES * 64), lds, st, a);
+        return launch_status("layer in one launch");
+    };
+    typedef std::integral_constant<int, 64> wide_t;
+    typedef std::integral_constant<int, 32> narrow_t;
+    if (fused)
+        return a.at.mask ? launch(wide_t(), std::true_type(), std::true_type()) : launch(wide_t(), std::false_type(), std::true_type());
+    if (wide)
+        return a.at.mask ? launch(wide_t(), std::true_type(), std::false_type()) : launch(wide_t(), std::false_type(), std::false_type());
+    return a.at.mask ? launch(narrow_t(), std::true_type(), std::false_type()) : launch(narrow_t(), std::false_type(), std::false_type());
 }

@@ -622,6 +622,38 @@ def test_layer_in_one_launch(request, d, H, dff, S, B, sp, lens, use_mask):
         del graph
 
 
+@pytest.mark.parametrize("d,H,dff,S,B,sp,lens,use_mask", [
+    (768, 12, 3072, 10, 9, 0.8, None, True),           # a head's projections and attention as a unit; more units than CUs
+    (768, 12, 3072, 33, 2, 0.9, [33, 1], False),       # ... a CU for every unit; one row behind two panels
+    (512, 8, 2048, 16, 5, 0.9, [16, 0, 7, 16, 0], True),  # empty sequences have no unit when packed
+    (256, 4, 1024, 96, 1, 0.0, None, False),           # dense lists short enough for a wave
+])
+def test_layer_in_one_launch_heads_as_units(request, d, H, dff, S, B, sp, lens, use_mask):
+    test_layer_in_one_launch(request, d, H, dff, S, B, sp, lens, use_mask)
+
+
+@pytest.mark.parametrize("d,H,dff,S,B,one_launch", [
+    (512, 8, 2048, 128, 1, True),      # 216 units
+    (512, 8, 2048, 75, 2, False),      # 276: beyond the line
+    (768, 12, 3072, 96, 1, True),      # 246
+    (768, 12, 3072, 112, 1, False),    # 285
+])
+def test_layer_in_one_launch_by_its_units(d, H, dff, S, B, one_launch):
+    """either side of the line, against the oracle; the separate launches write the workspace, the one launch does not"""
+    from et_amd import lib
+    from et_amd.encoder import Encoder_tile
+    if lib().et_device_cu_count() != 256:
+        pytest.skip("the line is one unit per compute unit of 256")
+    r = rng(1700 + d + S)
+    lins, ln = make_layer(r, d, dff, 0.8, seed=1800 + S, std=0.03, bias_std=0.05)
+    work = workspace(Encoder_tile, d, S, H, B).fill_(7.0)
+    enc = Encoder_tile(d, S, H, work, *build_linears(lins, B * S), *ln, None, B)
+    x = randn_h(r, (B * S, d))
+    got = host(enc.run(torch.empty_like(dev(x)), dev(x)))
+    assert (host(work) == 7.0).all() == one_launch
+    check_close(got, orc.encoder_tile_layer(x, lins, ln, None, S, H, B, None, 1.0), what="layer by its units")
+
+
 @pytest.mark.parametrize("d,S,B,sp,lens,use_mask,ls", [
     (64, 1, 1, 0.5, None, False, 1.0),                      # one row, one head
     (768, 16, 3, 0.8, None, True, 1.0),                     # whole panels; mask rows of whole loads
