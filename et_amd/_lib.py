@@ -56,6 +56,7 @@ PROTOTYPES = {
     "et_layer_flow_run": (_i, [_vp] * 7 + [_vp, _ip, _ip] + [_vp] * 4 + [_f, _vp]),
     "et_qkv_attention_pays": (_i, [_vp] * 3 + [_i] * 4),
     "et_qkv_attention": (_i, [_vp] * 6 + [_ip, _ip] + [_i] * 5 + [_f, _vp]),
+    "et_tile_plan_run_scatter_ln": (_i, [_vp, _vp, _vp, _vp, _ip, _i, _vp, _vp, _vp, _i, _i, _vp]),
     "et_wait_status_take": (_i, []),
     "et_wait_status_raise_for_test": (None, []),
     "et_tile_plan_run_multi": (_i, [C.POINTER(_vp), C.POINTER(_vp), _i, _vp, _i, _vp]),

@@ -9,7 +9,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libet_amd.so")
 
-SOURCES = ["runtime.hip", "formats.cpp", "skip_layernorm.hip", "tile_linear.hip", "tile_rows.hip", "tile_tail.hip", "dense_gemm.hip", "attention.hip", "qkv_attention.hip", "layer_flow.hip",
+SOURCES = ["runtime.hip", "formats.cpp", "skip_layernorm.hip", "tile_linear.hip", "tile_rows.hip", "tile_tail.hip", "dense_gemm.hip", "attention.hip", "qkv_attention.hip", "layer_flow.hip", "row_layernorm.hip",
            "encoder_capi.cpp"]
 
 # packed fp32 ops stay off: some of their forms have produced wrong results on

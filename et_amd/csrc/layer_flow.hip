@@ -63,6 +63,7 @@
 // from memory 0.9, LayerNorm of 16 rows 0.9), 0.7 for the stores to be
 // acknowledged and 0.4 until the counter is seen.
 #include "qkv_block.h"
+#include "row_ln.h"
 #include "tile_walk.h"
 
 #include <algorithm>
@@ -217,64 +218,18 @@ __device__ __forceinline__ void lf_finish(const LfArgs &a, f32x4 acc, f32x4 *red
     lf_put<GELU>(a, acc, bias, Y, N, bn, m0 + c16, g4);
 }
 
-// LayerNorm(y + skip) of one row, spread over the wave in 16-byte pieces (the math and the order of summation of
-// skip_layernorm.hip); a lane's pieces lie at lane and lane + 64, what is behind the row is not used.
-struct LfPieces {
-    f16x8 p[2];
-};
-__device__ __forceinline__ LfPieces lf_pieces(const LfArgs &a, const f16 *row, int lane) {
-    const int npiece = a.d >> 3;
-    LfPieces v;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-        v.p[i] = *reinterpret_cast<const f16x8 *>(row + min(lane + 64 * i, npiece - 1) * 8);
-    return v;
-}
+// rows of model width in a wave's registers (row_ln.h)
+typedef RowPieces<2> LfPieces;
+__device__ __forceinline__ LfPieces lf_pieces(const LfArgs &a, const f16 *row, int lane) { return row_pieces<2>(row, a.d >> 3, lane); }
 __device__ __forceinline__ const f16 *lf_row(const LfArgs &a, const f16 *rows, int row) {
     return rows + (size_t)min(row, a.M - 1) * a.d;
 }
-__device__ __forceinline__ LfPieces lf_layernorm(const LfArgs &a, LfPieces y, const LfPieces &skip, const LfPieces &gamma,
+__device__ __forceinline__ LfPieces lf_layernorm(const LfArgs &a, const LfPieces &y, const LfPieces &skip, const LfPieces &gamma,
                                                  const LfPieces &beta, int lane) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    const int npiece = a.d >> 3;
-    // (a half times 1.0 plus a float is one instruction; the multiplier is opaque, or it is a conversion and an addition)
-    float one = 1.0f;
-    asm("" : "+s"(one));
-    float sum = 0.f, var = 0.f;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        y.p[i] += skip.p[i]; // half add, one rounding
-        if (lane + 64 * i >= npiece)
-            y.p[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-        for (int j = 0; j < 8; j += 2)
-            sum = __builtin_amdgcn_fdot2(h2{y.p[i][j], y.p[i][j + 1]}, h2{(f16)1, (f16)1}, sum, false);
-    }
-    const float mean = wave_sum(sum) * a.inv_d;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-        if (lane + 64 * i < npiece) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float d = __builtin_fmaf((float)y.p[i][j], one, -mean);
-                var += d * d;
-            }
-        }
-    const float rstd = __builtin_amdgcn_rsqf(wave_sum(var) * a.inv_d + 1e-6f); // (never a denormal)
-    const float shift = -mean * rstd;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            y.p[i][j] = (f16)(__builtin_fmaf((float)y.p[i][j], rstd, shift) * (float)gamma.p[i][j] + (float)beta.p[i][j]);
-    return y;
+    return row_layernorm(y, skip, gamma, beta, a.d >> 3, a.inv_d, lane);
 }
-
 __device__ __forceinline__ void lf_put_row(const LfArgs &a, f16 *row, const LfPieces &v, int lane) {
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-        if (lane + 64 * i < a.d >> 3)
-            *reinterpret_cast<f16x8 *>(row + (lane + 64 * i) * 8) = v.p[i];
+    row_put(row, v, a.d >> 3, lane);
 }
 
 // rows of X -> panel, DMA; rows at or beyond M stay unwritten (they only feed rows that are never stored)

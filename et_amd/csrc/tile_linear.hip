@@ -61,6 +61,7 @@ int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *
                      bool raw, hipStream_t st);
 void set_flow_rows(int v);
 void set_qkv_attention(int v);
+void set_row_layernorm(int v);
 int tail_spin();
 
 constexpr int TL_THREADS = 512;
@@ -2230,6 +2231,10 @@ extern "C" int et_tuning_set(const char *key, int value) {
     }
     if (key && !strcmp(key, "qkv_attention")) {
         et::set_qkv_attention(value);
+        return ET_OK;
+    }
+    if (key && !strcmp(key, "row_layernorm")) {
+        et::set_row_layernorm(value);
         return ET_OK;
     }
     if (key && !strcmp(key, "ln_rows")) {

@@ -198,6 +198,18 @@ class Linear_row {
     void scatter(half *out, const half *compact, int rows, void *stream) const {
         etChk(et_scatter_cols(out, compact, row_id.get(), rows, row_id_size, nrow, out_feat, stream));
     }
+    // out = LayerNorm(scatter(this linear of `in`) + skip); `compact` [rows x nrow] where that takes two launches; out
+    // may alias skip
+    void run_rows_scatter_ln(half *out, half *in, half *compact, const half *skip, const half *gamma, const half *beta,
+                             int rows, void *stream) const {
+        if (plan && !is_gelu) {
+            etChk(et_tile_plan_run_scatter_ln(plan, out, in, compact, row_id.get(), row_id_size, skip, gamma, beta, out_feat,
+                                              rows, stream));
+            return;
+        }
+        run_rows(compact, in, rows, stream);
+        scatter_skip_layernorm(out, compact, skip, gamma, beta, rows, stream);
+    }
     // out = LayerNorm(scatter(compact) + skip) in one launch; out may alias skip
     void scatter_skip_layernorm(half *out, const half *compact, const half *skip, const half *gamma,
                                 const half *beta, int rows, void *stream) const {

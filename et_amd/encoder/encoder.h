@@ -312,13 +312,11 @@ class Encoder_attnaware : public Encoder_base {
             etChk(et_Prune_attention(buffers[3], buffers[0], buffers[1], buffers[2], Q_linear.head_ptr.get(),
                                      Q_linear.nrow, nullptr, nullptr, d_model, mask_ptr(), seq_len, d_model,
                                      nheads, batch, lens_ptr(), log2_scale, stream));
-        O_linear.run_rows(buffers[0], buffers[3], n, stream);
-        // expansion to model width, skip connection and LayerNorm in one launch
-        O_linear.scatter_skip_layernorm(buffers[1], buffers[0], in, ln_gamma[0].get(), ln_beta[0].get(), n, stream);
+        // (projection, expansion to model width, skip connection and LayerNorm)
+        O_linear.run_rows_scatter_ln(buffers[1], buffers[3], buffers[0], in, ln_gamma[0].get(), ln_beta[0].get(), n, stream);
         MLP1_linear.run_rows(buffers[2], buffers[1], n, stream); // compact hidden, spans units 2..4
-        MLP2_linear.run_rows(buffers[0], buffers[2], n, stream);
-        MLP2_linear.scatter_skip_layernorm(out, buffers[0], buffers[1], ln_gamma[1].get(), ln_beta[1].get(), n,
-                                           stream);
+        MLP2_linear.run_rows_scatter_ln(out, buffers[2], buffers[0], buffers[1], ln_gamma[1].get(), ln_beta[1].get(), n,
+                                        stream);
     }
 };
 

@@ -309,6 +309,14 @@ size_t et_tile_plan_tail_ws_bytes(const et_tile_plan *out, const et_tile_plan *f
  * default), so that Encoder_*::buffer_size is then the reference's five units */
 size_t et_tail_ws_bytes_for(int d_model, int rows);
 
+/* out[M x size] = LayerNorm(scatter(X W^T + bias) + skip): a row-pruned linear (plan: its compact rows, all tiles kept),
+ * its result expanded to model width (compact column j < n goes to column col_id[j], the others are zero) and the skip
+ * connection + LayerNorm behind it (steps 6-7 and 9-10 of a layer, encoder/encoder.cu:33-44, where those linears keep
+ * some rows).  One launch for plans of one column chunk and at most 384 outputs, size up to 1024, else et_tile_plan_run into `compact` [M x out_feat] and
+ * et_scatter_skip_layernorm.  col_id: device, ascending, n of them; skip and out are [M x size]; out may alias skip. */
+int et_tile_plan_run_scatter_ln(const et_tile_plan *plan, void *out, const void *X, void *compact, const int *col_id, int n,
+                                const void *skip, const void *gamma, const void *beta, int size, int M, void *stream);
+
 /* ---- a whole layer in one launch, for few rows ------------------------------
  * Q/K/V, attention, output projection, skip + LayerNorm, feed-forward block, skip + LayerNorm as units of work
  * of one grid (the steps of encoder/encoder.cu:20-45; what Encoder_tile and Encoder_length run where it pays).
@@ -520,6 +528,8 @@ int et_device_synchronize(void);
  *                     0: never
  *   "qkv_attention"   projections and attention of a head in one launch: 0 never, 1
  *                     wherever the form exists, -1 (default) where it pays
+ *   "row_layernorm"   row-pruned linear, expansion and LayerNorm in one launch: 0
+ *                     never, 1 (default) wherever the form exists
  *   "plan_dense"      plans of fully populated matrices as dense products: 0
  *                     never, 1 (default) where the estimated time is less, 2
  *                     always

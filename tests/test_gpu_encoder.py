@@ -353,6 +353,51 @@ def attnaware_case(S, B, balanced, sample, d=768, H=12, dff=3072):
     check_close(got, outd, what="Encoder_attnaware vs dense-with-zeroed-rows")
 
 
+@pytest.mark.parametrize("M,K,n,size,alias", [
+    (1, 64, 5, 64, False),              # one row, one block-row
+    (15, 768, 230, 768, True),          # the last block-row padded; out over the skip rows
+    (17, 624, 154, 768, False),         # an odd number of tiles in a list; rows of X narrower than the result
+    (1025, 1024, 384, 1024, False),     # three block-rows a wave, two pieces a lane
+    (4097, 928, 230, 768, True),        # 32 rows a workgroup, the last one with one
+    (4130, 512, 130, 512, False),       # one piece a lane
+    (8200, 768, 377, 768, False),       # 64 rows a workgroup
+    (40, 1104, 100, 768, False),        # two column chunks: the two launches
+    (40, 768, 385, 768, False),         # too wide: the two launches
+])
+def test_row_linear_scatter_layernorm(M, K, n, size, alias):
+    """row-pruned linear + expansion + skip + LayerNorm against the oracle's steps"""
+    import ctypes as C
+    from et_amd import lib
+    from et_amd._lib import check
+    r = rng(2500 + M + K)
+    N = (n + 15) // 16 * 16
+    W = np.zeros((N, K), np.float16)
+    W[:n] = randn_h(r, (n, K), 0.04)
+    bias = np.zeros(N, np.float16)
+    bias[:n] = randn_h(r, (n,), 0.1)
+    col = np.sort(r.permutation(size)[:n]).astype(np.int32)
+    X, skip = randn_h(r, (M, K)), randn_h(r, (M, size))
+    gamma, beta = randn_h(r, (size,), 0.2) + np.float16(1), randn_h(r, (size,), 0.2)
+    rows = np.unique(np.concatenate([np.arange(min(M, 40)), np.arange(max(M - 40, 0), M)]))
+    y = np.zeros((rows.size, size), np.float16)
+    y[:, col] = orc.row_linear(X[rows], W, bias)[:, :n]
+    want = orc.skip_layernorm(y, skip[rows], gamma, beta)
+    rp = (np.arange(N // 16 + 1) * (K // 16)).astype(np.int32)
+    ro = np.tile(np.arange(K // 16) * 16, N // 16).astype(np.int32)
+    data = orc.tile_pack(W, rp, ro)
+    L, p = lib(), C.c_void_p()
+    check(L.et_tile_plan_create(C.byref(p), K, N, ro.size, data.ctypes.data, rp.ctypes.data, ro.ctypes.data, bias.ctypes.data))
+    try:
+        Xd, sd, gd, bd, cd = dev(X), dev(skip), dev(gamma), dev(beta), dev(col)
+        out = sd if alias else torch.empty_like(sd)
+        compact = torch.empty((M, N), dtype=torch.float16, device="cuda")
+        check(L.et_tile_plan_run_scatter_ln(p, out.data_ptr(), Xd.data_ptr(), compact.data_ptr(), cd.data_ptr(), n, sd.data_ptr(),
+                                            gd.data_ptr(), bd.data_ptr(), size, M, torch.cuda.current_stream().cuda_stream))
+        check_close(host(out)[rows], want, what="row linear + LayerNorm")
+    finally:
+        L.et_tile_plan_destroy(p)
+
+
 def test_encoder_length_paths():
     from et_amd.encoder import Encoder_length
     r = rng(700)
