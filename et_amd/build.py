@@ -18,7 +18,9 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-W
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              # keep MFMA accumulators in VGPRs: the softmax / epilogue VALU work
              # reads them directly instead of copying from AGPRs
-             "-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+             "-mllvm", "-amdgpu-mfma-vgpr-form=1",
+             # the first scalar kernel parameters arrive in registers with the wave instead of by a load of its own
+             "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 
 def hipcc() -> str:

@@ -48,7 +48,20 @@ __device__ __forceinline__ int dg_swizzle(int r, int kc) { return kc ^ ((r >> 1)
 // 8192 rows 768 -> 768 18.5 -> 16.8, 768 -> 3072 53.0 -> 47.6, 3072 -> 768 49.7 -> 43.3, 928 -> 240 15.2 -> 10.2;
 // 16384 rows 1024 -> 4096 176 -> 132 (1040 TFLOP/s); 4096 x 4096 x 4096 151 -> 114 (1200 TFLOP/s).
 template <bool GELU, int WM, int WN, int TM, int TN, int ST>
-__global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(const DgArgs a) {
+__global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
+    // (what the first requests need arrives in registers with the wave)
+    const f16 *hot_X, const f16 *hot_W, int hot_M, int hot_K, int hot_N, int hot_per_xcd, int hot_total, int hot_div,
+    unsigned hot_div_magic, int hot_nlin, const DgArgs args) {
+    DgArgs a = args;
+    a.X = hot_X;
+    a.M = hot_M;
+    a.K = hot_K;
+    a.per_xcd = hot_per_xcd;
+    a.total = hot_total;
+    a.div = hot_div;
+    a.div_magic = hot_div_magic;
+    a.nlin = hot_nlin & 15;
+    a.by_column = hot_nlin >> 4;
     constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char dg_smem[];
     f16 *smem = reinterpret_cast<f16 *>(dg_smem);
@@ -60,15 +73,18 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(const DgArgs a)
         return;
     const int outer = div_magic(vid, a.div_magic), inner = vid - outer * a.div;
     const int tm = a.by_column ? inner : outer, tn_all = a.by_column ? outer : inner;
-    int lin = 0;
+    int lin = 0, tn = tn_all, N = hot_N;
+    const f16 *W = hot_W;
+    if (a.nlin > 1) { // (wave-uniform)
 #pragma unroll
-    for (int i = 1; i < DG_MAX_LIN; i++)
-        lin += (i < a.nlin && tn_all >= a.tile0[i]) ? 1 : 0;
-    const int tn = tn_all - (lin == 0 ? a.tile0[0] : lin == 1 ? a.tile0[1] : a.tile0[2]);
+        for (int i = 1; i < DG_MAX_LIN; i++)
+            lin += (i < a.nlin && tn_all >= a.tile0[i]) ? 1 : 0;
+        tn = tn_all - (lin == 0 ? a.tile0[0] : lin == 1 ? a.tile0[1] : a.tile0[2]);
+        W = lin == 0 ? a.W[0] : lin == 1 ? a.W[1] : a.W[2];
+        N = lin == 0 ? a.N[0] : lin == 1 ? a.N[1] : a.N[2];
+    }
     f16 *const Y = lin == 0 ? a.Y[0] : lin == 1 ? a.Y[1] : a.Y[2];
-    const f16 *const W = lin == 0 ? a.W[0] : lin == 1 ? a.W[1] : a.W[2];
     const f16 *const bias = lin == 0 ? a.bias[0] : lin == 1 ? a.bias[1] : a.bias[2];
-    const int N = lin == 0 ? a.N[0] : lin == 1 ? a.N[1] : a.N[2];
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -268,7 +284,8 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
     a.div_magic = magic_of(a.div);
     constexpr auto kern = &dense_gemm_kernel<GELU, WM, WN, TM, TN, ST>;
     ET_HIP(allow_lds<kern>(lds));
-    hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(WM * WN * 64), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(WM * WN * 64), lds, st, a.X, a.W[0], a.M, a.K, a.N[0],
+                       a.per_xcd, a.total, a.div, a.div_magic, a.nlin | a.by_column << 4, a);
     return launch_status("dense_gemm launch");
 }
 

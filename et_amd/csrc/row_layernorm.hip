@@ -44,7 +44,21 @@ struct RlArgs {
 };
 
 template <int NB, int MS, int NP>
-__global__ void __launch_bounds__(RL_WAVES * 64, NB < 3 ? 4 : 2) row_layernorm_kernel(const RlArgs a) {
+__global__ void __launch_bounds__(RL_WAVES * 64, NB < 3 ? 4 : 2) row_layernorm_kernel(
+    // (what the first requests need arrives in registers with the wave)
+    const f16 *hot_X, const f16 *hot_W, const f16 *hot_skip, int hot_M, int hot_K, int hot_nbr, int hot_ppb, int hot_size, int hot_ldx,
+    const f16 *hot_bias, const RlArgs args) {
+    RlArgs a = args;
+    a.X = hot_X;
+    a.W = hot_W;
+    a.skip = hot_skip;
+    a.M = hot_M;
+    a.K = hot_K;
+    a.nbr = hot_nbr;
+    a.ppb = hot_ppb;
+    a.size = hot_size;
+    a.ldx = hot_ldx;
+    a.bias = hot_bias;
     extern __shared__ __attribute__((aligned(16))) unsigned char rl_smem[];
     f16 *const xs = reinterpret_cast<f16 *>(rl_smem);
     constexpr int ROWS = 16 * MS / RL_WAVES; // of a wave: wave, wave + 8, ...
@@ -219,7 +233,8 @@ extern "C" int et_tile_plan_run_scatter_ln(const et_tile_plan *plan, void *out, 
         constexpr auto kern = &row_layernorm_kernel<decltype(nb_c)::value, decltype(ms_c)::value, decltype(np_c)::value>;
         if (lds > 64 * 1024) // (the default limit)
             ET_HIP(allow_lds<kern>(lds));
-        hipLaunchKernelGGL(kern, dim3((M + 16 * ms - 1) / (16 * ms)), dim3(RL_WAVES * 64), lds, st, a);
+        hipLaunchKernelGGL(kern, dim3((M + 16 * ms - 1) / (16 * ms)), dim3(RL_WAVES * 64), lds, st, a.X, a.W, a.skip, a.M, a.K,
+                           a.nbr, a.ppb, a.size, a.ldx, a.bias, a);
         return launch_status("row linear + LayerNorm launch");
     };
     typedef std::integral_constant<int, 1> c1;

@@ -116,6 +116,35 @@ struct TlArgs {
     int *status;               // fused feed-forward kernels: set when a bounded LDS wait gives up
     int spin;                  // ... after this many polls
 };
+// What a workgroup needs before its first requests stands in front of the struct as parameters of its own: the hardware
+// loads the first fourteen dwords of scalar parameters into registers while it starts a wave (build.py asks for it), a
+// struct is fetched from memory by the wave.  0.3-0.6 us a launch: 80 %, 37 rows 768->768 4.50 -> 4.12, 1536 rows
+// 768->768 + skip + LayerNorm 6.24 -> 5.90, 1000 rows 3072->768 10.5 -> 9.8.  (The fused feed-forward kernel runs for
+// 50 us and has no register to spare: its arguments stay in the struct.)
+#define TL_HOT_PARAMS                                                                             \
+    const f16 *hot_X, const int *hot_cptr, int hot_M, int hot_K, int hot_n, int hot_per_xcd, int hot_nwg, int hot_div,       \
+        unsigned hot_div_magic, unsigned hot_ncg_magic, int hot_ncg, int hot_ipw
+// (hot_n: outputs of the first linear for the resident kernel, whose one chunk is K wide, else the chunk's width)
+#define TL_HOT(a_, n_)                                                                            \
+    (a_).X, (a_).cptr[0], (a_).M, (a_).K, (a_).n_, (a_).per_xcd, (a_).nwg, (a_).div, (a_).div_magic, (a_).ncg_magic, (a_).ncg,  \
+        (a_).ipw | (a_).nlin << 24 | ((a_).by_group ? 1 << 30 : 0)
+constexpr int TL_HOT_BYTES = 2 * 8 + 10 * 4; // (the struct starts behind them)
+#define TL_HOT_TAKE(a_, args_, n_)                                                                \
+    TlArgs a_ = args_;                                                                            \
+    a_.X = hot_X;                                                                                 \
+    a_.cptr[0] = hot_cptr;                                                                        \
+    a_.M = hot_M;                                                                                 \
+    a_.K = hot_K;                                                                                 \
+    a_.n_ = hot_n;                                                                                \
+    a_.per_xcd = hot_per_xcd;                                                                     \
+    a_.nwg = hot_nwg;                                                                             \
+    a_.div = hot_div;                                                                             \
+    a_.div_magic = hot_div_magic;                                                                 \
+    a_.ncg_magic = hot_ncg_magic;                                                                 \
+    a_.ncg = hot_ncg;                                                                             \
+    a_.by_group = hot_ipw >> 30;                                                                  \
+    a_.nlin = hot_ipw >> 24 & 63;                                                                 \
+    a_.ipw = hot_ipw & 0xFFFFFF;
 #define TL_SEL(f) (lin == 0 ? a.f[0] : lin == 1 ? a.f[1] : lin == 2 ? a.f[2] : a.f[3])
 
 // tanh-form GELU of kernels/linear.cu:36-48: x^3 in half, the tanh argument
@@ -649,7 +678,8 @@ __device__ __forceinline__ void tl_ln_rows_at(const TlLnOperands<NB, NW, NLW> &o
 // ---------------------------------------------------------------------------
 
 template <int NB, bool GELU, int NW, bool LN>
-__global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(const TlArgs a) {
+__global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(TL_HOT_PARAMS, const TlArgs args) {
+    TL_HOT_TAKE(a, args, KC)
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
     f16 *xs = reinterpret_cast<f16 *>(tl_smem);
     TlCtx x;
@@ -796,7 +826,9 @@ __device__ __forceinline__ void tl_stage_tile(f16 *dst, int lds, f32x4 c0, f32x4
 }
 
 template <int NB, bool GELU, int NW, bool LN, int BM = TL_BM>
-__global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlArgs a) {
+__global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(TL_HOT_PARAMS, const TlArgs args) {
+    TL_HOT_TAKE(a, args, N[0])
+    a.KC = a.K;
     // BM = 64: 64-row panels and items (tl_stream64: four MFMAs per streamed W
     // pair), one workgroup per CU - the panel and the 64-row staging tiles fill
     // the LDS.  Chosen by the launcher where enough 64-row items exist.
@@ -867,11 +899,12 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
     // make the compiler copy it to scratch memory, and chains of selects over
     // its constant-indexed elements compile to long branch ladders.
     typedef const __attribute__((address_space(4))) char *KArg;
-    const KArg ka = (KArg)__builtin_amdgcn_kernarg_segment_ptr(); // TlArgs is the only argument
+    const KArg ka = (KArg)__builtin_amdgcn_kernarg_segment_ptr() + TL_HOT_BYTES;
 #define TL_KARG(type_, field_, lin_)                                                              \
     (*(const __attribute__((address_space(4))) type_ *)(ka + offsetof(TlArgs, field_) +           \
                                                          (lin_) * sizeof(type_)))
-    auto tl_item = [&](int lin, int cg) {
+    typedef const int *ListPtr;
+    auto tl_item = [&](int lin, int cg, ListPtr cptr, int N) {
         TlItem t;
         t.lin = lin;
         t.cg = cg;
@@ -879,30 +912,40 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(const TlA
         typedef f16 *YPtr;
         typedef const int *IPtr;
         typedef const f16 *HPtr;
-        t.Y = TL_KARG(YPtr, Y, lin);
-        t.cptr = TL_KARG(IPtr, cptr, lin);
-        t.poff = TL_KARG(IPtr, row_offset, lin);
-        t.data = TL_KARG(HPtr, data, lin);
-        t.bias = TL_KARG(HPtr, bias, lin);
-        t.N = TL_KARG(int, N, lin);
-        t.nbr = t.N >> 4;
+        t.cptr = cptr;
+        t.N = N;
+        t.nbr = N >> 4;
         typedef const __attribute__((address_space(4))) int *IConst;
         const IConst cp = (IConst)t.cptr;
-        t.q0 = cp[min(t.bn0, t.nbr)] >> 1;
-        t.qend = cp[min(t.bn0 + NB, t.nbr)] >> 1;
+        // (all of them requested before the first is waited for)
+        const int t0 = cp[min(t.bn0, t.nbr)], t1 = cp[min(t.bn0 + NB, t.nbr)];
+        t.data = TL_KARG(HPtr, data, lin);
+        t.poff = TL_KARG(IPtr, row_offset, lin);
+        t.bias = TL_KARG(HPtr, bias, lin);
+        t.Y = TL_KARG(YPtr, Y, lin);
+        __builtin_amdgcn_sched_barrier(0);
+        t.q0 = t0 >> 1;
+        t.qend = t1 >> 1;
         return t;
     };
     // the panel's next item
     auto tl_next = [&](const TlItem &t) {
         const bool cw = t.cg + 1 == a.ncg;
-        return tl_item(cw ? (t.lin + 1 == a.nlin ? 0 : t.lin + 1) : t.lin, cw ? 0 : t.cg + 1);
+        const int lin = cw ? (t.lin + 1 == a.nlin ? 0 : t.lin + 1) : t.lin;
+        return tl_item(lin, cw ? 0 : t.cg + 1, TL_KARG(ListPtr, cptr, lin), TL_KARG(int, N, lin));
     };
-    TlItem cur = tl_item(lin0, cg0);
+    TL_PANEL(rp) // (requested with what came with the wave; the rest of the arguments is on its way)
+    ListPtr cptr0 = hot_cptr;
+    int n0 = hot_n;
+    if (lin0 > 0) { // (wave-uniform)
+        cptr0 = TL_KARG(ListPtr, cptr, lin0);
+        n0 = TL_KARG(int, N, lin0);
+    }
+    TlItem cur = tl_item(lin0, cg0, cptr0, n0);
 
     int bvec = TL_BVEC(cur);
     f16x4 b4[NB];
     TL_BIAS(b4, cur)
-    TL_PANEL(rp)
     int q0, qend, qlast;
     const f16 *wdata;
     const int *wpoff;
@@ -1015,7 +1058,8 @@ constexpr int TL_FWAVES = 4; // fetching waves, eight panel rows each
 constexpr int TL_CTHREADS = (TL_CWAVES + TL_FWAVES) * 64;
 
 template <int NB, bool GELU, bool LN>
-__global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_kernel(const TlArgs a) {
+__global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_kernel(TL_HOT_PARAMS, const TlArgs args) {
+    TL_HOT_TAKE(a, args, KC)
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
     f16 *xs = reinterpret_cast<f16 *>(tl_smem);
     TlCtx x;
@@ -1534,11 +1578,11 @@ static int launch_inst(const TlArgs &a, size_t lds, hipStream_t st) {
         if (a.nchunk == 1) {
             constexpr auto k = &tile_linear_resident_kernel<PNB, GELU, TL_WAVES, false>;
             ET_HIP(allow_lds<k>(lds));
-            hipLaunchKernelGGL(k, grid, block, lds, st, a);
+            hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, N[0]), a);
         } else {
             constexpr auto k = &tile_linear_plan_kernel<PNB, GELU, TL_WAVES, false>;
             ET_HIP(allow_lds<k>(lds));
-            hipLaunchKernelGGL(k, grid, block, lds, st, a);
+            hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, KC), a);
         }
     } else {
         hipLaunchKernelGGL((tile_linear_generic_kernel<NB, GELU, MODE>), grid, block, lds, st, a);
@@ -1566,11 +1610,11 @@ static int launch_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     if (a.nchunk == 1) {
         constexpr auto k = &tile_linear_resident_kernel<NB, false, TL_LN_WAVES, true>;
         ET_HIP(allow_lds<k>(lds));
-        hipLaunchKernelGGL(k, grid, block, lds, st, a);
+        hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, N[0]), a);
     } else {
         constexpr auto k = &tile_linear_plan_kernel<NB, false, TL_LN_WAVES, true>;
         ET_HIP(allow_lds<k>(lds));
-        hipLaunchKernelGGL(k, grid, block, lds, st, a);
+        hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, KC), a);
     }
     return launch_status("tile_linear+LayerNorm launch");
 }
@@ -1586,7 +1630,7 @@ template <int NB>
 static int launch_chunked_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_chunked_kernel<NB, false, true>;
     ET_HIP(allow_lds<k>(lds));
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, a);
+    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
     return launch_status("tile_linear+LayerNorm (chunked) launch");
 }
 
@@ -1594,7 +1638,7 @@ template <int NB, bool GELU>
 static int launch_chunked_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_chunked_kernel<NB, GELU, false>;
     ET_HIP(allow_lds<k>(lds));
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, a);
+    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
     return launch_status("tile_linear (chunked) launch");
 }
 
@@ -1960,7 +2004,7 @@ template <int NB, bool GELU, int NW = TL_WAVES>
 static int launch_resident64(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_resident_kernel<NB, GELU, NW, false, TL_BM64>;
     ET_HIP(allow_lds<k>(lds));
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, a);
+    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, TL_HOT(a, N[0]), a);
     return launch_status("tile_linear (64-row panels) launch");
 }
 

@@ -61,7 +61,24 @@ __device__ __forceinline__ void tr_load_raw(TrSlots &p, const LfLinear &l, TrRaw
 }
 
 template <bool GELU, bool RAW>
-__global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(const TrArgs a) {
+__global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(
+    // (what comes before the first requests arrives in registers with the wave)
+    const f16 *hot_X, const int *hot_cptr, int hot_M, int hot_K, int hot_total, int hot_per_xcd, int hot_div, unsigned hot_div_magic,
+    int hot_ncg, unsigned hot_ncg_magic, int hot_form, int hot_nbr, const TrArgs args) {
+    TrArgs a = args;
+    a.X = hot_X;
+    a.M = hot_M;
+    a.K = hot_K;
+    a.ldx = hot_K + ((hot_K & 31) ? 0 : 16);
+    a.total = hot_total;
+    a.per_xcd = hot_per_xcd;
+    a.div = hot_div;
+    a.div_magic = hot_div_magic;
+    a.ncg = hot_ncg;
+    a.ncg_magic = hot_ncg_magic;
+    a.nb = hot_form & 15;
+    a.ls = hot_form >> 4 & 15;
+    a.by_group = hot_form >> 8;
     extern __shared__ __attribute__((aligned(16))) unsigned char tr_smem[];
     f16 *const xs = reinterpret_cast<f16 *>(tr_smem);
     // (consecutive ids on one XCD: the column groups of a panel, or, by_group, the panels of a column group)
@@ -75,28 +92,30 @@ __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(const TrArgs a
     const int panel = a.by_group ? inner : outer, rest = a.by_group ? outer : inner;
     const int lin = div_magic(rest, a.ncg_magic), cg = rest - lin * a.ncg;
     const int m0 = panel * TR_BM;
+    // the panel: wave w fetches row w, DMA
+    if (m0 + wave < a.M) {
+        const f16 *src = a.X + (size_t)(m0 + wave) * a.K;
+        f16 *dst = xs + wave * a.ldx;
+        const int npiece = a.K >> 3;
+        for (int c0 = 0; c0 < npiece; c0 += 64)
+            if (c0 + lane < npiece)
+                load_lds16(src + (c0 + lane) * 8, dst + c0 * 8);
+    }
     LfLinear l = a.l[0];
     f16 *Y = a.Y[0];
+    l.cptr = hot_cptr;
+    l.nbr = hot_nbr;
+    if (lin > 0) { // (wave-uniform)
 #pragma unroll
-    for (int i = 1; i < TR_MAX_LIN; i++)
-        if (lin == i) {
-            l = a.l[i];
-            Y = a.Y[i];
-        }
+        for (int i = 1; i < TR_MAX_LIN; i++)
+            if (lin == i) {
+                l = a.l[i];
+                Y = a.Y[i];
+            }
+    }
     const int N = l.nbr * 16;
     const int br = TR_WAVES >> a.ls, j = wave & (br - 1), sub = wave / br;
 
-    // the panel: wave w fetches row w, DMA; the first pairs are requested in front of it
-    auto panel_in = [&] {
-        if (m0 + wave < a.M) {
-            const f16 *src = a.X + (size_t)(m0 + wave) * a.K;
-            f16 *dst = xs + wave * a.ldx;
-            const int npiece = a.K >> 3;
-            for (int c0 = 0; c0 < npiece; c0 += 64)
-                if (c0 + lane < npiece)
-                    load_lds16(src + (c0 + lane) * 8, dst + c0 * 8);
-        }
-    };
     const char *const xlane = reinterpret_cast<const char *>(xs + c16 * a.ldx + khalf8);
     for (int ib = 0; ib < a.nb; ib++) {
         const int bn = (cg * a.nb + ib) * br + j;
@@ -132,7 +151,6 @@ __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(const TrArgs a
     }
         TR_GROUP(0, n > 0) TR_GROUP(2, n > 2) TR_GROUP(4, n > 4) TR_GROUP(6, n > 6)
         if (ib == 0) {
-            panel_in();
             __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): pairs and panel
             __syncthreads();
         }
@@ -273,7 +291,8 @@ int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *
     auto launch = [&](auto gelu_c, auto raw_c) -> int {
         constexpr auto kern = &tile_rows_kernel<decltype(gelu_c)::value, decltype(raw_c)::value>;
         ET_HIP(allow_lds<kern>(lds));
-        hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(TR_WAVES * 64), lds, st, a);
+        hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(TR_WAVES * 64), lds, st, a.X, a.l[0].cptr, a.M, a.K, a.total, a.per_xcd,
+                           a.div, a.div_magic, a.ncg, a.ncg_magic, a.nb | a.ls << 4 | a.by_group << 8, a.l[0].nbr, a);
         return launch_status("tile_linear (whole rows) launch");
     };
     if (raw)
