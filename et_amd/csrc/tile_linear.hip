@@ -351,45 +351,77 @@ __device__ __forceinline__ void tl_preload(const f16 *data, const int *poff, uns
 }
 
 
-// bvec: lane j holds the first pair of block-row j, lane NB the end of the
-// last one (read back with v_readlane)
-template <int NB, class Flush>
-__device__ __forceinline__ void tl_stream(const char *xlane, int xrow16, const f16 *data,
-                                          const int *poff, unsigned lane_w, unsigned hi, int q0,
-                                          int qend, int qlast, int bvec, f16x8 (&w)[TL_DEPTH],
-                                          int (&o)[TL_DEPTH], Flush &&flush
-) {
-    if (q0 >= qend)
+// Ends of a wave's block-rows: [k] is the first pair of block-row k, [NB] the end of the last one.  In scalar registers
+// throughout: kept in the lanes of a vector register, every block-row end cost reads of single lanes, and filling it a
+// select per end, all of them vector instructions, which is what the fused layer tail is bound by (8192 rows, 80 %:
+// 50.5 -> 48.4 us; 90 %: 42.5 -> 40.5; the Q/K/V launch of 64-row panels 15.7 -> 15.4).
+template <int NB> struct TlBounds {
+    int at[NB + 1];
+};
+// (bvec: lane k holds [k])
+template <int NB> __device__ __forceinline__ TlBounds<NB> tl_bounds(int bvec) {
+    TlBounds<NB> b;
+#pragma unroll
+    for (int k = 0; k <= NB; k++)
+        b.at[k] = __builtin_amdgcn_readlane(bvec, k);
+    return b;
+}
+
+// MS 16-row subtiles per pair: 2 (a 32-row panel), or 4 (64 rows: a W pair feeds four MFMAs, and a stream that is bound by
+// delivering W runs faster).  flush(j, sums) receives block-row j's MS sums.
+template <int NB, int MS, class Flush>
+__device__ __forceinline__ void tl_stream(const char *xlane, int xrow16, const f16 *data, const int *poff, unsigned lane_w,
+                                          unsigned hi, TlBounds<NB> bounds, f16x8 (&w)[TL_DEPTH], int (&o)[TL_DEPTH],
+                                          Flush &&flush) {
+    const int qend = bounds.at[NB];
+    int q = bounds.at[0];
+    if (q >= qend)
         return;
     __builtin_amdgcn_s_setprio(TL_PRIO);
-    f32x4 cur0 = f32x4{0.f, 0.f, 0.f, 0.f}, cur1 = f32x4{0.f, 0.f, 0.f, 0.f};
-    int j = 0;
-    int bend = __builtin_amdgcn_readlane(bvec, 1);
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 cur[MS];
 #pragma unroll
-    for (int t = 0; t < NB - 1; t++) { // leading empty block-rows
-        j += (bend == q0 && j + 1 < NB) ? 1 : 0;
-        bend = __builtin_amdgcn_readlane(bvec, j + 1);
+    for (int m = 0; m < MS; m++)
+        cur[m] = zero;
+    // j: the block-row that runs, ends at bend; the ends behind it move up as block-rows close
+    int j = 0, bend = bounds.at[1], ends[NB];
+#pragma unroll
+    for (int k = 0; k < NB; k++)
+        ends[k] = bounds.at[k + 2 < NB ? k + 2 : NB];
+    auto next_end = [&] {
+        j++;
+        bend = ends[0];
+#pragma unroll
+        for (int k = 0; k < NB - 1; k++)
+            ends[k] = ends[k + 1];
+    };
+#pragma unroll
+    for (int t = 0; t < NB - 1; t++) // leading empty block-rows
+        if (bend == q)
+            next_end();
+    f16x8 x[2][MS];
+#pragma unroll
+    for (int m = 0; m < MS; m++) {
+        x[0][m] = *reinterpret_cast<const f16x8 *>(xlane + o[0] + m * xrow16);
+        x[1][m] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
-    f16x8 xa[2], xb[2];
-    xa[0] = *reinterpret_cast<const f16x8 *>(xlane + o[0]);
-    xb[0] = *reinterpret_cast<const f16x8 *>(xlane + o[0] + xrow16);
-    xa[1] = xb[1] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    int q = q0;
     // running (wave-uniform) addresses of pair q + TL_DEPTH: a stage adds a
     // constant, which goes into the load's immediate offset
-    const char *wp = reinterpret_cast<const char *>(data) + (size_t)(q0 + TL_DEPTH) * 1024;
-    const char *op = reinterpret_cast<const char *>(poff) + (size_t)(q0 + TL_DEPTH) * 8;
+    const char *wp = reinterpret_cast<const char *>(data) + (size_t)(q + TL_DEPTH) * 1024;
+    const char *op = reinterpret_cast<const char *>(poff) + (size_t)(q + TL_DEPTH) * 8;
     unsigned lane_lo = hi * 4u, lane_lw = lane_w * 2u;
     auto stage = [&](auto ic, auto always) {
         constexpr int I = decltype(ic)::value;
         constexpr int S = I % TL_DEPTH, SN = (I + 1) % TL_DEPTH, P = I & 1;
-        xa[P ^ 1] = *reinterpret_cast<const f16x8 *>(xlane + o[SN]);
-        xb[P ^ 1] = *reinterpret_cast<const f16x8 *>(xlane + o[SN] + xrow16);
+#pragma unroll
+        for (int m = 0; m < MS; m++)
+            x[P ^ 1][m] = *reinterpret_cast<const f16x8 *>(xlane + o[SN] + m * xrow16);
         // keep the reads above the MFMAs: left alone, the scheduler sinks them
         // to the end of the stage and every stage then waits out the LDS latency
         __builtin_amdgcn_sched_barrier(0);
-        cur0 = mfma16x16x32(w[S], xa[P], cur0);
-        cur1 = mfma16x16x32(w[S], xb[P], cur1);
+#pragma unroll
+        for (int m = 0; m < MS; m++)
+            cur[m] = mfma16x16x32(w[S], x[P][m], cur[m]);
         // pair q + I + TL_DEPTH; the last stages of a stream request nothing:
         // a request still in flight when the stream ends would make the next
         // use of these registers wait out a full memory latency
@@ -397,17 +429,16 @@ __device__ __forceinline__ void tl_stream(const char *xlane, int xrow16, const f
             tl_load_pair_at(wp + I * 1024, op + I * 8, lane_lo, lane_lw, w[S], o[S]);
         if (q + I + 1 == bend) { // block-row j is complete
             __builtin_amdgcn_s_setprio(0);
-            flush(j, cur0, cur1);
+            flush(j, cur);
             __builtin_amdgcn_s_setprio(TL_PRIO);
-            cur0 = f32x4{0.f, 0.f, 0.f, 0.f};
-            cur1 = f32x4{0.f, 0.f, 0.f, 0.f};
-            j++;
-            bend = __builtin_amdgcn_readlane(bvec, min(j + 1, NB));
 #pragma unroll
-            for (int t = 0; t < NB - 2; t++) { // skip empty block-rows
-                j += (bend == q + I + 1 && j + 1 < NB) ? 1 : 0;
-                bend = __builtin_amdgcn_readlane(bvec, min(j + 1, NB));
-            }
+            for (int m = 0; m < MS; m++)
+                cur[m] = zero;
+            next_end();
+#pragma unroll
+            for (int t = 0; t < NB - 2; t++) // skip empty block-rows
+                if (bend == q + I + 1)
+                    next_end();
         }
     };
     for (; q + 2 * TL_DEPTH <= qend; q += TL_DEPTH) { // straight-line body: counted waits
@@ -420,79 +451,6 @@ __device__ __forceinline__ void tl_stream(const char *xlane, int xrow16, const f
             stage(ic, std::false_type());
     });
     __builtin_amdgcn_s_setprio(0);
-}
-
-// The same stream over a 64-row panel: every W pair is used for four 16-row
-// subtiles (four MFMAs per kilobyte of W instead of two: the stream is bound by
-// delivering W, so this is what raises its throughput).  flush(j, c0..c3).
-template <int NB, class Flush>
-__device__ __forceinline__ void tl_stream64(const char *xlane, int xrow16, const f16 *data,
-                                          const int *poff, unsigned lane_w, unsigned hi, int q0,
-                                          int qend, int qlast, int bvec, f16x8 (&w)[TL_DEPTH],
-                                          int (&o)[TL_DEPTH], Flush &&flush
-) {
-    if (q0 >= qend)
-        return;
-    f32x4 cur0 = f32x4{0.f, 0.f, 0.f, 0.f}, cur1 = cur0, cur2 = cur0, cur3 = cur0;
-    int j = 0;
-    int bend = __builtin_amdgcn_readlane(bvec, 1);
-#pragma unroll
-    for (int t = 0; t < NB - 1; t++) { // leading empty block-rows
-        j += (bend == q0 && j + 1 < NB) ? 1 : 0;
-        bend = __builtin_amdgcn_readlane(bvec, j + 1);
-    }
-    f16x8 xa[2], xb[2], xc[2], xd[2];
-    xa[0] = *reinterpret_cast<const f16x8 *>(xlane + o[0]);
-    xb[0] = *reinterpret_cast<const f16x8 *>(xlane + o[0] + xrow16);
-    xc[0] = *reinterpret_cast<const f16x8 *>(xlane + o[0] + 2 * xrow16);
-    xd[0] = *reinterpret_cast<const f16x8 *>(xlane + o[0] + 3 * xrow16);
-    xa[1] = xb[1] = xc[1] = xd[1] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    int q = q0;
-    // running (wave-uniform) addresses of pair q + TL_DEPTH: a stage adds a
-    // constant, which goes into the load's immediate offset
-    const char *wp = reinterpret_cast<const char *>(data) + (size_t)(q0 + TL_DEPTH) * 1024;
-    const char *op = reinterpret_cast<const char *>(poff) + (size_t)(q0 + TL_DEPTH) * 8;
-    unsigned lane_lo = hi * 4u, lane_lw = lane_w * 2u;
-    auto stage = [&](auto ic, auto always) {
-        constexpr int I = decltype(ic)::value;
-        constexpr int S = I % TL_DEPTH, SN = (I + 1) % TL_DEPTH, P = I & 1;
-        xa[P ^ 1] = *reinterpret_cast<const f16x8 *>(xlane + o[SN]);
-        xb[P ^ 1] = *reinterpret_cast<const f16x8 *>(xlane + o[SN] + xrow16);
-        xc[P ^ 1] = *reinterpret_cast<const f16x8 *>(xlane + o[SN] + 2 * xrow16);
-        xd[P ^ 1] = *reinterpret_cast<const f16x8 *>(xlane + o[SN] + 3 * xrow16);
-        // keep the reads above the MFMAs: left alone, the scheduler sinks them
-        // to the end of the stage and every stage then waits out the LDS latency
-        __builtin_amdgcn_sched_barrier(0);
-        cur0 = mfma16x16x32(w[S], xa[P], cur0);
-        cur1 = mfma16x16x32(w[S], xb[P], cur1);
-        cur2 = mfma16x16x32(w[S], xc[P], cur2);
-        cur3 = mfma16x16x32(w[S], xd[P], cur3);
-        // pair q + I + TL_DEPTH; the last stages of a stream request nothing:
-        // a request still in flight when the stream ends would make the next
-        // use of these registers wait out a full memory latency
-        if (decltype(always)::value || q + I + TL_DEPTH < qend)
-            tl_load_pair_at(wp + I * 1024, op + I * 8, lane_lo, lane_lw, w[S], o[S]);
-        if (q + I + 1 == bend) { // block-row j is complete
-            flush(j, cur0, cur1, cur2, cur3);
-            cur0 = cur1 = cur2 = cur3 = f32x4{0.f, 0.f, 0.f, 0.f};
-            j++;
-            bend = __builtin_amdgcn_readlane(bvec, min(j + 1, NB));
-#pragma unroll
-            for (int t = 0; t < NB - 2; t++) { // skip empty block-rows
-                j += (bend == q + I + 1 && j + 1 < NB) ? 1 : 0;
-                bend = __builtin_amdgcn_readlane(bvec, min(j + 1, NB));
-            }
-        }
-    };
-    for (; q + 2 * TL_DEPTH <= qend; q += TL_DEPTH) { // straight-line body: counted waits
-        tl_static_for<0, TL_DEPTH>([&](auto ic) { stage(ic, std::true_type()); });
-        wp += TL_DEPTH * 1024;
-        op += TL_DEPTH * 8;
-    }
-    tl_static_for<0, 2 * TL_DEPTH - 1>([&](auto ic) {
-        if (q + decltype(ic)::value < qend)
-            stage(ic, std::false_type());
-    });
 }
 
 // flush for kernels that keep NB static accumulators: acc[j] += cur with a
@@ -764,8 +722,8 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(TL_HOT_PARAMS
         f16x8 w[TL_DEPTH];
         int o[TL_DEPTH];
         tl_preload(data, poff, lane_w, hi, q0, qlast, w, o);
-        tl_stream<NB>(xlane, xrow16, data, poff, lane_w, hi, q0, qend, qlast, bvec, w, o,
-                      [&](int j, f32x4 c0, f32x4 c1) { tl_flush_acc<NB>(acc, j, c0, c1); });
+        tl_stream<NB, 2>(xlane, xrow16, data, poff, lane_w, hi, tl_bounds<NB>(bvec), w, o,
+                         [&](int j, const f32x4 (&c)[2]) { tl_flush_acc<NB>(acc, j, c[0], c[1]); });
     }
     tl_epilogue_wave<NB, GELU, !LN>(a, x, stage, Yp, N, nbr, acc, b4);
     if constexpr (LN) {
@@ -829,7 +787,7 @@ template <int NB, bool GELU, int NW, bool LN, int BM = TL_BM>
 __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(TL_HOT_PARAMS, const TlArgs args) {
     TL_HOT_TAKE(a, args, N[0])
     a.KC = a.K;
-    // BM = 64: 64-row panels and items (tl_stream64: four MFMAs per streamed W
+    // BM = 64: 64-row panels and items (four MFMAs per streamed W
     // pair), one workgroup per CU - the panel and the 64-row staging tiles fill
     // the LDS.  Chosen by the launcher where enough 64-row items exist.
     static_assert(BM == TL_BM || (BM == 2 * TL_BM && !LN), "64-row panels: without the LayerNorm epilogue");
@@ -972,23 +930,17 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_resident_kernel(TL_HOT_PA
                 bj += b4[k] * ((j == k) ? (f16)1 : (f16)0);
             return bj;
         };
-        if constexpr (BM == TL_BM) {
-            tl_stream<NB>(xlane, xrow16, wdata, wpoff, lane_w, hi, q0, qend, qlast, bvec, w, o,
-                          [&](int j, f32x4 c0, f32x4 c1) {
-                              tl_stage_tile<GELU>(stage_lane + j * 16, lds, c0, c1, bias_of(j));
-                          });
-        } else {
-            tl_stream64<NB>(xlane, xrow16, wdata, wpoff, lane_w, hi, q0, qend, qlast, bvec, w, o,
-                            [&](int j, f32x4 c0, f32x4 c1, f32x4 c2, f32x4 c3) {
-                                const f16x4 bj = bias_of(j);
-                                tl_stage_tile<GELU>(stage_lane + j * 16, lds, c0, c1, bj);
-                                tl_stage_tile<GELU>(stage_lane + 32 * lds + j * 16, lds, c2, c3, bj);
-                            });
-        }
+        const TlBounds<NB> bounds = tl_bounds<NB>(bvec);
+        tl_stream<NB, BM / 16>(xlane, xrow16, wdata, wpoff, lane_w, hi, bounds, w, o, [&](int j, const f32x4 (&c)[BM / 16]) {
+            const f16x4 bj = bias_of(j);
+#pragma unroll
+            for (int h = 0; h < BM / TL_BM; h++)
+                tl_stage_tile<GELU>(stage_lane + h * 32 * lds + j * 16, lds, c[2 * h], c[2 * h + 1], bj);
+        });
         // block-rows without any tile: bias only
 #pragma unroll
         for (int k = 0; k < NB; k++)
-            if (__builtin_amdgcn_readlane(bvec, k) == __builtin_amdgcn_readlane(bvec, k + 1)) {
+            if (bounds.at[k] == bounds.at[k + 1]) {
 #pragma unroll
                 for (int h = 0; h < BM / TL_BM; h++)
                     tl_stage_tile<GELU>(stage_lane + h * 32 * lds + k * 16, lds, f32x4{0.f, 0.f, 0.f, 0.f},
@@ -1151,8 +1103,8 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_kernel(TL_HOT
             const int bcur = bvec;
             tl_barrier_lds();
 
-            tl_stream<NB>(xlane, xrow16, data, poff, lane_w, hi, q0, qend, qlast, bcur, w, o,
-                          [&](int j, f32x4 c0, f32x4 c1) { tl_flush_acc<NB>(acc, j, c0, c1); });
+            tl_stream<NB, 2>(xlane, xrow16, data, poff, lane_w, hi, tl_bounds<NB>(bcur), w, o,
+                             [&](int j, const f32x4 (&c)[2]) { tl_flush_acc<NB>(acc, j, c[0], c[1]); });
             bvec = bvec_n;
         }
         f16 *stage = stage0 + x.wave * tl_wave_stage_halves<NB>();
@@ -1283,23 +1235,20 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
     const int *const cptr1 = a.cptr[L1], *const cptr2 = a.cptr[L2];
     const f16 *const data1 = a.data[L1], *const data2 = a.data[L2];
     const int *const poff1 = a.row_offset[L1], *const poff2 = a.row_offset[L2];
-    // pair-index boundaries of the wave's block-rows (lane j: start of block-row
-    // j, lane NB: end of the last one); block-rows past the phase's range or the
-    // matrix are empty
+    // pair-index boundaries of the wave's block-rows; block-rows past the
+    // phase's range or the matrix are empty
     // (read with scalar loads: they do not queue behind the weight pairs in
     // flight, and no wait for them drains those)
     typedef const __attribute__((address_space(4))) int *ScalarInts;
-    auto bvec_of = [&](ScalarInts base, int i0, int lim) {
-        int v = 0;
+    auto bounds_of = [&](ScalarInts base, int i0, int lim) {
+        TlBounds<NB> b;
 #pragma unroll
-        for (int k = NB; k >= 0; k--) {
-            const int s = base[min(i0 + k, lim)] >> 1;
-            v = (lane == k) ? s : v;
-        }
-        return v;
+        for (int k = 0; k <= NB; k++)
+            b.at[k] = base[min(i0 + k, lim)] >> 1;
+        return b;
     };
-#define TL_FFN_BVEC1(p_) bvec_of((ScalarInts)cptr1, (p_) * hbr + wave * NB, min(((p_) + 1) * hbr, nbr1))
-#define TL_FFN_BVEC2(p_) bvec_of((ScalarInts)cptr2 + (p_) * nbr2, wave * NB, nbr2)
+#define TL_FFN_BOUNDS1(p_) bounds_of((ScalarInts)cptr1, (p_) * hbr + wave * NB, min(((p_) + 1) * hbr, nbr1))
+#define TL_FFN_BOUNDS2(p_) bounds_of((ScalarInts)cptr2 + (p_) * nbr2, wave * NB, nbr2)
 #define TL_FFN_BIAS1(dst_, p_)                                                                    \
     _Pragma("unroll") for (int k = 0; k < NB; k++)                                                \
         dst_[k] = *reinterpret_cast<const f16x4 *>(                                               \
@@ -1315,29 +1264,28 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
 
     // One stream of the first linear: hidden columns of phase p_ (bias, GELU,
     // half) into hidden buffer p_ & 1.  w_/o_ hold its first pairs already.
-#define TL_FFN_FIRST(p_, bvec_, b1_, w_, o_)                                                      \
+#define TL_FFN_FIRST(p_, bounds_, b1_, w_, o_)                                                      \
     {                                                                                             \
         f16 *const hlane = hs + ((p_) & 1) * hbuf + c16 * ldh + wave * NB * 16 + g4 * 4;          \
-        const int q0_ = __builtin_amdgcn_readfirstlane(bvec_), qe_ = __builtin_amdgcn_readlane(bvec_, NB); \
-        tl_stream<NB>(xlane1, xrow1, data1, poff1, lane_w, hi, q0_, qe_, max(qe_ - 1, q0_), bvec_, w_, o_, \
-                      [&](int j, f32x4 c0, f32x4 c1) {                                            \
+        tl_stream<NB, 2>(xlane1, xrow1, data1, poff1, lane_w, hi, bounds_, w_, o_,                \
+                      [&](int j, const f32x4 (&c)[2]) {                                           \
                           f16x4 bj = f16x4{0, 0, 0, 0};                                           \
                           _Pragma("unroll") for (int k = 0; k < NB; k++)                          \
                               bj += b1_[k] * ((j == k) ? (f16)1 : (f16)0);                        \
-                          tl_stage_tile<true>(hlane + j * 16, ldh, c0, c1, bj);                   \
+                          tl_stage_tile<true>(hlane + j * 16, ldh, c[0], c[1], bj);               \
                       });                                                              \
         /* block-rows of this phase without any tile: bias only */                                \
         const int lim1 = min(((p_) + 1) * hbr, nbr1);                                             \
         _Pragma("unroll") for (int k = 0; k < NB; k++)                                            \
             if ((p_) * hbr + wave * NB + k < lim1 &&                                              \
-                __builtin_amdgcn_readlane(bvec_, k) == __builtin_amdgcn_readlane(bvec_, k + 1))   \
+                bounds_.at[k] == bounds_.at[k + 1])                                               \
                 tl_stage_tile<true>(hlane + k * 16, ldh, f32x4{0.f, 0.f, 0.f, 0.f},               \
                                     f32x4{0.f, 0.f, 0.f, 0.f}, b1_[k]);                           \
         tl_signal(ctr + (p_), lane);                                                              \
     }
-#define TL_FFN_PRELOAD(data_, poff_, bvec_, w_, o_)                                               \
+#define TL_FFN_PRELOAD(data_, poff_, bounds_, w_, o_)                                               \
     {                                                                                             \
-        const int q0_ = __builtin_amdgcn_readfirstlane(bvec_), qe_ = __builtin_amdgcn_readlane(bvec_, NB); \
+        const int q0_ = bounds_.at[0], qe_ = bounds_.at[NB];                                      \
         tl_preload(data_, poff_, lane_w, hi, q0_, max(qe_ - 1, q0_), w_, o_);                     \
     }
 
@@ -1351,13 +1299,13 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
     // Register set A serves F(0) and every S, set B every later F.
     f16x8 wA[TL_DEPTH], wB[TL_DEPTH];
     int oA[TL_DEPTH], oB[TL_DEPTH];
-    int bvecF = TL_FFN_BVEC1(0);
+    TlBounds<NB> boundsF = TL_FFN_BOUNDS1(0);
     f16x4 b1[NB];
     TL_FFN_BIAS1(b1, 0)
-    int bvecFn = TL_FFN_BVEC1(min(1, a.nchunk - 1));
+    TlBounds<NB> boundsFn = TL_FFN_BOUNDS1(min(1, a.nchunk - 1));
     f16x4 b1n[NB];
     TL_FFN_BIAS1(b1n, min(1, a.nchunk - 1))
-    int bvecS = TL_FFN_BVEC2(0);
+    TlBounds<NB> boundsS = TL_FFN_BOUNDS2(0);
     __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this wave's part of the panel has landed
     if constexpr (WITH_O) {
         // Linear 0 (the attention output projection) with its skip connection
@@ -1366,7 +1314,7 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
         // stores them) replace it in LDS as the feed-forward block's input and
         // as the skip operand of the final LayerNorm.
         const int NO = a.N[0], nbrO = NO >> 4; // == K
-        const int bvecO = bvec_of((ScalarInts)a.cptr[0], wave * NB, nbrO);
+        const TlBounds<NB> boundsO = bounds_of((ScalarInts)a.cptr[0], wave * NB, nbrO);
         f16x4 bO[NB];
 #pragma unroll
         for (int j = 0; j < NB; j++) {
@@ -1374,15 +1322,13 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
             if (x.bn0 + j < nbrO)
                 bO[j] = *reinterpret_cast<const f16x4 *>(a.bias[0] + (x.bn0 + j) * 16 + g4 * 4);
         }
-        TL_FFN_PRELOAD(a.data[0], a.row_offset[0], bvecO, wB, oB)
+        TL_FFN_PRELOAD(a.data[0], a.row_offset[0], boundsO, wB, oB)
         tl_barrier_lds(); // the whole panel has landed; the counters are zero
         {
-            const int q0_ = __builtin_amdgcn_readfirstlane(bvecO), qe_ = __builtin_amdgcn_readlane(bvecO, NB);
-            tl_stream<NB>(xlane1, xrow1, a.data[0], a.row_offset[0], lane_w, hi, q0_, qe_, max(qe_ - 1, q0_),
-                          bvecO, wB, oB,
-                          [&](int j, f32x4 c0, f32x4 c1) { TL_FFN_FLUSH(acc, j, c0, c1); });
+            tl_stream<NB, 2>(xlane1, xrow1, a.data[0], a.row_offset[0], lane_w, hi, boundsO, wB, oB,
+                             [&](int j, const f32x4 (&c)[2]) { TL_FFN_FLUSH(acc, j, c[0], c[1]); });
         }
-        TL_FFN_PRELOAD(data1, poff1, bvecF, wA, oA)
+        TL_FFN_PRELOAD(data1, poff1, boundsF, wA, oA)
         TlLnOperands<NB, NW, NW> lnop1; // (requested here: their latency runs under the wait for the other waves)
         tl_ln_fetch_at(lnop1, a.M, wave, lane, x.m0, NO, a.skip + (long)x.m0 * NO, (long)NO, a.gamma, a.beta);
         // staging tiles in the hidden buffers, which nobody uses yet
@@ -1396,26 +1342,26 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
         tl_barrier_lds(); // every wave's part is staged, and everyone has left the attention panel
         tl_ln_rows_at(lnop1, a.M, hs, wave, lane, x.m0, NO, xs, (long)ldx);
     } else {
-        TL_FFN_PRELOAD(data1, poff1, bvecF, wA, oA)
+        TL_FFN_PRELOAD(data1, poff1, boundsF, wA, oA)
     }
     tl_barrier_lds(); // the feed-forward input panel is complete (and the counters are zero)
     if (a.nchunk > 1)
-        TL_FFN_PRELOAD(data1, poff1, bvecFn, wB, oB)
-    TL_FFN_FIRST(0, bvecF, b1, wA, oA)
+        TL_FFN_PRELOAD(data1, poff1, boundsFn, wB, oB)
+    TL_FFN_FIRST(0, boundsF, b1, wA, oA)
 
     const int behind = (wave >> 2) & 1; // (a SIMD's waves are w, w+4, w+8, w+12)
     for (int p = 0; p < a.nchunk; p++) {
-        const int bvecSn = TL_FFN_BVEC2(min(p + 1, a.nchunk - 1));
-        TL_FFN_PRELOAD(data2, poff2, bvecS, wA, oA) // S(p), a stream ahead (unless no F runs in between)
+        const TlBounds<NB> boundsSn = TL_FFN_BOUNDS2(min(p + 1, a.nchunk - 1));
+        TL_FFN_PRELOAD(data2, poff2, boundsS, wA, oA) // S(p), a stream ahead (unless no F runs in between)
         const int fq = p + 1 - behind; // the first-linear phase this wave runs before S(p)
         if (fq >= 1 && fq < a.nchunk) {
-            const int bvecF2 = TL_FFN_BVEC1(min(fq + 1, a.nchunk - 1)); // (scalar loads, used after the stream)
+            const TlBounds<NB> boundsF2 = TL_FFN_BOUNDS1(min(fq + 1, a.nchunk - 1)); // (scalar loads, used after the stream)
             if (fq >= 2) // F(fq) overwrites the buffer that S(fq-2) read
                 tl_wait_count(ctr + TL_FFN_MAX_PHASES + fq - 2, NW, a.spin, a.status, lane);
-            TL_FFN_FIRST(fq, bvecFn, b1n, wB, oB)
-            bvecFn = bvecF2;
+            TL_FFN_FIRST(fq, boundsFn, b1n, wB, oB)
+            boundsFn = boundsF2;
             if (fq + 1 < a.nchunk) { // F(fq+1), a stream (or two) ahead
-                TL_FFN_PRELOAD(data1, poff1, bvecFn, wB, oB)
+                TL_FFN_PRELOAD(data1, poff1, boundsFn, wB, oB)
                 TL_FFN_BIAS1(b1n, fq + 1)
             }
         }
@@ -1423,15 +1369,14 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
         {
             const char *const xlane2 =
                 reinterpret_cast<const char *>(hs + (p & 1) * hbuf + c16 * ldh + x.khalf8);
-            const int q0_ = __builtin_amdgcn_readfirstlane(bvecS), qe_ = __builtin_amdgcn_readlane(bvecS, NB);
-            tl_stream<NB>(xlane2, xrow2, data2, poff2, lane_w, hi, q0_, qe_, max(qe_ - 1, q0_), bvecS, wA, oA,
-                          [&](int j, f32x4 c0, f32x4 c1) { TL_FFN_FLUSH(acc, j, c0, c1); });
+            tl_stream<NB, 2>(xlane2, xrow2, data2, poff2, lane_w, hi, boundsS, wA, oA,
+                             [&](int j, const f32x4 (&c)[2]) { TL_FFN_FLUSH(acc, j, c[0], c[1]); });
             tl_signal(ctr + TL_FFN_MAX_PHASES + p, lane);
         }
-        bvecS = bvecSn;
+        boundsS = boundsSn;
     }
-#undef TL_FFN_BVEC1
-#undef TL_FFN_BVEC2
+#undef TL_FFN_BOUNDS1
+#undef TL_FFN_BOUNDS2
 #undef TL_FFN_BIAS1
 #undef TL_FFN_FIRST
 #undef TL_FFN_PRELOAD
