@@ -185,7 +185,7 @@ template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false
           bool MASK = !PLAIN>
 static void attn_launch_one(const AttnArgs &a, hipStream_t st) {
     constexpr size_t lds = attn_lds_bytes<HD, QS, NW, PRUNED, HDK, VWIN>();
-    auto kern = attention_kernel<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, MASK>;
+    constexpr auto kern = &attention_kernel<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, MASK>;
     if (lds > 64 * 1024) { // above the default dynamic-LDS limit: opt in once per kernel
         static bool done = false;
         if (!done) {
@@ -194,7 +194,7 @@ static void attn_launch_one(const AttnArgs &a, hipStream_t st) {
             done = true;
         }
     }
-    hipLaunchKernelGGL(kern, dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, a);
+    launch_kernel<kern>(dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, a);
 }
 
 // Blocks of 128 query rows for packed sequences without a mask: K and V are read from LDS once per 32 queries of a wave
@@ -213,7 +213,7 @@ static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
     // a batch of 64 sequences of 32..512 rows; without it 154 and three)
     static_assert(QS == 1 || !MASK, "two subtiles a wave: without a mask");
     constexpr size_t lds = attn_lds_bytes<HD, QS, 4, false>();
-    auto kern = attention_packed_kernel<HD, QS, 4, MASK>;
+    constexpr auto kern = &attention_packed_kernel<HD, QS, 4, MASK>;
     if (lds > 64 * 1024) {
         static bool done = false;
         if (!done) {
@@ -224,7 +224,7 @@ static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
     }
     const long resident = (long)std::max(et_device_cu_count(), 1) * (QS == 2 ? 3 : HD <= 64 ? 4 : 2);
     const long wgs = std::min<long>(resident, a.total);
-    hipLaunchKernelGGL(kern, dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256), lds, st, a);
+    launch_kernel<kern>(dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256), lds, st, a);
 }
 
 // variant 0: 4 waves x 32 query rows; 1: 8 waves x 16 rows; 2: 4 waves x 16 rows
@@ -564,7 +564,7 @@ extern "C" int et_OTF_attention_noalloc(void *out, const void *Q, const void *K,
         return rc;
     // every word that the attention kernel reads for this seq_len is written
     // here first, so what an earlier call left in the array does not matter
-    hipLaunchKernelGGL(mask_summary_kernel, dim3((seq_len + 15) / 16), dim3(256), mask_summary_words(seq_len) * sizeof(unsigned), st, a.mask, seq_len,
+    launch_kernel<&mask_summary_kernel>(dim3((seq_len + 15) / 16), dim3(256), mask_summary_words(seq_len) * sizeof(unsigned), st, a.mask, seq_len,
                        summary, mask_summary_words(seq_len));
     const int rs = launch_status("et_OTF_attention_noalloc summary launch");
     if (rs != ET_OK)
@@ -723,7 +723,7 @@ extern "C" int et_attention_mask_summary(const void *mask, int seq_len, void *su
     using namespace et;
     ET_REQUIRE(mask && summary, ET_ERR_INVALID_ARG, "et_attention_mask_summary: null pointer");
     ET_REQUIRE(seq_len > 0, ET_ERR_INVALID_ARG, "et_attention_mask_summary: seq_len=%d", seq_len);
-    hipLaunchKernelGGL(mask_summary_kernel, dim3((seq_len + 15) / 16), dim3(256), mask_summary_words(seq_len) * sizeof(unsigned),
+    launch_kernel<&mask_summary_kernel>(dim3((seq_len + 15) / 16), dim3(256), mask_summary_words(seq_len) * sizeof(unsigned),
                        static_cast<hipStream_t>(stream), static_cast<const f16 *>(mask), seq_len,
                        static_cast<unsigned *>(summary), mask_summary_words(seq_len));
     return launch_status("et_attention_mask_summary launch");

@@ -704,7 +704,7 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
         constexpr auto kern = &layer_flow_kernel<decltype(hd_c)::value, decltype(mask_c)::value, decltype(fused_c)::value>;
         if (lds > 64 * 1024) // (the default limit)
             ET_HIP(allow_lds<kern>(lds));
-        hipLaunchKernelGGL(kern, dim3(total), dim3(LF_WAVES * 64), lds, st, a);
+        launch_kernel<kern>(dim3(total), dim3(LF_WAVES * 64), lds, st, a);
         return launch_status("layer in one launch");
     };
     typedef std::integral_constant<int, 64> wide_t;

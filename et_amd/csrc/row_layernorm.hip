@@ -233,7 +233,7 @@ extern "C" int et_tile_plan_run_scatter_ln(const et_tile_plan *plan, void *out, 
         constexpr auto kern = &row_layernorm_kernel<decltype(nb_c)::value, decltype(ms_c)::value, decltype(np_c)::value>;
         if (lds > 64 * 1024) // (the default limit)
             ET_HIP(allow_lds<kern>(lds));
-        hipLaunchKernelGGL(kern, dim3((M + 16 * ms - 1) / (16 * ms)), dim3(RL_WAVES * 64), lds, st, a.X, a.W, a.skip, a.M, a.K,
+        launch_kernel<kern>(dim3((M + 16 * ms - 1) / (16 * ms)), dim3(RL_WAVES * 64), lds, st, a.X, a.W, a.skip, a.M, a.K,
                            a.nbr, a.ppb, a.size, a.ldx, a.bias, a);
         return launch_status("row linear + LayerNorm launch");
     };

@@ -282,7 +282,7 @@ extern "C" int et_skip_layernorm(void *in_out, const void *skip, const void *gam
     const bool vec = (size % 8 == 0) && size <= 4096 && aligned16(in_out) &&
                      aligned16(skip) && aligned16(gamma) && aligned16(beta);
     if (!vec) {
-        hipLaunchKernelGGL(skip_layernorm_generic_kernel, dim3((num + 3) / 4), block, 0, st, a, s, g, b, num, size);
+        launch_kernel<&skip_layernorm_generic_kernel>(dim3((num + 3) / 4), block, 0, st, a, s, g, b, num, size);
     } else {
         const int nch8 = (size / 8 + 63) / 64;
         const float inv_n = 1.0f / (float)size;
@@ -298,15 +298,15 @@ extern "C" int et_skip_layernorm(void *in_out, const void *skip, const void *gam
 #define ET_LN_CASE(NCH_)                                                                          \
     {                                                                                             \
     if (nts)                                                                                      \
-        hipLaunchKernelGGL((skip_layernorm_vec_kernel<NCH_, 2, true, true>), grid, block, 0, st, a, s, g, b, num, size, inv_n); \
+        launch_kernel<&skip_layernorm_vec_kernel<NCH_, 2, true, true>>(grid, block, 0, st, a, s, g, b, num, size, inv_n); \
     else if (nt)                                                                                  \
-        hipLaunchKernelGGL((skip_layernorm_vec_kernel<NCH_, 2, true>), grid, block, 0, st, a, s, g, b, num, size, inv_n); \
+        launch_kernel<&skip_layernorm_vec_kernel<NCH_, 2, true>>(grid, block, 0, st, a, s, g, b, num, size, inv_n); \
     else if (rows >= 4)                                                                           \
-        hipLaunchKernelGGL((skip_layernorm_vec_kernel<NCH_, 4, false>), grid, block, 0, st, a, s, g, b, num, size, inv_n); \
+        launch_kernel<&skip_layernorm_vec_kernel<NCH_, 4, false>>(grid, block, 0, st, a, s, g, b, num, size, inv_n); \
     else if (rows >= 2)                                                                           \
-        hipLaunchKernelGGL((skip_layernorm_vec_kernel<NCH_, 2, false>), grid, block, 0, st, a, s, g, b, num, size, inv_n); \
+        launch_kernel<&skip_layernorm_vec_kernel<NCH_, 2, false>>(grid, block, 0, st, a, s, g, b, num, size, inv_n); \
     else                                                                                          \
-        hipLaunchKernelGGL((skip_layernorm_vec_kernel<NCH_, 1, false>), grid, block, 0, st, a, s, g, b, num, size, inv_n); \
+        launch_kernel<&skip_layernorm_vec_kernel<NCH_, 1, false>>(grid, block, 0, st, a, s, g, b, num, size, inv_n); \
     }
         {
             switch (nch8) { // size <= 4096: at most 8 chunks
@@ -349,7 +349,7 @@ extern "C" int et_scatter_skip_layernorm(void *out, const void *compact, const i
     const size_t lds = (size_t)4 * (size + 8) * sizeof(f16);
     const float inv_n = 1.0f / (float)size;
 #define ET_SLN_CASE(NCH_)                                                                         \
-    hipLaunchKernelGGL((scatter_skip_layernorm_kernel<NCH_>), grid, block, lds, st,               \
+    launch_kernel<&scatter_skip_layernorm_kernel<NCH_>>(grid, block, lds, st,               \
                        static_cast<f16 *>(out), static_cast<const f16 *>(compact), col_id, n, ld_in, \
                        static_cast<const f16 *>(skip), static_cast<const f16 *>(gamma),           \
                        static_cast<const f16 *>(beta), num, size, inv_n);                         \

@@ -1523,14 +1523,14 @@ static int launch_inst(const TlArgs &a, size_t lds, hipStream_t st) {
         if (a.nchunk == 1) {
             constexpr auto k = &tile_linear_resident_kernel<PNB, GELU, TL_WAVES, false>;
             ET_HIP(allow_lds<k>(lds));
-            hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, N[0]), a);
+            launch_kernel<k>(grid, block, lds, st, TL_HOT(a, N[0]), a);
         } else {
             constexpr auto k = &tile_linear_plan_kernel<PNB, GELU, TL_WAVES, false>;
             ET_HIP(allow_lds<k>(lds));
-            hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, KC), a);
+            launch_kernel<k>(grid, block, lds, st, TL_HOT(a, KC), a);
         }
     } else {
-        hipLaunchKernelGGL((tile_linear_generic_kernel<NB, GELU, MODE>), grid, block, lds, st, a);
+        launch_kernel<&tile_linear_generic_kernel<NB, GELU, MODE>>(grid, block, lds, st, a);
     }
     return launch_status("tile_linear launch");
 }
@@ -1555,11 +1555,11 @@ static int launch_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     if (a.nchunk == 1) {
         constexpr auto k = &tile_linear_resident_kernel<NB, false, TL_LN_WAVES, true>;
         ET_HIP(allow_lds<k>(lds));
-        hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, N[0]), a);
+        launch_kernel<k>(grid, block, lds, st, TL_HOT(a, N[0]), a);
     } else {
         constexpr auto k = &tile_linear_plan_kernel<NB, false, TL_LN_WAVES, true>;
         ET_HIP(allow_lds<k>(lds));
-        hipLaunchKernelGGL(k, grid, block, lds, st, TL_HOT(a, KC), a);
+        launch_kernel<k>(grid, block, lds, st, TL_HOT(a, KC), a);
     }
     return launch_status("tile_linear+LayerNorm launch");
 }
@@ -1575,7 +1575,7 @@ template <int NB>
 static int launch_chunked_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_chunked_kernel<NB, false, true>;
     ET_HIP(allow_lds<k>(lds));
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
+    launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
     return launch_status("tile_linear+LayerNorm (chunked) launch");
 }
 
@@ -1583,7 +1583,7 @@ template <int NB, bool GELU>
 static int launch_chunked_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_chunked_kernel<NB, GELU, false>;
     ET_HIP(allow_lds<k>(lds));
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
+    launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
     return launch_status("tile_linear (chunked) launch");
 }
 
@@ -1649,11 +1649,11 @@ static int tile_launch_ffn(const TlProblem *pO, const TlProblem &p1, const TlPro
     if (pO) {
         constexpr auto k = &tile_ffn_fused_kernel<3, true>;
         ET_HIP(allow_lds<k>(lds));
-        hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_FFN_WAVES * 64), lds, st, a);
+        launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_FFN_WAVES * 64), lds, st, a);
     } else {
         constexpr auto k = &tile_ffn_fused_kernel<3, false>;
         ET_HIP(allow_lds<k>(lds));
-        hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TL_FFN_WAVES * 64), lds, st, a);
+        launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_FFN_WAVES * 64), lds, st, a);
     }
     return launch_status("fused feed-forward launch");
 }
@@ -1949,7 +1949,7 @@ template <int NB, bool GELU, int NW = TL_WAVES>
 static int launch_resident64(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_resident_kernel<NB, GELU, NW, false, TL_BM64>;
     ET_HIP(allow_lds<k>(lds));
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, TL_HOT(a, N[0]), a);
+    launch_kernel<k>(dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, TL_HOT(a, N[0]), a);
     return launch_status("tile_linear (64-row panels) launch");
 }
 
