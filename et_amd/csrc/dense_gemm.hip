@@ -9,11 +9,11 @@
 // address is free per lane: the 16-byte pieces of a row are stored XOR-swizzled by (row / 2) % 8, which puts the sixteen
 // rows of a fragment read into sixteen different slots of 256 bytes without padding.
 //
-// What bounds it (measured with the DMA, the fragment reads and the MFMAs timed alone, 256 x 256 blocks, per step):
-// DMA 1.0 us, reads 0.5, MFMAs 1.0, all together 1.5 - the requests are issued in one go behind the barrier, and what
-// they miss in the XCD's L2 arrives late.  A second workgroup per CU fills these waits better than a third stage or
-// larger blocks, except where there is no work for a second one.  At K = 768 the twelve steps are a third of the time
-// of a launch; the rest is its start, the first step's latency and the result's way out.
+// What bounds it: in the middle of a large K the matrix unit at the clock it gets (256 x 192 blocks on every CU 1.25 us a
+// step, 1.29 PFLOP/s; 0.85 us while half of the CUs have none), at K = 768 the ends: the launch, the first step's
+// latency and the result's way out are 6 of 21 us.  A request occupies its wave while it goes out, and eight in one go
+// behind the barrier kept both waves of a SIMD from the matrix unit: they go out between the products (8192 rows 928 ->
+// 240 8.5 -> 7.1 us, 768 -> 768 14.1 -> 13.0, 2000 rows 768 -> 2304 12.5 -> 11.9, 16384 rows 4096 -> 1024 114 -> 109).
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -37,6 +37,13 @@ struct DgArgs {
     unsigned div_magic;
 };
 
+template <int B, int E, class F> __device__ __forceinline__ void dg_for(F &&f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>());
+        dg_for<B + 1, E>(f);
+    }
+}
+
 // where a row keeps its 16-byte piece kc of a step
 __device__ __forceinline__ int dg_swizzle(int r, int kc) { return kc ^ ((r >> 1) & 7); }
 
@@ -44,9 +51,8 @@ __device__ __forceinline__ int dg_swizzle(int r, int kc) { return kc ^ ((r >> 1)
 // step's second half of fragments is read while the first half multiplies, then the stage is handed back, the step ST
 // later requested into it and the next step's first fragments read while the second half multiplies: fragment reads and
 // the barrier run under MFMAs.
-// Against the kernel this replaced (128 x 128 by four waves, one stage ahead, reads between the MFMAs), us a launch:
-// 8192 rows 768 -> 768 18.5 -> 16.8, 768 -> 3072 53.0 -> 47.6, 3072 -> 768 49.7 -> 43.3, 928 -> 240 15.2 -> 10.2;
-// 16384 rows 1024 -> 4096 176 -> 132 (1040 TFLOP/s); 4096 x 4096 x 4096 151 -> 114 (1200 TFLOP/s).
+// us a launch: 8192 rows 768 -> 768 13.0, 768 -> 1536 21.2, 768 -> 3072 44.7, 3072 -> 768 40.2, 928 -> 240 7.1; 16384 rows
+// 1024 -> 4096 136 (1010 TFLOP/s), 4096 -> 1024 109 (1260 TFLOP/s).
 template <bool GELU, int WM, int WN, int TM, int TN, int ST>
 __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     // (what the first requests need arrives in registers with the wave)
@@ -112,25 +118,19 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     const char *const xbase = reinterpret_cast<const char *>(a.X + (size_t)m0 * a.K);
     const char *const wbase = reinterpret_cast<const char *>(W + (size_t)n0 * a.K);
     const int tail_cols = a.K - (nk - 1) * DG_BK; // 64, or 32: pieces beyond it re-read the step's first ones
-    auto fetch = [&](int kt, int slot) {
-        f16 *xn = smem + slot * STAGE;
-        const char *xs = xbase + (size_t)kt * (DG_BK * 2), *ws = wbase + (size_t)kt * (DG_BK * 2);
+    constexpr int PER = NXI + NWI; // requests of a stage per wave
+    auto request = [&](int kt, int slot, auto which) { // one of them
+        constexpr int Q = decltype(which)::value, I = Q < NXI ? Q : Q - NXI, PIECE = Q < NXI ? NXI : NWI;
+        f16 *dst = smem + slot * STAGE + (Q < NXI ? 0 : XT) + (wave * PIECE + I) * 512;
+        const char *src = (Q < NXI ? xbase : wbase) + (size_t)kt * (DG_BK * 2);
+        // (beyond a short last step: the swizzle flips bit 2 of a piece's number with the parity of its eight rows)
         const bool tail = kt == nk - 1 && tail_cols < DG_BK;
-        // (the swizzle flips bit 2 of a piece's number with the parity of its eight rows)
-        const unsigned even = tail && (lane & 4) ? 64u : 0u, odd = tail && !(lane & 4) ? 64u : 0u;
-#pragma unroll
-        for (int i = 0; i < NXI; i++) {
-            unsigned o = xoff[i];
-            asm volatile("" : "+v"(o)); // (a 32-bit offset off a uniform base, not a 64-bit pointer kept per piece)
-            load_lds16(xs + (o - (((wave * NXI + i) & 1) ? odd : even)), xn + (wave * NXI + i) * 512);
-        }
-#pragma unroll
-        for (int i = 0; i < NWI; i++) {
-            unsigned o = woff[i];
-            asm volatile("" : "+v"(o));
-            load_lds16(ws + (o - (((wave * NWI + i) & 1) ? odd : even)), xn + XT + (wave * NWI + i) * 512);
-        }
+        const unsigned back = tail && ((lane >> 2 ^ (wave * PIECE + I)) & 1) ? 64u : 0u;
+        unsigned o = Q < NXI ? xoff[Q < NXI ? I : 0] : woff[Q < NXI ? 0 : I];
+        asm volatile("" : "+v"(o)); // (a 32-bit offset off a uniform base, not a 64-bit pointer kept per piece)
+        load_lds16(src + (o - back), dst);
     };
+    auto fetch = [&](int kt, int slot) { dg_for<0, PER>([&](auto which) { request(kt, slot, which); }); };
     f32x4 acc[TN][TM]; // [feature subtile][row subtile]
 #pragma unroll
     for (int i = 0; i < TN; i++)
@@ -152,20 +152,22 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
         for (int j = 0; j < TM; j++)
             xf[H][j] = *reinterpret_cast<const f16x8 *>(s + px[H] + j * 2048);
     };
-    auto multiply = [&](auto half) {
+    auto multiply = [&](auto half, auto &&between) { // between(j): what goes out behind the products of row subtile j
         constexpr int H = decltype(half)::value;
         __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int j = 0; j < TM; j++)
+        dg_for<0, TM>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
 #pragma unroll
             for (int i = 0; i < TN; i++)
                 acc[i][j] = mfma16x16x32(wf[H][i], xf[H][j], acc[i][j]);
+            between(jc);
+        });
         __builtin_amdgcn_s_setprio(0);
     };
+    auto nothing = [](auto) {};
     typedef std::integral_constant<int, 0> h0;
     typedef std::integral_constant<int, 1> h1;
     auto barrier = [] { asm volatile("s_barrier" ::: "memory"); };
-    constexpr int PER = NXI + NWI; // requests of a stage per wave
     auto landed = [&](int behind) { // all but the youngest `behind` stages have arrived (this wave's part of them)
         if (behind >= 1 && ST > 2)
             __builtin_amdgcn_s_waitcnt(0x0070 | (PER & 15) | (PER >> 4 << 14)); // vmcnt(PER) lgkmcnt(0)
@@ -183,26 +185,41 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
         fetch(ST - 1, ST - 1);
     read(0, h0());
     int slot = 0;
-    auto turn = [&](int kt) { // stage kt has been read: wait for the next one, request into this one's place
-        landed(min(ST - 2, nk - 2 - kt));
-        barrier();
-        if (kt + ST < nk)
-            fetch(kt + ST, slot);
-        slot = slot == ST - 1 ? 0 : slot + 1;
-    };
-    for (int kt = 0; kt < nk; kt++) {
+    auto step = [&](int kt, auto more) {
         __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the first half's fragments, read a multiplication ago
         read(slot, h1());
         __builtin_amdgcn_sched_barrier(0);
-        multiply(h0());
-        if (kt + 1 < nk) {
-            turn(kt);
-            read(slot, h0());
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (kt < nk - 1 || tail_cols == DG_BK)
-            multiply(h1());
-    }
+        multiply(h0(), nothing);
+        // stage kt has been read: wait for the next one, request into this one's place
+        landed(min(ST - 2, nk - 2 - kt));
+        barrier();
+        const int freed = slot;
+        slot = slot == ST - 1 ? 0 : slot + 1;
+        read(slot, h0());
+        __builtin_amdgcn_sched_barrier(0);
+        // (a request occupies the wave while it goes out: between the products, where the matrix unit is busy meanwhile)
+        if constexpr (decltype(more)::value)
+            multiply(h1(), [&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                dg_for<j * PER / TM, (j + 1) * PER / TM>([&](auto which) { request(kt + ST, freed, which); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        else
+            multiply(h1(), nothing);
+    };
+    int kt = 0;
+    for (; kt < nk - ST; kt++)
+        step(kt, std::true_type());
+    for (; kt < nk - 1; kt++)
+        step(kt, std::false_type());
+    // (the last step apart: with a branch around the next stage's reads the compiler cannot tell which are in flight behind
+    // it, and waits for them before it multiplies)
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    read(slot, h1());
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(h0(), nothing);
+    if (tail_cols == DG_BK)
+        multiply(h1(), nothing);
     __builtin_amdgcn_s_waitcnt(0x0070);
     barrier(); // the stages are free: they stage the output block
 
@@ -290,29 +307,39 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
 }
 
 // The blocks there are and the time of each form in microseconds, without the launch.  A step takes longer with every
-// further workgroup of a CU; the figures are fits to 13 shapes (128 to 32768 rows, 768 to 4096 columns) within 15 %.  On
-// the 400 launches that bench/linear_forms.py times they are 15 % off in the mean, mostly alike for all forms: the block
-// they choose is 0.3 % behind the fastest in the mean, 6 % at most (768 -> 3072, 8863 rows: 58.2 against 54.9 us).
-// Small blocks win while they let more CUs take part, large ones where every CU has several.
-enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_FORMS };
+// further workgroup of a CU and with the share of the CUs that have one; the figures are fits to some 300 launches a form
+// (128 to 32768 rows, 512 to 4096 columns) within 10 %.  The block they choose is 0.3 % behind the fastest in the mean,
+// 14 % at most (3072 -> 768, 6000 rows: 39.4 against 34.6 us).  Small blocks win while they let more CUs take part, large
+// ones where every CU has several; 256 x 192 where one block a CU is all there is (768 -> 1536, 8192 rows: 21.2 against
+// 22.4 us in 128 x 192, 23.3 in 256 x 256).
+enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_256x192, DG_FORMS };
 static int g_dense_form = -1; // et_tuning_set("dense_form"): one of the above, -1 chooses
 static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
-    static const int bm[DG_FORMS] = {64, 128, 128, 128, 256}, bn[DG_FORMS] = {128, 128, 128, 192, 256};
+    static const int bm[DG_FORMS] = {64, 128, 128, 128, 256, 256}, bn[DG_FORMS] = {128, 128, 128, 192, 256, 192};
+    struct Form {
+        double ends;       // the first step's latency and the way out
+        double one, fill1; // a step while no CU has two blocks, per share of CUs that have one
+        double two, fill2; // ... while none has three
+        double more;       // ... a block
+    };
+    static const Form forms[DG_FORMS] = {
+        {0.6, 0.23, 0.08, 0.32, 0.13, 0.33}, // two per CU (72 KB)
+        {0.1, 0.40, 0.23, 0.53, 0.23, 0.56}, // two per CU (64 KB)
+        {1.3, 0.32, 0.11, 0.77, 0.13, 0.60}, // one per CU (96 KB)
+        {0.6, 0.54, 0.25, 0.65, 0.38, 0.75}, // two per CU (80 KB)
+        {4.3, 0.96, 0.54, 2.01, 0.70, 1.80}, // one per CU (128 KB)
+        {3.2, 0.80, 0.38, 1.92, 0.39, 1.44}, // one per CU (112 KB)
+    };
     const long cus = std::max(et_device_cu_count(), 1);
     long tiles = 0;
     for (int i = 0; i < nlin; i++)
         tiles += (Ns[i] + bn[form] - 1) / bn[form];
     tiles *= (M + bm[form] - 1) / bm[form];
-    const double n = (double)((tiles + cus - 1) / cus); // blocks of the busiest CU
-    double step = 0.0;
-    switch (form) {
-    case DG_64x128: step = n <= 1 ? 0.43 : n <= 2 ? 0.78 : 0.48 * n; break;                // two per CU (72 KB)
-    case DG_128x128: step = n <= 1 ? 0.69 : n <= 2 ? 0.58 * n : 0.65 * n; break;            // two per CU (64 KB)
-    case DG_128x128_DEEP: step = n <= 1 ? 0.57 : 0.83 * n; break;                           // one per CU (96 KB)
-    case DG_128x192: step = n <= 2 ? 0.15 + 0.68 * n : 0.87 * n; break;                     // two per CU (80 KB)
-    case DG_256x256: step = 1.95 * n; break;                                                // one per CU (128 KB)
-    }
-    return 1.6 + step * ((K + DG_BK - 1) / DG_BK);
+    const Form &f = forms[form];
+    const long n = (tiles + cus - 1) / cus; // blocks of the busiest CU
+    const double fill = (double)tiles / (double)cus;
+    const double step = n <= 1 ? f.one + f.fill1 * fill : n <= 2 ? f.two + f.fill2 * fill : f.more * (double)n;
+    return f.ends + step * ((K + DG_BK - 1) / DG_BK);
 }
 static int dg_choose(const int *Ns, int nlin, int M, int K, double *us) {
     int best = 0;
@@ -367,6 +394,7 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
         DG_CASE(DG_128x128_DEEP, 2, 4, 4, 2, 3)
         DG_CASE(DG_128x192, 2, 4, 4, 3, 2)
         DG_CASE(DG_256x256, 2, 4, 8, 4, 2)
+        DG_CASE(DG_256x192, 2, 4, 8, 3, 2)
 #undef DG_CASE
     }
     return ET_ERR_UNSUPPORTED;

@@ -2270,10 +2270,10 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 
 // Plans of fully populated matrices: the dense product where it is estimated to be the shorter launch, from some hundred
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
-// tile: their time is that of the choice among their forms.  The 2.4 us stand for the launch,
-// which dense_gemm_estimate leaves out.  Over 80 full plans (bench/linear_forms.py, launches of a graph) the choice is then
-// 0.7 % behind the faster side in the mean and 15 % at most; 0.9 and 32 % with nothing on top, 0.4 and 15 % with 1.2 us,
-// 1.2 and 21 % with 3.6.
+// tile: their time is that of the choice among their forms, whose figures are fits to launches of a graph and a tenth above
+// launches among others.  2.4 of the 2.6 us stand for the launch, which dense_gemm_estimate leaves out.  Over 176 full plans
+// the choice is then 0.5 % behind the faster side in the mean and 14 % at most; 1.9 and 20 % without the tenth, with it 0.9
+// and 17 % with 1 us more, 2 and 24 % with 1 us less.
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
@@ -2290,7 +2290,7 @@ static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool
         return true;
     const int K = plans[0]->in_feat, launches = join_launches(KC, nchunk, n, launch);
     const double tiles = tiles_estimate(Ns, ntile, nchunk, launch, launches, n, M, K, gelu);
-    return 2.4 + dense_gemm_estimate(Ns, n, M, K) < tiles;
+    return 2.6 + dense_gemm_estimate(Ns, n, M, K) < 0.9 * tiles;
 }
 static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
                            hipStream_t st) {

@@ -1261,6 +1261,17 @@ def test_full_plan_as_dense_product(K, form, M, Ns, Kd, gelu):
         assert np.abs(g.astype(np.float32) - t.astype(np.float32)).max() <= 2.0 ** -6
 
 
+@pytest.mark.parametrize("M,Ns,Kd,gelu", [
+    (256, (192,), 128, False),           # one whole block, as many steps as stages
+    (257, (208,), 96, True),             # a row and a piece into the next blocks; half a step at the end (GELU: one linear)
+    (100, (400,), 64, False),            # less than a block of rows, a single step
+    (520, (192, 384, 16), 1056, False),  # three linears; 16.5 steps
+])
+def test_full_plan_as_dense_product_256x192(K, M, Ns, Kd, gelu):
+    """the same for blocks of 256 x 192"""
+    test_full_plan_as_dense_product(K, 5, M, Ns, Kd, gelu)
+
+
 @pytest.mark.parametrize("M,Ns,Kd", [
     (1, (16,), 16), (33, (272, 16, 400), 768), (129, (400, 144), 1024), (200, (48, 784, 48), 512),
     (50, (336,), 2048),     # K in several chunks: whole rows in LDS
