@@ -32,7 +32,7 @@
 namespace et {
 
 template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
-          bool MASK = !PLAIN>
+          bool MASK = !PLAIN, int KS = 1>
 __global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 : 2) attention_kernel(const AttnArgs a) {
     // Workgroup ids go round-robin over the 8 XCDs.  XCD x works on the
     // (batch, head) pairs x, x+8, x+16, ... in that order, all query blocks of a
@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 : 2) attent
     const int bh = (rest / a.nqb) * 8 + xcd;
     if (bh >= a.nhead * a.batch)
         return;
-    attention_block<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, false, MASK>(a, bh / a.nhead, bh % a.nhead, qb);
+    attention_block<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, false, MASK, KS>(a, bh / a.nhead, bh % a.nhead, qb);
 }
 
 // Packed sequences of different lengths (cu_seqlens): a grid of one workgroup per
@@ -57,9 +57,9 @@ __global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 : 2) attent
 // sequence, which every wave keeps in registers (lane l: sequences l, l+64, ...;
 // at most 64*AT_PX sequences).
 constexpr int AT_PX = 4;
-template <int HD, int QS, int NW, bool MASK>
-__global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 : 2) attention_packed_kernel(const AttnArgs a) {
-    constexpr int QB = NW * 16 * QS;
+template <int HD, int QS, int NW, bool MASK, int KS = 1>
+__global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 / KS : 2) attention_packed_kernel(const AttnArgs a) {
+    constexpr int QB = NW / KS * 16 * QS;
     const int lane = threadIdx.x & 63;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, W = gridDim.x >> 3;
     int px[AT_PX], nbv[AT_PX]; // blocks before sequence (l + 64 r) in this XCD's list; its query blocks
@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 : 2) attent
         const int h = ((xcd - b * a.nhead) & 7) + 8 * (rem / max(nb, 1));
         if (nb <= 0 || rem < 0 || b >= a.batch || h >= a.nhead)
             continue; // (cannot happen with consistent counts; never index past the operands)
-        attention_block<HD, QS, NW, false, false, false, HD, false, false, MASK>(a, b, h, rem % nb);
+        attention_block<HD, QS, NW, false, false, false, HD, false, false, MASK, KS>(a, b, h, rem % nb);
         __syncthreads(); // the block's output staging in LDS is read before the next block's tiles land there
     }
 }
@@ -182,10 +182,10 @@ qk_scores_kernel(f16 *__restrict__ QK, const f16 *__restrict__ Q, const f16 *__r
 }
 
 template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
-          bool MASK = !PLAIN>
+          bool MASK = !PLAIN, int KS = 1>
 static void attn_launch_one(const AttnArgs &a, hipStream_t st) {
-    constexpr size_t lds = attn_lds_bytes<HD, QS, NW, PRUNED, HDK, VWIN>();
-    constexpr auto kern = &attention_kernel<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, MASK>;
+    constexpr size_t lds = attn_lds_bytes<HD, QS, NW, PRUNED, HDK, VWIN, KS>();
+    constexpr auto kern = &attention_kernel<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, MASK, KS>;
     if (lds > 64 * 1024) { // above the default dynamic-LDS limit: opt in once per kernel
         static bool done = false;
         if (!done) {
@@ -206,14 +206,25 @@ static bool packed_by_128(const AttnArgs &a) {
     return (long)((a.seq_len + 127) / 128) * a.nhead * a.batch >= 2 * 3 * (long)std::max(et_device_cu_count(), 1);
 }
 
+// Two groups of waves over the key tiles of a block of 64 query rows, where the chip has no block for its CUs' other
+// waves: a wave alone on its SIMD waits out every tile's latencies.  64 wide heads, one group / two, us: 12 blocks of 64
+// rows x 16 tiles (1 x 1024) no mask 11.5 / 9.9, padding 14.0 / 10.9, dense 17.1 / 13.1; 2 x 512 7.5 / 7.0, padding 8.5 /
+// 7.6, dense 10.2 / 8.8; 1 x 200 dense 6.8 / 6.5, others alike.  With more blocks than CUs only where there are many tiles:
+// 2 x 1000 (384 blocks) 14.4 / 13.7, padding 15.8 / 15.2, dense 19.6 / 18.0; 3 x 600 (360) 10.6 / 10.7, 11.7 / 11.7, 13.9 /
+// 13.3; 4 x 384 (288) 7.7 / 8.2, 8.9 / 9.1; 4 x 1000 (768) 19.4 / 21.0.  Four groups are not faster anywhere.
+static bool two_key_groups(const AttnArgs &a) {
+    const long cus = std::max(et_device_cu_count(), 1), tiles = (a.seq_len + AT_KT - 1) / AT_KT;
+    return (a.total <= cus && tiles >= 4) || (2 * a.total <= 3 * cus && tiles >= 12);
+}
+
 // packed sequences: as many workgroups (4 waves x 16 QS query rows) as the chip holds at once, or fewer
-template <int HD, bool MASK, int QS = 1>
+template <int HD, bool MASK, int QS = 1, int KS = 1>
 static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
     // (32 query rows per wave with the mask's bookkeeping needed 207 registers, two waves per SIMD: 63 us against 48 us on
     // a batch of 64 sequences of 32..512 rows; without it 154 and three)
     static_assert(QS == 1 || !MASK, "two subtiles a wave: without a mask");
-    constexpr size_t lds = attn_lds_bytes<HD, QS, 4, false>();
-    constexpr auto kern = &attention_packed_kernel<HD, QS, 4, MASK>;
+    constexpr size_t lds = attn_lds_bytes<HD, QS, 4 * KS, false, HD, false, KS>();
+    constexpr auto kern = &attention_packed_kernel<HD, QS, 4 * KS, MASK, KS>;
     if (lds > 64 * 1024) {
         static bool done = false;
         if (!done) {
@@ -222,14 +233,26 @@ static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
             done = true;
         }
     }
-    const long resident = (long)std::max(et_device_cu_count(), 1) * (QS == 2 ? 3 : HD <= 64 ? 4 : 2);
+    const long resident = (long)std::max(et_device_cu_count(), 1) * (QS == 2 ? 3 : HD <= 64 ? 4 / KS : 2);
     const long wgs = std::min<long>(resident, a.total);
-    launch_kernel<kern>(dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256), lds, st, a);
+    launch_kernel<kern>(dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256 * KS), lds, st, a);
 }
 
-// variant 0: 4 waves x 32 query rows; 1: 8 waves x 16 rows; 2: 4 waves x 16 rows
+// variant 0: 4 waves x 32 query rows; 1: 8 waves x 16 rows; 2: 4 waves x 16 rows; 3: 4 waves x 16 rows in each of two key
+// groups
 template <int HD, bool PRUNED, bool SHAREDQK, int HDK = HD>
 static void attn_launch_variant(int variant, bool plain, bool no_mask, const AttnArgs &a, hipStream_t st) {
+    if constexpr (HD == 64 && HDK == 64 && !PRUNED && !SHAREDQK) {
+        if (variant == 3) {
+            if (plain)
+                attn_launch_one<HD, 1, 8, false, false, true, HDK, false, false, 2>(a, st);
+            else if (no_mask)
+                attn_launch_one<HD, 1, 8, false, false, false, HDK, false, false, 2>(a, st);
+            else
+                attn_launch_one<HD, 1, 8, false, false, false, HDK, false, true, 2>(a, st);
+            return;
+        }
+    }
     if constexpr (!PRUNED && !SHAREDQK) {
         if (plain) {
             if (variant == 0)
@@ -408,14 +431,19 @@ static int attention_dispatch(AttnArgs a, int d_model, bool pruned, bool sharedq
         if (a.cu_seqlens)
             variant = 2; // packed sequences of different lengths: 64-row blocks waste fewer padded query rows
                          // (64 sequences of 32 to 512 rows: 50 us against 53-57 us with 128-row blocks)
+        if (g_attn_variant == 3)
+            variant = 2;
         if (g_attn_variant >= 0 && g_attn_variant <= 2 && !(hd == 128 && g_attn_variant == 0))
             variant = g_attn_variant;
     }
-    const int QB = variant == 2 ? 64 : 128;
+    const int QB = variant == 2 ? 64 : 128; // (3: chosen below, from 2)
     const bool plain = no_mask && !a.seq_lens && !a.cu_seqlens && a.seq_len % QB == 0;
     a.nqb = (a.seq_len + QB - 1) / QB;
     a.total = a.nqb * a.nhead * a.batch;
     a.per_xcd = (a.nhead * a.batch + 7) / 8 * a.nqb;
+    if (variant == 2 && hd == 64 && hd_data == 64 && !pruned && !sharedqk && !(qk_width && qk_width != hd_data) &&
+        (g_attn_variant < 0 ? two_key_groups(a) : g_attn_variant == 3))
+        variant = 3;
 #define ET_ATTN_CASE(HDV)                                                                         \
     if (hd == HDV) {                                                                              \
         if (sharedqk) attn_launch_variant<HDV, false, true>(variant, false, false, a, st);                     \
@@ -437,9 +465,11 @@ static int attention_dispatch(AttnArgs a, int d_model, bool pruned, bool sharedq
     }
     // packed sequences: the grid the chip holds, every workgroup walks its share of the query blocks that exist
     // (variant 2 counts the blocks of 64)
-    if (a.cu_seqlens && !pruned && !sharedqk && variant == 2 && a.batch <= 64 * AT_PX && g_attn_packed) {
+    if (a.cu_seqlens && !pruned && !sharedqk && variant >= 2 && a.batch <= 64 * AT_PX && g_attn_packed) {
         if (hd == 32)
             no_mask ? attn_launch_packed<32, false>(a, st) : attn_launch_packed<32, true>(a, st);
+        else if (variant == 3)
+            no_mask ? attn_launch_packed<64, false, 1, 2>(a, st) : attn_launch_packed<64, true, 1, 2>(a, st);
         else if (hd == 64)
             no_mask ? (packed_by_128(a) ? attn_launch_packed<64, false, 2>(a, st) : attn_launch_packed<64, false>(a, st)) : attn_launch_packed<64, true>(a, st);
         else

@@ -125,15 +125,18 @@ __device__ __forceinline__ void transpose_pieces_4x4(f16x4 (&p)[4]) {
 // are stored past the XCD's own L2 (store_agent8).
 // One workgroup's work: the NW*16*QS query rows of block qb of (sequence b, head h).
 // MASK: there may be a mask.  Without one (and not PLAIN: ragged lengths) nothing of its bookkeeping is compiled in.
+// KS: the waves form KS groups over the same query rows; group k takes key tiles k, k + KS, ... through tile buffers of its
+// own, and the groups' partial results meet in LDS behind the loop.
 template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
-          bool FLOW = false, bool MASK = !PLAIN>
+          bool FLOW = false, bool MASK = !PLAIN, int KS = 1>
 __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, const int h, const int qb) {
     static_assert(!PLAIN || ((!PRUNED || VWIN) && !SHAREDQK), "the plain form exists for the DMA-staged kernels only");
     static_assert(!PLAIN || !MASK, "the plain form has no mask");
     static_assert(HDK == HD || (!PRUNED && !SHAREDQK && HDK % 32 == 0), "narrow Q/K heads: on-the-fly kernel only");
     static_assert(!VWIN || (PRUNED && HD == 64), "the value-window form exists for the pruned kernel with 64-wide heads");
-    constexpr int AT_THREADS = NW * 64; // NW waves, each owning 16*QS query rows
-    constexpr int AT_WAVES = NW;
+    static_assert(KS == 1 || (!PRUNED && !SHAREDQK && QS == 1 && NW % KS == 0), "key groups: the DMA-staged form, a subtile a wave");
+    constexpr int AT_WAVES = NW / KS;         // of a group, each owning 16*QS query rows
+    constexpr int AT_THREADS = AT_WAVES * 64; // of a group
     constexpr int DK = HDK / 32;   // k-steps of Q K^T
     constexpr int DV = VWIN ? 5 : HD / 16; // 16-wide column subtiles of the output (of the 80-column window)
     // LDS row strides.  K rows are read with ds_read_b128 by 16 lanes at a
@@ -157,7 +160,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
     constexpr int SM = SM_KV > SM_O ? SM_KV : SM_O;
     extern __shared__ __attribute__((aligned(16))) unsigned char at_smem[];
     f16 *smem = reinterpret_cast<f16 *>(at_smem);
-    static_assert(SM * 2 <= 160 * 1024, "LDS budget");
+    static_assert(KS * SM * 2 <= 160 * 1024, "LDS budget");
 
     const int bh = b * a.nhead + h;
 
@@ -212,9 +215,11 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
         nv += vskip; // columns of the window up to the head's last one
     }
 
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
+    const int group = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / AT_WAVES;
+    const int tid = threadIdx.x - group * AT_THREADS;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - group * AT_WAVES;
+    const int lane = threadIdx.x & 63;
+    smem += group * SM;
     const int c16 = lane & 15;
     const int g4 = lane >> 4;
     f16 *obase = a.out + (size_t)row0 * a.ldo + h * hw;
@@ -255,10 +260,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
         // maximum is raised (after the first tiles: almost never): the start vector of the score
         // products, four copies of -m (zero while the row has no maximum yet), and the amount a
         // tile's maximum has to exceed before the row's is raised (-inf until then, 8 binades after).
-        // Only the forms without a mask keep them (there they save a dozen vector instructions per tile); with
-        // mask handling they would be ten registers too many for three waves per SIMD, and the masked
-        // forms work both out from m_run in every tile.
-        constexpr bool KEEP_START = !MASK && !SHAREDQK;
+        // They save a dozen vector instructions per tile.  With mask handling and two subtiles they would be ten registers
+        // too many for three waves per SIMD, and those forms work both out from m_run in every tile (a subtile, 1 x 1024
+        // rows: padding mask 14.7 -> 14.0 us, dense 17.4 -> 17.1; 2 x 1000 16.6 -> 15.8, 20.3 -> 19.6).
+        constexpr bool KEEP_START = (!MASK || (QS == 1 && DMA)) && !SHAREDQK;
         f32x4 neg_m4[QS];
         float raise_over[QS];
         f32x4 l_acc[QS]; // row sums of P, accumulated by the matrix unit (all 16 rows of the tile equal)
@@ -495,9 +500,9 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
         auto fast_tile = [&](int kb) { return kb + AT_KT <= len && (!SHAREDQK || (wave_rows_ok && qk_vec)); };
         bool has_mask_cur = false;
         auto mask_ahead = [&] { // the first tile's
-            has_mask_cur = MASK && !wave_idle && a.mask && tile_has_mask(0);
+            has_mask_cur = MASK && !wave_idle && a.mask && group < nt && tile_has_mask(group);
             if (has_mask_cur)
-                load_mask(0);
+                load_mask(group * AT_KT);
         };
 
         // One key tile.  FAST: all 64 keys and all of the wave's query rows are
@@ -618,9 +623,9 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
                             st[ksub][qs][r] = __builtin_fmaf((float)mk[qs][ksub][r], one, st[ksub][qs][r]);
             }
             if (MASK && a.mask) { // next tile's mask
-                has_mask_next = kb + AT_KT < len && tile_has_mask((kb + AT_KT) / AT_KT);
+                has_mask_next = kb + KS * AT_KT < len && tile_has_mask((kb + KS * AT_KT) / AT_KT);
                 if (has_mask_next)
-                    load_mask(kb + AT_KT);
+                    load_mask(kb + KS * AT_KT);
             }
             // the lane's part of each row maximum (of s - m_ref); the row's other three
             // parts only matter when some row of the wave has to raise its maximum
@@ -763,11 +768,12 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
         // Everything the first tiles need is requested before anything is waited for: K and V of the first tile, Q, the
         // first mask values, K and V of the second tile (whose wait is the first tile's end).
         if (DMA) {
-            dma_tile(0, 0);
+            if (KS == 1 || group < nt)
+                dma_tile(group * AT_KT, 0);
             load_q();
             mask_ahead();
-            if (nt > 1) {
-                dma_tile(AT_KT, 1);
+            if (nt > group + KS) {
+                dma_tile((group + KS) * AT_KT, 1);
                 constexpr int BEHIND = DMA_NTOT / AT_WAVES; // at least so many requests of this wave are the second tile's
                 __builtin_amdgcn_s_waitcnt(0x0F70 | (BEHIND & 15) | (BEHIND >> 4 << 14)); // vmcnt(BEHIND)
             } else {
@@ -786,20 +792,20 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
 
         // Without a mask: the full tiles in a loop of their own, the last one behind it (the bounds as a branch inside
         // the loop cost 0.15 us a tile: 2 x 1024 rows with lengths 15.9 us, without 13.4).
-        constexpr bool PEEL = DMA && !MASK && !SHAREDQK && !PLAIN;
-        const int nloop = PEEL ? len / AT_KT : nt;
+        constexpr bool PEEL = DMA && !MASK && !SHAREDQK && !PLAIN && KS == 1;
+        const int nloop = PEEL ? len / AT_KT : (nt + KS - 1) / KS;
         for (int t = 0; t < nloop; t++) {
-            const int kb = t * AT_KT;
+            const int kb = (t * KS + group) * AT_KT;
             const f16 *ks = smem + (t & 1) * (KBUF + VBUF);
             const f16 *vt = ks + KBUF;
-            const bool more = t + 1 < nt;
+            const bool more = (t + 1) * KS + group < nt;
             // tile t+1 goes into the other buffer (last read in iteration t-1,
             // which every wave left before the previous barrier) while tile t is
             // consumed: by DMA straight away, or through registers that are
             // stored after the tile body
             if (more) {
                 if (DMA && t > 0) // (the second tile is on its way)
-                    dma_tile(kb + AT_KT, (t + 1) & 1);
+                    dma_tile(kb + KS * AT_KT, (t + 1) & 1);
                 else if (DMA)
                     ;
                 else if (kb + 2 * AT_KT <= len)
@@ -807,7 +813,9 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
                 else
                     load_tile(kb + AT_KT, no_t{});
             }
-            if constexpr (PLAIN)
+            if (KS > 1 && kb >= len) // (the other groups' last step)
+                ;
+            else if constexpr (PLAIN)
                 tile_body(kb, ks, vt, true, false);
             else if (PEEL) {
                 if (!wave_idle)
@@ -831,16 +839,45 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
             __syncthreads();
         }
 
+        if constexpr (KS > 1) { // the groups' sums, each under its own maximum
+            constexpr int PART = AT_THREADS * (DV * 4 + 2); // floats of a group
+            static_assert(PART * 4 <= SM * 2, "a group's sums fit its tile buffers");
+            f32x4 *const part = reinterpret_cast<f32x4 *>(smem);
+            float *const stat = reinterpret_cast<float *>(part + DV * AT_THREADS);
+            if (group > 0) {
+#pragma unroll
+                for (int d = 0; d < DV; d++)
+                    part[d * AT_THREADS + tid] = ot[d][0];
+                stat[tid] = m_run[0];
+                stat[AT_THREADS + tid] = l_acc[0][0];
+            }
+            __syncthreads();
+            if (group == 0) {
+#pragma unroll
+                for (int g = 1; g < KS; g++) {
+                    const f32x4 *const other = part + g * (SM / 8);
+                    const float *const ostat = stat + g * (SM / 2);
+                    const float m_o = ostat[tid], m_new = fmaxf(m_run[0], m_o), m_fin = m_new == -INFINITY ? 0.f : m_new;
+                    const float mine = __builtin_amdgcn_exp2f((m_run[0] - m_fin) * ls), its = __builtin_amdgcn_exp2f((m_o - m_fin) * ls);
+                    m_run[0] = m_new;
+                    l_acc[0] = l_acc[0] * mine + ostat[AT_THREADS + tid] * its;
+#pragma unroll
+                    for (int d = 0; d < DV; d++)
+                        ot[d][0] = ot[d][0] * mine + other[d * AT_THREADS + tid] * its;
+                }
+            }
+        }
         // ---- normalise and stage the output block in LDS (all waves are past
         // the loop's final barrier, so the tile buffers are free)
-        f16 *os = smem;
+        f16 *os = smem - group * SM;
         if (PRUNED) { // columns that no kept V column maps to must read as zero
             for (int i = tid; i < SM_O / 8; i += AT_THREADS)
                 reinterpret_cast<f16x8 *>(os)[i] = zero8;
             __syncthreads();
         }
+        if (KS == 1 || group == 0)
 #pragma unroll
-        for (int qs = 0; qs < QS; qs++) {
+            for (int qs = 0; qs < QS; qs++) {
             const float l = l_acc[qs][0];
             const float inv = l > 0.f ? 1.0f / l : 0.f;
             const int ql = (wave * QS + qs) * 16 + c16;
@@ -873,7 +910,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
             }
         }
         __syncthreads();
-        for (int idx = tid; idx < QB * CPR; idx += AT_THREADS) {
+        for (int idx = threadIdx.x; idx < QB * CPR; idx += NW * 64) {
             const int ql = idx / CPR, dc = idx % CPR;
             const int q = q0 + ql;
             if (q < rows_alloc && dc * 8 < hw) {
@@ -886,7 +923,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
     } else {
         // whole query block is padding: rows exist (padded layout) and read as zero
         constexpr int CPR = HD / 8;
-        for (int idx = tid; idx < QB * CPR; idx += AT_THREADS) {
+        for (int idx = threadIdx.x; idx < QB * CPR; idx += NW * 64) {
             const int ql = idx / CPR, dc = idx % CPR;
             const int q = q0 + ql;
             if (q < rows_alloc && dc * 8 < hw)
@@ -896,11 +933,11 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
 }
 
 // LDS bytes of one workgroup (mirrors the constants inside attention_block)
-template <int HD, int QS, int NW, bool PRUNED, int HDK = HD, bool VWIN = false> constexpr size_t attn_lds_bytes() {
+template <int HD, int QS, int NW, bool PRUNED, int HDK = HD, bool VWIN = false, int KS = 1> constexpr size_t attn_lds_bytes() {
     // (must agree with the kernel's KBUF / VBUF)
     constexpr int KV = 2 * (AT_KT * (HDK + 16) + ((PRUNED && !VWIN) ? HD * (AT_KT + 8) : AT_KT * (HD + 16)));
-    constexpr int O = NW * 16 * QS * (HD + 8);
-    return sizeof(f16) * (size_t)(KV > O ? KV : O) + (VWIN ? 5 * 16 * sizeof(int) : 0); // (+ the window's column table)
+    constexpr int O = NW / KS * 16 * QS * (HD + 8);
+    return sizeof(f16) * (size_t)KS * (KV > O ? KV : O) + (VWIN ? 5 * 16 * sizeof(int) : 0); // (+ the window's column table)
 }
 
 // what a launcher fills in besides the operands (attention.hip): head scale,

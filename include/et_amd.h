@@ -545,7 +545,8 @@ int et_device_synchronize(void);
  *                     single-buffer kernel; 1 (default): the double-buffered one
  *   "ln_rows"         rows per wave of et_skip_layernorm (1, 2, 4)
  *   "attn_variant"    0: 4 waves x 32 query rows, 1: 8 waves x 16 rows,
- *                     2: 4 waves x 16 rows; -1 automatic
+ *                     2: 4 waves x 16 rows, 3: the same in two groups over the
+ *                     key tiles (64 columns a head); -1 automatic
  *   "attn_vwin"       0: et_Prune_attention always stages K and V through
  *                     registers; 1 (default): dense Q/K with a compact V whose
  *                     pitch is a multiple of 8 take the DMA-staged kernel

@@ -891,6 +891,53 @@ def test_otf_attention_varlen_blocks_of_128_rows(K, S, H, lens, walked_by):
         check_close(walked[rows], want, max_abs=5e-3, mean_rel=1e-3, what="varlen attention, 128-row blocks")
 
 
+@pytest.mark.parametrize("S,H,B,lens,use_mask,packed", [
+    (64, 2, 1, None, True, False),             # one tile: the second group has none
+    (65, 3, 2, None, False, False),            # a key into the second group's only tile
+    (192, 4, 1, None, False, False),           # an odd number of whole tiles
+    (200, 12, 2, [200, 129], True, False),     # ragged lengths
+    (300, 2, 4, [300, 64, 1, 0], False, False),
+    (1000, 1, 2, None, True, False),
+    (130, 4, 3, [130, 128, 63], True, True),   # packed rows
+    (513, 2, 5, [513, 512, 257, 64, 1], False, True),
+])
+def test_otf_attention_two_key_groups(K, S, H, B, lens, use_mask, packed):
+    """two groups of waves over the key tiles of a query block, against the oracle and one group (fp32 sums in another
+    order, probabilities rounded to half under another maximum: the oracle's tolerance)"""
+    from et_amd._lib import lib
+    r = rng(90 + S + B)
+    d = H * 64
+    lens_np = None if lens is None else np.array(lens, np.int32)
+    cu = np.concatenate([[0], np.cumsum(lens_np)]).astype(np.int32) if packed else None
+    rows = int(cu[-1]) if packed else B * S
+    Q, Kk, V = (randn_h(r, (rows, d)) for _ in range(3))
+    mask = randn_h(r, (S, S)) if use_mask else None
+    dm = None if mask is None else dev(mask)
+
+    def run():
+        if packed:
+            return host(K.OTF_attention_varlen(dev(Q), dev(Kk), dev(V), dm, dev(cu), S, H, LOG2E))
+        return host(K.OTF_attention(dev(Q), dev(Kk), dev(V), dm, S, H, B, None if lens is None else dev(lens_np), LOG2E))
+
+    try:
+        lib().et_tuning_set(b"attn_variant", 2)
+        one = run()
+        lib().et_tuning_set(b"attn_variant", 3)
+        two = run()
+    finally:
+        lib().et_tuning_set(b"attn_variant", -1)
+    check_close(two, one, max_abs=5e-3, mean_rel=1e-3, what="two key groups against one")
+    for b in range(B):
+        n = S if lens is None else int(lens[b])
+        at = slice(int(cu[b]), int(cu[b + 1])) if packed else slice(b * S, b * S + n)
+        if n:
+            want = orc.otf_attention(Q[at], Kk[at], V[at], None if mask is None else np.ascontiguousarray(mask[:n, :n]), n, H, 1, None,
+                                     LOG2E, f64=True)
+            check_close(two[at], want, max_abs=5e-3, mean_rel=1e-3, what=f"two key groups, sequence {b}")
+        if not packed:
+            assert (two[b * S + n:(b + 1) * S] == 0).all()
+
+
 @pytest.mark.parametrize("S,keep,value", [(512, 300, -30000.0), (512, 64, -65504.0), (256, 200, -1000.0), (192, 1, -30000.0)])
 def test_otf_attention_padding_mask_with_dead_tiles(K, S, keep, value):
     """a padding mask that blanks the keys from `keep` on: key tiles that lie wholly behind it add nothing (every
