@@ -165,6 +165,42 @@ inline hipError_t allow_lds(size_t lds) {
     return e;
 }
 
+// What a launcher worked out for sizes it has seen: a choice among a kernel's forms weighs up to a hundred of them, 1 us of
+// the host's time at every launch, and a program calls with few sizes.  By value of the sizes alone, a table of its own
+// for every thread and choice, 64 entries that displace each other.
+template <class Value, int N> struct KeptChoices {
+    struct Key {
+        int v[N];
+        bool operator==(const Key &o) const {
+            for (int i = 0; i < N; i++)
+                if (v[i] != o.v[i])
+                    return false;
+            return true;
+        }
+    };
+    struct Entry {
+        Key key;
+        Value value;
+        bool used;
+    };
+    Entry entries[64];
+    Entry &at(const Key &k) {
+        unsigned h = 0;
+        for (int i = 0; i < N; i++)
+            h = (h ^ (unsigned)k.v[i]) * 0x9E3779B1u;
+        return entries[h >> 26];
+    }
+    template <class Work> Value get(const Key &k, Work &&work) {
+        Entry &e = at(k);
+        if (!e.used || !(e.key == k)) {
+            e.value = work();
+            e.key = k;
+            e.used = true;
+        }
+        return e.value;
+    }
+};
+
 // A launch through the kernel's function handle, which is looked up once per kernel instance and device instead of by its
 // host address at every launch: 0.16 us less of host time a launch (13 parameters: 2.47 -> 2.31 us, 3.59 -> 3.48 while
 // the host is slow), where a call's smallest sizes are bound by the host.  Errors are left for launch_status, as with <<<>>>.

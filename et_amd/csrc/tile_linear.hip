@@ -1793,8 +1793,7 @@ struct TlChoice {
     size_t lds;
     double us;
 };
-static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, int nbr_max, bool gelu) {
-    const int cus = std::max(et_device_cu_count(), 1);
+static TlChoice weigh_resident(const TlProblem *probs, int nlin, int M, int K, int nbr_max, bool gelu, int cus) {
     double pairs = 0.0, w_mb = 0.0, result = 0.0; // tile pairs per block-row; W and the result of all linears
     for (int i = 0; i < nlin; i++) {
         const double p = 0.5 * probs[i].ntile / probs[i].nbr;
@@ -1882,8 +1881,7 @@ static double estimate_chunked(int M, double pairs, double x_mb, double w_mb, in
                              0.00429 * std::min(TL_CWAVES * nb, nbr_max) * pairs) +
            0.0980 * tl_traffic_mb(x_mb, w_mb, panels, ncg, 1.75);
 }
-static int choose_chunked(const TlProblem *probs, int nlin, int M, int K, int nchunk, int nbr_max, double *us) {
-    const long cus = std::max(et_device_cu_count(), 1);
+static int weigh_chunked(const TlProblem *probs, int nlin, int M, int K, int nchunk, int nbr_max, long cus, double *us) {
     double pairs = 0.0, w_mb = 0.0;
     for (int i = 0; i < nlin; i++) {
         const double p = 0.5 * probs[i].ntile / probs[i].nbr;
@@ -1918,6 +1916,41 @@ static int choose_chunked(const TlProblem *probs, int nlin, int M, int K, int nc
     if (rows_fit && g_tile_rows_most < 0)
         take(TL_BY_ROWS);
     return best;
+}
+
+// The two choices, kept for sizes that come again (100 rows 768 -> 768, bound by the host: 5.4 -> 4.9 us a call).
+static std::atomic<int> g_tunings{0}; // et_tuning_set was called so many times
+typedef KeptChoices<TlChoice, 6 + 3 * TL_MAX_LIN> ResidentChoices;
+struct ChunkedChoice {
+    int which;
+    double us;
+};
+typedef KeptChoices<ChunkedChoice, 6 + 3 * TL_MAX_LIN> ChunkedChoices;
+template <class Key> static Key choice_key(const TlProblem *probs, int nlin, int M, int K, int more, int cus) {
+    Key k = {{nlin, M, K, more, cus, g_tunings.load(std::memory_order_relaxed)}};
+    for (int i = 0; i < nlin; i++) {
+        k.v[6 + 3 * i] = probs[i].N;
+        k.v[7 + 3 * i] = probs[i].nbr;
+        k.v[8 + 3 * i] = probs[i].ntile;
+    }
+    return k;
+}
+static TlChoice choose_resident(const TlProblem *probs, int nlin, int M, int K, int nbr_max, bool gelu) {
+    static thread_local ResidentChoices kept;
+    const int cus = std::max(et_device_cu_count(), 1);
+    return kept.get(choice_key<ResidentChoices::Key>(probs, nlin, M, K, gelu, cus),
+                    [&] { return weigh_resident(probs, nlin, M, K, nbr_max, gelu, cus); });
+}
+static int choose_chunked(const TlProblem *probs, int nlin, int M, int K, int nchunk, int nbr_max, double *us) {
+    static thread_local ChunkedChoices kept;
+    const int cus = std::max(et_device_cu_count(), 1);
+    const ChunkedChoice c = kept.get(choice_key<ChunkedChoices::Key>(probs, nlin, M, K, nchunk, cus), [&] {
+        ChunkedChoice v;
+        v.which = weigh_chunked(probs, nlin, M, K, nchunk, nbr_max, cus, &v.us);
+        return v;
+    });
+    *us = c.us;
+    return c.which;
 }
 
 // the tile kernels' estimated time for planned linears over one input, launches of their own added up (join_launches)
@@ -2138,6 +2171,7 @@ static int raw_tile_linear(void *Y, const void *X, const int *row_ptr, const int
 static int g_tail_pair_min_wgs = 0; // et_tuning_set("tile_tail_pair_min_wgs"): 0 = three quarters of the CUs
 
 extern "C" int et_tuning_set(const char *key, int value) {
+    et::g_tunings.fetch_add(1, std::memory_order_relaxed); // (kept choices are weighed again)
     if (key && !strcmp(key, "tile_splitk_rows")) {
         et::g_tile_rows_most = value;
         return ET_OK;
