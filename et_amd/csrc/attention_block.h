@@ -260,10 +260,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs &a, const int b, 
         // maximum is raised (after the first tiles: almost never): the start vector of the score
         // products, four copies of -m (zero while the row has no maximum yet), and the amount a
         // tile's maximum has to exceed before the row's is raised (-inf until then, 8 binades after).
-        // They save a dozen vector instructions per tile.  With mask handling and two subtiles they would be ten registers
-        // too many for three waves per SIMD, and those forms work both out from m_run in every tile (a subtile, 1 x 1024
-        // rows: padding mask 14.7 -> 14.0 us, dense 17.4 -> 17.1; 2 x 1000 16.6 -> 15.8, 20.3 -> 19.6).
-        constexpr bool KEEP_START = (!MASK || (QS == 1 && DMA)) && !SHAREDQK;
+        // They save a dozen vector instructions per tile (padding mask: 1 x 1024 rows 14.7 -> 14.0 us, 2 x 1000 16.6 -> 15.8;
+        // two subtiles a wave, 157 registers: 8 x 700 24.7 -> 23.9, 6 x 1024 31.3 -> 30.3).  The register-staged forms with a
+        // mask, and heads of 128 with two subtiles, have none to spare and work both out from m_run in every tile.
+        constexpr bool KEEP_START = (!MASK || (DMA && (QS == 1 || HD <= 64))) && !SHAREDQK;
         f32x4 neg_m4[QS];
         float raise_over[QS];
         f32x4 l_acc[QS]; // row sums of P, accumulated by the matrix unit (all 16 rows of the tile equal)
