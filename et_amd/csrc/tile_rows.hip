@@ -178,6 +178,21 @@ __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(
                 acc1 = mfma16x16x32(p.w[I + 1], x1, acc1);
             }
         };
+        // Long lists of the caller's own: as long as a round's pairs are all in flight and as many to come, it asks nothing
+        // and its waits are counted - a request that may not have gone out makes the compiler wait for all of them, a round
+        // trip for every two pairs.  3072 -> 768: 1067 rows 80 % 8.4 -> 7.7 us, 50 % 13.1 -> 12.1, dense 26.8 -> 21.7; 4096
+        // rows 20.6 -> 18.6, 43.4 -> 34.8, 74.7 -> 58.9; 4096 -> 1024, 1067 rows, dense 64.5 -> 48.4.  (A plan's lists may
+        // step into the next column chunk at every pair, which is a branch again: no faster.)
+        if constexpr (RAW) {
+            while (n == LF_D && pairs_left() >= LF_D) {
+#define TR_ROUND(i_)                                                                              \
+    multiply(std::integral_constant<int, i_>());                                                  \
+    load(std::integral_constant<int, i_>());                                                      \
+    load(std::integral_constant<int, i_ + 1>());
+                TR_ROUND(0) TR_ROUND(2) TR_ROUND(4) TR_ROUND(6)
+#undef TR_ROUND
+            }
+        }
         while (n > 0) {
             int m = 0; // pairs in the slots of the next round
 #define TR_STEP(i_)                                                                               \

@@ -635,6 +635,23 @@ def test_row_linear(K, M, N, Kd):
     check_close(got, want, max_abs=max(np.abs(want.astype(np.float64)).max() * 2.0 ** -10, 1e-3), mean_rel=5e-4, what="row linear")
 
 
+@pytest.mark.parametrize("M,gelu", [(16, False), (700, True), (2065, False)])  # a block-row split over waves, and whole
+def test_raw_lists_of_any_length_on_whole_rows(K, M, gelu):
+    """the caller's own unsorted tile lists over 4096 columns, of lengths around one and several rounds of eight pairs,
+    odd ones among them, against the oracle"""
+    r = rng(31 + M)
+    Kd, counts = 4096, [0, 1, 15, 16, 17, 31, 32, 33, 34, 47, 48, 49, 63, 64, 65, 96, 97, 127, 128, 255, 256]
+    N = 16 * len(counts)
+    row_ptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    row_offset = np.concatenate([r.permutation(Kd // 16)[:c] * 16 for c in counts]).astype(np.int32)
+    data = (randn_h(r, (row_offset.size * 256,)).astype(np.float32) * 0.02).astype(np.float16)
+    bias, X = randn_h(r, (N,)), randn_h(r, (M, Kd))
+    got = host(K.tile_spmm_add_bias(dev(X), dev(row_ptr), dev(row_offset), dev(data), dev(bias), N, gelu=gelu))
+    rows = np.unique(np.concatenate([np.arange(min(M, 20)), np.arange(max(M - 20, 0), M)]))
+    want = orc.tile_linear(X[rows], row_ptr, row_offset, data, bias, N, gelu=gelu, f64=True)
+    check_close(got[rows], want, max_abs=8e-3, mean_rel=5e-4, what="raw lists on whole rows")
+
+
 # ------------------------------------------------------------------ attention
 ATT_CASES = [
     # S, H, d_model, batch, lens, mask, log2_scale
