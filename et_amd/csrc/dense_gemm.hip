@@ -307,9 +307,9 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
 }
 
 // The blocks there are and the time of each form in microseconds, without the launch.  A step takes longer with every
-// further workgroup of a CU and with the share of the CUs that have one; the figures are fits to some 300 launches a form
-// (128 to 32768 rows, 512 to 4096 columns) within 10 %.  The block they choose is 0.3 % behind the fastest in the mean,
-// 14 % at most (3072 -> 768, 6000 rows: 39.4 against 34.6 us).  Small blocks win while they let more CUs take part, large
+// further workgroup of a CU and with the share of the CUs that have one; the figures are fits to 385 shapes (128 to 32768
+// rows, 512 to 4096 columns), the forms near the fastest weighing most.  The block they choose is 0.2 % behind the fastest
+// in the mean, 14 % at most (3072 -> 768, 8192 rows: 40.6 against 35.7 us).  Small blocks win while they let more CUs take part, large
 // ones where every CU has several; 256 x 192 where one block a CU is all there is (768 -> 1536, 8192 rows: 21.2 against
 // 22.4 us in 128 x 192, 23.3 in 256 x 256).
 enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_256x192, DG_FORMS };
@@ -323,12 +323,12 @@ static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
         double more;       // ... a block
     };
     static const Form forms[DG_FORMS] = {
-        {0.6, 0.23, 0.08, 0.32, 0.13, 0.33}, // two per CU (72 KB)
-        {0.1, 0.40, 0.23, 0.53, 0.23, 0.56}, // two per CU (64 KB)
-        {1.3, 0.32, 0.11, 0.77, 0.13, 0.60}, // one per CU (96 KB)
-        {0.6, 0.54, 0.25, 0.65, 0.38, 0.75}, // two per CU (80 KB)
-        {4.3, 0.96, 0.54, 2.01, 0.70, 1.80}, // one per CU (128 KB)
-        {3.2, 0.80, 0.38, 1.92, 0.39, 1.44}, // one per CU (112 KB)
+        {0.7, 0.23, 0.08, 0.31, 0.16, 0.37}, // two per CU (72 KB)
+        {1.3, 0.24, 0.21, 0.38, 0.25, 0.57}, // two per CU (64 KB)
+        {1.6, 0.25, 0.14, 0.70, 0.19, 0.60}, // one per CU (96 KB)
+        {1.2, 0.41, 0.34, 0.63, 0.36, 0.74}, // two per CU (80 KB)
+        {6.1, 0.67, 0.87, 1.82, 0.73, 1.56}, // one per CU (128 KB)
+        {4.0, 0.68, 0.51, 1.50, 0.66, 1.33}, // one per CU (112 KB)
     };
     const long cus = std::max(et_device_cu_count(), 1);
     long tiles = 0;

@@ -2306,7 +2306,7 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
 // tile: their time is that of the choice among their forms, whose figures are fits to launches of a graph and a tenth above
 // launches among others.  2.4 of the 2.6 us stand for the launch, which dense_gemm_estimate leaves out.  Over 176 full plans
-// the choice is then 0.5 % behind the faster side in the mean and 14 % at most; 1.9 and 20 % without the tenth, with it 0.9
+// the choice is then 0.3 % behind the faster side in the mean and 14 % at most; 1 and 20 % without the tenth, with it 0.8
 // and 17 % with 1 us more, 2 and 24 % with 1 us less.
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
