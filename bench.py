@@ -39,7 +39,7 @@ TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "encoder_layer_b16_s512_hbm_tra
 KERNEL_SOURCES = tuple(sorted(f for f in os.listdir(os.path.join(ROOT, "et_amd", "csrc")) if f.endswith((".hip", ".h"))))
 TRAFFIC_KERNELS = {  # bench line -> kernel instance in the profile summary (the default workload's launches)
     "tile_linear qkv (3 x 768->768, one launch)": "et::tile_linear_resident_kernel<2, false, 12, false, 64>",
-    "attention (on-the-fly)": "et::attention_kernel<64, 2, 4, false, false, true, 64, false, false, 1>",
+    "attention (on-the-fly)": "et::attention_kernel<64, 2, 4, false, false, true, 64, false, false>",
     "layer tail: o + skip + LayerNorm + feed-forward (gelu) + skip + LayerNorm, fused": "et::tile_ffn_fused_kernel<3, true>",
 }
 

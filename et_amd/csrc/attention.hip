@@ -31,19 +31,30 @@
 
 namespace et {
 
-template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
-          bool MASK = !PLAIN, int KS = 1>
-__global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 : 2) attention_kernel(const AttnArgs a) {
-    // Workgroup ids go round-robin over the 8 XCDs.  XCD x works on the
-    // (batch, head) pairs x, x+8, x+16, ... in that order, all query blocks of a
-    // pair together (they share its K and V in that XCD's L2): with sequences of
-    // different lengths every XCD gets an even mix, and pairs keep their order.
+// A workgroup's query block qb of pair bh; false: none.  Workgroup ids go round-robin over the 8 XCDs.  XCD x works on
+// the (batch, head) pairs x, x+8, x+16, ... in that order, all query blocks of a pair together (they share its K and V in
+// that XCD's L2): with sequences of different lengths every XCD gets an even mix, and pairs keep their order.
+__device__ __forceinline__ bool attn_place(const AttnArgs &a, int &bh, int &qb) {
     const int xcd = blockIdx.x & 7, rest = blockIdx.x >> 3; // rest < per_xcd = ceil(pairs / 8) * nqb
-    const int qb = rest % a.nqb;
-    const int bh = (rest / a.nqb) * 8 + xcd;
-    if (bh >= a.nhead * a.batch)
-        return;
-    attention_block<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, false, MASK, KS>(a, bh / a.nhead, bh % a.nhead, qb);
+    qb = rest % a.nqb;
+    bh = (rest / a.nqb) * 8 + xcd;
+    return bh < a.nhead * a.batch;
+}
+
+template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
+          bool MASK = !PLAIN>
+__global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 : 2) attention_kernel(const AttnArgs a) {
+    int bh, qb;
+    if (attn_place(a, bh, qb))
+        attention_block<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, false, MASK>(a, bh / a.nhead, bh % a.nhead, qb);
+}
+
+// the same in two groups of four waves over the key tiles of a block of 64 query rows (two_key_groups)
+template <int HD, bool PLAIN, bool MASK>
+__global__ void __launch_bounds__(512, 4) attention_two_groups_kernel(const AttnArgs a) {
+    int bh, qb;
+    if (attn_place(a, bh, qb))
+        attention_block<HD, 1, 8, false, false, PLAIN, HD, false, false, MASK, 2>(a, bh / a.nhead, bh % a.nhead, qb);
 }
 
 // Packed sequences of different lengths (cu_seqlens): a grid of one workgroup per
@@ -181,20 +192,26 @@ qk_scores_kernel(f16 *__restrict__ QK, const f16 *__restrict__ Q, const f16 *__r
     }
 }
 
-template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
-          bool MASK = !PLAIN, int KS = 1>
-static void attn_launch_one(const AttnArgs &a, hipStream_t st) {
-    constexpr size_t lds = attn_lds_bytes<HD, QS, NW, PRUNED, HDK, VWIN, KS>();
-    constexpr auto kern = &attention_kernel<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, MASK, KS>;
+template <auto KERN> static void attn_launch_grid(size_t lds, int threads, const AttnArgs &a, hipStream_t st) {
     if (lds > 64 * 1024) { // above the default dynamic-LDS limit: opt in once per kernel
         static bool done = false;
         if (!done) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             done = true;
         }
     }
-    launch_kernel<kern>(dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, a);
+    launch_kernel<KERN>(dim3(a.per_xcd * 8), dim3(threads), lds, st, a);
+}
+template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
+          bool MASK = !PLAIN>
+static void attn_launch_one(const AttnArgs &a, hipStream_t st) {
+    constexpr auto kern = &attention_kernel<HD, QS, NW, PRUNED, SHAREDQK, PLAIN, HDK, VWIN, MASK>;
+    attn_launch_grid<kern>(attn_lds_bytes<HD, QS, NW, PRUNED, HDK, VWIN>(), NW * 64, a, st);
+}
+template <int HD, bool PLAIN, bool MASK> static void attn_launch_two_groups(const AttnArgs &a, hipStream_t st) {
+    constexpr auto kern = &attention_two_groups_kernel<HD, PLAIN, MASK>;
+    attn_launch_grid<kern>(attn_lds_bytes<HD, 1, 8, false, HD, false, 2>(), 512, a, st);
 }
 
 // Blocks of 128 query rows for packed sequences without a mask: K and V are read from LDS once per 32 queries of a wave
@@ -245,11 +262,11 @@ static void attn_launch_variant(int variant, bool plain, bool no_mask, const Att
     if constexpr (HD == 64 && HDK == 64 && !PRUNED && !SHAREDQK) {
         if (variant == 3) {
             if (plain)
-                attn_launch_one<HD, 1, 8, false, false, true, HDK, false, false, 2>(a, st);
+                attn_launch_two_groups<HD, true, false>(a, st);
             else if (no_mask)
-                attn_launch_one<HD, 1, 8, false, false, false, HDK, false, false, 2>(a, st);
+                attn_launch_two_groups<HD, false, false>(a, st);
             else
-                attn_launch_one<HD, 1, 8, false, false, false, HDK, false, true, 2>(a, st);
+                attn_launch_two_groups<HD, false, true>(a, st);
             return;
         }
     }
