@@ -193,14 +193,8 @@ qk_scores_kernel(f16 *__restrict__ QK, const f16 *__restrict__ Q, const f16 *__r
 }
 
 template <auto KERN> static void attn_launch_grid(size_t lds, int threads, const AttnArgs &a, hipStream_t st) {
-    if (lds > 64 * 1024) { // above the default dynamic-LDS limit: opt in once per kernel
-        static bool done = false;
-        if (!done) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            done = true;
-        }
-    }
+    if (lds > 64 * 1024 && allow_lds<KERN>(lds) != hipSuccess) // (above the default limit)
+        return; // (the error is left for launch_status)
     launch_kernel<KERN>(dim3(a.per_xcd * 8), dim3(threads), lds, st, a);
 }
 template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
@@ -242,14 +236,8 @@ static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
     static_assert(QS == 1 || !MASK, "two subtiles a wave: without a mask");
     constexpr size_t lds = attn_lds_bytes<HD, QS, 4 * KS, false, HD, false, KS>();
     constexpr auto kern = &attention_packed_kernel<HD, QS, 4 * KS, MASK, KS>;
-    if (lds > 64 * 1024) {
-        static bool done = false;
-        if (!done) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            done = true;
-        }
-    }
+    if (lds > 64 * 1024 && allow_lds<kern>(lds) != hipSuccess)
+        return;
     const long resident = (long)std::max(et_device_cu_count(), 1) * (QS == 2 ? 3 : HD <= 64 ? 4 / KS : 2);
     const long wgs = std::min<long>(resident, a.total);
     launch_kernel<kern>(dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256 * KS), lds, st, a);

@@ -1,0 +1,146 @@
+// A HIP runtime of two devices without any: host memory, launches that are checked and written down instead of run.  Loaded
+// ahead of libet_amd.so it answers the calls that the library makes, so that what the launchers do per device, per stream
+// and per thread can be tested where there is no GPU.  Kernels need the opt-in to more than 64 KB of LDS on each device,
+// and a launch takes a function of its stream's device, as the runtime documents.
+#include <cstdint>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <utility>
+#include <vector>
+
+namespace {
+constexpr int OK = 0, INVALID_VALUE = 1, INVALID_DEVICE = 101, INVALID_HANDLE = 400;
+struct Stream {
+    int device;
+};
+struct Function {
+    const void *symbol;
+    int device;
+};
+struct Launch {
+    int device;
+    unsigned grid, block, lds;
+    const void *symbol;
+    void *third; // the third parameter's eight bytes, where there is one
+};
+std::mutex lock;
+std::map<std::pair<const void *, int>, int> allowed; // (kernel, device) -> dynamic LDS
+std::map<std::pair<const void *, int>, Function *> functions;
+std::vector<Launch> launches;
+unsigned char symbols[2][1 << 16]; // a device variable's stand-in on either device
+thread_local int current = 0, last_error = OK;
+
+int fail(int e) {
+    if (e != OK)
+        last_error = e;
+    return e;
+}
+int device_of(void *stream) { return stream ? static_cast<Stream *>(stream)->device : current; }
+int launch(const void *symbol, int device, unsigned grid, unsigned block, unsigned lds, void **params, bool has_third) {
+    std::lock_guard<std::mutex> l(lock);
+    if (lds > 64 * 1024 && allowed[{symbol, device}] < (int)lds)
+        return fail(INVALID_VALUE);
+    void *third = nullptr;
+    if (has_third)
+        memcpy(&third, params[2], sizeof(third));
+    if (launches.size() < 4096)
+        launches.push_back({device, grid, block, lds, symbol, third});
+    return OK;
+}
+struct Dim {
+    unsigned x, y, z;
+};
+} // namespace
+
+extern "C" {
+// ---- what the tests ask
+void two_devices_stream(int device, void **stream) { *stream = new Stream{device}; }
+int two_devices_launches() {
+    std::lock_guard<std::mutex> l(lock);
+    return (int)launches.size();
+}
+void two_devices_clear() {
+    std::lock_guard<std::mutex> l(lock);
+    launches.clear();
+}
+void two_devices_launch(int i, int *device, unsigned *block, unsigned *lds) {
+    std::lock_guard<std::mutex> l(lock);
+    *device = launches[i].device;
+    *block = launches[i].block;
+    *lds = launches[i].lds;
+}
+// whose copy of a device variable the launch was handed as its third parameter; -1: none
+int two_devices_variable_of(int i) {
+    std::lock_guard<std::mutex> l(lock);
+    const unsigned char *p = static_cast<unsigned char *>(launches[i].third);
+    for (int d = 0; d < 2; d++)
+        if (p >= symbols[d] && p < symbols[d] + sizeof(symbols[d]))
+            return d;
+    return -1;
+}
+
+// ---- the runtime
+int hipGetDevice(int *d) { return *d = current, OK; }
+int hipSetDevice(int d) { return d < 0 || d > 1 ? fail(INVALID_DEVICE) : (current = d, OK); }
+int hipStreamGetDevice(void *s, int *d) { return *d = device_of(s), OK; }
+int hipGetLastError() {
+    const int e = last_error;
+    last_error = OK;
+    return e;
+}
+const char *hipGetErrorString(int) { return "refused by the two devices"; }
+int hipDeviceGetAttribute(int *v, int, int) { return *v = 256, OK; } // (compute units)
+int hipDeviceSynchronize() { return OK; }
+int hipStreamSynchronize(void *) { return OK; }
+int hipStreamCreate(void **s) { return two_devices_stream(current, s), OK; }
+int hipStreamDestroy(void *s) { return delete static_cast<Stream *>(s), OK; }
+int hipMalloc(void **p, size_t n) { return posix_memalign(p, 256, n ? n : 1) ? fail(2) : OK; }
+int hipFree(void *p) { return free(p), OK; }
+int hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+int hipHostFree(void *p) { return hipFree(p); }
+int hipHostGetDevicePointer(void **d, void *h, unsigned) { return *d = h, OK; }
+int hipMemcpy(void *d, const void *s, size_t n, int) { return memcpy(d, s, n), OK; }
+int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) { return memcpy(d, s, n), OK; }
+int hipGetSymbolAddress(void **p, const void *) { return *p = symbols[current], OK; }
+int hipFuncSetAttribute(const void *symbol, int, int value) {
+    std::lock_guard<std::mutex> l(lock);
+    allowed[{symbol, current}] = value;
+    return OK;
+}
+int hipGetFuncBySymbol(void **fn, const void *symbol) {
+    std::lock_guard<std::mutex> l(lock);
+    Function *&f = functions[{symbol, current}];
+    if (!f)
+        f = new Function{symbol, current};
+    *fn = f;
+    return OK;
+}
+int hipModuleLaunchKernel(void *fn, unsigned gx, unsigned, unsigned, unsigned bx, unsigned, unsigned, unsigned lds, void *stream,
+                          void **params, void **) {
+    const Function *f = static_cast<Function *>(fn);
+    if (f->device != device_of(stream))
+        return fail(INVALID_HANDLE);
+    return launch(f->symbol, f->device, gx, bx, lds, params, true);
+}
+int hipLaunchKernel(const void *symbol, Dim grid, Dim block, void **params, size_t lds, void *stream) {
+    return launch(symbol, device_of(stream), grid.x, block.x, (unsigned)lds, params, false);
+}
+static thread_local struct {
+    Dim grid, block;
+    size_t lds;
+    void *stream;
+} call;
+int __hipPushCallConfiguration(Dim grid, Dim block, size_t lds, void *stream) {
+    call = {grid, block, lds, stream};
+    return OK;
+}
+int __hipPopCallConfiguration(Dim *grid, Dim *block, size_t *lds, void **stream) {
+    *grid = call.grid;
+    *block = call.block;
+    *lds = call.lds;
+    *stream = call.stream;
+    return OK;
+}
+}
