@@ -193,8 +193,6 @@ qk_scores_kernel(f16 *__restrict__ QK, const f16 *__restrict__ Q, const f16 *__r
 }
 
 template <auto KERN> static void attn_launch_grid(size_t lds, int threads, const AttnArgs &a, hipStream_t st) {
-    if (lds > 64 * 1024 && allow_lds<KERN>(lds) != hipSuccess) // (above the default limit)
-        return; // (the error is left for launch_status)
     launch_kernel<KERN>(dim3(a.per_xcd * 8), dim3(threads), lds, st, a);
 }
 template <int HD, int QS, int NW, bool PRUNED, bool SHAREDQK, bool PLAIN = false, int HDK = HD, bool VWIN = false,
@@ -236,8 +234,6 @@ static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
     static_assert(QS == 1 || !MASK, "two subtiles a wave: without a mask");
     constexpr size_t lds = attn_lds_bytes<HD, QS, 4 * KS, false, HD, false, KS>();
     constexpr auto kern = &attention_packed_kernel<HD, QS, 4 * KS, MASK, KS>;
-    if (lds > 64 * 1024 && allow_lds<kern>(lds) != hipSuccess)
-        return;
     const long resident = (long)std::max(et_device_cu_count(), 1) * (QS == 2 ? 3 : HD <= 64 ? 4 / KS : 2);
     const long wgs = std::min<long>(resident, a.total);
     launch_kernel<kern>(dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256 * KS), lds, st, a);
@@ -547,14 +543,16 @@ constexpr int NOALLOC_MAX_DEVICES = 64;
 static unsigned *g_scratch_ptr[NOALLOC_MAX_DEVICES];
 static std::mutex g_scratch_mutex;
 
-static int noalloc_scratch(unsigned **ptr) {
+static int noalloc_scratch(unsigned **ptr, hipStream_t st) {
     int dev = -1;
-    ET_HIP(hipGetDevice(&dev));
+    ET_HIP(stream_device(st, &dev));
     ET_REQUIRE(dev >= 0 && dev < NOALLOC_MAX_DEVICES, ET_ERR_UNSUPPORTED,
                "et_OTF_attention_noalloc: device index %d beyond %d", dev, NOALLOC_MAX_DEVICES);
     std::lock_guard<std::mutex> lock(g_scratch_mutex);
     if (!g_scratch_ptr[dev]) {
         void *p = nullptr;
+        const OnDevice on(dev);
+        ET_HIP(on.error);
         ET_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
         ET_REQUIRE(p != nullptr, ET_ERR_HIP, "et_OTF_attention_noalloc: no address for the scratch array");
         g_scratch_ptr[dev] = static_cast<unsigned *>(p);
@@ -594,7 +592,7 @@ extern "C" int et_OTF_attention_noalloc(void *out, const void *Q, const void *K,
                "et_OTF_attention_noalloc: seq_len %d beyond the %d that the static scratch array covers",
                seq_len, NOALLOC_MAX_SEQ);
     unsigned *summary = nullptr;
-    const int rc = noalloc_scratch(&summary);
+    const int rc = noalloc_scratch(&summary, st);
     if (rc != ET_OK)
         return rc;
     // every word that the attention kernel reads for this seq_len is written

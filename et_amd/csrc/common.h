@@ -33,10 +33,14 @@ static inline bool aligned16(const void *p) {
     return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
 
+// What kept launch_kernel from launching, for the launch_status behind it.
+inline thread_local hipError_t g_not_launched = hipSuccess;
+
 static inline int launch_status(const char *what) {
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
-        return hip_fail(e, what);
+    const hipError_t kept = g_not_launched, last = hipGetLastError();
+    g_not_launched = hipSuccess;
+    if (kept != hipSuccess || last != hipSuccess)
+        return hip_fail(kept != hipSuccess ? kept : last, what);
     return ET_OK;
 }
 
@@ -146,24 +150,30 @@ __device__ __forceinline__ float f16_bits_to_float(uint16_t b) {
 inline unsigned magic_of(int d) { return d == 1 ? 0u : 0xFFFFFFFFu / (unsigned)d + 1u; }
 __device__ __forceinline__ int div_magic(int n, unsigned magic) { return magic ? (int)__umulhi((unsigned)n, magic) : n; }
 
-// Dynamic LDS above the 64 KB default has to be allowed per kernel.  The call
-// goes to the driver, so it is made only when a kernel needs more than it was
-// last given (one record per kernel instance and device).
-template <auto KERN>
-inline hipError_t allow_lds(size_t lds) {
-    static size_t allowed[16] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16)
-        return hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (lds <= allowed[dev])
-        return hipSuccess;
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERN),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e == hipSuccess)
-        allowed[dev] = lds;
-    return e;
+// The device that a stream's work runs on, whichever is current; the null stream and the per-thread one are the current
+// device's.
+inline hipError_t stream_device(hipStream_t st, int *dev) {
+    return !st || st == hipStreamLegacy || st == hipStreamPerThread ? hipGetDevice(dev) : hipStreamGetDevice(st, dev);
 }
+// `dev` is the current device while this lives
+class OnDevice {
+    int before = -1;
+
+  public:
+    hipError_t error;
+    explicit OnDevice(int dev) : error(hipGetDevice(&before)) {
+        if (error == hipSuccess && before != dev)
+            error = hipSetDevice(dev);
+        else
+            before = -1;
+    }
+    ~OnDevice() {
+        if (before >= 0)
+            (void)hipSetDevice(before);
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+};
 
 // What a launcher worked out for sizes it has seen: a choice among a kernel's forms weighs up to a hundred of them, 1 us of
 // the host's time at every launch, and a program calls with few sizes.  By value of the sizes alone, a table of its own
@@ -201,9 +211,19 @@ template <class Value, int N> struct KeptChoices {
     }
 };
 
-// A launch through the kernel's function handle, which is looked up once per kernel instance and device instead of by its
-// host address at every launch: 0.16 us less of host time a launch (13 parameters: 2.47 -> 2.31 us, 3.59 -> 3.48 while
-// the host is slow), where a call's smallest sizes are bound by the host.  Errors are left for launch_status, as with <<<>>>.
+// A launch through the kernel's function handle on the stream's device, which is looked up once per kernel instance and
+// device instead of by its host address at every launch: 0.16 us less of host time a launch (13 parameters: 2.47 -> 2.31
+// us, 3.59 -> 3.48 while the host is slow), where a call's smallest sizes are bound by the host.  Dynamic LDS above the
+// 64 KB default has to be allowed per kernel and device, by a call to the driver: made when a launch needs more than any
+// before it.  What goes wrong is left for launch_status, as with <<<>>>.
+constexpr size_t DEFAULT_LDS = 64 * 1024;
+struct KernelOnDevice {
+    std::atomic<hipFunction_t> fn{nullptr};
+    std::atomic<size_t> lds{DEFAULT_LDS}; // dynamic LDS that launches may ask for
+};
+// runtime.hip: makes both of the record good for such a launch
+hipError_t kernel_on_device(KernelOnDevice &k, const void *kernel, int dev, size_t lds);
+
 template <class... P, class... A>
 inline hipError_t launch_function(hipFunction_t fn, void (*)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, const A &...args) {
     static_assert(sizeof...(P) == sizeof...(A), "as many arguments as the kernel has parameters");
@@ -214,19 +234,22 @@ inline hipError_t launch_function(hipFunction_t fn, void (*)(P...), dim3 grid, d
 }
 template <auto KERN, class... A>
 inline void launch_kernel(dim3 grid, dim3 block, size_t lds, hipStream_t st, const A &...args) {
-    static std::atomic<hipFunction_t> known[16] = {};
+    static KernelOnDevice known[16];
+    KernelOnDevice beyond; // (devices of a higher number: looked up each time)
     int dev = 0;
-    hipFunction_t fn = nullptr;
-    const bool kept = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 16;
-    if (kept)
-        fn = known[dev].load(std::memory_order_acquire);
-    if (!fn) {
-        if (hipGetFuncBySymbol(&fn, reinterpret_cast<const void *>(KERN)) != hipSuccess)
-            return;
-        if (kept)
-            known[dev].store(fn, std::memory_order_release);
+    hipError_t e = stream_device(st, &dev);
+    if (e == hipSuccess) {
+        KernelOnDevice &k = dev >= 0 && dev < 16 ? known[dev] : beyond;
+        hipFunction_t fn = k.fn.load(std::memory_order_acquire);
+        if (!fn || lds > k.lds.load(std::memory_order_acquire)) {
+            e = kernel_on_device(k, reinterpret_cast<const void *>(KERN), dev, lds);
+            fn = k.fn.load(std::memory_order_acquire);
+        }
+        if (e == hipSuccess)
+            e = launch_function(fn, KERN, grid, block, lds, st, args...);
     }
-    (void)launch_function(fn, KERN, grid, block, lds, st, args...);
+    if (e != hipSuccess)
+        g_not_launched = e;
 }
 
 } // namespace et

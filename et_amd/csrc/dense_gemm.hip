@@ -300,7 +300,6 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
     a.div = a.by_column ? a.tiles_m : a.tiles_n;
     a.div_magic = magic_of(a.div);
     constexpr auto kern = &dense_gemm_kernel<GELU, WM, WN, TM, TN, ST>;
-    ET_HIP(allow_lds<kern>(lds));
     launch_kernel<kern>(dim3(a.per_xcd * 8), dim3(WM * WN * 64), lds, st, a.X, a.W[0], a.M, a.K, a.N[0],
                        a.per_xcd, a.total, a.div, a.div_magic, a.nlin | a.by_column << 4, a);
     return launch_status("dense_gemm launch");

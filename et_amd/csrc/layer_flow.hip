@@ -702,8 +702,6 @@ extern "C" int et_layer_flow_run(et_layer_flow *f, void *out, const void *in, vo
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto launch = [&](auto hd_c, auto mask_c, auto fused_c) -> int {
         constexpr auto kern = &layer_flow_kernel<decltype(hd_c)::value, decltype(mask_c)::value, decltype(fused_c)::value>;
-        if (lds > 64 * 1024) // (the default limit)
-            ET_HIP(allow_lds<kern>(lds));
         launch_kernel<kern>(dim3(total), dim3(LF_WAVES * 64), lds, st, a);
         return launch_status("layer in one launch");
     };

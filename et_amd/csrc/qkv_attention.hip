@@ -119,7 +119,6 @@ extern "C" int et_qkv_attention(void *out, const void *X, const et_tile_plan *q,
     hipStream_t s = static_cast<hipStream_t>(stream);
     auto launch = [&](auto mask_c) -> int {
         constexpr auto kern = &qkv_attention_kernel<decltype(mask_c)::value>;
-        ET_HIP(allow_lds<kern>(lds));
         launch_kernel<kern>(dim3(grid), dim3(QA_WAVES * 64), lds, s, a);
         return launch_status("et_qkv_attention launch");
     };

@@ -231,8 +231,6 @@ extern "C" int et_tile_plan_run_scatter_ln(const et_tile_plan *plan, void *out, 
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto launch = [&](auto nb_c, auto ms_c, auto np_c) -> int {
         constexpr auto kern = &row_layernorm_kernel<decltype(nb_c)::value, decltype(ms_c)::value, decltype(np_c)::value>;
-        if (lds > 64 * 1024) // (the default limit)
-            ET_HIP(allow_lds<kern>(lds));
         launch_kernel<kern>(dim3((M + 16 * ms - 1) / (16 * ms)), dim3(RL_WAVES * 64), lds, st, a.X, a.W, a.skip, a.M, a.K,
                            a.nbr, a.ppb, a.size, a.ldx, a.bias, a);
         return launch_status("row linear + LayerNorm launch");

@@ -23,6 +23,28 @@ int hip_fail(hipError_t e, const char *what) {
     return ET_ERR_HIP;
 }
 
+hipError_t kernel_on_device(KernelOnDevice &k, const void *kernel, int dev, size_t lds) {
+    static std::mutex mutex; // (a smaller value must not follow a larger one)
+    std::lock_guard<std::mutex> lock(mutex);
+    const OnDevice on(dev); // (both calls are about the current device's copy of the kernel)
+    if (on.error != hipSuccess)
+        return on.error;
+    if (!k.fn.load(std::memory_order_relaxed)) {
+        hipFunction_t fn = nullptr;
+        const hipError_t e = hipGetFuncBySymbol(&fn, kernel);
+        if (e != hipSuccess)
+            return e;
+        k.fn.store(fn, std::memory_order_release);
+    }
+    if (lds > k.lds.load(std::memory_order_relaxed)) {
+        const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess)
+            return e;
+        k.lds.store(lds, std::memory_order_release);
+    }
+    return hipSuccess;
+}
+
 // The wait-status word: pinned host memory that the device sees, allocated
 // once per process (by the first plan that is created, never inside a run).
 static int *g_status_host = nullptr, *g_status_dev = nullptr;

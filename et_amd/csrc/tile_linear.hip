@@ -1522,11 +1522,9 @@ static int launch_inst(const TlArgs &a, size_t lds, hipStream_t st) {
         constexpr int PNB = NB > 3 ? 3 : NB;
         if (a.nchunk == 1) {
             constexpr auto k = &tile_linear_resident_kernel<PNB, GELU, TL_WAVES, false>;
-            ET_HIP(allow_lds<k>(lds));
             launch_kernel<k>(grid, block, lds, st, TL_HOT(a, N[0]), a);
         } else {
             constexpr auto k = &tile_linear_plan_kernel<PNB, GELU, TL_WAVES, false>;
-            ET_HIP(allow_lds<k>(lds));
             launch_kernel<k>(grid, block, lds, st, TL_HOT(a, KC), a);
         }
     } else {
@@ -1554,11 +1552,9 @@ static int launch_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     const dim3 grid(a.per_xcd * 8), block(TL_LN_WAVES * 64);
     if (a.nchunk == 1) {
         constexpr auto k = &tile_linear_resident_kernel<NB, false, TL_LN_WAVES, true>;
-        ET_HIP(allow_lds<k>(lds));
         launch_kernel<k>(grid, block, lds, st, TL_HOT(a, N[0]), a);
     } else {
         constexpr auto k = &tile_linear_plan_kernel<NB, false, TL_LN_WAVES, true>;
-        ET_HIP(allow_lds<k>(lds));
         launch_kernel<k>(grid, block, lds, st, TL_HOT(a, KC), a);
     }
     return launch_status("tile_linear+LayerNorm launch");
@@ -1574,7 +1570,6 @@ static int ln_block_rows(int nbr) {
 template <int NB>
 static int launch_chunked_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_chunked_kernel<NB, false, true>;
-    ET_HIP(allow_lds<k>(lds));
     launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
     return launch_status("tile_linear+LayerNorm (chunked) launch");
 }
@@ -1582,7 +1577,6 @@ static int launch_chunked_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
 template <int NB, bool GELU>
 static int launch_chunked_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_chunked_kernel<NB, GELU, false>;
-    ET_HIP(allow_lds<k>(lds));
     launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
     return launch_status("tile_linear (chunked) launch");
 }
@@ -1648,11 +1642,9 @@ static int tile_launch_ffn(const TlProblem *pO, const TlProblem &p1, const TlPro
     const size_t lds = ffn_lds_bytes(K1, KC2);
     if (pO) {
         constexpr auto k = &tile_ffn_fused_kernel<3, true>;
-        ET_HIP(allow_lds<k>(lds));
         launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_FFN_WAVES * 64), lds, st, a);
     } else {
         constexpr auto k = &tile_ffn_fused_kernel<3, false>;
-        ET_HIP(allow_lds<k>(lds));
         launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_FFN_WAVES * 64), lds, st, a);
     }
     return launch_status("fused feed-forward launch");
@@ -1981,7 +1973,6 @@ static double tiles_estimate(const int *out_feat, const int *ntile, const int *n
 template <int NB, bool GELU, int NW = TL_WAVES>
 static int launch_resident64(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_resident_kernel<NB, GELU, NW, false, TL_BM64>;
-    ET_HIP(allow_lds<k>(lds));
     launch_kernel<k>(dim3(a.per_xcd * 8), dim3(NW * 64), lds, st, TL_HOT(a, N[0]), a);
     return launch_status("tile_linear (64-row panels) launch");
 }

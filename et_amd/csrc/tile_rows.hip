@@ -305,7 +305,6 @@ int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *
     const size_t lds = tile_rows_lds(K);
     auto launch = [&](auto gelu_c, auto raw_c) -> int {
         constexpr auto kern = &tile_rows_kernel<decltype(gelu_c)::value, decltype(raw_c)::value>;
-        ET_HIP(allow_lds<kern>(lds));
         launch_kernel<kern>(dim3(a.per_xcd * 8), dim3(TR_WAVES * 64), lds, st, a.X, a.l[0].cptr, a.M, a.K, a.total, a.per_xcd,
                            a.div, a.div_magic, a.ncg, a.ncg_magic, a.nb | a.ls << 4 | a.by_group << 8, a.l[0].nbr, a);
         return launch_status("tile_linear (whole rows) launch");

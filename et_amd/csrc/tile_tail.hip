@@ -933,8 +933,7 @@ int tail_pair_prepare(const et_tile_plan *pO, const et_tile_plan *p1, et_tile_pl
 template <int D, int MS>
 static int tt_launch(const TtArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_tail_pair_kernel<D, MS>;
-    ET_HIP(allow_lds<k>(lds));
-    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(TT_WAVES * 64), lds, st, a);
+    launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TT_WAVES * 64), lds, st, a);
     return launch_status("layer tail (pairs) launch");
 }
 

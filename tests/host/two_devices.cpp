@@ -21,14 +21,15 @@ struct Function {
 };
 struct Launch {
     int device;
-    unsigned grid, block, lds;
-    const void *symbol;
-    void *third; // the third parameter's eight bytes, where there is one
+    unsigned block, lds;
+    void *third; // the third parameter's eight bytes (two_devices_third)
 };
 std::mutex lock;
 std::map<std::pair<const void *, int>, int> allowed; // (kernel, device) -> dynamic LDS
 std::map<std::pair<const void *, int>, Function *> functions;
 std::vector<Launch> launches;
+bool refuse_lds = false; // the opt-in to large LDS fails
+unsigned third_lds = 0; // launches with that much LDS have at least three parameters, others may have one
 unsigned char symbols[2][1 << 16]; // a device variable's stand-in on either device
 thread_local int current = 0, last_error = OK;
 
@@ -38,17 +39,7 @@ int fail(int e) {
     return e;
 }
 int device_of(void *stream) { return stream ? static_cast<Stream *>(stream)->device : current; }
-int launch(const void *symbol, int device, unsigned grid, unsigned block, unsigned lds, void **params, bool has_third) {
-    std::lock_guard<std::mutex> l(lock);
-    if (lds > 64 * 1024 && allowed[{symbol, device}] < (int)lds)
-        return fail(INVALID_VALUE);
-    void *third = nullptr;
-    if (has_third)
-        memcpy(&third, params[2], sizeof(third));
-    if (launches.size() < 4096)
-        launches.push_back({device, grid, block, lds, symbol, third});
-    return OK;
-}
+bool lds_allowed(const void *symbol, int device, size_t lds) { return lds <= 64 * 1024 || allowed[{symbol, device}] >= (int)lds; }
 struct Dim {
     unsigned x, y, z;
 };
@@ -61,6 +52,8 @@ int two_devices_launches() {
     std::lock_guard<std::mutex> l(lock);
     return (int)launches.size();
 }
+void two_devices_refuse(int on) { refuse_lds = on; }
+void two_devices_third(unsigned lds) { third_lds = lds; }
 void two_devices_clear() {
     std::lock_guard<std::mutex> l(lock);
     launches.clear();
@@ -71,7 +64,7 @@ void two_devices_launch(int i, int *device, unsigned *block, unsigned *lds) {
     *block = launches[i].block;
     *lds = launches[i].lds;
 }
-// whose copy of a device variable the launch was handed as its third parameter; -1: none
+// whose copy of a device variable the launch was handed as its third parameter; -1: nobody's
 int two_devices_variable_of(int i) {
     std::lock_guard<std::mutex> l(lock);
     const unsigned char *p = static_cast<unsigned char *>(launches[i].third);
@@ -106,6 +99,8 @@ int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) { return memcp
 int hipGetSymbolAddress(void **p, const void *) { return *p = symbols[current], OK; }
 int hipFuncSetAttribute(const void *symbol, int, int value) {
     std::lock_guard<std::mutex> l(lock);
+    if (refuse_lds)
+        return fail(INVALID_VALUE);
     allowed[{symbol, current}] = value;
     return OK;
 }
@@ -117,15 +112,25 @@ int hipGetFuncBySymbol(void **fn, const void *symbol) {
     *fn = f;
     return OK;
 }
-int hipModuleLaunchKernel(void *fn, unsigned gx, unsigned, unsigned, unsigned bx, unsigned, unsigned, unsigned lds, void *stream,
+int hipModuleLaunchKernel(void *fn, unsigned, unsigned, unsigned, unsigned bx, unsigned, unsigned, unsigned lds, void *stream,
                           void **params, void **) {
     const Function *f = static_cast<Function *>(fn);
+    std::lock_guard<std::mutex> l(lock);
     if (f->device != device_of(stream))
         return fail(INVALID_HANDLE);
-    return launch(f->symbol, f->device, gx, bx, lds, params, true);
+    if (!lds_allowed(f->symbol, f->device, lds))
+        return fail(INVALID_VALUE);
+    void *third = nullptr;
+    if (lds && lds == third_lds)
+        memcpy(&third, params[2], sizeof(third));
+    if (launches.size() < 4096)
+        launches.push_back({f->device, bx, lds, third});
+    return OK;
 }
-int hipLaunchKernel(const void *symbol, Dim grid, Dim block, void **params, size_t lds, void *stream) {
-    return launch(symbol, device_of(stream), grid.x, block.x, (unsigned)lds, params, false);
+// (finds its device by itself: not written down)
+int hipLaunchKernel(const void *symbol, Dim, Dim, void **, size_t lds, void *stream) {
+    std::lock_guard<std::mutex> l(lock);
+    return lds_allowed(symbol, device_of(stream), lds) ? OK : fail(INVALID_VALUE);
 }
 static thread_local struct {
     Dim grid, block;

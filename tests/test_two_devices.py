@@ -45,7 +45,14 @@ def plan(K, N, sparsity):
     check(L.et_tile_plan_create(C.byref(p), K, N, n, data.ctypes.data, rp.ctypes.data, ro.ctypes.data, bias.ctypes.data))
     return p
 
-x = buf(1 << 20)
+def flow(rows):
+    f = C.c_void_p()
+    plans = [plan(768, 768, 0.8) for _ in range(4)] + [plan(768, 3072, 0.8), plan(3072, 768, 0.8)]
+    check(L.et_layer_flow_create(C.byref(f), *plans, rows, 12, 1))
+    assert f.value
+    return f
+
+x, y = buf(1 << 20), buf(1 << 20)
 """
 
 
@@ -84,4 +91,66 @@ for device in (0, 1, 0):
     check({ATTENTION[form]})
     ls = launches()
     assert len(ls) == 1 and ls[0][0] == device and ls[0][2] > 64 * 1024, ls
+""")
+
+
+OTHER_STREAM = {
+    "attention": "[L.et_OTF_attention(x, x, x, x, None, 1024, 768, 12, 1, None, 1.0, s)]",
+    "packed attention": "[L.et_OTF_attention_varlen(x, x, x, x, x, x, 1024, 768, 12, 1, 1.0, s)]",
+    "linear, 64-row panels": "[L.et_tile_plan_run(plan(768, 3072, 0.8), x, x, 4096, 1, s)]",
+    "linear, chunks": "[L.et_tile_plan_run(plan(3072, 768, 0.8), x, x, m, 0, s) for m in (100, 3300, 16384)]",
+    "linear + LayerNorm": "[L.et_tile_plan_run_ln(plan(k, 768, 0.8), x, x, x, x, x, 8192, s) for k in (768, 3072)]",
+    "raw linear": "[L.et_tile_spmm_add_bias(x, x, x, x, x, m, 768, k, x, s) for m, k in ((64, 768), (4096, 768), (64, 3072))]",
+    "dense product": "[L.et_row_spmm_add_bias(x, x, x, x, m, 768, 3072, s) for m in (2000, 8192, 65536)]",
+    "projections and attention": "[L.et_qkv_attention(x, x, *[plan(768, 768, 0.8) for _ in range(3)], m, None, None, 128, 128, 768,"
+                                 " 12, 4, 1.0, s) for m in (None, x)]",
+    "layer tail": "[L.et_tile_plan_run_tail(plan(768, 768, 0.8), plan(768, 3072, 0.8), plan(3072, 768, 0.8), *[x] * 9, 8192, s)]",
+    "layer tail in pairs": "[L.et_tile_plan_run_tail_ws(plan(768, 768, 0.8), plan(768, 3072, 0.8), plan(3072, 768, 0.8), *[x] * 9,"
+                           " 2048, y, 1 << 27, s) for v in (1, 2, 3) if not L.et_tuning_set(b'tile_tail_pair', v)]",
+    "layer": "[L.et_layer_flow_run(flow(37), x, x, x, x, x, x, m, None, None, x, x, x, x, 1.0, s) for m in (None, x)]",
+    "compact linear + LayerNorm": "[L.et_tile_plan_run_scatter_ln(plan(k, 384, 0.0), x, x, y, x, 384, x, x, x, 768, 8192, s)"
+                                  " for k in (768, 1024)]",
+    "LayerNorm": "[L.et_skip_layernorm(x, x, x, x, 1000, 768, s)]",
+}
+
+
+@pytest.mark.parametrize("op", OTHER_STREAM)
+def test_launches_take_the_device_of_their_stream(runtime, op):
+    """a stream of the second device while the first one is current: functions, and the opt-in to large LDS, of the second
+    device, whichever of the two was used first; the current device stays"""
+    run(runtime, f"""
+d = C.c_int()
+for device in (1, 0, 1):
+    s = stream(device)
+    rt.two_devices_clear()
+    for rc in {OTHER_STREAM[op]}:
+        check(rc)
+    ls = launches()
+    assert ls and all(l[0] == device for l in ls), ls
+    rt.hipGetDevice(C.byref(d))
+    assert d.value == 0
+""")
+
+
+def test_static_scratch_is_that_of_the_streams_device(runtime):
+    """et_OTF_attention_noalloc: every device has its own copy of the mask summary's array"""
+    run(runtime, """
+rt.two_devices_third(4)  # (the summary kernel: a word for 200 keys; mask, rows, summary, words)
+for device in (1, 0):
+    rt.two_devices_clear()
+    check(L.et_OTF_attention_noalloc(x, x, x, x, x, 200, 768, 12, 1, None, 1.0, stream(device)))
+    assert [l[0] for l in launches()] == [device, device]
+    assert rt.two_devices_variable_of(0) == device
+""")
+
+
+def test_a_refused_opt_in_is_reported_and_nothing_launched(runtime):
+    run(runtime, """
+rt.two_devices_refuse(1)
+for s in (None, stream(1)):
+    assert L.et_OTF_attention(x, x, x, x, None, 1024, 768, 12, 1, None, 1.0, s) == -4
+    assert L.et_tile_plan_run(plan(768, 3072, 0.8), x, x, 4096, 1, s) == -4
+assert launches() == []
+rt.two_devices_refuse(0)
+check(L.et_OTF_attention(x, x, x, x, None, 1024, 768, 12, 1, None, 1.0, None))
 """)
