@@ -312,7 +312,7 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
 // ones where every CU has several; 256 x 192 where one block a CU is all there is (768 -> 1536, 8192 rows: 21.2 against
 // 22.4 us in 128 x 192, 23.3 in 256 x 256).
 enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_256x192, DG_FORMS };
-static int g_dense_form = -1; // et_tuning_set("dense_form"): one of the above, -1 chooses
+static std::atomic<int> g_dense_form{-1}; // et_tuning_set("dense_form"): one of the above, -1 chooses
 static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
     static const int bm[DG_FORMS] = {64, 128, 128, 128, 256, 256}, bn[DG_FORMS] = {128, 128, 128, 192, 256, 192};
     struct Form {
@@ -353,8 +353,9 @@ static int dg_choose(const int *Ns, int nlin, int M, int K, double *us) {
 }
 double dense_gemm_estimate(const int *Ns, int nlin, int M, int K) {
     double us = 0.0;
-    if (g_dense_form >= 0)
-        return dg_estimate(g_dense_form, Ns, nlin, M, K);
+    const int set = g_dense_form;
+    if (set >= 0)
+        return dg_estimate(set, Ns, nlin, M, K);
     dg_choose(Ns, nlin, M, K, &us);
     return us;
 }
@@ -384,7 +385,7 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
     a.M = M;
     a.K = K;
     double us;
-    const int form = g_dense_form >= 0 ? g_dense_form : dg_choose(Ns, nlin, M, K, &us);
+    const int set = g_dense_form, form = set >= 0 ? set : dg_choose(Ns, nlin, M, K, &us);
     switch (form) {
 #define DG_CASE(form_, ...)                                                                                            \
     case form_: return gelu ? dg_launch_inst<true, __VA_ARGS__>(a, st) : dg_launch_inst<false, __VA_ARGS__>(a, st);

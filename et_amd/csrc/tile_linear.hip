@@ -1582,7 +1582,7 @@ static int launch_chunked_inst(const TlArgs &a, size_t lds, hipStream_t st) {
 }
 
 static int g_tile_ln_chunked = 1;
-static int g_tile_chunked = -1; // et_tuning_set("tile_chunked")
+static std::atomic<int> g_tile_chunked{-1}; // et_tuning_set("tile_chunked")
 static int g_tile_fuse_ffn = 2; // et_tuning_set("tile_fuse_ffn"): 1 feed-forward block, 2 whole layer tail
 
 // LDS bytes of the fused feed-forward kernel: X panel, two hidden buffers (the
@@ -1699,11 +1699,12 @@ static int tile_launch_ln(const TlProblem &p, const f16 *X, int M, int K, int KC
     }
 }
 
-// Tuning knobs (et_tuning_set): 0 = automatic.
-static int g_tile_nb = 0;
-static int g_tile_min_wgs = 512;
-static int g_tile_ipw = 0;
-static int g_tile_form = -1; // et_tuning_set("tile_form"): index in tl_forms
+// Tuning knobs (et_tuning_set): 0 = automatic.  Those that the choice of a form reads may be set while another thread
+// launches: that launch takes the old or the new value, later ones the new.
+static std::atomic<int> g_tile_nb{0};
+static std::atomic<int> g_tile_min_wgs{512};
+static std::atomic<int> g_tile_ipw{0};
+static std::atomic<int> g_tile_form{-1}; // et_tuning_set("tile_form"): index in tl_forms
 static int g_tile_fuse_ln = 1;
 static int g_tile_min_panels = 0; // fewest panels of the fused linear + LayerNorm and layer tail kernels, 0 = automatic
 // the layer tail's choice is forced (a layer then runs its steps as separate launches)
@@ -1729,25 +1730,26 @@ static int choose_nb(int nrp, int nbr_max, int nlin) {
 }
 
 constexpr int TL_BM64 = 2 * TL_BM;
-static int g_tile_bm64 = 1; // et_tuning_set("tile_bm64")
+static std::atomic<int> g_tile_bm64{1}; // et_tuning_set("tile_bm64")
 // rows from which the row-pruned linear runs the register-blocked GEMM (et_tuning_set("row_gemm_min_rows");
 // below, 128 x 128 blocks leave most CUs without work and the tile kernels win)
 static int g_row_gemm_min_rows = 1024;
 // fully populated plans as dense products: 1 by size, 0 never, 2 always (et_tuning_set("plan_dense"))
 static int g_plan_dense = 1;
 
-static int g_tile_rows_most = -1; // et_tuning_set("tile_splitk_rows"): most rows for which a plan runs on whole rows, -1 automatic
+static std::atomic<int> g_tile_rows_most{-1}; // et_tuning_set("tile_splitk_rows"): most rows for which a plan runs on whole rows, -1 automatic
 static int g_tile_splitk_k1 = 0;  // et_tuning_set("tile_splitk_k1"): also plans of one chunk, up to that many rows (automatic: 128)
 
-static int g_tile_order = 1; // et_tuning_set("tile_order"): 0 panels slowest, 2 column groups slowest, 1 fewer bytes
+static std::atomic<int> g_tile_order{1}; // et_tuning_set("tile_order"): 0 panels slowest, 2 column groups slowest, 1 fewer bytes
 // Whether consecutive workgroups walk the panels of a column group (tl_place): X and W in bytes, numbers of panels
 // and of workgroups per panel.  Every L2 that has part of the work takes what all of the work shares, so W times eight
 // is what bounds a launch of few rows: 256 rows, 1024 -> 4096: dense 14.2 -> 6.6 us, 50 % 10.0 -> 5.6; 768 -> 3072
 // dense 9.7 -> 5.9; 128 rows 3072 -> 768 dense 9.8 -> 6.8.  Only up to x_most bytes of X: beyond, the L2s have time
 // enough for W and the launch is up to 10 % slower in this order (1536 rows, 1024 -> 4096, 50 %: 18.7 and 20.9).
 bool tl_order(double x_bytes, double w_bytes, long panels, long groups, double x_most) {
-    if (g_tile_order != 1)
-        return g_tile_order == 2;
+    const int order = g_tile_order;
+    if (order != 1)
+        return order == 2;
     return x_bytes <= x_most && std::min(groups, 8L) * x_bytes + w_bytes < x_bytes + std::min(panels, 8L) * w_bytes;
 }
 double tl_traffic_mb(double x_mb, double w_mb, long panels, long groups, double x_most) {
@@ -1794,20 +1796,20 @@ static TlChoice weigh_resident(const TlProblem *probs, int nlin, int M, int K, i
         result += (double)M * probs[i].N;
     }
     const double x_mb = 2e-6 * M * K;
-    const int fnb = g_tile_nb >= 1 && g_tile_nb <= 3 ? g_tile_nb : 0;
+    const int nb_set = g_tile_nb, form_set = g_tile_form, ipw_set = g_tile_ipw, bm64 = g_tile_bm64;
+    const int fnb = nb_set >= 1 && nb_set <= 3 ? nb_set : 0;
     TlChoice best = {};
     auto lds_of = [&](const TlForm &f) {
         return (size_t)f.rows * (K + ((K & 31) ? 0 : TL_PAD)) * sizeof(f16) +
                (size_t)f.waves * f.rows * (16 * f.nb + 8) * sizeof(f16);
     };
     const TlForm *only = nullptr; // (tuning)
-    if (g_tile_form >= 0 && g_tile_form < (int)(sizeof(tl_forms) / sizeof(tl_forms[0])) &&
-        lds_of(tl_forms[g_tile_form]) <= 160 * 1024)
-        only = &tl_forms[g_tile_form];
+    if (form_set >= 0 && form_set < (int)(sizeof(tl_forms) / sizeof(tl_forms[0])) && lds_of(tl_forms[form_set]) <= 160 * 1024)
+        only = &tl_forms[form_set];
     for (const TlForm &f : tl_forms) {
         if (only ? &f != only
-                 : (f.rows == TL_BM ? (fnb ? f.nb != fnb : g_tile_bm64 == 2) : fnb || g_tile_bm64 == 0) ||
-                       (f.waves == 12 && g_tile_bm64 == 4))
+                 : (f.rows == TL_BM ? (fnb ? f.nb != fnb : bm64 == 2) : fnb || bm64 == 0) ||
+                       (f.waves == 12 && bm64 == 4))
             continue; // (tuning; a form of either height fits every K of one chunk)
         const size_t lds = lds_of(f);
         if (lds > 160 * 1024)
@@ -1823,8 +1825,8 @@ static TlChoice weigh_resident(const TlProblem *probs, int nlin, int M, int K, i
         // (beyond 16 items a workgroup the tail of the launch shows; a tuning value counts down to a whole number of
         // workgroups per panel)
         int first = 1, last = std::min(per_panel, 16);
-        if (g_tile_ipw > 0) {
-            first = std::min(g_tile_ipw, per_panel);
+        if (ipw_set > 0) {
+            first = std::min(ipw_set, per_panel);
             while (per_panel % first)
                 first--;
             last = first;
@@ -1887,11 +1889,12 @@ static int weigh_chunked(const TlProblem *probs, int nlin, int M, int K, int nch
                                      : estimate_chunked(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, which, cus);
     };
     const bool rows_fit = tile_rows_fits(K);
+    const int rows_most = g_tile_rows_most, chunked = g_tile_chunked;
     int best = TL_BY_PLAN;
-    if (rows_fit && g_tile_rows_most >= 0 && M <= g_tile_rows_most)
+    if (rows_fit && rows_most >= 0 && M <= rows_most)
         best = TL_BY_ROWS; // (tuning)
-    else if (g_tile_chunked > 0)
-        best = std::min(g_tile_chunked, 4);
+    else if (chunked > 0)
+        best = std::min(chunked, 4);
     *us = estimate(best);
     if (best != TL_BY_PLAN)
         return best;
@@ -1902,16 +1905,16 @@ static int weigh_chunked(const TlProblem *probs, int nlin, int M, int K, int nch
             best = which;
         }
     };
-    if (g_tile_chunked < 0)
+    if (chunked < 0)
         for (int nb = 1; nb <= 4; nb++)
             take(nb);
-    if (rows_fit && g_tile_rows_most < 0)
+    if (rows_fit && rows_most < 0)
         take(TL_BY_ROWS);
     return best;
 }
 
 // The two choices, kept for sizes that come again (100 rows 768 -> 768, bound by the host: 5.4 -> 4.9 us a call).
-static std::atomic<int> g_tunings{0}; // et_tuning_set was called so many times
+static std::atomic<int> g_tunings{0}; // et_tuning_set has returned so many times
 typedef KeptChoices<TlChoice, 6 + 3 * TL_MAX_LIN> ResidentChoices;
 struct ChunkedChoice {
     int which;
@@ -1919,7 +1922,7 @@ struct ChunkedChoice {
 };
 typedef KeptChoices<ChunkedChoice, 6 + 3 * TL_MAX_LIN> ChunkedChoices;
 template <class Key> static Key choice_key(const TlProblem *probs, int nlin, int M, int K, int more, int cus) {
-    Key k = {{nlin, M, K, more, cus, g_tunings.load(std::memory_order_relaxed)}};
+    Key k = {{nlin, M, K, more, cus, g_tunings.load(std::memory_order_acquire)}};
     for (int i = 0; i < nlin; i++) {
         k.v[6 + 3 * i] = probs[i].N;
         k.v[7 + 3 * i] = probs[i].nbr;
@@ -2002,11 +2005,12 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
     // Whole rows in LDS (tile_rows.hip).  Plans: see choose_chunked.  Raw lists: always where K is beyond the generic
     // kernel's panel (it filters every list once per chunk: three to eight times slower), else while there is no more
     // than one workgroup per CU (16 rows x 16 block-rows each).
+    const int rows_most = g_tile_rows_most;
     int which = TL_BY_PLAN;
     if (mode == TL_PLAN && nchunk > 1) {
         double us;
         which = g_tile_nb == 0 ? choose_chunked(probs, nlin, M, K, nchunk, nbr_max, &us) : TL_BY_PLAN;
-    } else if (mode == TL_PLAN && g_tile_splitk_k1 && tile_rows_fits(K) && M <= (g_tile_rows_most < 0 ? 128 : g_tile_rows_most)) {
+    } else if (mode == TL_PLAN && g_tile_splitk_k1 && tile_rows_fits(K) && M <= (rows_most < 0 ? 128 : rows_most)) {
         which = TL_BY_ROWS;
     } else if (g_tile_nb == 0 && tile_rows_fits(K) && (mode == TL_RAW || mode == TL_FILTER)) {
         const long panels = (M + 15) / 16;
@@ -2161,8 +2165,7 @@ static int raw_tile_linear(void *Y, const void *X, const int *row_ptr, const int
 
 static int g_tail_pair_min_wgs = 0; // et_tuning_set("tile_tail_pair_min_wgs"): 0 = three quarters of the CUs
 
-extern "C" int et_tuning_set(const char *key, int value) {
-    et::g_tunings.fetch_add(1, std::memory_order_relaxed); // (kept choices are weighed again)
+static int set_knob(const char *key, int value) {
     if (key && !strcmp(key, "tile_splitk_rows")) {
         et::g_tile_rows_most = value;
         return ET_OK;
@@ -2269,6 +2272,12 @@ extern "C" int et_tuning_set(const char *key, int value) {
     }
     et::set_error("et_tuning_set: unknown key");
     return ET_ERR_INVALID_ARG;
+}
+extern "C" int et_tuning_set(const char *key, int value) {
+    const int rc = set_knob(key, value);
+    // Kept choices are weighed again.  Counted behind the write: a choice kept under the new number has read the new value.
+    et::g_tunings.fetch_add(1, std::memory_order_release);
+    return rc;
 }
 
 extern "C" int et_tile_spmm_add_bias(void *Y, const void *X, const int *W_row_ptr,

@@ -565,7 +565,10 @@ int et_device_synchronize(void);
  *                     up sets a status word, the launch's result is wrong, and
  *                     the next launch of that kind returns ET_ERR_HIP once.  0
  *                     makes every wait give up at once (for testing the report)
- * Not thread-safe; results never depend on these beyond fp32 summation
+ * A launch that begins after the call has returned sees the value, on any thread.
+ * "tile_nb", "tile_min_wgs", "tile_ipw", "tile_form", "tile_bm64", "tile_order",
+ * "tile_chunked", "tile_splitk_rows" and "dense_form" may be set while other threads
+ * launch; the others may not.  Results never depend on these beyond fp32 summation
  * order. */
 int et_tuning_set(const char *key, int value);
 /* The fused layer-tail kernels order their waves with bounded waits on LDS

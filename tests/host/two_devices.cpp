@@ -2,11 +2,12 @@
 // ahead of libet_amd.so it answers the calls that the library makes, so that what the launchers do per device, per stream
 // and per thread can be tested where there is no GPU.  Kernels need the opt-in to more than 64 KB of LDS on each device,
 // and a launch takes a function of its stream's device, as the runtime documents.
-#include <cstdint>
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -27,7 +28,8 @@ struct Launch {
 std::mutex lock;
 std::map<std::pair<const void *, int>, int> allowed; // (kernel, device) -> dynamic LDS
 std::map<std::pair<const void *, int>, Function *> functions;
-std::vector<Launch> launches;
+std::vector<Launch> launches; // the first few thousand
+Launch latest;
 bool refuse_lds = false; // the opt-in to large LDS fails
 unsigned third_lds = 0; // launches with that much LDS have at least three parameters, others may have one
 unsigned char symbols[2][1 << 16]; // a device variable's stand-in on either device
@@ -72,6 +74,29 @@ int two_devices_variable_of(int i) {
         if (p >= symbols[d] && p < symbols[d] + sizeof(symbols[d]))
             return d;
     return -1;
+}
+// One thread launches the plan again and again while this one sets a key, to two values in turn.  Returns how often a launch
+// that began after the key was set did not have the value's threads a workgroup.
+int two_devices_race(int (*set)(const char *, int), int (*run)(const void *, void *, const void *, int, int, void *),
+                     const void *plan, void *x, int rows, const char *key, const int *values, const unsigned *threads, int times) {
+    std::atomic<bool> stop{false};
+    std::atomic<int> done{0};
+    std::thread runs([&] {
+        for (; !stop; done++)
+            run(plan, x, x, rows, 1, nullptr);
+    });
+    int wrong = 0;
+    for (int i = 0; i < times; i++) {
+        set(key, values[i & 1]);
+        const int before = done;
+        while (done < before + 2) // (the first of them may have begun earlier)
+            ;
+        std::lock_guard<std::mutex> l(lock);
+        wrong += latest.block != threads[i & 1];
+    }
+    stop = true;
+    runs.join();
+    return wrong;
 }
 
 // ---- the runtime
@@ -123,8 +148,9 @@ int hipModuleLaunchKernel(void *fn, unsigned, unsigned, unsigned, unsigned bx, u
     void *third = nullptr;
     if (lds && lds == third_lds)
         memcpy(&third, params[2], sizeof(third));
+    latest = {f->device, bx, lds, third};
     if (launches.size() < 4096)
-        launches.push_back({f->device, bx, lds, third});
+        launches.push_back(latest);
     return OK;
 }
 // (finds its device by itself: not written down)

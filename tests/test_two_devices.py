@@ -154,3 +154,20 @@ assert launches() == []
 rt.two_devices_refuse(0)
 check(L.et_OTF_attention(x, x, x, x, None, 1024, 768, 12, 1, None, 1.0, None))
 """)
+
+
+def test_a_tuning_key_holds_from_its_return_on_other_threads_too(runtime):
+    """choices are kept per thread under the number of et_tuning_set calls: a launch that is being weighed while a key is
+    set must not keep the old value's choice under the new number"""
+    run(runtime, """
+rows, values, threads = 4096, (C.c_int * 2)(0, 2), (C.c_uint * 2)()
+p = plan(768, 3072, 0.8)
+for i in range(2):
+    check(L.et_tuning_set(b"tile_bm64", values[i]))  # 32-row panels, 64-row panels
+    check(L.et_tile_plan_run(p, x, x, rows, 1, None))
+    threads[i] = launches()[-1][1]
+assert threads[0] != threads[1]
+as_pointer = lambda f: C.cast(f, C.c_void_p)
+assert rt.two_devices_race(as_pointer(L.et_tuning_set), as_pointer(L.et_tile_plan_run), p, x, rows, b"tile_bm64", values, threads,
+                           20000) == 0
+""")
