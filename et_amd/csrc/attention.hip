@@ -68,8 +68,11 @@ __global__ void __launch_bounds__(512, 4) attention_two_groups_kernel(const Attn
 // sequence, which every wave keeps in registers (lane l: sequences l, l+64, ...;
 // at most 64*AT_PX sequences).
 constexpr int AT_PX = 4;
+// workgroups that a CU holds at once, by which the launcher sizes the grid: the registers have to allow them (the bound
+// counts waves of a SIMD)
+constexpr int packed_on_cu(int HD, int QS, int KS) { return QS == 2 ? 3 : HD <= 64 ? 4 / KS : 2; }
 template <int HD, int QS, int NW, bool MASK, int KS = 1>
-__global__ void __launch_bounds__(NW * 64, (QS == 1 && HD <= 64) ? 4 / KS : 2) attention_packed_kernel(const AttnArgs a) {
+__global__ void __launch_bounds__(NW * 64, packed_on_cu(HD, QS, KS) * NW / 4) attention_packed_kernel(const AttnArgs a) {
     constexpr int QB = NW / KS * 16 * QS;
     const int lane = threadIdx.x & 63;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, W = gridDim.x >> 3;
@@ -234,7 +237,7 @@ static void attn_launch_packed(const AttnArgs &a, hipStream_t st) {
     static_assert(QS == 1 || !MASK, "two subtiles a wave: without a mask");
     constexpr size_t lds = attn_lds_bytes<HD, QS, 4 * KS, false, HD, false, KS>();
     constexpr auto kern = &attention_packed_kernel<HD, QS, 4 * KS, MASK, KS>;
-    const long resident = (long)std::max(et_device_cu_count(), 1) * (QS == 2 ? 3 : HD <= 64 ? 4 / KS : 2);
+    const long resident = (long)std::max(et_device_cu_count(), 1) * packed_on_cu(HD, QS, KS);
     const long wgs = std::min<long>(resident, a.total);
     launch_kernel<kern>(dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256 * KS), lds, st, a);
 }
