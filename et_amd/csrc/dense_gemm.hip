@@ -13,7 +13,9 @@
 // step, 1.29 PFLOP/s; 0.85 us while half of the CUs have none), at K = 768 the ends: the launch, the first step's
 // latency and the result's way out are 6 of 21 us.  A request occupies its wave while it goes out, and eight in one go
 // behind the barrier kept both waves of a SIMD from the matrix unit: they go out between the products (8192 rows 928 ->
-// 240 8.5 -> 7.1 us, 768 -> 768 14.1 -> 13.0, 2000 rows 768 -> 2304 12.5 -> 11.9, 16384 rows 4096 -> 1024 114 -> 109).
+// 240 9.5 -> 8.1 us, 768 -> 768 15.3 -> 13.9, 2000 rows 768 -> 2304 14.1 -> 12.8, 16384 rows 1024 -> 4096 135 -> 127, 4096 ->
+// 1024 111 -> 106; 3072 -> 768 43.0 -> 42.8 and 768 -> 3072 45.1 -> 42.6).  All figures here are of normally distributed
+// operands: with weights that are all alike the same launches are up to a sixth shorter.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -51,8 +53,8 @@ __device__ __forceinline__ int dg_swizzle(int r, int kc) { return kc ^ ((r >> 1)
 // step's second half of fragments is read while the first half multiplies, then the stage is handed back, the step ST
 // later requested into it and the next step's first fragments read while the second half multiplies: fragment reads and
 // the barrier run under MFMAs.
-// us a launch: 8192 rows 768 -> 768 13.0, 768 -> 1536 21.2, 768 -> 3072 44.7, 3072 -> 768 40.2, 928 -> 240 7.1; 16384 rows
-// 1024 -> 4096 136 (1010 TFLOP/s), 4096 -> 1024 109 (1260 TFLOP/s).
+// us a launch: 8192 rows 768 -> 768 13.9, 768 -> 1536 23.0, 768 -> 3072 42.6, 3072 -> 768 42.8, 928 -> 240 8.1; 16384 rows
+// 1024 -> 4096 127 (1080 TFLOP/s), 4096 -> 1024 106 (1290); 4096 x 4096 x 4096 107 (1280), 8192 x 8192 x 8192 909 (1210).
 template <bool GELU, int WM, int WN, int TM, int TN, int ST>
 __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     // (what the first requests need arrives in registers with the wave)
@@ -307,10 +309,11 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
 
 // The blocks there are and the time of each form in microseconds, without the launch.  A step takes longer with every
 // further workgroup of a CU and with the share of the CUs that have one; the figures are fits to 385 shapes (128 to 32768
-// rows, 512 to 4096 columns), the forms near the fastest weighing most.  The block they choose is 0.2 % behind the fastest
-// in the mean, 14 % at most (3072 -> 768, 8192 rows: 40.6 against 35.7 us).  Small blocks win while they let more CUs take part, large
-// ones where every CU has several; 256 x 192 where one block a CU is all there is (768 -> 1536, 8192 rows: 21.2 against
-// 22.4 us in 128 x 192, 23.3 in 256 x 256).
+// rows, 512 to 4096 columns; equal weights), the forms near the fastest weighing most.  On the 80 full plans of
+// bench/linear_forms.py (random weights, two runs) the block they choose is 0.2 to 0.3 % behind the fastest in the mean, 8 %
+// at most (512 -> 512, 9182 rows: 10.1 against 9.4 us), and its estimate with the launch 7 % off; over all blocks, also those
+// that nobody would choose, 12 %.  Small blocks win while they let more CUs take part, large ones where every CU has several;
+// 256 x 192 where one block a CU is all there is (768 -> 1536, 8192 rows: 22.0 against 22.6 us in 128 x 192, 23.8 in 256 x 256).
 enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_256x192, DG_FORMS };
 static std::atomic<int> g_dense_form{-1}; // et_tuning_set("dense_form"): one of the above, -1 chooses
 static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {

@@ -1738,7 +1738,7 @@ static int g_row_gemm_min_rows = 1024;
 static int g_plan_dense = 1;
 
 static std::atomic<int> g_tile_rows_most{-1}; // et_tuning_set("tile_splitk_rows"): most rows for which a plan runs on whole rows, -1 automatic
-static int g_tile_splitk_k1 = 0;  // et_tuning_set("tile_splitk_k1"): also plans of one chunk, up to that many rows (automatic: 128)
+static int g_tile_splitk_k1 = 0;  // et_tuning_set("tile_splitk_k1"): 1: also plans of one chunk, up to tile_splitk_rows rows (-1: 128)
 
 static std::atomic<int> g_tile_order{1}; // et_tuning_set("tile_order"): 0 panels slowest, 2 column groups slowest, 1 fewer bytes
 // Whether consecutive workgroups walk the panels of a column group (tl_place): X and W in bytes, numbers of panels
@@ -1767,9 +1767,9 @@ double tl_traffic_mb(double x_mb, double w_mb, long panels, long groups, double 
 // are then moved by up to a factor of two where that brings the choice closer to the fastest form: 0.5 % from it in the
 // mean, 13 % at most (0.6 % where half of the row counts was left out); the rule before, a number of workgroups to aim
 // for, was 6.3 %.  bench/linear_forms.py times the forms and fits the terms anew: on its 320 linears (launches of a graph)
-// the estimates are 4 to 7 % off and all choices of this file together 1.3 % behind the fastest form, 20 % at most (2048
-// -> 512 dense, 1343 rows: 12.7 against 10.6 us).  1536 rows 768 -> 3072, 50 %: 13.8 -> 11.7 us; 3500 rows 768 -> 768, 90 %: 7.3 -> 5.8; 2700 rows
-// 768 -> 3072, 80 %: 16.1 -> 12.4.
+// the estimates are 6 to 8 % off and all choices of this file together 1.4 % behind the fastest form, 19 % at most (2048
+// -> 512 dense, 1343 rows: 12.4 against 10.4 us).  1536 rows 768 -> 3072, 50 %: 13.8 -> 11.7 us; 3500 rows 768 -> 768, 90 %:
+// 7.3 -> 5.8; 2700 rows 768 -> 3072, 80 %: 16.1 -> 12.4.
 struct TlForm {
     int rows, waves, nb;
 };
@@ -1856,8 +1856,8 @@ static TlChoice weigh_resident(const TlProblem *probs, int nlin, int M, int K, i
 // Terms: launch, rounds of workgroups and their chunks, the stream of a wave's pairs, the work of the busiest CU, and
 // the megabytes that the L2s take in; fitted like the single-panel forms to 1600 launches (2048 -> 512, 3072 -> 768,
 // 4096 -> 1024, 0 to 90 % pruned, 48 to 16384 rows): 5 to 6 % off in the mean, the choice 0.2 % behind the fastest
-// kernel, 9 % at most (the rule before: 10.9 %).  The 576 launches that bench/linear_forms.py times in graphs: 14, 6 and
-// 9 % off.
+// kernel, 9 % at most (the rule before: 10.9 %).  The 576 launches that bench/linear_forms.py times in graphs (plan kernel,
+// fetching waves, whole rows): 15, 8 and 13 % off.
 enum { TL_BY_ROWS = -1, TL_BY_PLAN = 0 }; // or 1 .. 4: fetching waves, that many block-rows per computing wave
 static double estimate_plan_kernel(int M, double pairs, double x_mb, double w_mb, int nchunk, int nbr_max, int nlin, long cus) {
     const long panels = (M + TL_BM - 1) / TL_BM;
@@ -2305,9 +2305,10 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 // Plans of fully populated matrices: the dense product where it is estimated to be the shorter launch, from some hundred
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
 // tile: their time is that of the choice among their forms, whose figures are fits to launches of a graph and a tenth above
-// launches among others.  2.4 of the 2.6 us stand for the launch, which dense_gemm_estimate leaves out.  Over 176 full plans
-// the choice is then 0.3 % behind the faster side in the mean and 14 % at most; 1 and 20 % without the tenth, with it 0.8
-// and 17 % with 1 us more, 2 and 24 % with 1 us less.
+// launches among others.  2.4 of the 2.6 us stand for the launch, which dense_gemm_estimate leaves out.  On the 80 full plans of
+// bench/linear_forms.py (random weights, launches of a graph, two runs) the choice is then 0.1 to 0.2 % behind the faster side
+// in the mean and 9 % at most, with 1 us more 0.8 and 19 %, with 1 us less 3 and 24 %: the line is steep on one side.  It was
+// drawn on 176 full plans of equal weights (0.3 and 14 %).
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
