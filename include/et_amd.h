@@ -345,7 +345,9 @@ int et_layer_flow_run(et_layer_flow *flow, void *out, const void *in, void *Q, v
  * sequences of at most 128 rows; Q, K and V are not written anywhere.  Plans of d_model x d_model in one column chunk
  * (d_model up to 1024).  Sequences: cu_seqlens (device row offsets of batch + 1, packed rows, each sequence of at most
  * max_len rows) or a padded batch of seq_len rows each (max_len == seq_len) with optional seq_lens (device).  mask,
- * log2_scale as in et_OTF_attention.  out must not overlap X.
+ * log2_scale as in et_OTF_attention.  out must not overlap X.  Not the bits of et_tile_plan_run_multi +
+ * et_OTF_attention: tile pairs are added in another order, and probabilities are rounded to half under their row's
+ * largest score instead of the largest one so far.  As far from the exact result as those.
  * et_qkv_attention_pays: 1 where the form exists and is the one to take (et_tuning_set "qkv_attention"). */
 int et_qkv_attention_pays(const et_tile_plan *q, const et_tile_plan *k, const et_tile_plan *v, int max_len,
                           int d_model, int nheads, int batch);
@@ -568,8 +570,9 @@ int et_device_synchronize(void);
  * A launch that begins after the call has returned sees the value, on any thread.
  * "tile_nb", "tile_min_wgs", "tile_ipw", "tile_form", "tile_bm64", "tile_order",
  * "tile_chunked", "tile_splitk_rows" and "dense_form" may be set while other threads
- * launch; the others may not.  Results never depend on these beyond fp32 summation
- * order. */
+ * launch; the others may not.  Results depend on these by fp32 summation order, and
+ * by the maximum under which attention takes a row's probabilities before it
+ * rounds them to half ("qkv_attention", "layer_flow_rows", "attn_variant"). */
 int et_tuning_set(const char *key, int value);
 /* The fused layer-tail kernels order their waves with bounded waits on LDS
  * counters, the one-launch layer its workgroups with bounded waits on counters
