@@ -222,8 +222,8 @@ extern "C" int et_tile_plan_run_scatter_ln(const et_tile_plan *plan, void *out, 
     a.ldx = a.K + ((a.K & 31) ? 0 : 16); // row stride == 32 (mod 64) bytes: conflict-free
     a.lde = size + 8;
     a.inv_n = 1.0f / (float)size;
-    // 16 rows a workgroup while that is one per CU, then 32, of which two share a CU's registers; with three block-rows a
-    // wave they do not, and beyond a round 64 rows cost less: 16384 x 768 -> 384 29.4 -> 25.3 us, 8224 rows 23.7 -> 19.1
+    // 16 rows a workgroup while that is one per CU, then 32: one per CU up to 8192 rows, beyond them two share its registers;
+    // with three block-rows a wave they do not, and beyond a round 64 rows cost less: 16384 x 768 -> 384 29.4 -> 25.3 us, 8224 rows 23.7 -> 19.1
     // (with two block-rows 16384 rows 21.7 -> 22.1)
     const int nb = (a.nbr + RL_WAVES - 1) / RL_WAVES, cus = std::max(et_device_cu_count(), 1);
     const int ms = M <= 16 * cus ? 1 : M <= 32 * cus || nb < 3 ? 2 : 4;

@@ -3,6 +3,7 @@
 // and per thread can be tested where there is no GPU.  Kernels need the opt-in to more than 64 KB of LDS on each device,
 // and a launch takes a function of its stream's device, as the runtime documents.
 #include <atomic>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -76,7 +77,8 @@ int two_devices_variable_of(int i) {
     return -1;
 }
 // One thread launches the plan again and again while this one sets a key, to two values in turn.  Returns how often a launch
-// that began after the key was set did not have the value's threads a workgroup.
+// that began after the key was set did not have the value's threads a workgroup.  (A few seconds at most: on one processor
+// the two threads hardly meet.)
 int two_devices_race(int (*set)(const char *, int), int (*run)(const void *, void *, const void *, int, int, void *),
                      const void *plan, void *x, int rows, const char *key, const int *values, const unsigned *threads, int times) {
     std::atomic<bool> stop{false};
@@ -86,11 +88,12 @@ int two_devices_race(int (*set)(const char *, int), int (*run)(const void *, voi
             run(plan, x, x, rows, 1, nullptr);
     });
     int wrong = 0;
-    for (int i = 0; i < times; i++) {
+    const auto end = std::chrono::steady_clock::now() + std::chrono::seconds(5);
+    for (int i = 0; i < times && std::chrono::steady_clock::now() < end; i++) {
         set(key, values[i & 1]);
         const int before = done;
         while (done < before + 2) // (the first of them may have begun earlier)
-            ;
+            std::this_thread::yield();
         std::lock_guard<std::mutex> l(lock);
         wrong += latest.block != threads[i & 1];
     }
