@@ -876,6 +876,26 @@ def test_otf_attention_varlen_walks_existing_blocks(K, S, H, d, lens):
     check_close(walked, want[sel], max_abs=5e-3, mean_rel=1e-3, what="varlen attention, walked blocks")
 
 
+@pytest.mark.parametrize("S,H,n,use_mask", [(1024, 12, 1024, False), (200, 12, 199, True), (130, 9, 65, False), (64, 8, 1, False)])
+def test_otf_attention_varlen_one_sequence(K, S, H, n, use_mask):
+    """one packed sequence: more heads than XCDs (some have a pair more than others), as many, and blocks that the
+    sequence does not reach, == one workgroup per possible block == the oracle"""
+    from et_amd._lib import lib
+    r, d = rng(31 + S + H), H * 64
+    Q, Kk, V = (randn_h(r, (n, d)) for _ in range(3))
+    mask = randn_h(r, (S, S), 0.5) if use_mask else None
+    args = (dev(Q), dev(Kk), dev(V), None if mask is None else dev(mask), dev(np.array([0, n], np.int32)), S, H, 1.0)
+    walked = host(K.OTF_attention_varlen(*args))
+    try:
+        lib().et_tuning_set(b"attn_packed", 0)
+        grid = host(K.OTF_attention_varlen(*args))
+    finally:
+        lib().et_tuning_set(b"attn_packed", 1)
+    assert np.array_equal(walked, grid)
+    want = orc.otf_attention(Q, Kk, V, None if mask is None else np.ascontiguousarray(mask[:n, :n]), n, H, 1, None, 1.0, f64=True)
+    check_close(walked, want, max_abs=5e-3, mean_rel=1e-3, what="varlen attention, one sequence")
+
+
 @pytest.mark.parametrize("S,H,lens,walked_by", [
     (80, 16, [80 - (i % 81) for i in range(96)], 128),          # 1536 possible blocks of 128: just over the line; empty ones
     (300, 8, [300, 257, 256, 255, 129, 128, 127, 65, 64, 63, 33, 1, 0] * 5, 128),  # block and tile edges
