@@ -1308,6 +1308,25 @@ def test_tile_linear_multi_of_different_column_chunks(K, M, Kd, Ns, sp):
         check_close(host(o)[rows], want, max_abs=4e-3, mean_rel=5e-4, what=f"multi, {Kd} -> {l['N']}")
 
 
+@pytest.mark.parametrize("M,N", [(4161, 1040), (1024, 5392), (4096, 1152)])
+def test_dense_product_walks_groups_of_tiles(K, M, N):
+    """more blocks of 64 x 128 than the chip holds at once: row tiles (the second size: column tiles) in groups, the last
+    group smaller (66 = 8 x 8 + 2, 43 = 5 x 8 + 3) or not"""
+    from et_amd import lib
+    if lib().et_device_cu_count() != 256:
+        pytest.skip("the group counts the workgroups of 256 compute units")
+    r = rng(91 + M)
+    X, W, b = randn_h(r, (M, 32)), randn_h(r, (N, 32), 0.2), randn_h(r, (N,), 0.2)
+    try:
+        lib().et_tuning_set(b"dense_form", 0)
+        got = host(K.row_spmm_add_bias(dev(X), dev(W), dev(b)))
+    finally:
+        lib().et_tuning_set(b"dense_form", -1)
+    want = X.astype(np.float64) @ W.astype(np.float64).T + b.astype(np.float64)
+    # 32 fp16 products summed in fp32, one rounding to half: half a unit in the last place of up to 8
+    assert np.abs(got.astype(np.float64) - want).max() <= 2.0 ** -11 * max(8.0, np.abs(want).max())
+
+
 @pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("M,Ns,Kd,gelu", [
     (1, (16,), 32, False),               # half a step of 64 columns, one piece of a block
