@@ -202,7 +202,7 @@ def measure(path):
                         keys(plan_dense=1)
                         line("auto+dense", 0)
                         keys(plan_dense=2)
-                        for k in range(6):
+                        for k in range(8):
                             keys(dense_form=k)
                             line(f"dense{k}", 0, dense=True)
                     automatic()

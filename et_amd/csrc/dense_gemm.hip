@@ -4,18 +4,20 @@
 //
 // Both operands are contiguous along K, which is the layout the 16x16x32 MFMA wants for A and for B (8 consecutive k
 // per lane), so neither is transposed.  The product is issued as W X^T so that a lane ends with four consecutive output
-// features of one row.  K is walked in steps of 64 through two or three LDS stages filled by DMA
+// features of one row.  K is walked in steps of 64 through two to six LDS stages filled by DMA
 // (global_load_lds_dwordx4, no registers).  A DMA instruction writes 64 x 16 bytes to consecutive LDS, the source
 // address is free per lane: the 16-byte pieces of a row are stored XOR-swizzled by (row / 2) % 8, which puts the sixteen
 // rows of a fragment read into sixteen different slots of 256 bytes without padding.
 //
-// What bounds it: in the middle of a large K the matrix unit at the clock it gets (256 x 192 blocks on every CU 1.25 us a
-// step, 1.29 PFLOP/s; 0.85 us while half of the CUs have none), at K = 768 the ends: the launch, the first step's
-// latency and the result's way out are 6 of 21 us.  A request occupies its wave while it goes out, and eight in one go
-// behind the barrier kept both waves of a SIMD from the matrix unit: they go out between the products (8192 rows 928 ->
-// 240 9.5 -> 8.1 us, 768 -> 768 15.3 -> 13.9, 2000 rows 768 -> 2304 14.1 -> 12.8, 16384 rows 1024 -> 4096 135 -> 127, 4096 ->
-// 1024 111 -> 106; 3072 -> 768 43.0 -> 42.8 and 768 -> 3072 45.1 -> 42.6).  All figures here are of normally distributed
-// operands: with weights that are all alike the same launches are up to a sixth shorter.
+// What bounds it: in the middle of a large K the way of the operands into LDS and registers - a launch of 8192 x 8192 x 8192
+// whose loop fetches nothing takes three quarters of the time, one that reads no fragments either two thirds, which is the
+// matrix unit at the clock it gets (1.9 PFLOP/s); at K = 768 the ends: the launch, the first step's latency and the result's
+// way out are 6 of 20 us.  A wave issues in order, and a memory instruction holds it until it is out, with both waves of a
+// SIMD at the same place: so nothing goes out in one go, requests and LDS reads stand between the products.  Two stages of 64
+// columns are requested half a step to a step before they are needed, which is a round trip to memory under load: where the
+// LDS has room for more stages, and every CU has one block, they are taken.  (Stages of 32 columns, four to eight of them,
+// are slower: a row's 64 bytes are half a cache line, which is fetched twice.)  All figures here are of normally
+// distributed operands: with weights that are all alike the same launches are up to a sixth shorter.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -53,10 +55,15 @@ __device__ __forceinline__ int dg_swizzle(int r, int kc) { return kc ^ ((r >> 1)
 
 // WM x WN waves of TM x TN MFMA tiles: a block of 16 WM TM rows and 16 WN TN features.  ST stages of 64 columns; a
 // step's second half of fragments is read while the first half multiplies, then the stage is handed back, the step ST
-// later requested into it and the next step's first fragments read while the second half multiplies: fragment reads and
-// the barrier run under MFMAs.
-// us a launch: 8192 rows 768 -> 768 13.9, 768 -> 1536 23.0, 768 -> 3072 42.6, 3072 -> 768 42.8, 928 -> 240 8.1; 16384 rows
-// 1024 -> 4096 127 (1080 TFLOP/s), 4096 -> 1024 106 (1290); 4096 x 4096 x 4096 107 (1280), 8192 x 8192 x 8192 909 (1210).
+// later requested into it and the next step's first fragments read while the second half multiplies: fragment reads,
+// requests and the barrier run under MFMAs.
+// us a launch, with LDS reads and at most three stages' requests in one go or half of a step / as here, in turn on one
+// machine: 8192 rows 768 -> 768 13.0 / 12.8, 768 -> 928 15.6 / 15.6, 768 -> 1536 22.4 / 21.7, 768 -> 3072 42.1 / 42.6, 3072 ->
+// 768 42.3 / 36.2; 2000 rows 768 -> 2304 12.0 / 11.5, 3072 -> 768 17.3 / 16.1; 2003 rows 3072 -> 3072 44.5 / 39.8; 1200 rows 4096
+// -> 1024 21.8 / 19.1; 16384 rows 1024 -> 4096 126.8 / 122.4 (1120 TFLOP/s), 4096 -> 1024 104.8 / 100.3 (1370); 4096 x 4096 x
+// 4096 106.0 / 101.7 (1350), 8192 x 8192 x 8192 838 / 780 (1410).  Of that, as the mean over 60 shapes: reads between the
+// products 256 x 256 6 %, 256 x 192 4 %, else 2 %; requests over the whole step, with three stages and more, 4 to 5 %; the
+// barrier in front of a half's last products 1 to 3 % where a CU has one workgroup.
 template <bool GELU, int WM, int WN, int TM, int TN, int ST>
 __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     // (what the first requests need arrives in registers with the wave)
@@ -163,9 +170,28 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
         for (int j = 0; j < TM; j++)
             xf[H][j] = *reinterpret_cast<const f16x8 *>(s + px[H] + j * 2048);
     };
+    // (LDS reads in one go keep the wave from its products until the last one is out: a half's fragments are read behind the
+    // products of the other half's first OVER row subtiles)
+    constexpr int FRAG = TM + TN, OVER = TM >= 4 ? TM / 2 : TM;
+    auto read_some = [&](int slot, auto half, auto jc) {
+        constexpr int H = decltype(half)::value, j = decltype(jc)::value;
+        const char *s = reinterpret_cast<const char *>(smem) + slot * (STAGE * 2);
+        if constexpr (j < OVER)
+            dg_for<j * FRAG / OVER, (j + 1) * FRAG / OVER>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (i < TN)
+                    wf[H][i] = *reinterpret_cast<const f16x8 *>(s + pw[H] + i * 2048);
+                else
+                    xf[H][i - TN] = *reinterpret_cast<const f16x8 *>(s + px[H] + (i - TN) * 2048);
+            });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // (two workgroups on a CU: the one that multiplies goes first, and it has the other one's work while its waves wait)
+    constexpr bool SHARED = ST * STAGE * 2 <= 80 * 1024;
     auto multiply = [&](auto half, auto &&between) { // between(j): what goes out behind the products of row subtile j
         constexpr int H = decltype(half)::value;
-        __builtin_amdgcn_s_setprio(1);
+        if (SHARED)
+            __builtin_amdgcn_s_setprio(1);
         dg_for<0, TM>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
 #pragma unroll
@@ -173,56 +199,79 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
                 acc[i][j] = mfma16x16x32(wf[H][i], xf[H][j], acc[i][j]);
             between(jc);
         });
-        __builtin_amdgcn_s_setprio(0);
+        if (SHARED)
+            __builtin_amdgcn_s_setprio(0);
     };
     auto nothing = [](auto) {};
     typedef std::integral_constant<int, 0> h0;
     typedef std::integral_constant<int, 1> h1;
     auto barrier = [] { asm volatile("s_barrier" ::: "memory"); };
-    auto landed = [&](int behind) { // all but the youngest `behind` stages have arrived (this wave's part of them)
-        if (behind >= 1 && ST > 2)
-            __builtin_amdgcn_s_waitcnt(0x0070 | (PER & 15) | (PER >> 4 << 14)); // vmcnt(PER) lgkmcnt(0)
-        else
-            __builtin_amdgcn_s_waitcnt(0x0070); // vmcnt(0) lgkmcnt(0)
+    auto landed = [&](auto behind) { // all but the youngest `behind` stages have arrived (this wave's part of them)
+        constexpr int V = decltype(behind)::value * PER;
+        static_assert(V < 64, "what vmcnt counts");
+        __builtin_amdgcn_s_waitcnt(0x0070 | (V & 15) | (V >> 4 << 14)); // vmcnt(V) lgkmcnt(0)
     };
-    static_assert(ST == 2 || ST == 3, "stages");
 #pragma unroll
     for (int t = 0; t < ST - 1; t++)
         if (t < nk)
             fetch(t, t);
-    landed(min(ST - 2, nk - 1));
+    if (nk >= ST - 1)
+        landed(std::integral_constant<int, ST - 2>());
+    else
+        landed(h0());
     barrier();
-    if (ST - 1 < nk)
-        fetch(ST - 1, ST - 1);
-    read(0, h0());
-    int slot = 0;
-    auto step = [&](int kt, auto more) {
-        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the first half's fragments, read a multiplication ago
-        read(slot, h1());
+    // A stage's requests go out between the products as well, while the matrix unit is busy: with more than two stages the
+    // first EARLY of them in the step that frees the place, the others in the first half of the next one.
+    constexpr int EARLY = ST > 2 ? (PER + 1) / 2 : PER;
+    // The barrier that hands a step's stage over stands in front of the first half's last products, so that the matrix unit
+    // has work while the waves wait for each other.  (What is requested in this half goes out before it: it is counted.)
+    constexpr int BEFORE = TM >= 4 && !SHARED ? TM - 1 : TM; // row subtiles in front of the barrier
+    auto request_some = [&](int stage, int slot, auto jc, auto over, auto from, auto to) { // behind the products of row subtile j
+        constexpr int j = decltype(jc)::value, OV = decltype(over)::value, F = decltype(from)::value, N = decltype(to)::value - F;
+        if constexpr (j < OV)
+            dg_for<F + j * N / OV, F + (j + 1) * N / OV>([&](auto which) { request(stage, slot, which); });
         __builtin_amdgcn_sched_barrier(0);
-        multiply(h0(), nothing);
-        // stage kt has been read: wait for the next one, request into this one's place
-        landed(min(ST - 2, nk - 2 - kt));
-        barrier();
-        const int freed = slot;
-        slot = slot == ST - 1 ? 0 : slot + 1;
-        read(slot, h0());
-        __builtin_amdgcn_sched_barrier(0);
-        // (a request occupies the wave while it goes out: between the products, where the matrix unit is busy meanwhile)
-        if constexpr (decltype(more)::value)
-            multiply(h1(), [&](auto jc) {
-                constexpr int j = decltype(jc)::value;
-                dg_for<j * PER / TM, (j + 1) * PER / TM>([&](auto which) { request(kt + ST, freed, which); });
-                __builtin_amdgcn_sched_barrier(0);
-            });
-        else
-            multiply(h1(), nothing);
     };
+    typedef std::integral_constant<int, TM> every_t;
+    typedef std::integral_constant<int, BEFORE> before_t;
+    typedef std::integral_constant<int, 0> none_t;
+    typedef std::integral_constant<int, EARLY> early_t;
+    typedef std::integral_constant<int, PER> all_t;
+    if (ST - 1 < nk)
+        dg_for<0, EARLY>([&](auto which) { request(ST - 1, ST - 1, which); });
+    read(0, h0());
+    int slot = 0, freed = ST - 1;
+    auto step = [&](int kt, auto late, auto early, auto behind) {
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the first half's fragments, read a multiplication ago
+        multiply(h0(), [&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            read_some(slot, h1(), jc);
+            if constexpr (decltype(late)::value && EARLY < PER)
+                request_some(kt - 1 + ST, freed, jc, before_t(), early_t(), all_t());
+            if constexpr (j == BEFORE - 1) { // this wave has the step's fragments and its part of the next stage
+                landed(behind);
+                barrier();
+            }
+        });
+        freed = slot;
+        slot = slot == ST - 1 ? 0 : slot + 1;
+        multiply(h1(), [&](auto jc) {
+            read_some(slot, h0(), jc);
+            if constexpr (decltype(early)::value)
+                request_some(kt + ST, freed, jc, every_t(), none_t(), early_t());
+        });
+    };
+    typedef std::integral_constant<int, ST - 2> steady_t;
     int kt = 0;
     for (; kt < nk - ST; kt++)
-        step(kt, std::true_type());
-    for (; kt < nk - 1; kt++)
-        step(kt, std::false_type());
+        step(kt, std::true_type(), std::true_type(), steady_t());
+    if (kt == nk - ST)
+        step(kt++, std::true_type(), std::false_type(), steady_t());
+    dg_for<0, ST - 2>([&](auto ic) { // everything has been requested
+        constexpr int BEHIND = ST - 3 - decltype(ic)::value;
+        if (nk - 2 - kt == BEHIND)
+            step(kt++, std::false_type(), std::false_type(), std::integral_constant<int, BEHIND>());
+    });
     // (the last step apart: with a branch around the next stage's reads the compiler cannot tell which are in flight behind
     // it, and waits for them before it multiplies)
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -344,16 +393,15 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
 }
 
 // The blocks there are and the time of each form in microseconds, without the launch.  A step takes longer with every
-// further workgroup of a CU and with the share of the CUs that have one; the figures are fits to 385 shapes (128 to 32768
-// rows, 512 to 4096 columns; equal weights), the forms near the fastest weighing most.  On the 80 full plans of
-// bench/linear_forms.py (random weights, two runs) the block they choose is 0.2 to 0.3 % behind the fastest in the mean, 8 %
-// at most (512 -> 512, 9182 rows: 10.1 against 9.4 us), and its estimate with the launch 7 % off; over all blocks, also those
-// that nobody would choose, 12 %.  Small blocks win while they let more CUs take part, large ones where every CU has several;
-// 256 x 192 where one block a CU is all there is (768 -> 1536, 8192 rows: 22.0 against 22.6 us in 128 x 192, 23.8 in 256 x 256).
-enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_256x192, DG_FORMS };
+// further workgroup of a CU and with the share of the CUs that have one; the figures are fits to 260 shapes (1024 to 19000
+// rows, 512 to 4096 columns, random weights), the forms near the fastest weighing most.  On 400 other shapes the block they
+// choose is 0.06 % behind the fastest in the mean, 7 % at most (512 -> 4096, 13421 rows: 72.7 against 68.1 us), and its
+// estimate with 3.0 us for the launch 4 % off.  Small blocks win while they let more CUs take part, large ones where every
+// CU has several; of the small ones those with more stages where a CU has one of them.
+enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_256x192, DG_128x192_DEEP, DG_64x128_DEEP, DG_FORMS };
 static std::atomic<int> g_dense_form{-1}; // et_tuning_set("dense_form"): one of the above, -1 chooses
 static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
-    static const int bm[DG_FORMS] = {64, 128, 128, 128, 256, 256}, bn[DG_FORMS] = {128, 128, 128, 192, 256, 192};
+    static const int bm[DG_FORMS] = {64, 128, 128, 128, 256, 256, 128, 64}, bn[DG_FORMS] = {128, 128, 128, 192, 256, 192, 192, 128};
     struct Form {
         double ends;       // the first step's latency and the way out
         double one, fill1; // a step while no CU has two blocks, per share of CUs that have one
@@ -361,12 +409,14 @@ static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
         double more;       // ... a block
     };
     static const Form forms[DG_FORMS] = {
-        {0.7, 0.23, 0.08, 0.31, 0.16, 0.37}, // two per CU (72 KB)
-        {1.3, 0.24, 0.21, 0.38, 0.25, 0.57}, // two per CU (64 KB)
-        {1.6, 0.25, 0.14, 0.70, 0.19, 0.60}, // one per CU (96 KB)
-        {1.2, 0.41, 0.34, 0.63, 0.36, 0.74}, // two per CU (80 KB)
-        {6.1, 0.67, 0.87, 1.82, 0.73, 1.56}, // one per CU (128 KB)
-        {4.0, 0.68, 0.51, 1.50, 0.66, 1.33}, // one per CU (112 KB)
+        {0.0, 0.245, 0.055, 0.325, 0.119, 0.310}, // two per CU (72 KB)
+        {0.8, 0.274, 0.221, 0.418, 0.254, 0.506}, // two per CU (64 KB)
+        {0.7, 0.274, 0.143, 0.553, 0.220, 0.517}, // one per CU (128 KB)
+        {0.8, 0.351, 0.373, 0.612, 0.385, 0.712}, // two per CU (80 KB)
+        {4.9, 0.652, 0.733, 1.577, 0.788, 1.537}, // one per CU (128 KB)
+        {3.7, 0.537, 0.537, 1.505, 0.448, 1.356}, // one per CU (112 KB)
+        {1.6, 0.276, 0.342, 0.771, 0.299, 0.706}, // one per CU (120 KB)
+        {0.4, 0.212, 0.075, 0.518, 0.062, 0.350}, // one per CU (144 KB)
     };
     const long cus = std::max(et_device_cu_count(), 1);
     long tiles = 0;
@@ -430,10 +480,12 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
     case form_: return gelu ? dg_launch_inst<true, __VA_ARGS__>(a, st) : dg_launch_inst<false, __VA_ARGS__>(a, st);
         DG_CASE(DG_64x128, 2, 4, 2, 2, 3)
         DG_CASE(DG_128x128, 2, 4, 4, 2, 2)
-        DG_CASE(DG_128x128_DEEP, 2, 4, 4, 2, 3)
+        DG_CASE(DG_128x128_DEEP, 2, 4, 4, 2, 4)
         DG_CASE(DG_128x192, 2, 4, 4, 3, 2)
         DG_CASE(DG_256x256, 2, 4, 8, 4, 2)
         DG_CASE(DG_256x192, 2, 4, 8, 3, 2)
+        DG_CASE(DG_128x192_DEEP, 2, 4, 4, 3, 3)
+        DG_CASE(DG_64x128_DEEP, 2, 4, 2, 2, 6)
 #undef DG_CASE
     }
     return ET_ERR_UNSUPPORTED;

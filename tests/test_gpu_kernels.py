@@ -1308,6 +1308,24 @@ def test_tile_linear_multi_of_different_column_chunks(K, M, Kd, Ns, sp):
         check_close(host(o)[rows], want, max_abs=4e-3, mean_rel=5e-4, what=f"multi, {Kd} -> {l['N']}")
 
 
+@pytest.mark.parametrize("form", range(8))
+def test_dense_product_stages(K, form):
+    """every block size, from fewer steps of 64 columns than stages (two to six) to more, whole and half last steps"""
+    from et_amd import lib
+    r = rng(90)
+    M, N = 1025, 400
+    try:
+        lib().et_tuning_set(b"dense_form", form)
+        for Kd in (32, 64, 96, 128, 160, 192, 224, 256, 320, 384, 416, 448, 512, 608):
+            X, W, b = randn_h(r, (M, Kd)), randn_h(r, (N, Kd), Kd ** -0.5), randn_h(r, (N,), 0.2)
+            got = host(K.row_spmm_add_bias(dev(X), dev(W), dev(b)))
+            want = X.astype(np.float64) @ W.astype(np.float64).T + b.astype(np.float64)
+            # fp16 products summed in fp32, one rounding to half: half a unit in the last place of up to 8
+            assert np.abs(got.astype(np.float64) - want).max() <= 2.0 ** -11 * max(8.0, np.abs(want).max()), Kd
+    finally:
+        lib().et_tuning_set(b"dense_form", -1)
+
+
 @pytest.mark.parametrize("M,N", [(4161, 1040), (1024, 5392), (4096, 1152)])
 def test_dense_product_walks_groups_of_tiles(K, M, N):
     """more blocks of 64 x 128 than the chip holds at once: row tiles (the second size: column tiles) in groups, the last
