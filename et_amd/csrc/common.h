@@ -125,6 +125,31 @@ __device__ __forceinline__ float wave_sum(float v) {
     return (r0 + r1) + (r2 + r3);
 }
 
+// A row in 32 lanes: `lo` is what lanes 0..31 of a whole wave would hold, `hi` what lanes 32..63 would; the sum of each half
+// of the wave to its lanes, in the order of wave_sum.
+__device__ __forceinline__ float half_wave_sum(float lo, float hi) {
+    float v[2] = {lo, hi};
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        v[i] += dpp_move<0xB1>(v[i]);
+        v[i] += dpp_move<0x4E>(v[i]);
+        v[i] += dpp_move<0x141>(v[i]);
+        v[i] += dpp_move<0x140>(v[i]);
+    }
+    // rows of 16 lanes: (lo 0, lo 1) and (hi 0, hi 1) -> (lo 0, hi 0) and (lo 1, hi 1)
+    // (the additions are written out: the compiler takes the two results of a swap that meet in one for equal)
+    auto swap_add = [](unsigned x, unsigned y) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        unsigned t = r[0];
+        asm("v_add_f32 %0, %0, %1" : "+v"(t) : "v"(r[1]));
+        return t;
+    };
+    const unsigned s = swap_add(__builtin_bit_cast(unsigned, v[0]), __builtin_bit_cast(unsigned, v[1]));
+    unsigned t = s;
+    asm("" : "+v"(t));
+    return __builtin_bit_cast(float, swap_add(s, t));
+}
+
 // GELU of four halves: x^3 in (packed) half, the sigmoid form of
 // 0.5(1+tanh u) = 1/(1+exp(-2u)) in fp32, rounded to half, times x in half
 // (kernels/linear.cu:36-48).

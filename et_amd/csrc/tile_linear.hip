@@ -502,35 +502,48 @@ __device__ __forceinline__ void tl_flush_acc_branch(f32x4 (&acc)[NB][2], int j, 
 // math of skip_layernorm.hip: x = half(y + skip), fp32 mean and biased
 // two-pass variance, eps 1e-6).  The workgroup covers the whole row: wave k's
 // staging tile holds columns [k*16*NB, (k+1)*16*NB), k < NW.  Wave w of the NLW
-// waves that take part normalises rows w, w+NLW, ..., a row spread over its 64
-// lanes in 16-byte pieces.  The operands that come from global memory (the
+// waves that take part normalises rows w, w+NLW, ..., two at a time, each spread
+// over 32 lanes in 16-byte pieces (rows wider than 1024: one over 64, for the
+// registers).  A row of 768 is one and a half pieces for 64 lanes and three for
+// 32, and two rows share the sums' exchanges: 140 vector instructions a wave and
+// LayerNorm fewer than row after row, and the layer tail keeps its registers out of
+// memory.  Whole layers of 16 x 512 rows 83.2 -> 78.1 us, with pruned values 83.1 ->
+// 80.0, the stack of 64 ragged sequences 2277 -> 2219.  The operands that come from global memory (the
 // skip rows, gamma, beta) are requested by tl_ln_fetch, which a wave calls
 // BEFORE the barrier that ends the staging writes, so that their latency runs
 // under the wait for the other waves.
 template <int NB, int NW, int NLW>
 struct TlLnOperands {
-    static constexpr int NCH = (NW * NB * 2 + 63) / 64;    // 16-byte pieces per lane and row
-    static constexpr int ROWS = (TL_BM + NLW - 1) / NLW;   // rows per wave
-    f16x8 skip[ROWS][NCH], gamma[NCH], beta[NCH];
+    static constexpr int LPR = NW * NB > 64 ? 64 : 32;                         // lanes per row
+    static constexpr int NP = (NW * NB * 2 + LPR - 1) / LPR;                   // 16-byte pieces per lane
+    static constexpr int STEPS = ((TL_BM + NLW - 1) / NLW * LPR + 63) / 64;    // rows, or pairs of them, per wave
+    f16x8 skip[STEPS][NP], gamma[NP], beta[NP];
 };
 
 // (skip0 / Y0 point at the panel's first row, in global memory or in LDS, with
 // row pitches ldskip / ldy in halves)
 template <int NB, int NW, int NLW>
-__device__ __forceinline__ void tl_ln_fetch_at(TlLnOperands<NB, NW, NLW> &op, int M, int wave, int lane,
-                                               int m0, int N, const f16 *skip0, long ldskip,
-                                               const f16 *gamma, const f16 *beta) {
-    constexpr int NCH = TlLnOperands<NB, NW, NLW>::NCH;
-    constexpr int ROWS = TlLnOperands<NB, NW, NLW>::ROWS;
-    const int npiece = N >> 3;
+__device__ __forceinline__ void tl_ln_fetch_skip(TlLnOperands<NB, NW, NLW> &op, int M, int wave, int lane,
+                                                 int m0, int N, const f16 *skip0, long ldskip) {
+    typedef TlLnOperands<NB, NW, NLW> Op;
 #pragma unroll
-    for (int i = 0; i < NCH; i++) {
-        const int ch = min(lane + 64 * i, npiece - 1); // (clamped pieces are never used)
+    for (int i = 0; i < Op::NP; i++) {
+        const int ch = min((lane & (Op::LPR - 1)) + Op::LPR * i, (N >> 3) - 1); // (clamped pieces are never used)
 #pragma unroll
-        for (int k = 0; k < ROWS; k++) {
-            const long r = min((long)wave + k * NLW, (long)M - 1 - m0);
+        for (int k = 0; k < Op::STEPS; k++) {
+            const long r = min(wave + (64 / Op::LPR * k + lane / Op::LPR) * NLW, min(TL_BM, M - m0) - 1);
             op.skip[k][i] = *reinterpret_cast<const f16x8 *>(skip0 + r * ldskip + ch * 8);
         }
+    }
+}
+// (behind the epilogue: its accumulators' registers are free then)
+template <int NB, int NW, int NLW>
+__device__ __forceinline__ void tl_ln_fetch_scale(TlLnOperands<NB, NW, NLW> &op, int lane, int N, const f16 *gamma,
+                                                  const f16 *beta) {
+#pragma unroll
+    for (int i = 0; i < TlLnOperands<NB, NW, NLW>::NP; i++) {
+        constexpr int LPR = TlLnOperands<NB, NW, NLW>::LPR;
+        const int ch = min((lane & (LPR - 1)) + LPR * i, (N >> 3) - 1);
         op.gamma[i] = *reinterpret_cast<const f16x8 *>(gamma + ch * 8);
         op.beta[i] = *reinterpret_cast<const f16x8 *>(beta + ch * 8);
     }
@@ -539,7 +552,8 @@ __device__ __forceinline__ void tl_ln_fetch_at(TlLnOperands<NB, NW, NLW> &op, in
 template <int NB, int NW, int NLW>
 __device__ __forceinline__ void tl_ln_fetch(TlLnOperands<NB, NW, NLW> &op, const TlArgs &a, int wave,
                                             int lane, int m0, int N) {
-    tl_ln_fetch_at(op, a.M, wave, lane, m0, N, a.skip + (long)m0 * N, (long)N, a.gamma, a.beta);
+    tl_ln_fetch_skip(op, a.M, wave, lane, m0, N, a.skip + (long)m0 * N, (long)N);
+    tl_ln_fetch_scale(op, lane, N, a.gamma, a.beta);
 }
 
 template <int NB, int NW, int NLW>
@@ -558,58 +572,59 @@ __device__ __forceinline__ void tl_ln_rows_at(const TlLnOperands<NB, NW, NLW> &o
                                               const f16 *stage0, int wave, int lane, int m0, int N,
                                               f16 *Y0, long ldy) {
     constexpr int lds = 16 * NB + 8;
-    constexpr int NCH = TlLnOperands<NB, NW, NLW>::NCH;
-    constexpr int ROWS = TlLnOperands<NB, NW, NLW>::ROWS;
+    typedef TlLnOperands<NB, NW, NLW> Op;
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    constexpr int LPR = Op::LPR, HALF = LPR == 32;
     const int npiece = N >> 3;
     const float inv_n = 1.0f / (float)N;
-    const f16x8 zero8 = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    auto row_sum = [](const float (&v)[2]) { return LPR == 32 ? half_wave_sum(v[0], v[1]) : wave_sum(v[0]); };
+    // (a half times 1.0 plus a float is one instruction; the multiplier is opaque, or it is a conversion and an addition)
+    float one = 1.0f;
+    asm("" : "+s"(one));
 #pragma unroll
-    for (int k = 0; k < ROWS; k++) {
-        const int r = wave + k * NLW;
-        if (r >= TL_BM || m0 + r >= M)
+    for (int k = 0; k < Op::STEPS; k++) {
+        if (m0 + wave + 64 / LPR * k * NLW >= M) // (wave-uniform)
             break;
-        f16x8 xv[NCH];
-        float sum = 0.f;
+        const int r = wave + (64 / LPR * k + lane / LPR) * NLW, rc = min(r, TL_BM - 1);
+        f16x8 xv[Op::NP];
+        // (32 lanes: the sums of the pieces that a whole wave would hold in lanes 0..31 and in lanes 32..63 are kept apart,
+        // since skip_layernorm.hip adds in that order)
+        float sum[2] = {0.f, 0.f}, var[2] = {0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < NCH; i++) {
-            const int ch = lane + 64 * i;
-            xv[i] = zero8;
-            if (ch < npiece) {
-                const int tile = ch / (2 * NB), c = ch - tile * (2 * NB);
-                const f16x8 y = *reinterpret_cast<const f16x8 *>(
-                    stage0 + tile * tl_wave_stage_halves<NB>() + r * lds + c * 8);
-                xv[i] = y + op.skip[k][i]; // half add, one rounding (kernels/skip_layernorm.cu:20)
-            }
+        for (int i = 0; i < Op::NP; i++) {
+            const int ch = (lane & (LPR - 1)) + LPR * i;
+            const int tile = ch / (2 * NB), c = ch - tile * (2 * NB);
+            xv[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            if (ch < npiece)
+                xv[i] = *reinterpret_cast<const f16x8 *>(stage0 + tile * tl_wave_stage_halves<NB>() + rc * lds + c * 8) +
+                        op.skip[k][i]; // half add, one rounding (kernels/skip_layernorm.cu:20)
             // (pairs of halves summed in fp32 by the dot-product unit: no conversions)
-            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 #pragma unroll
             for (int j = 0; j < 8; j += 2)
-                sum = __builtin_amdgcn_fdot2(h2{xv[i][j], xv[i][j + 1]}, h2{(f16)1, (f16)1}, sum, false);
+                sum[i & HALF] = __builtin_amdgcn_fdot2(h2{xv[i][j], xv[i][j + 1]}, h2{(f16)1, (f16)1}, sum[i & HALF], false);
         }
-        const float mean = wave_sum(sum) * inv_n;
-        float var = 0.f;
+        const float mean = row_sum(sum) * inv_n;
 #pragma unroll
-        for (int i = 0; i < NCH; i++)
-            if (lane + 64 * i < npiece) {
+        for (int i = 0; i < Op::NP; i++)
+            if ((lane & (LPR - 1)) + LPR * i < npiece) {
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
-                    const float d = (float)xv[i][j] - mean;
-                    var += d * d;
+                    const float d = __builtin_fmaf((float)xv[i][j], one, -mean);
+                    var[i & HALF] += d * d;
                 }
             }
-        const float rstd = rsqrtf(wave_sum(var) * inv_n + 1e-6f);
+        const float rstd = __builtin_amdgcn_rsqf(row_sum(var) * inv_n + 1e-6f); // (never a denormal)
         const float shift = -mean * rstd;
+        const bool store = r < min(TL_BM, M - m0);
 #pragma unroll
-        for (int i = 0; i < NCH; i++) {
-            const int ch = lane + 64 * i;
-            if (ch < npiece) {
-                f16x8 o;
+        for (int i = 0; i < Op::NP; i++) {
+            const int ch = (lane & (LPR - 1)) + LPR * i;
+            f16x8 o;
 #pragma unroll
-                for (int j = 0; j < 8; j++) // ((x - mean) * rstd) * gamma + beta, the first step as one fma
-                    o[j] = (f16)(__builtin_fmaf((float)xv[i][j], rstd, shift) * (float)op.gamma[i][j] +
-                                 (float)op.beta[i][j]);
+            for (int j = 0; j < 8; j++) // ((x - mean) * rstd) * gamma + beta, the first step as one fma
+                o[j] = (f16)(__builtin_fmaf((float)xv[i][j], rstd, shift) * (float)op.gamma[i][j] + (float)op.beta[i][j]);
+            if (store && ch < npiece)
                 *reinterpret_cast<f16x8 *>(Y0 + r * ldy + ch * 8) = o;
-            }
         }
     }
 }
@@ -1330,7 +1345,7 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
         }
         TL_FFN_PRELOAD(data1, poff1, boundsF, wA, oA)
         TlLnOperands<NB, NW, NW> lnop1; // (requested here: their latency runs under the wait for the other waves)
-        tl_ln_fetch_at(lnop1, a.M, wave, lane, x.m0, NO, a.skip + (long)x.m0 * NO, (long)NO, a.gamma, a.beta);
+        tl_ln_fetch_skip(lnop1, a.M, wave, lane, x.m0, NO, a.skip + (long)x.m0 * NO, (long)NO);
         // staging tiles in the hidden buffers, which nobody uses yet
         tl_epilogue_wave<NB, false, false>(a, x, hs + wave * tl_wave_stage_halves<NB>(), nullptr, NO, nbrO, acc,
                                            bO);
@@ -1339,6 +1354,7 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
             acc[j][0] = f32x4{0.f, 0.f, 0.f, 0.f};
             acc[j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
+        tl_ln_fetch_scale(lnop1, lane, NO, a.gamma, a.beta);
         tl_barrier_lds(); // every wave's part is staged, and everyone has left the attention panel
         tl_ln_rows_at(lnop1, a.M, hs, wave, lane, x.m0, NO, xs, (long)ldx);
     } else {
@@ -1384,10 +1400,12 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
     // output rows -> staging tiles over the (now unused) panel and hidden
     // buffers, then skip connection + LayerNorm over whole rows
     TlLnOperands<NB, NW, NW> lnop;
-    if constexpr (WITH_O) // the skip operand is the panel in LDS
-        tl_ln_fetch_at(lnop, a.M, wave, lane, x.m0, N2, xs, (long)ldx, a.gamma2, a.beta2);
-    else
+    if constexpr (WITH_O) { // the skip operand is the panel in LDS
+        tl_ln_fetch_skip(lnop, a.M, wave, lane, x.m0, N2, xs, (long)ldx);
+        tl_ln_fetch_scale(lnop, lane, N2, a.gamma2, a.beta2);
+    } else {
         tl_ln_fetch(lnop, a, wave, lane, x.m0, N2);
+    }
     f16x4 b2[NB];
 #pragma unroll
     for (int j = 0; j < NB; j++) {

@@ -198,6 +198,31 @@ def test_tile_linear_fused_skip_layernorm(K, M, N, Kd, sp):
         assert (inplace != got).mean() < 0.02
 
 
+@pytest.mark.parametrize("M,N", [(1, 16), (16, 240), (17, 272), (31, 512), (47, 768), (33, 784), (32, 1024), (49, 1040), (18, 1536)])
+def test_tile_linear_layernorm_rows_in_pairs(K, M, N):
+    """the LayerNorm behind a linear has the bits of skip_layernorm, whichever lanes hold the row: one tile per block-row, so
+    that the linear's sums do not depend on its form"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile
+    r = rng(7100 + M + N)
+    lin = make_tile_linear(r, N, 16, 0.0, seed=M + N, std=0.3, bias_std=0.2)
+    X, skip = dev(randn_h(r, (M, 16))), randn_h(r, (M, N))
+    g, b = dev(randn_h(r, (N,), 0.3) + np.float16(1)), dev(randn_h(r, (N,), 0.3))
+    lt = Linear_tile(16, N, M, lin["row_offset"].size, lin["data"], lin["row_ptr"], lin["row_offset"], lin["bias"], False)
+    want = lt.run(X)
+    K.skip_layernorm(want, dev(skip), g, b)
+    try:
+        lib().et_tuning_set(b"tile_ln_min_panels", 1)
+        lib().et_tuning_set(b"plan_dense", 0)
+        got = host(lt.run_ln(X, dev(skip), g, b))
+        sk = dev(skip)
+        lt.run_ln(X, sk, g, b, out=sk)
+    finally:
+        lib().et_tuning_set(b"tile_ln_min_panels", 0)
+        lib().et_tuning_set(b"plan_dense", 1)
+    assert np.array_equal(got, host(want)) and np.array_equal(host(sk), got)
+
+
 FFN_CASES = [
     # M, d (in = out), hidden, sparsity, fused kernel expected
     (128, 768, 3072, 0.8, True),    # BERT-base block: four hidden chunks of 768
