@@ -24,9 +24,8 @@ PANEL = ((512, (512,), 0), (512, (2048,), 1), (768, (768,), 0), (768, (768, 768,
 CHUNKS = ((2048, (512,), 0), (3072, (768,), 0), (4096, (1024,), 0))
 SPARSITIES = (0.0, 0.5, 0.8, 0.9)
 FORMS = ((32, 8, 1), (32, 8, 2), (32, 8, 3), (64, 12, 2), (64, 8, 3), (64, 8, 2), (64, 8, 1))  # rows, waves, block-rows
-DENSE_LAUNCH = 2.6  # us that the library adds to the dense product's estimate when it is weighed against the tile kernels
-LAUNCH = 2.4        # ... of which so many are the launch, which the dense product's estimate leaves out
-TILES_SHARE = 0.9   # ... of whose estimate it takes this much
+DENSE_LAUNCH = 3.5  # us that the library adds to the dense product's estimate when it is weighed against the tile kernels
+LAUNCH = 3.0        # ... of which so many are the launch, which the dense product's estimate leaves out
 TERMS = {  # kernel -> its cost terms, in the order of features()
     "32 rows": "launch traffic traffic_over round item item_nb item_stream panel out gelu mfma result wg".split(),
     "64 rows": "launch traffic traffic_over round item item_nb item_stream panel out gelu mfma result wg".split(),
@@ -202,7 +201,7 @@ def measure(path):
                         keys(plan_dense=1)
                         line("auto+dense", 0)
                         keys(plan_dense=2)
-                        for k in range(8):
+                        for k in range(11):
                             keys(dense_form=k)
                             line(f"dense{k}", 0, dense=True)
                     automatic()
@@ -276,8 +275,8 @@ def report(lines):
             elif l["form"].startswith("dense"):
                 if l["est"] < b.get("est_dense", 1e30):
                     b["est_dense"], b["dense"] = l["est"], l["us"]
-    for extra in (DENSE_LAUNCH - 1, DENSE_LAUNCH, DENSE_LAUNCH + 1):
-        lost = [(b["dense"] if extra + b["est_dense"] < TILES_SHARE * b["est_tiles"] else b["tiles"]) / min(b["dense"], b["tiles"]) - 1
+    for extra in (DENSE_LAUNCH - 0.3, DENSE_LAUNCH, DENSE_LAUNCH + 0.3):
+        lost = [(b["dense"] if extra + b["est_dense"] < b["est_tiles"] else b["tiles"]) / min(b["dense"], b["tiles"]) - 1
                 for b in both.values() if "est_dense" in b]
         if lost:
             print(f"full plans, {extra:.1f} us on top of the dense product's estimate: {100 * sum(lost) / len(lost):.1f} % behind the "

@@ -4,7 +4,7 @@
 //
 // Both operands are contiguous along K, which is the layout the 16x16x32 MFMA wants for A and for B (8 consecutive k
 // per lane), so neither is transposed.  The product is issued as W X^T so that a lane ends with four consecutive output
-// features of one row.  K is walked in steps of 64 through two to six LDS stages filled by DMA
+// features of one row.  K is walked in steps of 64 through two to twelve LDS stages filled by DMA
 // (global_load_lds_dwordx4, no registers).  A DMA instruction writes 64 x 16 bytes to consecutive LDS, the source
 // address is free per lane: the 16-byte pieces of a row are stored XOR-swizzled by (row / 2) % 8, which puts the sixteen
 // rows of a fragment read into sixteen different slots of 256 bytes without padding.
@@ -286,7 +286,7 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     // acc[i][j][r] = Y[row = m0 + wm*16*TM + j*16 + c16][col = n0 + wn*16*TN + i*16 + g4*4 + r]
     // -> the wave's rows in LDS, 64 at a time ([row][16 TN halves + 8]), then 16-byte stores
     constexpr int LDO = 16 * TN + 8, CH = 2 * TN; // 16-byte pieces per row
-    constexpr int TR = TM < 4 ? TM : 4;           // row subtiles per pass
+    constexpr int TR = TM < 4 ? TM : TM % 4 == 0 ? 4 : 3; // row subtiles per pass
     static_assert(TM % TR == 0 && (size_t)NW * TR * 16 * LDO <= ST * (size_t)STAGE, "the output staging fits the stages");
     f16 *os = smem + wave * TR * 16 * LDO;
     f32x4 bf[TN];
@@ -313,9 +313,11 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         // (the staging block is the wave's own: LDS operations of one wave execute in order)
 #pragma unroll
-        for (int t = 0; t < TR * 16 * CH / 64; t++) {
+        for (int t = 0; t < (TR * 16 * CH + 63) / 64; t++) {
             const int q = t * 64 + lane, r = q / CH, pc = q % CH;
             const int row = m0 + wm * TM * 16 + p * TR * 16 + r, col = n0 + wn * TN * 16 + pc * 8;
+            if (TR * 16 * CH % 64 != 0 && r >= TR * 16) // (three subtiles of three: the last pieces are half a wave's)
+                continue;
             if (row < a.M && col < N) // N is a multiple of 16: a piece is inside or outside as a whole
                 *reinterpret_cast<u32x4 *>(Y + (size_t)row * N + col) = *reinterpret_cast<const u32x4 *>(os + r * LDO + pc * 8);
         }
@@ -342,7 +344,7 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 
 // How many row tiles (or column tiles, whichever the launch has as its outer ones) are walked together.  What an XCD's
 // workgroups fetch at the same time should be few tiles: a block of rows x columns of them, not one row.  Best of 1, 2, 4 ..
-// 16 by what the blocks at work take in per step; it is the group measured best for all block sizes but 256 x 192 (1 to 4
+// 16 by what the blocks at work take in per step; it is the group measured best for the blocks of 64 x 128 to 256 x 256 (1 to 4
 // within 2 %).  8192 x 8192 x 8192 931 -> 863 us (64 x 128 blocks 2370 -> 1240, 128 x 192 1190 -> 930), 2003 rows 3072 -> 3072
 // 46.4 -> 44.6, 16384 rows 1024 -> 4096 128.8 -> 126.7.  Not where all blocks are at work at once: 2000 rows 768 -> 2304 (192
 // blocks) took 12.5 us instead of 12.0.
@@ -393,30 +395,44 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
 }
 
 // The blocks there are and the time of each form in microseconds, without the launch.  A step takes longer with every
-// further workgroup of a CU and with the share of the CUs that have one; the figures are fits to 260 shapes (1024 to 19000
-// rows, 512 to 4096 columns, random weights), the forms near the fastest weighing most.  On 400 other shapes the block they
-// choose is 0.06 % behind the fastest in the mean, 7 % at most (512 -> 4096, 13421 rows: 72.7 against 68.1 us), and its
-// estimate with 3.0 us for the launch 4 % off.  Small blocks win while they let more CUs take part, large ones where every
-// CU has several; of the small ones those with more stages where a CU has one of them.
-enum { DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_256x192, DG_128x192_DEEP, DG_64x128_DEEP, DG_FORMS };
+// further workgroup of a CU and with the share of the CUs that have one; the figures are fits to 860 shapes (150 to 18000
+// rows, 512 to 4096 columns, random weights, a quarter of them with GELU), the forms near the fastest weighing most.  Fitted
+// to one half, the block they choose for the other is 0.2 % behind the fastest in the mean, 17 % at most (512 -> 768, 5453
+// rows: 10.6 against 9.0 us), and its estimate with 3.0 us for the launch 3 % off.  What decides is how many bytes of X and
+// W the busiest CU takes in, at about 100 GB/s by DMA, and that no CU has a block more than the others: small blocks win
+// while they let more CUs take part, large ones where every CU has several, and of those near in size the one whose count
+// fills its last round.  (Blocks of 192 x 192 were the shorter launch for some hundred of 860 shapes, by 2 %; 6144 rows
+// 768 -> 3072 inside a layer took 5 us more.)  The blocks of 32 to 96 rows x 64 or 96 and of 192 x 256 against the others alone, us: 3072
+// -> 768 512 rows 14.8 / 11.0, 1024 16.3 / 12.9, 2000 16.3 / 15.3, 3000 20.6 / 18.2; 4096 -> 1024 512 rows 18.9 / 14.2, 1024
+// 19.7 / 16.5; 2048 -> 512 1200 rows 10.8 / 8.9; 1024 -> 4096 3000 rows 30.3 / 27.4, 6000 57.0 / 50.9; 512 -> 2048 6000 rows
+// 20.2 / 18.0; the 640 shapes without GELU 10.5 % in the geometric mean.
+enum {
+    DG_64x128 = 0, DG_128x128, DG_128x128_DEEP, DG_128x192, DG_256x256, DG_192x256, DG_128x192_DEEP, DG_64x64, DG_32x64,
+    DG_96x64, DG_96x96, DG_FORMS
+};
 static std::atomic<int> g_dense_form{-1}; // et_tuning_set("dense_form"): one of the above, -1 chooses
-static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
-    static const int bm[DG_FORMS] = {64, 128, 128, 128, 256, 256, 128, 64}, bn[DG_FORMS] = {128, 128, 128, 192, 256, 192, 192, 128};
+static double dg_estimate(int form, const int *Ns, int nlin, int M, int K, bool gelu) {
+    static const int bm[DG_FORMS] = {64, 128, 128, 128, 256, 192, 128, 64, 32, 96, 96};
+    static const int bn[DG_FORMS] = {128, 128, 128, 192, 256, 256, 192, 64, 64, 64, 96};
     struct Form {
-        double ends;       // the first step's latency and the way out
-        double one, fill1; // a step while no CU has two blocks, per share of CUs that have one
-        double two, fill2; // ... while none has three
-        double more;       // ... a block
+        double ends;        // the first step's latency and the way out
+        double one, fill1;  // a step while no CU has two blocks, per share of CUs that have one
+        double two, fill2;  // ... while none has three
+        double more, fill3; // ... a block, per block that the CUs have in the mean
+        double gelu;        // of 128 x 128 results
     };
     static const Form forms[DG_FORMS] = {
-        {0.0, 0.245, 0.055, 0.325, 0.119, 0.310}, // two per CU (72 KB)
-        {0.8, 0.274, 0.221, 0.418, 0.254, 0.506}, // two per CU (64 KB)
-        {0.7, 0.274, 0.143, 0.553, 0.220, 0.517}, // one per CU (128 KB)
-        {0.8, 0.351, 0.373, 0.612, 0.385, 0.712}, // two per CU (80 KB)
-        {4.9, 0.652, 0.733, 1.577, 0.788, 1.537}, // one per CU (128 KB)
-        {3.7, 0.537, 0.537, 1.505, 0.448, 1.356}, // one per CU (112 KB)
-        {1.6, 0.276, 0.342, 0.771, 0.299, 0.706}, // one per CU (120 KB)
-        {0.4, 0.212, 0.075, 0.518, 0.062, 0.350}, // one per CU (144 KB)
+        {0.118, 0.226, 0.091, 0.541, 0.072, 0.238, 0.144, 1.165}, // one per CU (144 KB)
+        {0.918, 0.279, 0.234, 0.323, 0.338, 0.292, 0.275, 0.827}, // two per CU (64 KB)
+        {0.708, 0.269, 0.189, 0.682, 0.186, 0.237, 0.372, 1.096}, // one per CU (128 KB)
+        {1.425, 0.303, 0.494, 0.579, 0.441, 0.429, 0.352, 0.745}, // two per CU (80 KB)
+        {5.481, 0.677, 0.784, 1.777, 0.821, 1.479, 0.301, 0.890}, // one per CU (128 KB)
+        {4.006, 0.535, 0.631, 1.451, 0.617, 0.759, 0.735, 0.859}, // one per CU (112 KB)
+        {1.758, 0.294, 0.361, 0.778, 0.344, 0.415, 0.418, 1.088}, // one per CU (120 KB)
+        {0.000, 0.166, 0.049, 0.425, 0.037, 0.135, 0.136, 0.619}, // one per CU (128 KB)
+        {0.000, 0.133, 0.034, 0.332, 0.035, 0.151, 0.067, 0.037}, // one per CU (144 KB)
+        {0.041, 0.211, 0.056, 0.532, 0.012, 0.189, 0.122, 1.351}, // one per CU (140 KB)
+        {0.401, 0.250, 0.082, 0.551, 0.082, 0.134, 0.286, 1.423}, // one per CU (144 KB)
     };
     const long cus = std::max(et_device_cu_count(), 1);
     long tiles = 0;
@@ -426,13 +442,13 @@ static double dg_estimate(int form, const int *Ns, int nlin, int M, int K) {
     const Form &f = forms[form];
     const long n = (tiles + cus - 1) / cus; // blocks of the busiest CU
     const double fill = (double)tiles / (double)cus;
-    const double step = n <= 1 ? f.one + f.fill1 * fill : n <= 2 ? f.two + f.fill2 * fill : f.more * (double)n;
-    return f.ends + step * ((K + DG_BK - 1) / DG_BK);
+    const double step = n <= 1 ? f.one + f.fill1 * fill : n <= 2 ? f.two + f.fill2 * fill : f.more * (double)n + f.fill3 * fill;
+    return f.ends + step * ((K + DG_BK - 1) / DG_BK) + (gelu ? f.gelu * (double)n * bm[form] * bn[form] / 16384.0 : 0.0);
 }
-static int dg_choose(const int *Ns, int nlin, int M, int K, double *us) {
+static int dg_choose(const int *Ns, int nlin, int M, int K, bool gelu, double *us) {
     int best = 0;
     for (int f = 0; f < DG_FORMS; f++) {
-        const double t = dg_estimate(f, Ns, nlin, M, K);
+        const double t = dg_estimate(f, Ns, nlin, M, K, gelu);
         if (f == 0 || t < *us) {
             *us = t;
             best = f;
@@ -440,12 +456,12 @@ static int dg_choose(const int *Ns, int nlin, int M, int K, double *us) {
     }
     return best;
 }
-double dense_gemm_estimate(const int *Ns, int nlin, int M, int K) {
+double dense_gemm_estimate(const int *Ns, int nlin, int M, int K, bool gelu) {
     double us = 0.0;
     const int set = g_dense_form;
     if (set >= 0)
-        return dg_estimate(set, Ns, nlin, M, K);
-    dg_choose(Ns, nlin, M, K, &us);
+        return dg_estimate(set, Ns, nlin, M, K, gelu);
+    dg_choose(Ns, nlin, M, K, gelu, &us);
     return us;
 }
 void set_dense_form(int v) { g_dense_form = v < DG_FORMS ? v : -1; }
@@ -474,18 +490,22 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
     a.M = M;
     a.K = K;
     double us;
-    const int set = g_dense_form, form = set >= 0 ? set : dg_choose(Ns, nlin, M, K, &us);
+    const int set = g_dense_form, form = set >= 0 ? set : dg_choose(Ns, nlin, M, K, gelu, &us);
     switch (form) {
 #define DG_CASE(form_, ...)                                                                                            \
     case form_: return gelu ? dg_launch_inst<true, __VA_ARGS__>(a, st) : dg_launch_inst<false, __VA_ARGS__>(a, st);
-        DG_CASE(DG_64x128, 2, 4, 2, 2, 3)
+        DG_CASE(DG_64x128, 2, 4, 2, 2, 6)
         DG_CASE(DG_128x128, 2, 4, 4, 2, 2)
         DG_CASE(DG_128x128_DEEP, 2, 4, 4, 2, 4)
         DG_CASE(DG_128x192, 2, 4, 4, 3, 2)
         DG_CASE(DG_256x256, 2, 4, 8, 4, 2)
-        DG_CASE(DG_256x192, 2, 4, 8, 3, 2)
         DG_CASE(DG_128x192_DEEP, 2, 4, 4, 3, 3)
-        DG_CASE(DG_64x128_DEEP, 2, 4, 2, 2, 6)
+        // (four waves: a block of 64 x 64 in eight is 3 % slower, its waves read more fragments for a product)
+        DG_CASE(DG_64x64, 2, 2, 2, 2, 8)
+        DG_CASE(DG_32x64, 2, 2, 1, 2, 12)
+        DG_CASE(DG_96x64, 2, 2, 3, 2, 7)
+        DG_CASE(DG_96x96, 2, 2, 3, 3, 6)
+        DG_CASE(DG_192x256, 2, 4, 6, 4, 2)
 #undef DG_CASE
     }
     return ET_ERR_UNSUPPORTED;

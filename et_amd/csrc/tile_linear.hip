@@ -2317,16 +2317,17 @@ namespace et {
 // dense_gemm.hip
 int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, const void *const *biases,
                       const int *Ns, int nlin, int M, int K, bool gelu, hipStream_t st);
-double dense_gemm_estimate(const int *Ns, int nlin, int M, int K);
+double dense_gemm_estimate(const int *Ns, int nlin, int M, int K, bool gelu);
 int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int nchunk, int nbr); // null stream
 
 // Plans of fully populated matrices: the dense product where it is estimated to be the shorter launch, from some hundred
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
-// tile: their time is that of the choice among their forms, whose figures are fits to launches of a graph and a tenth above
-// launches among others.  2.4 of the 2.6 us stand for the launch, which dense_gemm_estimate leaves out.  On the 80 full plans of
-// bench/linear_forms.py (random weights, launches of a graph, two runs) the choice is then 0.1 to 0.2 % behind the faster side
-// in the mean and 9 % at most, with 1 us more 0.8 and 19 %, with 1 us less 3 and 24 %: the line is steep on one side.  It was
-// drawn on 176 full plans of equal weights (0.3 and 14 %).
+// tile.  3.0 of the 3.5 us stand for the launch, which dense_gemm_estimate leaves out.  On 252 full plans (16 to 16384 rows,
+// random weights, launches of a graph) the choice is then 0.1 % behind the faster side in the mean and 8 % at most, on the
+// 80 of bench/linear_forms.py 0.1 and 3 %; with 0.3 us less 0.2 and 17 %, with 0.3 more 1.5 and 14 %.  Those launches find
+// their operands in the caches; where they are too large to stay there inside a layer the tile kernels, which read W more
+// often, take a tenth more than estimated and above (12288 rows, 768 -> 3072: the layer 285 us on them, 267 on the product).
+constexpr double DENSE_LAUNCH_US = 3.5;
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
@@ -2343,7 +2344,10 @@ static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool
         return true;
     const int K = plans[0]->in_feat, launches = join_launches(KC, nchunk, n, launch);
     const double tiles = tiles_estimate(Ns, ntile, nchunk, launch, launches, n, M, K, gelu);
-    return 2.6 + dense_gemm_estimate(Ns, n, M, K) < 0.9 * tiles;
+    double mb = K * 2e-6 * M;
+    for (int i = 0; i < n; i++)
+        mb += Ns[i] * 2e-6 * M;
+    return DENSE_LAUNCH_US + dense_gemm_estimate(Ns, n, M, K, gelu) < tiles * (mb > 48.0 ? 1.1 : 1.0);
 }
 static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
                            hipStream_t st) {
@@ -2619,7 +2623,7 @@ extern "C" int et_tile_plan_estimate(int in_feat, const int *out_feat, const int
     }
     const int launches = join_launches(KC, nchunk, n, launch);
     *tiles_us = tiles_estimate(out_feat, ntile, nchunk, launch, launches, n, M, in_feat, gelu != 0);
-    *dense_us = dense_gemm_estimate(out_feat, n, M, in_feat);
+    *dense_us = dense_gemm_estimate(out_feat, n, M, in_feat, gelu != 0);
     return ET_OK;
 }
 
@@ -2713,10 +2717,29 @@ extern "C" int et_tile_plan_ffn_fusable(const et_tile_plan *p1, const et_tile_pl
                : 0;
 }
 
-// Dense feed-forward products against the fused tail, which streams all of W past every 32 or 64 rows: wherever both
-// products are the shorter launch by themselves (768 wide, 3072 rows: 157 -> 99 us a layer; 8192 rows: 206 -> 181).
-static bool ffn_runs_dense(const et_tile_plan *p1, const et_tile_plan *p2, int M) {
-    return et::plans_run_dense(&p1, 1, M, true) && et::plans_run_dense(&p2, 1, M, false);
+// Full feed-forward plans: whether the steps of the block (pO: of the whole tail), one after the other, take less than the
+// fused kernel, whose round streams all of W past its panels.  A fused round of full plans takes 14 us and 10.7 per MB of
+// W, and inside a layer a tenth more: 256 wide 26, 384 38 to 42, 512 58 to 65, 640 90 to 100, 768 117 to 130.  Tail fused / by steps, us: 8192 rows 256 wide 27.9 /
+// 33.7, 384 41.8 / 46.9, 512 65.3 / 63.7 (the layer 105.6 / 99.9), 768 130 / 110; 16384 rows 512 wide 131 / 110, 768 258 / 200.
+static bool ffn_runs_dense(const et_tile_plan *pO, const et_tile_plan *p1, const et_tile_plan *p2, int M) {
+    using namespace et;
+    if (!g_plan_dense || !p1->d_dense || !p2->d_dense)
+        return false;
+    if (g_plan_dense == 2)
+        return true;
+    auto linear = [](const et_tile_plan *p, int rows, bool gelu) {
+        int launch = 0;
+        const double tiles = tiles_estimate(&p->out_feat, &p->ntile, &p->nchunk, &launch, 1, 1, rows, p->in_feat, gelu);
+        return p->d_dense ? std::min(tiles, DENSE_LAUNCH_US + dense_gemm_estimate(&p->out_feat, 1, rows, p->in_feat, gelu)) : tiles;
+    };
+    auto steps = [&](int rows) { // (a LayerNorm: 5.5 TB/s behind its launch)
+        const double ln = 3.0 + 1.1e-6 * rows * p2->out_feat;
+        return linear(p1, rows, true) + linear(p2, rows, false) + ln + (pO ? linear(pO, rows, false) + ln : 0.0);
+    };
+    const int cus = std::max(et_device_cu_count(), 1), full = M / (cus * TL_BM), rest = M - full * cus * TL_BM;
+    const double round = 15.5 + 11.7 * 512e-6 * ((double)p1->ntile + p2->ntile + (pO ? pO->ntile : 0));
+    // (behind full rounds the rest may run by steps in either case)
+    return steps(M) < full * round + (rest == 0 ? 0.0 : full == 0 ? round : std::min(round, steps(rest)));
 }
 
 extern "C" int et_tile_plan_run_ffn_ln(const et_tile_plan *p1, const et_tile_plan *p2, void *Y,
@@ -2735,7 +2758,7 @@ extern "C" int et_tile_plan_run_ffn_ln(const et_tile_plan *p1, const et_tile_pla
     if (M == 0)
         return ET_OK;
     const bool fusable = et_tile_plan_ffn_fusable(p1, p2) != 0;
-    if (!fusable || (hidden && (!ln_fusion_pays(M) || ffn_runs_dense(p1, p2, M)))) {
+    if (!fusable || (hidden && (!ln_fusion_pays(M) || ffn_runs_dense(nullptr, p1, p2, M)))) {
         // the three steps one after the other, through the caller's buffer
         ET_REQUIRE(hidden, ET_ERR_UNSUPPORTED,
                    "et_tile_plan_run_ffn_ln: these shapes need the hidden buffer (%d x %d halves)", M,
@@ -2791,7 +2814,7 @@ extern "C" int et_tile_plan_run_tail(const et_tile_plan *pO, const et_tile_plan 
                ET_ERR_ALIGNMENT, "et_tile_plan_run_tail: pointers must be 16-byte aligned");
     if (M == 0)
         return ET_OK;
-    if (!et_tile_plan_tail_fusable(pO, p1, p2) || (mid && ((M + TL_BM - 1) / TL_BM < tail_min_panels(pO, p1, p2) || ffn_runs_dense(p1, p2, M)))) {
+    if (!et_tile_plan_tail_fusable(pO, p1, p2) || (mid && ((M + TL_BM - 1) / TL_BM < tail_min_panels(pO, p1, p2) || ffn_runs_dense(pO, p1, p2, M)))) {
         // step by step through the caller's buffers
         ET_REQUIRE(mid, ET_ERR_UNSUPPORTED,
                    "et_tile_plan_run_tail: these shapes need the mid buffer (%d x %d halves)", M, pO->out_feat);
@@ -2908,7 +2931,7 @@ extern "C" int et_tile_plan_run_tail_ws(const et_tile_plan *pO, const et_tile_pl
     using namespace et;
     ET_REQUIRE(pO && p1 && p2 && Y && attn && input && gamma1 && beta1 && gamma2 && beta2,
                ET_ERR_INVALID_ARG, "et_tile_plan_run_tail_ws: null pointer");
-    if (ws && M > 0 && tail_pair_applies(pO, p1, p2) && !(mid && hidden && ffn_runs_dense(p1, p2, M))) {
+    if (ws && M > 0 && tail_pair_applies(pO, p1, p2) && !(mid && hidden && ffn_runs_dense(pO, p1, p2, M))) {
         const size_t need = tail_pair_ws_bytes(pO, p1, p2, M);
         const int cus = std::max(et_device_cu_count(), 1);
         const int wgs = 2 * ((M + 63) / 64);

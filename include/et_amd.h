@@ -535,10 +535,10 @@ int et_device_synchronize(void);
  *   "plan_dense"      plans of fully populated matrices as dense products: 0
  *                     never, 1 (default) where the estimated time is less, 2
  *                     always
- *   "dense_form"      block of the dense kernel: 0 .. 7: 64 x 128, 128 x 128 with
- *                     two and four stages, 128 x 192, 256 x 256, 256 x 192, 128 x
- *                     192 with three stages, 64 x 128 with six; -1 (default): the
- *                     least estimated time
+ *   "dense_form"      block of the dense kernel: 0 .. 10: 64 x 128, 128 x 128 with
+ *                     two and four stages, 128 x 192, 256 x 256, 192 x 256, 128 x
+ *                     192 with three stages, 64 x 64, 32 x 64, 96 x 64, 96 x 96; -1
+ *                     (default): the least estimated time
  *   "row_gemm_min_rows" rows from which et_row_spmm_add_bias runs the dense
  *                     GEMM kernel (default 1024; 0: never)
  *   "tile_fuse_ffn"   0: et_tile_plan_ffn_fusable answers no (the feed-forward

@@ -327,6 +327,41 @@ def test_tile_layer_tail_fused(K, M, d, F, sp, fused):
         assert np.array_equal(host(ad), got)
 
 
+@pytest.mark.parametrize("d,M,one_launch", [
+    (256, 7200, True),     # a round of the fused kernel is shorter than the five steps
+    (512, 7200, False),    # ... and longer
+    (256, 8225, False),    # one row into a second round
+])
+def test_layer_tail_of_full_plans_fused_or_by_steps(K, d, M, one_launch):
+    """full plans with the caller's buffers at hand, either side of the line between the fused tail and the steps (which write
+    the hidden buffer), against the steps"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile
+    if lib().et_device_cu_count() != 256:
+        pytest.skip("a round is one panel per compute unit of 256")
+    r = rng(2900 + d + M)
+    mk = lambda n, k, gelu, i: (lambda l: Linear_tile(k, n, M, l["row_offset"].size, l["data"], l["row_ptr"], l["row_offset"], l["bias"],
+                                                      gelu))(make_tile_linear(r, n, k, 0.0, seed=i, std=0.05, bias_std=0.2))
+    to, t1, t2 = mk(d, d, False, 1), mk(4 * d, d, True, 2), mk(d, 4 * d, False, 3)
+    attn, inp = dev(randn_h(r, (M, d))), dev(randn_h(r, (M, d)))
+    ln = [dev(t) for t in (randn_h(r, (d,), 0.3) + np.float16(1), randn_h(r, (d,), 0.3)) * 2]
+
+    def run():
+        hid = torch.full((M, 4 * d), 7.0, dtype=torch.float16, device="cuda")
+        out = host(Linear_tile.run_tail(to, t1, t2, attn, inp, *ln, mid=torch.empty_like(attn), hidden=hid))
+        return out, bool((hid == 7.0).all())
+
+    got, untouched = run()
+    assert untouched == one_launch
+    try:
+        lib().et_tuning_set(b"tile_fuse_ffn", 0)
+        want, untouched = run()
+    finally:
+        lib().et_tuning_set(b"tile_fuse_ffn", 2)
+    assert not untouched
+    check_close(got, want, max_abs=3e-2, mean_rel=2e-3, what="tail of full plans")  # (as against the oracle, above)
+
+
 PAIR_CASES = [
     (640, 768, 3072, 0.8),     # BERT-base widths, ten 64-row panels
     (200, 256, 1024, 0.5),     # a ragged last panel (8 rows), two block-rows per wave
@@ -1416,6 +1451,23 @@ def test_full_plan_as_dense_product(K, form, M, Ns, Kd, gelu):
 def test_full_plan_as_dense_product_256x192(K, M, Ns, Kd, gelu):
     """the same for blocks of 256 x 192"""
     test_full_plan_as_dense_product(K, 5, M, Ns, Kd, gelu)
+
+
+@pytest.mark.parametrize("form", [8, 9, 10])
+def test_dense_product_stages_of_small_blocks(K, form):
+    """the same for the blocks of four waves, with six to twelve stages"""
+    test_dense_product_stages(K, form)
+
+
+@pytest.mark.parametrize("form", [5, 6, 7, 8, 9, 10])
+@pytest.mark.parametrize("M,Ns,Kd,gelu", [
+    (1, (16,), 32, False),
+    (33, (80, 16, 400), 96, False),      # a row into the second block of 32; three linears, none a multiple of a block
+    (193, (272, 112), 832, False),       # a row into the second (third) block; thirteen steps: one more than the most stages
+    (97, (208,), 1056, True),            # 16.5 steps; a plan of two chunks with odd counts
+])
+def test_full_plan_as_dense_product_small_blocks(K, form, M, Ns, Kd, gelu):
+    test_full_plan_as_dense_product(K, form, M, Ns, Kd, gelu)
 
 
 @pytest.mark.parametrize("M,Ns,Kd", [
