@@ -32,6 +32,8 @@ TERMS = {  # kernel -> its cost terms, in the order of features()
     "64 rows, 12 waves": "launch traffic traffic_over round item item_nb item_stream panel out gelu mfma result wg".split(),
     "chunk by chunk": "launch round*chunk round*nb*pairs cu*chunk cu*nb*pairs cu*nb traffic".split(),
     "fetching waves": "launch round round*chunk round*nb*chunk round*nb*pairs round*fill*nb*pairs round*group*pairs traffic".split(),
+    "48 rows": "launch round round*chunk round*nb*chunk round*nb*pairs round*fill*nb*pairs round*group*pairs traffic".split(),
+    "48 rows, two waves a block-row": "launch round round*chunk round*nb*chunk round*nb*pairs round*fill*nb*pairs round*group*pairs traffic".split(),
     "whole rows": "launch traffic round round*K round*group*pairs round*nb round*fill".split(),
 }
 
@@ -97,6 +99,14 @@ def features(line, cus=256):
         return "fetching waves", [1, rounds, rounds * nchunk, rounds * nb * nchunk, rounds * nb * pairs,
                                   rounds * fill * nb * pairs, rounds * min(12 * nb, nbr) * pairs,
                                   traffic(x, w, panels, ncg, 1.75)]
+    if form.startswith("tall"):
+        group = {5: 12, 6: 6, 7: 24, 8: 36}[int(form[4:])]
+        panels, nb = up(M, 48), group / 12
+        ncg = up(nbr, group) * nlin
+        rounds, fill = up(panels * ncg, cus), min(1.0, panels * ncg / cus)
+        return "48 rows, two waves a block-row" if group == 6 else "48 rows", [
+            1, rounds, rounds * nchunk, rounds * nb * nchunk, rounds * nb * pairs, rounds * fill * nb * pairs,
+            rounds * min(group, nbr) * pairs, traffic(x, w, panels, ncg, 1.75)]
     if form == "rows":
         b, s = rows_shape(M, K, nbr, nlin, pairs, cus)
         group, panels = (16 >> s) * b, up(M, 16)
@@ -194,6 +204,9 @@ def measure(path):
                         for nb in range(5):
                             keys(tile_chunked=nb, tile_splitk_rows=0)
                             line(f"fetch{nb}" if nb else "chunk", 0)
+                        for form in range(5, 9):
+                            keys(tile_chunked=form, tile_splitk_rows=0)
+                            line(f"tall{form}", 0)
                         keys(tile_chunked=-1, tile_splitk_rows=most)
                         line("rows", 0)
                         keys(tile_splitk_rows=-1)

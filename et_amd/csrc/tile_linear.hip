@@ -1134,6 +1134,152 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_kernel(TL_HOT
 }
 
 // ---------------------------------------------------------------------------
+// The chunked kernel on 48-row panels: a computing wave has one block-row, or
+// (SPLIT) two waves share one, each with half of the pairs of every chunk.
+//
+// What bounds these kernels is what a CU takes in - X by DMA, W past the vector
+// memory path, 100 to 120 GB/s together - so the best workgroup is the one whose
+// panel and lists are equally large.  1536 rows 3072 -> 768 at 50 %: 32 rows x 192
+// columns are 197 KB of X and 590 of W on 192 CUs, 48 x 96 are 295 and 295 on 256;
+// 2000 rows 4096 -> 1024 at 80 %: 32 x 384 are 262 and 627 on 189, 48 x 192 393 and
+// 313 on 252.  us, the other kernels / this: 3072 -> 768 50 % 2791 rows 20.1 / 16.1, 4523 32.4
+// / 22.6, 10111 57.2 / 44.8; 80 % 4523 19.1 / 15.2, 10111 35.3 / 29.8; 4096 -> 1024 50 % 770 17.4 / 15.3, 2000
+// 23.4 / 20.3, 5134 48.7 / 40.1; 80 % 5134 29.7 / 24.6; 2048 -> 512 80 % 8345 21.7 / 15.6.  With two block-rows
+// a wave and more (NB) the panels of all rows fit fewer rounds.
+// The panel buffer of the chunk before the last, which everyone has left, stages
+// the result (and, SPLIT, the second waves' sums): whole rows of the column
+// group, stored line-wise by all sixteen waves.
+// ---------------------------------------------------------------------------
+constexpr int TL_TALL = 3; // subtiles of a panel
+
+template <int NB, bool SPLIT, bool GELU>
+__global__ void __launch_bounds__(TL_CTHREADS) tile_linear_tall_kernel(TL_HOT_PARAMS, const TlArgs args) {
+    static_assert(!SPLIT || NB == 1, "two waves share one block-row");
+    TL_HOT_TAKE(a, args, KC)
+    constexpr int MS = TL_TALL, BM = 16 * MS, BRS = SPLIT ? TL_CWAVES / 2 : TL_CWAVES * NB; // block-rows of a workgroup
+    extern __shared__ __attribute__((aligned(16))) unsigned char tl_smem[];
+    f16 *xs = reinterpret_cast<f16 *>(tl_smem);
+    int rp, lin, cg;
+    if (!tl_place(a, rp, lin, cg))
+        return;
+    const int m0 = rp * BM;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int c16 = lane & 15, g4 = lane >> 4, khalf8 = (g4 & 1) * 8, hi = lane >> 5;
+    const int ldx = a.KC + ((a.KC & 31) ? 0 : TL_PAD);
+    const int pbuf = BM * ldx; // halves per panel buffer
+    f16 *const Y = TL_SEL(Y);
+    const int N = TL_SEL(N), nbr = N >> 4;
+    constexpr int LDS = 16 * BRS + 8; // halves per staged row
+    f16 *const stage = xs + (a.nchunk & 1) * pbuf;
+    f32x4 *const red = reinterpret_cast<f32x4 *>(stage + BM * LDS);
+    static_assert(BM * LDS * 2 % 16 == 0, "aligned sums");
+    if (wave >= TL_CWAVES) {
+        // ---- the fetching waves ----
+        const int row0 = (wave - TL_CWAVES) * (BM / TL_FWAVES);
+        auto fetch = [&](int c) {
+            const int pk0 = c * a.KC, pcpr = min(a.KC, a.K - pk0) >> 3; // 16-byte pieces per row, <= 96
+            f16 *dst = xs + (c & 1) * pbuf;
+            const int row1 = min(row0 + BM / TL_FWAVES, a.M - m0);
+            for (int row = row0; row < row1; row++) {
+                const f16 *src = a.X + (size_t)(m0 + row) * a.K + pk0;
+                if (lane < pcpr)
+                    load_lds16(src + lane * 8, dst + row * ldx);
+                if (64 + lane < pcpr)
+                    load_lds16(src + (64 + lane) * 8, dst + row * ldx + 512);
+            }
+        };
+        fetch(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+        if (a.nchunk > 1)
+            fetch(1);
+        tl_barrier_lds(); // chunk 0 is in LDS
+        for (int c = 1; c < a.nchunk; c++) {
+            __builtin_amdgcn_s_waitcnt(0x0F70); // chunk c has landed
+            tl_barrier_lds();                   // ... and every wave has left chunk c-1
+            if (c + 1 < a.nchunk)
+                fetch(c + 1);
+        }
+        if (SPLIT)
+            tl_barrier_lds();
+    } else {
+        // ---- the computing waves ----
+        const int br = SPLIT ? wave >> 1 : wave * NB, half = SPLIT ? wave & 1 : 0, bn = cg * BRS + br;
+        const int *const cptr = TL_SEL(cptr);
+        const f16 *const data = TL_SEL(data);
+        const int *const poff = TL_SEL(row_offset);
+        const f16 *const bias = TL_SEL(bias);
+        f32x4 acc[NB][MS];
+        f16x4 b4[NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+#pragma unroll
+            for (int m = 0; m < MS; m++)
+                acc[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+            b4[j] = *reinterpret_cast<const f16x4 *>(bias + min(bn + j, nbr - 1) * 16 + g4 * 4);
+        }
+        const unsigned lane_w = hi * 256 + c16 * 16 + khalf8;
+        // lane k: first pair of block-row k in a chunk, then the end of the last one; the next chunk's are requested a chunk ahead
+        auto ends = [&](int c) { return cptr[min(c, a.nchunk - 1) * nbr + min(bn + min(lane, NB), nbr)] >> 1; };
+        int bvec = ends(0);
+        for (int c = 0; c < a.nchunk; c++) {
+            const char *const xlane = reinterpret_cast<const char *>(xs + (c & 1) * pbuf + c16 * ldx + khalf8);
+            TlBounds<NB> b = tl_bounds<NB>(bvec);
+            if (SPLIT) {
+                const int st = b.at[0], len = b.at[1] - st;
+                b.at[0] = st + ((len * half) >> 1);
+                b.at[1] = st + ((len * (half + 1)) >> 1);
+            }
+            f16x8 w[TL_DEPTH];
+            int o[TL_DEPTH];
+            tl_preload(data, poff, lane_w, hi, b.at[0], max(b.at[NB] - 1, b.at[0]), w, o);
+            bvec = ends(c + 1);
+            tl_barrier_lds();
+            tl_stream<NB, MS>(xlane, 16 * ldx * 2, data, poff, lane_w, hi, b, w, o, [&](int j, const f32x4 (&s)[MS]) {
+#pragma unroll
+                for (int k = 0; k < NB; k++) {
+                    const float mk = k == j ? 1.0f : 0.0f;
+#pragma unroll
+                    for (int m = 0; m < MS; m++)
+                        acc[k][m] = NB == 1 ? acc[k][m] + s[m] : __builtin_elementwise_fma(s[m], f32x4{mk, mk, mk, mk}, acc[k][m]);
+                }
+            });
+        }
+        if (SPLIT) {
+            if (half)
+#pragma unroll
+                for (int m = 0; m < MS; m++)
+                    red[(br * MS + m) * 64 + lane] = acc[0][m];
+            tl_barrier_lds();
+            if (!half)
+#pragma unroll
+                for (int m = 0; m < MS; m++)
+                    acc[0][m] += red[(br * MS + m) * 64 + lane];
+        }
+        if (!half)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int m = 0; m < MS; m++) {
+                    f16x4 v;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        v[r] = (f16)(acc[j][m][r] + (float)b4[j][r]);
+                        if (GELU)
+                            v[r] = gelu_h(v[r]);
+                    }
+                    *reinterpret_cast<f16x4 *>(stage + (m * 16 + c16) * LDS + (br + j) * 16 + g4 * 4) = v;
+                }
+    }
+    tl_barrier_lds(); // the rows are staged
+    const int col0 = cg * BRS * 16, cpr = 2 * BRS; // 16-byte pieces per row
+    for (int i = threadIdx.x; i < BM * cpr; i += TL_CTHREADS) {
+        const int r = i / cpr, c = i - r * cpr;
+        if (m0 + r < a.M && col0 + c * 8 < N)
+            *reinterpret_cast<u32x4 *>(Y + (size_t)(m0 + r) * N + col0 + c * 8) = *reinterpret_cast<const u32x4 *>(stage + r * LDS + c * 8);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Fused feed-forward block: Y = LayerNorm(skip + W2 * gelu(W1 * X + b1) + b2)
 // in ONE launch (encoder/encoder.cu:36-44 runs it as MLP1, MLP2 and
 // skip_layernorm with the [rows x ffn] intermediate written to and read back
@@ -1592,6 +1738,14 @@ static int launch_chunked_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     return launch_status("tile_linear+LayerNorm (chunked) launch");
 }
 
+template <int NB, bool SPLIT, bool GELU>
+static int launch_tall(const TlArgs &a, hipStream_t st) {
+    constexpr auto k = &tile_linear_tall_kernel<NB, SPLIT, GELU>;
+    const size_t lds = 2 * (size_t)16 * TL_TALL * (a.KC + ((a.KC & 31) ? 0 : TL_PAD)) * sizeof(f16);
+    launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
+    return launch_status("tile_linear (48-row panels) launch");
+}
+
 template <int NB, bool GELU>
 static int launch_chunked_inst(const TlArgs &a, size_t lds, hipStream_t st) {
     constexpr auto k = &tile_linear_chunked_kernel<NB, GELU, false>;
@@ -1876,7 +2030,10 @@ static TlChoice weigh_resident(const TlProblem *probs, int nlin, int M, int K, i
 // 4096 -> 1024, 0 to 90 % pruned, 48 to 16384 rows): 5 to 6 % off in the mean, the choice 0.2 % behind the fastest
 // kernel, 9 % at most (the rule before: 10.9 %).  The 576 launches that bench/linear_forms.py times in graphs (plan kernel,
 // fetching waves, whole rows): 15, 8 and 13 % off.
-enum { TL_BY_ROWS = -1, TL_BY_PLAN = 0 }; // or 1 .. 4: fetching waves, that many block-rows per computing wave
+enum { TL_BY_ROWS = -1, TL_BY_PLAN = 0, TL_BY_TALL = 5, TL_BY_TALL_SPLIT, TL_BY_TALL_2, TL_BY_TALL_3, TL_BY_LAST = TL_BY_TALL_3 }; // or 1 .. 4: fetching waves, that many block-rows per computing wave
+static int tall_block_rows(int which) { // of a workgroup
+    return which == TL_BY_TALL_SPLIT ? TL_CWAVES / 2 : TL_CWAVES * (which == TL_BY_TALL ? 1 : which - TL_BY_TALL);
+}
 static double estimate_plan_kernel(int M, double pairs, double x_mb, double w_mb, int nchunk, int nbr_max, int nlin, long cus) {
     const long panels = (M + TL_BM - 1) / TL_BM;
     const int nb = choose_nb((int)panels, nbr_max, nlin), ncg = (nbr_max + TL_WAVES * nb - 1) / (TL_WAVES * nb) * nlin;
@@ -1893,6 +2050,22 @@ static double estimate_chunked(int M, double pairs, double x_mb, double w_mb, in
                              0.00429 * std::min(TL_CWAVES * nb, nbr_max) * pairs) +
            0.0980 * tl_traffic_mb(x_mb, w_mb, panels, ncg, 1.75);
 }
+// 48-row panels.  The fit (775 launches of 1536 -> 768, 2048 -> 512 and 1536, 3072 -> 768, 4096 -> 1024, 50 to 90 % pruned,
+// 250 to 16384 rows: 2 to 5 % off) times 1.15: the figures above are 6 to 12 % high on the same launches, and with less the
+// choice is up to 24 % behind what it was without these forms, with this 1.6 %.  It is 3.6 % faster in the mean over all of
+// these launches, and 1 % behind the fastest kernel.
+static double estimate_tall(int which, int M, double pairs, double x_mb, double w_mb, int nchunk, int nbr_max, int nlin, long cus) {
+    const long panels = (M + 16 * TL_TALL - 1) / (16 * TL_TALL);
+    const int brs = tall_block_rows(which), ncg = (nbr_max + brs - 1) / brs * nlin;
+    const double nb = (double)brs / TL_CWAVES;
+    const long wgs = panels * ncg;
+    const double rounds = (double)((wgs + cus - 1) / cus), fill = std::min(1.0, (double)wgs / cus);
+    const double traffic = tl_traffic_mb(x_mb, w_mb, panels, ncg, 1.75);
+    if (which == TL_BY_TALL_SPLIT)
+        return 1.15 * (1.468 + rounds * (2.068 + 1.277 * nchunk + 0.0512 * fill * nb * pairs + 0.00231 * std::min(brs, nbr_max) * pairs) +
+                       0.0332 * traffic);
+    return 1.15 * (1.094 + rounds * (2.931 + (0.4926 + 0.2443 * nb) * nchunk + (0.0840 + 0.0414 * fill) * nb * pairs) + 0.0736 * traffic);
+}
 static int weigh_chunked(const TlProblem *probs, int nlin, int M, int K, int nchunk, int nbr_max, long cus, double *us) {
     double pairs = 0.0, w_mb = 0.0;
     for (int i = 0; i < nlin; i++) {
@@ -1904,6 +2077,7 @@ static int weigh_chunked(const TlProblem *probs, int nlin, int M, int K, int nch
     auto estimate = [&](int which) {
         return which == TL_BY_ROWS   ? tile_rows_estimate(M, K, nbr_max, nlin, pairs, w_mb)
                : which == TL_BY_PLAN ? estimate_plan_kernel(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, cus)
+               : which >= TL_BY_TALL ? estimate_tall(which, M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, cus)
                                      : estimate_chunked(M, pairs, x_mb, w_mb, nchunk, nbr_max, nlin, which, cus);
     };
     const bool rows_fit = tile_rows_fits(K);
@@ -1912,7 +2086,7 @@ static int weigh_chunked(const TlProblem *probs, int nlin, int M, int K, int nch
     if (rows_fit && rows_most >= 0 && M <= rows_most)
         best = TL_BY_ROWS; // (tuning)
     else if (chunked > 0)
-        best = std::min(chunked, 4);
+        best = std::min(chunked, (int)TL_BY_LAST);
     *us = estimate(best);
     if (best != TL_BY_PLAN)
         return best;
@@ -1924,8 +2098,8 @@ static int weigh_chunked(const TlProblem *probs, int nlin, int M, int K, int nch
         }
     };
     if (chunked < 0)
-        for (int nb = 1; nb <= 4; nb++)
-            take(nb);
+        for (int which = 1; which <= TL_BY_LAST; which++)
+            take(which);
     if (rows_fit && rows_most < 0)
         take(TL_BY_ROWS);
     return best;
@@ -2088,6 +2262,18 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         order = c.by_group;
     } else {
         const int nrp = (M + TL_BM - 1) / TL_BM;
+        if (which >= TL_BY_TALL) {
+            const int brs = tall_block_rows(which);
+            a.ncg = (nbr_max + brs - 1) / brs;
+            a.ipw = 1;
+            place(16 * TL_TALL, -1);
+            switch (which) {
+            case TL_BY_TALL: return gelu ? launch_tall<1, false, true>(a, st) : launch_tall<1, false, false>(a, st);
+            case TL_BY_TALL_2: return gelu ? launch_tall<2, false, true>(a, st) : launch_tall<2, false, false>(a, st);
+            case TL_BY_TALL_3: return gelu ? launch_tall<3, false, true>(a, st) : launch_tall<3, false, false>(a, st);
+            default: return gelu ? launch_tall<1, true, true>(a, st) : launch_tall<1, true, false>(a, st);
+            }
+        }
         if (which > 0) {
             const int cnb = which;
             a.ncg = (nbr_max + TL_CWAVES * cnb - 1) / (TL_CWAVES * cnb);

@@ -523,8 +523,9 @@ int et_device_synchronize(void);
  *   "tile_splitk_k1"  1: whole rows also for K of one chunk, up to
  *                     "tile_splitk_rows" rows (-1: 128); 0 (default)
  *   "tile_chunked"    a planned linear with K in several chunks on the kernel with
- *                     fetching waves: 1 .. 4 block-rows per computing wave; 0: never; -1
- *                     (default): by estimated time
+ *                     fetching waves: 1 .. 4 block-rows per computing wave on 32-row
+ *                     panels, 5, 7, 8: one to three on 48-row panels, 6: two waves
+ *                     a block-row; 0: never; -1 (default): by estimated time
  *   "layer_flow_rows" most rows for which an encoder layer runs as one launch
  *                     (et_layer_flow_pays); -1 (default): by size and density;
  *                     0: never

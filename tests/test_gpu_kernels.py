@@ -1573,6 +1573,38 @@ def test_tile_linear_fetching_waves(K, nb, M, N, Kd, gelu):
     assert np.array_equal(got, chunks)
 
 
+@pytest.mark.parametrize("form,Ns", [(5, (16, 208)), (6, (112, 96)), (7, (784, 48)), (8, (592,))])
+@pytest.mark.parametrize("M,Kd,sp,gelu", [
+    (1, 1040, 0.7, True),      # one row; a second chunk of 272 columns
+    (49, 1552, 0.97, False),   # a row into the second panel; three chunks, most runs empty or of one pair
+    (143, 3072, 0.5, True),    # four full chunks, the last panel one row short
+])
+def test_tile_linear_tall_panels(K, form, Ns, M, Kd, sp, gelu):
+    """48-row panels of one to three block-rows a wave, or two waves a block-row, widths either side of a column group: the
+    oracle, and the bits of the kernel that fetches chunk by chunk where a block-row is one wave's"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile, run_multi
+    r = rng(89 + M + form)
+    mats = [make_tile_linear(r, N, Kd, sp, seed=M + Kd + N, std=0.05, bias_std=0.2) for N in Ns]
+    X = randn_h(r, (M, Kd))
+    lts = [Linear_tile(Kd, N, M, m["row_offset"].size, m["data"], m["row_ptr"], m["row_offset"], m["bias"], gelu) for N, m in zip(Ns, mats)]
+    run = lambda: [host(y) for y in (run_multi(lts, dev(X)) if len(lts) > 1 and not gelu else [l.run(dev(X)) for l in lts])]
+    try:
+        lib().et_tuning_set(b"tile_splitk_rows", 0)
+        lib().et_tuning_set(b"tile_chunked", 0)
+        chunks = run()
+        lib().et_tuning_set(b"tile_chunked", form)
+        got = run()
+    finally:
+        lib().et_tuning_set(b"tile_splitk_rows", -1)
+        lib().et_tuning_set(b"tile_chunked", -1)
+    for g, c, N, m in zip(got, chunks, Ns, mats):
+        want = orc.tile_linear(X, m["row_ptr"], m["row_offset"], m["data"], m["bias"], N, gelu=gelu, f64=True)
+        check_close(g, want, max_abs=4e-3, mean_rel=5e-4, what=f"48-row panels, N={N}")
+        if form != 6:
+            assert np.array_equal(g, c)
+
+
 @pytest.mark.parametrize("form", ["planned", "raw"])
 @pytest.mark.parametrize("M,N,Kd", [
     (5, 160, 2048),       # a block-row's pairs split over many waves

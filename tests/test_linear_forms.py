@@ -70,6 +70,20 @@ def test_chunk_terms_follow_the_estimate(K, Ns, gelu, rows):
         assert sum(c * v for c, v in zip(const, terms)) == pytest.approx(library_estimate(line, **keys), rel=1e-6), form
 
 
+@pytest.mark.parametrize("rows", [37, 700, 9000])
+@pytest.mark.parametrize("K,Ns,gelu", lf.CHUNKS)
+def test_tall_panel_terms_follow_the_estimate(K, Ns, gelu, rows):
+    cus = max(lib().et_device_cu_count(), 1)
+    split, whole = (1.468, 2.068, 1.277, 0, 0, 0.0512, 0.00231, 0.0332), (1.094, 2.931, 0.4926, 0.2443, 0.0840, 0.0414, 0, 0.0736)
+    for form in (5, 6, 7, 8):
+        line = dict(inputs=K, outputs=Ns, gelu=gelu, sparsity=0.5, rows=rows, form=f"tall{form}", d=0)
+        name, terms = lf.features(line, cus)
+        assert len(terms) == len(lf.TERMS[name])
+        const = split if form == 6 else whole
+        assert 1.15 * sum(c * v for c, v in zip(const, terms)) == pytest.approx(
+            library_estimate(line, tile_chunked=(form, -1), tile_splitk_rows=(0, -1)), rel=1e-6), form
+
+
 def test_times_are_read_back(tmp_path):
     p = tmp_path / "times.txt"
     p.write_text("A heading.\n\n768 768+768 1 0.8 100 panel3 2 7.25 6.90\n768 768+768 1 0.8 100 auto 0 7.10 6.90\n")
