@@ -13,9 +13,11 @@
 // features, W in the plan's tile pairs (a full list: pair j of a block-row is
 // columns 32j .. 32j + 31), four pairs of each block-row in flight.  The results
 // are rounded to half and scattered over zeroed rows of model width in the
-// panel's LDS; then a wave normalises 2 * MS rows.
+// panel's LDS; then a wave normalises 2 * MS rows, two at a time in 32 lanes each (row after row over 64 lanes a quarter of
+// the vector work of a 768-wide row was for lanes without a piece: attention-aware layer 32 x 256 86.8 -> 85.5 us, 4 x 100 33.2 ->
+// 32.6).
 // What bounds it: one phase after the other in a workgroup - panel, W (370 KB for
-// 240 x 768 past every workgroup, 3 us at 64 bytes a clock), LayerNorm (2.5 us for
+// 240 x 768 past every workgroup, 3 us at 64 bytes a clock), LayerNorm (2 us for
 // 32 rows on a CU), store.  Linear and expansion + LayerNorm as two launches / this
 // one, back to back, us: 768 -> 240 (230 kept): 256 rows 8.9 / 7.5, 4096 11.8 / 9.1,
 // 8192 16.8 / 12.5, 16384 25.0 / 21.7; 928 -> 240: 8192 17.6 / 14.0; 624 -> 160: 8192
@@ -101,10 +103,11 @@ __global__ void __launch_bounds__(RL_WAVES * 64, NB < 3 ? 4 : 2) row_layernorm_k
         for (int r = 0; r < 4; r++)
             col[nb][r] = a.col[min(f + r, a.ncol - 1)];
     }
-    RowPieces<NP> skip[ROWS];
+    // (a pair of rows: 32 lanes each)
+    RowPieces<NP> skip[ROWS / 2];
 #pragma unroll
-    for (int k = 0; k < ROWS; k++)
-        skip[k] = row_pieces<NP>(a.skip + (size_t)min(m0 + wave + k * RL_WAVES, a.M - 1) * a.size, npiece, lane);
+    for (int k = 0; k < ROWS / 2; k++)
+        skip[k] = row_pieces<NP, 32>(a.skip + (size_t)min(m0 + wave + (2 * k + hi) * RL_WAVES, a.M - 1) * a.size, npiece, lane);
     const char *const xlane = reinterpret_cast<const char *>(xs + c16 * a.ldx + khalf8);
     f32x4 acc[NB][MS];
 #pragma unroll
@@ -133,15 +136,15 @@ __global__ void __launch_bounds__(RL_WAVES * 64, NB < 3 ? 4 : 2) row_layernorm_k
                 request(w[i], s + RL_DEPTH);
             }
     }
-    const RowPieces<NP> gamma = row_pieces<NP>(a.gamma, npiece, lane), beta = row_pieces<NP>(a.beta, npiece, lane);
+    const RowPieces<NP> gamma = row_pieces<NP, 32>(a.gamma, npiece, lane), beta = row_pieces<NP, 32>(a.beta, npiece, lane);
     __syncthreads(); // X has been read
 #pragma unroll
-    for (int k = 0; k < ROWS; k++) {
+    for (int k = 0; k < ROWS / 2; k++) {
         RowPieces<NP> zero;
 #pragma unroll
         for (int i = 0; i < NP; i++)
             zero.p[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        row_put(xs + (wave + k * RL_WAVES) * a.lde, zero, npiece, lane);
+        row_put<NP, 32>(xs + (wave + (2 * k + hi) * RL_WAVES) * a.lde, zero, npiece, lane);
     }
     __syncthreads();
 #pragma unroll
@@ -159,11 +162,11 @@ __global__ void __launch_bounds__(RL_WAVES * 64, NB < 3 ? 4 : 2) row_layernorm_k
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < ROWS; k++) {
-        const int r = wave + k * RL_WAVES;
-        const RowPieces<NP> v = row_layernorm(row_pieces<NP>(xs + r * a.lde, npiece, lane), skip[k], gamma, beta, npiece, a.inv_n, lane);
+    for (int k = 0; k < ROWS / 2; k++) {
+        const int r = wave + (2 * k + hi) * RL_WAVES;
+        const RowPieces<NP> v = row_layernorm<NP, 32>(row_pieces<NP, 32>(xs + r * a.lde, npiece, lane), skip[k], gamma, beta, npiece, a.inv_n, lane);
         if (m0 + r < a.M)
-            row_put(a.out + (size_t)(m0 + r) * a.size, v, npiece, lane);
+            row_put<NP, 32>(a.out + (size_t)(m0 + r) * a.size, v, npiece, lane);
     }
 }
 
@@ -238,7 +241,7 @@ extern "C" int et_tile_plan_run_scatter_ln(const et_tile_plan *plan, void *out, 
     typedef std::integral_constant<int, 1> c1;
     typedef std::integral_constant<int, 2> c2;
     typedef std::integral_constant<int, 3> c3;
-    auto by_np = [&](auto nb_c, auto ms_c) { return size <= 512 ? launch(nb_c, ms_c, c1()) : launch(nb_c, ms_c, c2()); };
+    auto by_np = [&](auto nb_c, auto ms_c) { return size <= 512 ? launch(nb_c, ms_c, c2()) : size <= 768 ? launch(nb_c, ms_c, c3()) : launch(nb_c, ms_c, std::integral_constant<int, 4>()); };
     auto by_ms = [&](auto nb_c) { return ms == 1 ? by_np(nb_c, c1()) : by_np(nb_c, c2()); };
     if (ms == 4)
         return by_np(c3(), std::integral_constant<int, 4>());

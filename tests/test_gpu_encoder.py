@@ -398,6 +398,18 @@ def test_row_linear_scatter_layernorm(M, K, n, size, alias):
         L.et_tile_plan_destroy(p)
 
 
+@pytest.mark.parametrize("M,K,n,size,alias", [
+    (1, 64, 3, 8, True),                # one piece in all
+    (17, 64, 20, 264, False),           # a piece behind the first 32 lanes
+    (31, 128, 40, 520, True),           # ... and behind two whole pieces; the last pair of rows has one
+    (33, 64, 50, 776, False),           # four pieces a lane, the last one lane's
+    (4104, 96, 30, 1016, True),         # 32 rows a workgroup, two pairs a wave
+])
+def test_row_linear_scatter_layernorm_rows_in_pairs(M, K, n, size, alias):
+    """two rows of a wave at once, 32 lanes each: widths that leave lanes without a piece"""
+    test_row_linear_scatter_layernorm(M, K, n, size, alias)
+
+
 def test_encoder_length_paths():
     from et_amd.encoder import Encoder_length
     r = rng(700)
