@@ -445,24 +445,31 @@ static double dg_estimate(int form, const int *Ns, int nlin, int M, int K, bool 
     const double step = n <= 1 ? f.one + f.fill1 * fill : n <= 2 ? f.two + f.fill2 * fill : f.more * (double)n + f.fill3 * fill;
     return f.ends + step * ((K + DG_BK - 1) / DG_BK) + (gelu ? f.gelu * (double)n * bm[form] * bn[form] / 16384.0 : 0.0);
 }
-static int dg_choose(const int *Ns, int nlin, int M, int K, bool gelu, double *us) {
-    int best = 0;
-    for (int f = 0; f < DG_FORMS; f++) {
-        const double t = dg_estimate(f, Ns, nlin, M, K, gelu);
-        if (f == 0 || t < *us) {
-            *us = t;
-            best = f;
+// The choice, kept for sizes that come again: a plan's launch asks twice, for the line to the tile kernels and for the
+// block (61 rows 768 -> 768 without pruning, bound by the host: 5.0 us a call weighed each time, 4.4 so).
+struct DenseChoice {
+    int form;
+    double us;
+};
+typedef KeptChoices<DenseChoice, 5 + DG_MAX_LIN> DenseChoices;
+static DenseChoice dg_choose(const int *Ns, int nlin, int M, int K, bool gelu) {
+    static thread_local DenseChoices kept;
+    DenseChoices::Key k = {{nlin, M, K, gelu, std::max(et_device_cu_count(), 1)}};
+    for (int i = 0; i < nlin; i++)
+        k.v[5 + i] = Ns[i];
+    return kept.get(k, [&] {
+        DenseChoice best = {0, dg_estimate(0, Ns, nlin, M, K, gelu)};
+        for (int f = 1; f < DG_FORMS; f++) {
+            const double us = dg_estimate(f, Ns, nlin, M, K, gelu);
+            if (us < best.us)
+                best = DenseChoice{f, us};
         }
-    }
-    return best;
+        return best;
+    });
 }
 double dense_gemm_estimate(const int *Ns, int nlin, int M, int K, bool gelu) {
-    double us = 0.0;
     const int set = g_dense_form;
-    if (set >= 0)
-        return dg_estimate(set, Ns, nlin, M, K, gelu);
-    dg_choose(Ns, nlin, M, K, gelu, &us);
-    return us;
+    return set >= 0 ? dg_estimate(set, Ns, nlin, M, K, gelu) : dg_choose(Ns, nlin, M, K, gelu).us;
 }
 void set_dense_form(int v) { g_dense_form = v < DG_FORMS ? v : -1; }
 
@@ -489,8 +496,7 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
     a.nlin = nlin;
     a.M = M;
     a.K = K;
-    double us;
-    const int set = g_dense_form, form = set >= 0 ? set : dg_choose(Ns, nlin, M, K, gelu, &us);
+    const int set = g_dense_form, form = set >= 0 ? set : dg_choose(Ns, nlin, M, K, gelu).form;
     switch (form) {
 #define DG_CASE(form_, ...)                                                                                            \
     case form_: return gelu ? dg_launch_inst<true, __VA_ARGS__>(a, st) : dg_launch_inst<false, __VA_ARGS__>(a, st);

@@ -3,6 +3,7 @@ import ctypes as C
 import os
 import re
 import sys
+import threading
 
 import pytest
 
@@ -82,6 +83,36 @@ def test_tall_panel_terms_follow_the_estimate(K, Ns, gelu, rows):
         const = split if form == 6 else whole
         assert 1.15 * sum(c * v for c, v in zip(const, terms)) == pytest.approx(
             library_estimate(line, tile_chunked=(form, -1), tile_splitk_rows=(0, -1)), rel=1e-6), form
+
+
+def test_dense_choice_is_kept_by_its_sizes():
+    """More shapes than the table of kept choices has entries, in two orders and from two threads: always the least block."""
+    L = lib()
+    shapes = [(K, Ns, gelu, rows) for K, Ns, gelu in ((768, (768,), 0), (768, (3072,), 1), (1024, (1024,) * 3, 0), *lf.CHUNKS)
+              for rows in (16, 37, 61, 104, 250, 345, 700, 1300, 2048, 5000, 9000, 16384)]
+    assert len(shapes) > 64
+
+    def dense_us(K, Ns, gelu, rows):
+        n, t, g = len(Ns), C.c_double(), C.c_double()
+        assert L.et_tile_plan_estimate(K, (C.c_int * n)(*Ns), (C.c_int * n)(*[(K // 16) * (v // 16) for v in Ns]), n, rows,
+                                       gelu, C.byref(t), C.byref(g)) == 0
+        return g.value
+
+    def block_us(form):
+        assert L.et_tuning_set(b"dense_form", form) == 0
+        return [dense_us(*s) for s in shapes]
+
+    try:
+        want = [min(v) for v in zip(*(block_us(f) for f in range(11)))]
+    finally:
+        L.et_tuning_set(b"dense_form", -1)
+    assert [dense_us(*s) for s in shapes] == want
+    got = []
+    other = threading.Thread(target=lambda: got.extend(dense_us(*s) for s in reversed(shapes)))
+    other.start()
+    assert [dense_us(*s) for s in reversed(shapes)] == want[::-1]
+    other.join()
+    assert got == want[::-1]
 
 
 def test_times_are_read_back(tmp_path):
