@@ -7,6 +7,7 @@
 #include <stdio.h>
 
 #include "../../include/et_amd.h"
+#include "tile_order.h"
 
 namespace et {
 
@@ -169,11 +170,6 @@ __device__ __forceinline__ f16x4 gelu4(f16x4 v) {
 __device__ __forceinline__ float f16_bits_to_float(uint16_t b) {
     return (float)__builtin_bit_cast(f16, b);
 }
-
-// n / d by one scalar multiplication: exact while n * d < 2^32 (magic 0: d = 1).  A division in front of a kernel's
-// first request costs tens of vector instructions, fetched cold at every launch.
-inline unsigned magic_of(int d) { return d == 1 ? 0u : 0xFFFFFFFFu / (unsigned)d + 1u; }
-__device__ __forceinline__ int div_magic(int n, unsigned magic) { return magic ? (int)__umulhi((unsigned)n, magic) : n; }
 
 // The device that a stream's work runs on, whichever is current; the null stream and the per-thread one are the current
 // device's.

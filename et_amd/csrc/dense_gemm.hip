@@ -36,11 +36,9 @@ struct DgArgs {
     int N[DG_MAX_LIN];
     int tile0[DG_MAX_LIN + 1]; // first column tile of each linear in the launch's tile list
     const f16 *X;
-    int nlin, M, K, tiles_m, tiles_n, per_xcd, total;
+    int nlin, M, K, tiles_m, tiles_n, per_xcd;
     int by_column;
-    int group, last; // row tiles (by_column: column tiles) that are walked together; of the last such group
-    int div;         // blocks of a group
-    unsigned div_magic, group_magic, last_magic;
+    GroupWalk walk; // row tiles (by_column: column tiles) are the outer ones
 };
 
 template <int B, int E, class F> __device__ __forceinline__ void dg_for(F &&f) {
@@ -74,12 +72,12 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     a.M = hot_M;
     a.K = hot_K;
     a.per_xcd = hot_per_xcd;
-    a.total = hot_total;
-    a.div = hot_div;
-    a.div_magic = hot_div_magic;
+    a.walk.total = hot_total;
+    a.walk.div = hot_div;
+    a.walk.div_magic = hot_div_magic;
     a.nlin = hot_nlin & 15;
     a.by_column = hot_nlin >> 4 & 1;
-    a.group = hot_nlin >> 5;
+    a.walk.group = hot_nlin >> 5;
     constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char dg_smem[];
     f16 *smem = reinterpret_cast<f16 *>(dg_smem);
@@ -87,15 +85,10 @@ __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     // consecutive ids on one XCD walk the column tiles of a group of row tiles (dg_group), whose X tiles stay in that
     // XCD's L2 meanwhile, and W is everywhere - or, where X is the smaller one, the other way round
     const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-    if (vid >= a.total)
+    if (vid >= a.walk.total)
         return;
-    int outer = div_magic(vid, a.div_magic), inner = vid - outer * a.div;
-    if (a.group > 1) { // (only then: the rest of the struct is a round trip to memory)
-        const int g = outer, in_group = inner;
-        const bool last = (g + 1) * a.div > a.total;
-        inner = div_magic(in_group, last ? a.last_magic : a.group_magic);
-        outer = g * a.group + in_group - inner * (last ? a.last : a.group);
-    }
+    int outer, inner;
+    group_walk_at(a.walk, vid, outer, inner); // (one tile a group: only what came in registers, the rest is a round trip to memory)
     const int tm = a.by_column ? inner : outer, tn_all = a.by_column ? outer : inner;
     int lin = 0, tn = tn_all, N = hot_N;
     const f16 *W = hot_W;
@@ -377,20 +370,14 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
             n += a.N[i];
         }
     }
-    a.total = a.tiles_m * a.tiles_n;
-    a.per_xcd = (a.total + 7) / 8;
     // (every L2 that has part of the work takes the operand that all of the work shares)
     a.by_column = tl_order(2.0 * a.M * a.K, 2.0 * a.K * n, a.tiles_m, a.tiles_n, 4.5e6);
     const int outer = a.by_column ? a.tiles_n : a.tiles_m, inner = a.by_column ? a.tiles_m : a.tiles_n;
-    a.group = dg_group(outer, inner, a.by_column ? BN : BM, a.by_column ? BM : BN, lds <= 80 * 1024 ? 2 : 1);
-    a.last = outer - (outer - 1) / a.group * a.group;
-    a.div = a.group * inner;
-    a.div_magic = magic_of(a.div);
-    a.group_magic = magic_of(a.group);
-    a.last_magic = magic_of(a.last);
+    a.walk = group_walk(outer, inner, dg_group(outer, inner, a.by_column ? BN : BM, a.by_column ? BM : BN, lds <= 80 * 1024 ? 2 : 1));
+    a.per_xcd = (a.walk.total + 7) / 8;
     constexpr auto kern = &dense_gemm_kernel<GELU, WM, WN, TM, TN, ST>;
     launch_kernel<kern>(dim3(a.per_xcd * 8), dim3(WM * WN * 64), lds, st, a.X, a.W[0], a.M, a.K, a.N[0],
-                       a.per_xcd, a.total, a.div, a.div_magic, a.nlin | a.by_column << 4 | a.group << 5, a);
+                       a.per_xcd, a.walk.total, a.walk.div, a.walk.div_magic, a.nlin | a.by_column << 4 | a.walk.group << 5, a);
     return launch_status("dense_gemm launch");
 }
 

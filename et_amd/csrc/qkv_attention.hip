@@ -24,12 +24,13 @@ template <bool MASK>
 __global__ void __launch_bounds__(QA_WAVES * 64) qkv_attention_kernel(const QaArgs a) {
     int b, h;
     if (a.by_seq) {
-        const int i = blockIdx.x >> 3, s = div_magic(i, a.nhead_magic);
-        h = i - s * a.nhead;
-        b = s * 8 + (blockIdx.x & 7);
+        const QuotRem of = quot_rem(blockIdx.x >> 3, a.nhead, a.nhead_magic);
+        h = of.r;
+        b = of.q * 8 + (blockIdx.x & 7);
     } else {
-        b = div_magic(blockIdx.x, a.nhead_magic);
-        h = blockIdx.x - b * a.nhead;
+        const QuotRem of = quot_rem(blockIdx.x, a.nhead, a.nhead_magic);
+        h = of.r;
+        b = of.q;
     }
     if (b < a.batch)
         qkv_attention_block<QA_WAVES, QA_PAIRS, MASK, false>(a, b, h);

@@ -168,11 +168,11 @@ __device__ __forceinline__ bool tl_place(const TlArgs &a, int &rp, int &lin, int
     const int vid = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
     if (vid >= a.nwg)
         return false;
-    const int outer = div_magic(vid, a.div_magic), inner = vid - outer * a.div;
-    rp = a.by_group ? inner : outer;
-    const int rest = (a.by_group ? outer : inner) * a.ipw;
-    lin = div_magic(rest, a.ncg_magic);
-    cg = rest - lin * a.ncg;
+    const QuotRem of = quot_rem(vid, a.div, a.div_magic);
+    rp = a.by_group ? of.r : of.q;
+    const QuotRem rest = quot_rem((a.by_group ? of.q : of.r) * a.ipw, a.ncg, a.ncg_magic);
+    lin = rest.q;
+    cg = rest.r;
     return true;
 }
 

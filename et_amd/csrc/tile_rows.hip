@@ -88,9 +88,10 @@ __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int c16 = lane & 15, g4 = lane >> 4, khalf8 = (g4 & 1) * 8, hi = lane >> 5;
     const unsigned lane_w2 = (unsigned)(hi * 256 + c16 * 16 + khalf8) * 2, hi4 = hi * 4;
-    const int outer = div_magic(vid, a.div_magic), inner = vid - outer * a.div;
-    const int panel = a.by_group ? inner : outer, rest = a.by_group ? outer : inner;
-    const int lin = div_magic(rest, a.ncg_magic), cg = rest - lin * a.ncg;
+    const QuotRem of = quot_rem(vid, a.div, a.div_magic);
+    const int panel = a.by_group ? of.r : of.q;
+    const QuotRem rest = quot_rem(a.by_group ? of.q : of.r, a.ncg, a.ncg_magic);
+    const int lin = rest.q, cg = rest.r;
     const int m0 = panel * TR_BM;
     // the panel: wave w fetches row w, DMA
     if (m0 + wave < a.M) {
