@@ -453,30 +453,18 @@ __device__ __forceinline__ void tl_stream(const char *xlane, int xrow16, const f
     __builtin_amdgcn_s_setprio(0);
 }
 
-// flush for kernels that keep NB static accumulators: acc[j] += cur with a
-// 0/1 mask per accumulator (branch-free; a branch per j makes the compiler
-// keep a copy of every accumulator per pipeline stage)
-template <int NB>
-__device__ __forceinline__ void tl_flush_acc(f32x4 (&acc)[NB][2], int j, f32x4 cur0, f32x4 cur1) {
-#pragma unroll
-    for (int k = 0; k < NB; k++) {
-        const float mk = (k == j) ? 1.0f : 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            acc[k][0][r] = __builtin_fmaf(cur0[r], mk, acc[k][0][r]);
-            acc[k][1][r] = __builtin_fmaf(cur1[r], mk, acc[k][1][r]);
-        }
-    }
-}
-
-// The same with a branch per accumulator instead of NB masked multiply-adds
-// (eight adds per flush instead of 8 NB fused multiply-adds and NB selects).
-// Two things keep the compiler from undoing it: the adds are inline assembly
-// with tied operands (the sum replaces the accumulator in its own registers;
-// otherwise every accumulator gets a second set of registers behind the
-// branches), and the cases are independent ifs with something opaque between
-// them (as an if / else chain they become a switch, whose lowering copies the
-// accumulators around or addresses them through scratch memory).
+// flush for kernels that keep NB static accumulators: acc[j] += cur by a
+// branch per accumulator.  (A factor of 0 or 1 per accumulator makes NaN of an
+// infinite sum in block-rows that it does not belong to; a mask on the sums'
+// bits is two instructions for each value of every accumulator.  48-row panels,
+// factor / mask / branch, us: 5134 rows 4096 -> 1024 80 % 23.6 / 24.6 / 23.4, 16000
+// rows 3072 -> 768 90 % 39.5 / 40.9 / 39.1, 10000 rows 2048 -> 512 50 % 23.1 / 23.4 /
+// 23.1.)  Two things keep the compiler from undoing the branches: the adds are
+// inline assembly with tied operands (the sum replaces the accumulator in its
+// own registers; otherwise every accumulator gets a second set of registers
+// behind the branches), and the cases are independent ifs with something opaque
+// between them (as an if / else chain they become a switch, whose lowering
+// copies the accumulators around or addresses them through scratch memory).
 template <int K>
 __device__ __forceinline__ void tl_add_tied(f32x4 &a, const f32x4 &c) {
     float a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
@@ -486,16 +474,23 @@ __device__ __forceinline__ void tl_add_tied(f32x4 &a, const f32x4 &c) {
                  : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "n"(K));
     a = f32x4{a0, a1, a2, a3};
 }
-template <int NB>
-__device__ __forceinline__ void tl_flush_acc_branch(f32x4 (&acc)[NB][2], int j, const f32x4 &cur0, const f32x4 &cur1) {
-    tl_static_for<0, NB>([&](auto kc) {
-        constexpr int k = decltype(kc)::value;
-        if (j == k) {
-            tl_add_tied<k>(acc[k][0], cur0);
-            tl_add_tied<k>(acc[k][1], cur1);
-        }
-        asm volatile("; after case %0" ::"n"(k));
-    });
+template <int NB, int MS>
+__device__ __forceinline__ void tl_flush_acc(f32x4 (&acc)[NB][MS], int j, const f32x4 (&cur)[MS]) {
+    if constexpr (NB == 1) {
+#pragma unroll
+        for (int m = 0; m < MS; m++)
+            acc[0][m] += cur[m];
+    } else {
+        tl_static_for<0, NB>([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            if (j == k) {
+#pragma unroll
+                for (int m = 0; m < MS; m++)
+                    tl_add_tied<k>(acc[k][m], cur[m]);
+            }
+            asm volatile("; after case %0" ::"n"(k));
+        });
+    }
 }
 
 // Fused skip connection + LayerNorm over a workgroup's 32 finished rows (the
@@ -738,7 +733,7 @@ __global__ void __launch_bounds__(NW * 64) tile_linear_plan_kernel(TL_HOT_PARAMS
         int o[TL_DEPTH];
         tl_preload(data, poff, lane_w, hi, q0, qlast, w, o);
         tl_stream<NB, 2>(xlane, xrow16, data, poff, lane_w, hi, tl_bounds<NB>(bvec), w, o,
-                         [&](int j, const f32x4 (&c)[2]) { tl_flush_acc<NB>(acc, j, c[0], c[1]); });
+                         [&](int j, const f32x4 (&c)[2]) { tl_flush_acc(acc, j, c); });
     }
     tl_epilogue_wave<NB, GELU, !LN>(a, x, stage, Yp, N, nbr, acc, b4);
     if constexpr (LN) {
@@ -1119,7 +1114,7 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_chunked_kernel(TL_HOT
             tl_barrier_lds();
 
             tl_stream<NB, 2>(xlane, xrow16, data, poff, lane_w, hi, tl_bounds<NB>(bcur), w, o,
-                             [&](int j, const f32x4 (&c)[2]) { tl_flush_acc<NB>(acc, j, c[0], c[1]); });
+                             [&](int j, const f32x4 (&c)[2]) { tl_flush_acc(acc, j, c); });
             bvec = bvec_n;
         }
         f16 *stage = stage0 + x.wave * tl_wave_stage_halves<NB>();
@@ -1234,15 +1229,8 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_tall_kernel(TL_HOT_PA
             tl_preload(data, poff, lane_w, hi, b.at[0], max(b.at[NB] - 1, b.at[0]), w, o);
             bvec = ends(c + 1);
             tl_barrier_lds();
-            tl_stream<NB, MS>(xlane, 16 * ldx * 2, data, poff, lane_w, hi, b, w, o, [&](int j, const f32x4 (&s)[MS]) {
-#pragma unroll
-                for (int k = 0; k < NB; k++) {
-                    const float mk = k == j ? 1.0f : 0.0f;
-#pragma unroll
-                    for (int m = 0; m < MS; m++)
-                        acc[k][m] = NB == 1 ? acc[k][m] + s[m] : __builtin_elementwise_fma(s[m], f32x4{mk, mk, mk, mk}, acc[k][m]);
-                }
-            });
+            tl_stream<NB, MS>(xlane, 16 * ldx * 2, data, poff, lane_w, hi, b, w, o,
+                              [&](int j, const f32x4 (&s)[MS]) { tl_flush_acc(acc, j, s); });
         }
         if (SPLIT) {
             if (half)
@@ -1303,11 +1291,6 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_tall_kernel(TL_HOT_PA
 // K = input width, KC / nchunk = the second plan's chunking; skip / gamma /
 // beta belong to the first LayerNorm that runs, gamma2 / beta2 to the second.
 // ---------------------------------------------------------------------------
-#ifdef TL_FFN_MASKED_FLUSH
-#define TL_FFN_FLUSH(acc_, j_, c0_, c1_) tl_flush_acc<NB>(acc_, j_, c0_, c1_)
-#else
-#define TL_FFN_FLUSH(acc_, j_, c0_, c1_) tl_flush_acc_branch<NB>(acc_, j_, c0_, c1_)
-#endif
 constexpr int TL_FFN_WAVES = 16;
 constexpr int TL_FFN_MAX_PHASES = 16;
 
@@ -1487,7 +1470,7 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
         tl_barrier_lds(); // the whole panel has landed; the counters are zero
         {
             tl_stream<NB, 2>(xlane1, xrow1, a.data[0], a.row_offset[0], lane_w, hi, boundsO, wB, oB,
-                             [&](int j, const f32x4 (&c)[2]) { TL_FFN_FLUSH(acc, j, c[0], c[1]); });
+                             [&](int j, const f32x4 (&c)[2]) { tl_flush_acc(acc, j, c); });
         }
         TL_FFN_PRELOAD(data1, poff1, boundsF, wA, oA)
         TlLnOperands<NB, NW, NW> lnop1; // (requested here: their latency runs under the wait for the other waves)
@@ -1532,7 +1515,7 @@ __global__ void __launch_bounds__(TL_FFN_WAVES * 64) tile_ffn_fused_kernel(const
             const char *const xlane2 =
                 reinterpret_cast<const char *>(hs + (p & 1) * hbuf + c16 * ldh + x.khalf8);
             tl_stream<NB, 2>(xlane2, xrow2, data2, poff2, lane_w, hi, boundsS, wA, oA,
-                             [&](int j, const f32x4 (&c)[2]) { TL_FFN_FLUSH(acc, j, c[0], c[1]); });
+                             [&](int j, const f32x4 (&c)[2]) { tl_flush_acc(acc, j, c); });
             tl_signal(ctr + TL_FFN_MAX_PHASES + p, lane);
         }
         boundsS = boundsSn;

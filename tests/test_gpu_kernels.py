@@ -1640,3 +1640,32 @@ def test_tile_linear_whole_rows_infinite_activations(K, form, M, N, Kd):
     assert np.isfinite(fin).all()
     assert np.array_equal(inf[:, ~hit], fin[:, ~hit])
     assert not np.isfinite(inf[:, hit]).any()
+
+
+@pytest.mark.parametrize("form", range(9))
+@pytest.mark.parametrize("M,N,Kd", [(49, 592, 2048), (33, 1024, 1552)])
+def test_tile_linear_chunked_infinite_activations(K, form, M, N, Kd):
+    """the same for the kernels that walk K chunk by chunk, of one to four block-rows a wave: a block-row's sums reach
+    no other block-row of its wave"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile
+    r = rng(1950 + M)
+    lin = make_tile_linear(r, N, Kd, 0.85, seed=M + N, std=0.05, bias_std=0.2)
+    rp, ro = lin["row_ptr"], lin["row_offset"]
+    col = Kd // 2 // 16 * 16
+    hit = np.array([np.isin([0, col], ro[rp[b]:rp[b + 1]]).any() for b in range(N // 16)])
+    assert hit.any() and not hit.all()
+    lt = Linear_tile(Kd, N, M, ro.size, lin["data"], rp, ro, lin["bias"])
+    X = randn_h(r, (M, Kd))
+    Xi, rows = X.copy(), np.arange(M) % 5 == 1
+    Xi[np.ix_(rows, [3, col + 7])] = np.inf
+    try:
+        lib().et_tuning_set(b"tile_splitk_rows", 0)
+        lib().et_tuning_set(b"tile_chunked", form)
+        fin, inf = (host(lt.run(dev(x))).reshape(M, N // 16, 16) for x in (X, Xi))
+    finally:
+        lib().et_tuning_set(b"tile_splitk_rows", -1)
+        lib().et_tuning_set(b"tile_chunked", -1)
+    assert np.isfinite(fin).all()
+    assert np.array_equal(inf[:, ~hit], fin[:, ~hit]) and np.array_equal(inf[~rows], fin[~rows])
+    assert not np.isfinite(inf[rows][:, hit]).any()
