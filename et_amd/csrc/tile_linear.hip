@@ -1168,6 +1168,7 @@ __global__ void __launch_bounds__(TL_CTHREADS) tile_linear_tall_kernel(TL_HOT_PA
     f16 *const stage = xs + (a.nchunk & 1) * pbuf;
     f32x4 *const red = reinterpret_cast<f32x4 *>(stage + BM * LDS);
     static_assert(BM * LDS * 2 % 16 == 0, "aligned sums");
+    static_assert(BM * LDS * 2 + (SPLIT ? BRS * MS * 64 * 16 : 0) <= BM * TL_CHUNK * 2, "the staged rows and sums fit a panel buffer");
     if (wave >= TL_CWAVES) {
         // ---- the fetching waves ----
         const int row0 = (wave - TL_CWAVES) * (BM / TL_FWAVES);
@@ -1723,6 +1724,7 @@ static int launch_chunked_ln_inst(const TlArgs &a, size_t lds, hipStream_t st) {
 
 template <int NB, bool SPLIT, bool GELU>
 static int launch_tall(const TlArgs &a, hipStream_t st) {
+    ET_REQUIRE(a.KC == TL_CHUNK, ET_ERR_UNSUPPORTED, "48-row panels of %d columns instead of %d", a.KC, TL_CHUNK); // (what the kernel stages over)
     constexpr auto k = &tile_linear_tall_kernel<NB, SPLIT, GELU>;
     const size_t lds = 2 * (size_t)16 * TL_TALL * (a.KC + ((a.KC & 31) ? 0 : TL_PAD)) * sizeof(f16);
     launch_kernel<k>(dim3(a.per_xcd * 8), dim3(TL_CTHREADS), lds, st, TL_HOT(a, KC), a);
