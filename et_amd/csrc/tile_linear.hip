@@ -2499,6 +2499,17 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 // their operands in the caches; where they are too large to stay there inside a layer the tile kernels, which read W more
 // often, take a tenth more than estimated and above (12288 rows, 768 -> 3072: the layer 285 us on them, 267 on the product).
 constexpr double DENSE_LAUNCH_US = 3.5;
+struct FullPlansTime {
+    double tiles, dense; // us, with what the line adds
+};
+static FullPlansTime full_plans_time(const int *Ns, const int *ntile, const int *nchunk, const int *launch, int launches, int n,
+                                     int M, int K, bool gelu) {
+    double mb = K * 2e-6 * M;
+    for (int i = 0; i < n; i++)
+        mb += Ns[i] * 2e-6 * M;
+    return {tiles_estimate(Ns, ntile, nchunk, launch, launches, n, M, K, gelu) * (mb > 48.0 ? 1.1 : 1.0),
+            DENSE_LAUNCH_US + dense_gemm_estimate(Ns, n, M, K, gelu)};
+}
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
     if (!g_plan_dense || n > 3)
         return false;
@@ -2513,12 +2524,9 @@ static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool
     }
     if (g_plan_dense == 2)
         return true;
-    const int K = plans[0]->in_feat, launches = join_launches(KC, nchunk, n, launch);
-    const double tiles = tiles_estimate(Ns, ntile, nchunk, launch, launches, n, M, K, gelu);
-    double mb = K * 2e-6 * M;
-    for (int i = 0; i < n; i++)
-        mb += Ns[i] * 2e-6 * M;
-    return DENSE_LAUNCH_US + dense_gemm_estimate(Ns, n, M, K, gelu) < tiles * (mb > 48.0 ? 1.1 : 1.0);
+    const int launches = join_launches(KC, nchunk, n, launch);
+    const FullPlansTime t = full_plans_time(Ns, ntile, nchunk, launch, launches, n, M, plans[0]->in_feat, gelu);
+    return t.dense < t.tiles;
 }
 static int run_plans_dense(const et_tile_plan *const *plans, void *const *Ys, int n, const void *X, int M, bool gelu,
                            hipStream_t st) {
@@ -2889,9 +2897,15 @@ extern "C" int et_tile_plan_ffn_fusable(const et_tile_plan *p1, const et_tile_pl
 }
 
 // Full feed-forward plans: whether the steps of the block (pO: of the whole tail), one after the other, take less than the
-// fused kernel, whose round streams all of W past its panels.  A fused round of full plans takes 14 us and 10.7 per MB of
-// W, and inside a layer a tenth more: 256 wide 26, 384 38 to 42, 512 58 to 65, 640 90 to 100, 768 117 to 130.  Tail fused / by steps, us: 8192 rows 256 wide 27.9 /
-// 33.7, 384 41.8 / 46.9, 512 65.3 / 63.7 (the layer 105.6 / 99.9), 768 130 / 110; 16384 rows 512 wide 131 / 110, 768 258 / 200.
+// fused kernel, whose round streams all of W past its panels; a last round costs as much as a full one, unless the tail's
+// rest runs by steps (et_tile_plan_run_tail).
+// A fused round of the tail takes 14 us and 10.7 per MB of W, and inside a layer a tenth more: 256 wide 26, 384 38 to 42, 512
+// 58 to 65, 640 90 to 100, 768 117 to 130.  Tail fused / by steps, us: 8192 rows 256 wide 27.9 / 33.7, 384 41.8 / 46.9, 512 65.3 / 63.7
+// (the layer 105.6 / 99.9), 768 130 / 110; 16384 rows 512 wide 131 / 110, 768 258 / 200.
+// Of the block alone: 9.4 us, 10.5 per MB and 2.9 for each further chunk of hidden columns, where the steps' estimates are
+// 7 % high.  Fused / by steps, us: 128 -> 512 7200 rows 12.4 / 15.2, 12700 rows (the second round) 23.2 / 17.7; 256 -> 512 8192 14.7 /
+// 16.2, 256 -> 1024 23.6 / 21.5, 384 -> 768 21.5 / 23.2, 12700 rows 38.3 / 31.9, 384 -> 1536 8192 rows 36.9 / 33.6, 640 -> 1280 49.3 / 43.7; from
+// 512 wide on the steps.  Over these widths and 5000 to 16384 rows every choice is the faster one.
 static bool ffn_runs_dense(const et_tile_plan *pO, const et_tile_plan *p1, const et_tile_plan *p2, int M) {
     using namespace et;
     if (!g_plan_dense || !p1->d_dense || !p2->d_dense)
@@ -2899,18 +2913,21 @@ static bool ffn_runs_dense(const et_tile_plan *pO, const et_tile_plan *p1, const
     if (g_plan_dense == 2)
         return true;
     auto linear = [](const et_tile_plan *p, int rows, bool gelu) {
-        int launch = 0;
-        const double tiles = tiles_estimate(&p->out_feat, &p->ntile, &p->nchunk, &launch, 1, 1, rows, p->in_feat, gelu);
-        return p->d_dense ? std::min(tiles, DENSE_LAUNCH_US + dense_gemm_estimate(&p->out_feat, 1, rows, p->in_feat, gelu)) : tiles;
+        const int launch = 0;
+        const FullPlansTime t = full_plans_time(&p->out_feat, &p->ntile, &p->nchunk, &launch, 1, 1, rows, p->in_feat, gelu);
+        return p->d_dense ? std::min(t.tiles, t.dense) : t.tiles;
     };
     auto steps = [&](int rows) { // (a LayerNorm: 5.5 TB/s behind its launch)
         const double ln = 3.0 + 1.1e-6 * rows * p2->out_feat;
         return linear(p1, rows, true) + linear(p2, rows, false) + ln + (pO ? linear(pO, rows, false) + ln : 0.0);
     };
-    const int cus = std::max(et_device_cu_count(), 1), full = M / (cus * TL_BM), rest = M - full * cus * TL_BM;
-    const double round = 15.5 + 11.7 * 512e-6 * ((double)p1->ntile + p2->ntile + (pO ? pO->ntile : 0));
-    // (behind full rounds the rest may run by steps in either case)
-    return steps(M) < full * round + (rest == 0 ? 0.0 : full == 0 ? round : std::min(round, steps(rest)));
+    const int cus = std::max(et_device_cu_count(), 1), panels = (M + TL_BM - 1) / TL_BM, full = panels / cus, rest = panels - full * cus;
+    const double w_mb = 512e-6 * ((double)p1->ntile + p2->ntile + (pO ? pO->ntile : 0));
+    const double round = pO ? 15.5 + 11.7 * w_mb : (9.4 + 10.5 * w_mb + 2.9 * (p2->nchunk - 1)) * 1.07;
+    double fused = round * full;
+    if (rest > 0)
+        fused += pO && full > 0 && rest < tail_min_panels(pO, p1, p2) ? steps(M - full * cus * TL_BM) : round;
+    return steps(M) < fused;
 }
 
 extern "C" int et_tile_plan_run_ffn_ln(const et_tile_plan *p1, const et_tile_plan *p2, void *Y,

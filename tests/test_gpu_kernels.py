@@ -362,6 +362,43 @@ def test_layer_tail_of_full_plans_fused_or_by_steps(K, d, M, one_launch):
     check_close(got, want, max_abs=3e-2, mean_rel=2e-3, what="tail of full plans")  # (as against the oracle, above)
 
 
+@pytest.mark.parametrize("d,F,M,one_launch", [
+    (128, 512, 7200, True),      # a round of the fused kernel is shorter than two linears and a LayerNorm
+    (256, 512, 8192, True),
+    (384, 768, 8192, True),
+    (384, 768, 12700, False),    # ... two rounds are not
+    (256, 1024, 8192, False),
+])
+def test_ffn_of_full_plans_fused_or_by_steps(K, d, F, M, one_launch):
+    """the feed-forward block of full plans with the hidden buffer at hand, either side of the line between the fused kernel
+    and the steps (which write the buffer), against the steps"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile
+    if lib().et_device_cu_count() != 256:
+        pytest.skip("a round is one panel per compute unit of 256")
+    r = rng(3000 + d + M)
+    mk = lambda n, k, gelu, i: (lambda l: Linear_tile(k, n, M, l["row_offset"].size, l["data"], l["row_ptr"], l["row_offset"], l["bias"],
+                                                      gelu))(make_tile_linear(r, n, k, 0.0, seed=i, std=0.05, bias_std=0.2))
+    t1, t2 = mk(F, d, True, 1), mk(d, F, False, 2)
+    x, skip = dev(randn_h(r, (M, d))), dev(randn_h(r, (M, d)))
+    ln = [dev(t) for t in (randn_h(r, (d,), 0.3) + np.float16(1), randn_h(r, (d,), 0.3))]
+
+    def run():
+        hid = torch.full((M, F), 7.0, dtype=torch.float16, device="cuda")
+        out = host(Linear_tile.run_ffn_ln(t1, t2, x, skip, *ln, hidden=hid))
+        return out, bool((hid == 7.0).all())
+
+    got, untouched = run()
+    assert untouched == one_launch
+    try:
+        lib().et_tuning_set(b"tile_fuse_ffn", 0)
+        want, untouched = run()
+    finally:
+        lib().et_tuning_set(b"tile_fuse_ffn", 2)
+    assert not untouched
+    check_close(got, want, max_abs=3e-2, mean_rel=2e-3, what="feed-forward block of full plans")  # (as against the oracle, above)
+
+
 PAIR_CASES = [
     (640, 768, 3072, 0.8),     # BERT-base widths, ten 64-row panels
     (200, 256, 1024, 0.5),     # a ragged last panel (8 rows), two block-rows per wave
