@@ -170,7 +170,7 @@ __device__ __forceinline__ bool tl_place(const TlArgs &a, int &rp, int &lin, int
         return false;
     const QuotRem of = quot_rem(vid, a.div, a.div_magic);
     rp = a.by_group ? of.r : of.q;
-    const QuotRem rest = quot_rem((a.by_group ? of.q : of.r) * a.ipw, a.ncg, a.ncg_magic);
+    const QuotRem rest = quot_rem_small((a.by_group ? of.q : of.r) * a.ipw, a.ncg, a.ncg_magic); // (at most four linears)
     lin = rest.q;
     cg = rest.r;
     return true;

@@ -13,15 +13,19 @@ namespace et {
 
 // A division in front of a kernel's first request costs tens of vector instructions, fetched cold at every launch; this is
 // a scalar multiplication, and another one for the rest.  magic_of(d) is 2^32 / d rounded up (0: d = 1), too large by less
-// than one part in 2^32 / d, so for n < 2^31 the product's high half is the quotient or one more than it: the rest tells.
+// than one part in 2^32 / d: while n * d < 2^32 the product's high half is the quotient, for every other n < 2^31 it is the
+// quotient or one more, and the rest tells.
 inline unsigned magic_of(int d) { return d == 1 ? 0u : 0xFFFFFFFFu / (unsigned)d + 1u; }
 struct QuotRem {
     int q, r;
 };
-ET_BOTH QuotRem quot_rem(int n, int d, unsigned magic) {
+ET_BOTH QuotRem quot_rem_small(int n, int d, unsigned magic) { // n * d < 2^32
     const unsigned q = magic ? (unsigned)((uint64_t)(unsigned)n * magic >> 32) : (unsigned)n;
-    const int r = (int)((unsigned)n - q * (unsigned)d);
-    return r < 0 ? QuotRem{(int)q - 1, r + d} : QuotRem{(int)q, r};
+    return QuotRem{(int)q, (int)((unsigned)n - q * (unsigned)d)};
+}
+ET_BOTH QuotRem quot_rem(int n, int d, unsigned magic) {
+    const QuotRem v = quot_rem_small(n, d, magic);
+    return v.r < 0 ? QuotRem{v.q - 1, v.r + d} : v;
 }
 
 // Outer x inner tiles, walked in groups of `group` outer ones: block `vid` goes through a group's outer tiles first, then to
@@ -41,7 +45,7 @@ ET_BOTH void group_walk_at(const GroupWalk &w, int vid, int &outer, int &inner) 
     inner = of.r;
     if (w.group > 1) {
         const bool last = vid - of.r > w.total - w.div;
-        const QuotRem in = last ? quot_rem(of.r, w.last, w.last_magic) : quot_rem(of.r, w.group, w.group_magic);
+        const QuotRem in = last ? quot_rem_small(of.r, w.last, w.last_magic) : quot_rem_small(of.r, w.group, w.group_magic);
         outer = of.q * w.group + in.r;
         inner = in.q;
     }

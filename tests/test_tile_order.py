@@ -14,6 +14,11 @@ extern "C" void rest(int n, int d, int *out) {
     out[0] = v.q;
     out[1] = v.r;
 }
+extern "C" void rest_small(int n, int d, int *out) {
+    const et::QuotRem v = et::quot_rem_small(n, d, et::magic_of(d));
+    out[0] = v.q;
+    out[1] = v.r;
+}
 extern "C" void walk(int outer, int inner, int group, const int *vid, int n, int *out) {
     const et::GroupWalk w = et::group_walk(outer, inner, group);
     for (int i = 0; i < n; i++)
@@ -72,3 +77,13 @@ def test_grouped_walk_of_many_blocks(order, outer, inner, group):
         g, k = divmod(v, div)
         n = min(group, outer - g * group)
         assert got == (g * group + k % n, k // n), v
+
+
+def test_quotient_of_few_linears(order):
+    """the form without the correction, for up to four linears' column groups: the product stays below 2^32"""
+    out = (C.c_int * 2)()
+    for d in (1, 2, 3, 7, 33, 390, 4095, 4096, 16383):
+        for n in {0, 1, d - 1, d, d + 1, 2 * d - 1, 2 * d, 3 * d - 1, 3 * d, 4 * d - 1}:
+            assert 4 * d * d < 2 ** 32
+            order.rest_small(n, d, out)
+            assert tuple(out) == divmod(n, d), (n, d)
