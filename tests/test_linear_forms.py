@@ -86,10 +86,17 @@ def test_tall_panel_terms_follow_the_estimate(K, Ns, gelu, rows):
 
 
 def test_dense_choice_is_kept_by_its_sizes():
-    """More shapes than the table of kept choices has entries, in two orders and from two threads: always the least block."""
+    """More shapes than the table of kept choices has entries, in two orders and from two threads, neighbours that differ in
+    one thing among them: always the least block."""
     L = lib()
     shapes = [(K, Ns, gelu, rows) for K, Ns, gelu in ((768, (768,), 0), (768, (3072,), 1), (1024, (1024,) * 3, 0), *lf.CHUNKS)
               for rows in (16, 37, 61, 104, 250, 345, 700, 1300, 2048, 5000, 9000, 16384)]
+    one_thing = [(768, (3072,), 0, 2048), (768, (3072,), 1, 2048),                             # GELU
+                 (768, (768,), 0, 2048), (768, (768, 768), 0, 2048), (768, (768,) * 3, 0, 2048),  # linears
+                 (768, (768, 3072), 0, 2048), (768, (768, 768), 0, 2048),                      # the second one's width
+                 (768, (768, 768, 3072), 0, 2048), (768, (768,) * 3, 0, 2048),                 # the third one's
+                 (3072, (768,) * 3, 0, 2048), (3072, (768,) * 3, 0, 1024)]                     # inputs, rows
+    shapes += one_thing * 2
     assert len(shapes) > 64
 
     def dense_us(K, Ns, gelu, rows):
@@ -106,6 +113,7 @@ def test_dense_choice_is_kept_by_its_sizes():
         want = [min(v) for v in zip(*(block_us(f) for f in range(11)))]
     finally:
         L.et_tuning_set(b"dense_form", -1)
+    assert all(a != b for a, b in zip(want[-len(one_thing):], want[-len(one_thing) + 1:]))
     assert [dense_us(*s) for s in shapes] == want
     got = []
     other = threading.Thread(target=lambda: got.extend(dense_us(*s) for s in reversed(shapes)))
