@@ -60,6 +60,7 @@ PROTOTYPES = {
     "et_wait_status_take": (_i, []),
     "et_wait_status_raise_for_test": (None, []),
     "et_tile_plan_run_multi": (_i, [C.POINTER(_vp), C.POINTER(_vp), _i, _vp, _i, _vp]),
+    "et_tile_plan_prefers_dense": (_i, [_i, _ip, _i, _i, _i]),
     "et_tile_plan_estimate": (_i, [_i, _ip, _ip, _i, _i, _i, C.POINTER(C.c_double), C.POINTER(C.c_double)]),
     "et_tile_plan_launches": (_i, [_i, _ip, _i, _ip, _ip, _ip]),
     "et_tile_plan_query": (_i, [_vp, C.POINTER(_i), C.POINTER(_i), C.POINTER(_i), C.POINTER(_i), C.POINTER(_i)]),

@@ -26,6 +26,7 @@ SPARSITIES = (0.0, 0.5, 0.8, 0.9)
 FORMS = ((32, 8, 1), (32, 8, 2), (32, 8, 3), (64, 12, 2), (64, 8, 3), (64, 8, 2), (64, 8, 1))  # rows, waves, block-rows
 DENSE_LAUNCH = 3.5  # us that the library adds to the dense product's estimate when it is weighed against the tile kernels
 LAUNCH = 3.0        # ... of which so many are the launch, which the dense product's estimate leaves out
+TILES_BEYOND_MB, TILES_BEYOND = 48.0, 1.1  # the tile kernels' share of their estimate where input and result are larger
 TERMS = {  # kernel -> its cost terms, in the order of features()
     "32 rows": "launch traffic traffic_over round item item_nb item_stream panel out gelu mfma result wg".split(),
     "64 rows": "launch traffic traffic_over round item item_nb item_stream panel out gelu mfma result wg".split(),
@@ -279,7 +280,7 @@ def report(lines):
     both = {}
     for l in lines:
         if l["form"] == "auto+dense":
-            both.setdefault(shape_of(l), {})["est_tiles"] = l["est"]
+            both.setdefault(shape_of(l), {"of": (l["inputs"], l["outputs"], l["rows"])})["est_tiles"] = l["est"]
     for l in lines:
         if shape_of(l) in both:
             b = both[shape_of(l)]
@@ -289,11 +290,17 @@ def report(lines):
                 if l["est"] < b.get("est_dense", 1e30):
                     b["est_dense"], b["dense"] = l["est"], l["us"]
     for extra in (DENSE_LAUNCH - 0.3, DENSE_LAUNCH, DENSE_LAUNCH + 0.3):
-        lost = [(b["dense"] if extra + b["est_dense"] < b["est_tiles"] else b["tiles"]) / min(b["dense"], b["tiles"]) - 1
+        lost = [(b["dense"] if takes_dense(*b["of"], b["est_tiles"], b["est_dense"], extra) else b["tiles"]) / min(b["dense"], b["tiles"]) - 1
                 for b in both.values() if "est_dense" in b]
         if lost:
             print(f"full plans, {extra:.1f} us on top of the dense product's estimate: {100 * sum(lost) / len(lost):.1f} % behind the "
                   f"faster of the two, {100 * max(lost):.0f} % at most")
+
+
+def takes_dense(K, Ns, rows, est_tiles, est_dense, extra=DENSE_LAUNCH):
+    """the library's line for full plans (et_tile_plan_prefers_dense)"""
+    mb = 2e-6 * rows * (K + sum(Ns))
+    return extra + est_dense < est_tiles * (TILES_BEYOND if mb > TILES_BEYOND_MB else 1.0)
 
 
 def fit(lines):

@@ -2495,10 +2495,13 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
 // tile.  3.0 of the 3.5 us stand for the launch, which dense_gemm_estimate leaves out.  On 252 full plans (16 to 16384 rows,
 // random weights, launches of a graph) the choice is then 0.1 % behind the faster side in the mean and 8 % at most, on the
-// 80 of bench/linear_forms.py 0.1 and 3 %; with 0.3 us less 0.2 and 17 %, with 0.3 more 1.5 and 14 %.  Those launches find
-// their operands in the caches; where they are too large to stay there inside a layer the tile kernels, which read W more
-// often, take a tenth more than estimated and above (12288 rows, 768 -> 3072: the layer 285 us on them, 267 on the product).
-constexpr double DENSE_LAUNCH_US = 3.5;
+// 80 of bench/linear_forms.py 0.2 and 8 %; with 0.3 us less 0.4 and 15 %, with 0.3 more 1.3 and 14 %.  Those launches find
+// their operands in the caches; where input and result do not stay there the tile kernels, which read W more often, take
+// longer than estimated: from 48 MB on they count a tenth more.  99 plans of 256 to 1024 inputs for which that tenth decides,
+// or would with a lower line, by stream, how much longer than the product the tile kernels take on the same operands / on
+// operands that change: 10 to 16 MB +1 / -4 %, 16 to 24 +2 / +1, 40 to 48 +4 / +4 (from -3 to +15), 48 to 64 +8 / +6, 64 to 110 +1
+// / +14, 110 to 200 +6 / +12.
+constexpr double DENSE_LAUNCH_US = 3.5, TILES_BEYOND_MB = 48.0, TILES_BEYOND = 1.1;
 struct FullPlansTime {
     double tiles, dense; // us, with what the line adds
 };
@@ -2507,7 +2510,7 @@ static FullPlansTime full_plans_time(const int *Ns, const int *ntile, const int 
     double mb = K * 2e-6 * M;
     for (int i = 0; i < n; i++)
         mb += Ns[i] * 2e-6 * M;
-    return {tiles_estimate(Ns, ntile, nchunk, launch, launches, n, M, K, gelu) * (mb > 48.0 ? 1.1 : 1.0),
+    return {tiles_estimate(Ns, ntile, nchunk, launch, launches, n, M, K, gelu) * (mb > TILES_BEYOND_MB ? TILES_BEYOND : 1.0),
             DENSE_LAUNCH_US + dense_gemm_estimate(Ns, n, M, K, gelu)};
 }
 static bool plans_run_dense(const et_tile_plan *const *plans, int n, int M, bool gelu) {
@@ -2804,6 +2807,24 @@ extern "C" int et_tile_plan_estimate(int in_feat, const int *out_feat, const int
     *tiles_us = tiles_estimate(out_feat, ntile, nchunk, launch, launches, n, M, in_feat, gelu != 0);
     *dense_us = dense_gemm_estimate(out_feat, n, M, in_feat, gelu != 0);
     return ET_OK;
+}
+
+extern "C" int et_tile_plan_prefers_dense(int in_feat, const int *out_feat, int n, int M, int gelu) {
+    using namespace et;
+    if (!g_plan_dense || !out_feat || n < 1 || n > 3 || M <= 0 || in_feat <= 0 || in_feat % 32 != 0)
+        return 0;
+    int ntile[3], KC[3], nchunk[3], launch[3];
+    for (int i = 0; i < n; i++) {
+        if (out_feat[i] <= 0 || out_feat[i] % 16 != 0)
+            return 0;
+        ntile[i] = (in_feat / 16) * (out_feat[i] / 16);
+        plan_chunking(in_feat, out_feat[i], &KC[i], &nchunk[i]);
+    }
+    if (g_plan_dense == 2)
+        return 1;
+    const int launches = join_launches(KC, nchunk, n, launch);
+    const FullPlansTime t = full_plans_time(out_feat, ntile, nchunk, launch, launches, n, M, in_feat, gelu != 0);
+    return t.dense < t.tiles;
 }
 
 extern "C" int et_tile_plan_launches(int in_feat, const int *out_feat, int n, int *launch, int *nchunk, int *chunk_cols) {

@@ -372,6 +372,8 @@ int et_tile_plan_launches(int in_feat, const int *out_feat, int n, int *launch,
  * Follows the tuning keys: a forced form's own estimate. */
 int et_tile_plan_estimate(int in_feat, const int *out_feat, const int *ntile, int n, int M, int gelu,
                           double *tiles_us, double *dense_us);
+/* Host only: whether plans of full in_feat x out_feat[i] matrices (n <= 3) run as a dense product over M rows. */
+int et_tile_plan_prefers_dense(int in_feat, const int *out_feat, int n, int M, int gelu);
 /* a plan's sizes and its column chunks */
 int et_tile_plan_query(const et_tile_plan *plan, int *in_feat, int *out_feat,
                        int *ntile, int *nchunk, int *chunk_cols);

@@ -123,6 +123,37 @@ def test_dense_choice_is_kept_by_its_sizes():
     assert got == want[::-1]
 
 
+def test_line_of_full_plans_is_the_librarys():
+    """the program's line between tile kernels and dense product, among others where input and result beyond 48 MB decide"""
+    L, beyond = lib(), 0
+    for K, Ns, gelu in ((256, (1024,), 1), (512, (512,), 0), (768, (768,), 0), (768, (3072,), 1), (768, (768,) * 3, 0), (640, (640,) * 3, 0), (512, (1024,), 0), *lf.CHUNKS):
+        for rows in [16, 100, 1000, 3000, *range(4000, 40000, 311)]:
+            n, t, g = len(Ns), C.c_double(), C.c_double()
+            assert L.et_tile_plan_estimate(K, (C.c_int * n)(*Ns), (C.c_int * n)(*[(K // 16) * (v // 16) for v in Ns]), n, rows,
+                                           gelu, C.byref(t), C.byref(g)) == 0
+            takes = lf.takes_dense(K, Ns, rows, t.value, g.value)
+            beyond += takes != (lf.DENSE_LAUNCH + g.value < t.value)
+            assert L.et_tile_plan_prefers_dense(K, (C.c_int * n)(*Ns), n, rows, gelu) == takes, (K, Ns, rows)
+    if L.et_device_cu_count() in (0, 256):  # (without a device the estimates count one compute unit)
+        assert beyond > 0
+
+
+def test_prefers_dense_follows_its_key_and_the_plans_that_have_a_dense_form():
+    L, one = lib(), lambda *v: (C.c_int * len(v))(*v)
+    sizes = (768, one(768), 1, 16, 0)
+    try:
+        assert L.et_tuning_set(b"plan_dense", 2) == 0
+        assert L.et_tile_plan_prefers_dense(*sizes) == 1
+        assert L.et_tile_plan_prefers_dense(784, one(768), 1, 16, 0) == 0  # K not a multiple of 32: no row-major W
+        assert L.et_tile_plan_prefers_dense(768, one(768, 768, 768, 768), 4, 16, 0) == 0
+        assert L.et_tile_plan_prefers_dense(768, one(760), 1, 16, 0) == 0 and L.et_tile_plan_prefers_dense(768, None, 1, 16, 0) == 0
+        assert L.et_tile_plan_prefers_dense(768, one(768), 1, 0, 0) == 0
+        assert L.et_tuning_set(b"plan_dense", 0) == 0
+        assert L.et_tile_plan_prefers_dense(*sizes) == 0
+    finally:
+        L.et_tuning_set(b"plan_dense", 1)
+
+
 def test_times_are_read_back(tmp_path):
     p = tmp_path / "times.txt"
     p.write_text("A heading.\n\n768 768+768 1 0.8 100 panel3 2 7.25 6.90\n768 768+768 1 0.8 100 auto 0 7.10 6.90\n")
