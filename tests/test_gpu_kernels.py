@@ -1407,13 +1407,14 @@ def test_tile_linear_multi_of_different_column_chunks(K, M, Kd, Ns, sp):
 
 @pytest.mark.parametrize("form", range(8))
 def test_dense_product_stages(K, form):
-    """every block size, from fewer steps of 64 columns than stages (two to six) to more, whole and half last steps"""
+    """every block size, from fewer steps of 64 columns than stages (two to eight here, up to twelve below) to more, whole and
+    half last steps"""
     from et_amd import lib
     r = rng(90)
     M, N = 1025, 400
     try:
         lib().et_tuning_set(b"dense_form", form)
-        for Kd in (32, 64, 96, 128, 160, 192, 224, 256, 320, 384, 416, 448, 512, 608):
+        for Kd in (32, 64, 96, 128, 160, 192, 224, 256, 320, 384, 416, 448, 512, 608, 672, 704, 736, 768, 832):
             X, W, b = randn_h(r, (M, Kd)), randn_h(r, (N, Kd), Kd ** -0.5), randn_h(r, (N,), 0.2)
             got = host(K.row_spmm_add_bias(dev(X), dev(W), dev(b)))
             want = X.astype(np.float64) @ W.astype(np.float64).T + b.astype(np.float64)
@@ -1480,19 +1481,21 @@ def test_full_plan_as_dense_product(K, form, M, Ns, Kd, gelu):
 
 
 @pytest.mark.parametrize("M,Ns,Kd,gelu", [
-    (256, (192,), 128, False),           # one whole block, as many steps as stages
-    (257, (208,), 96, True),             # a row and a piece into the next blocks; half a step at the end (GELU: one linear)
+    (192, (256,), 128, False),           # one whole block, as many steps as stages
+    (193, (272,), 96, True),             # a row and a piece into the next blocks; half a step at the end (GELU: one linear)
+    (256, (192,), 128, False),           # a block and a third of the rows, three quarters of one's columns
+    (257, (208,), 96, True),
     (100, (400,), 64, False),            # less than a block of rows, a single step
     (520, (192, 384, 16), 1056, False),  # three linears; 16.5 steps
 ])
-def test_full_plan_as_dense_product_256x192(K, M, Ns, Kd, gelu):
-    """the same for blocks of 256 x 192"""
+def test_full_plan_as_dense_product_192x256(K, M, Ns, Kd, gelu):
+    """the same for blocks of 192 x 256"""
     test_full_plan_as_dense_product(K, 5, M, Ns, Kd, gelu)
 
 
 @pytest.mark.parametrize("form", [8, 9, 10])
 def test_dense_product_stages_of_small_blocks(K, form):
-    """the same for the blocks of four waves, with six to twelve stages"""
+    """the same for the other blocks of four waves, with six, seven and twelve stages: as many as 768 columns have steps"""
     test_dense_product_stages(K, form)
 
 
