@@ -55,13 +55,14 @@ __device__ __forceinline__ int dg_swizzle(int r, int kc) { return kc ^ ((r >> 1)
 // step's second half of fragments is read while the first half multiplies, then the stage is handed back, the step ST
 // later requested into it and the next step's first fragments read while the second half multiplies: fragment reads,
 // requests and the barrier run under MFMAs.
-// us a launch, with LDS reads and at most three stages' requests in one go or half of a step / as here, in turn on one
-// machine: 8192 rows 768 -> 768 13.0 / 12.8, 768 -> 928 15.6 / 15.6, 768 -> 1536 22.4 / 21.7, 768 -> 3072 42.1 / 42.6, 3072 ->
-// 768 42.3 / 36.2; 2000 rows 768 -> 2304 12.0 / 11.5, 3072 -> 768 17.3 / 16.1; 2003 rows 3072 -> 3072 44.5 / 39.8; 1200 rows 4096
-// -> 1024 21.8 / 19.1; 16384 rows 1024 -> 4096 126.8 / 122.4 (1120 TFLOP/s), 4096 -> 1024 104.8 / 100.3 (1370); 4096 x 4096 x
-// 4096 106.0 / 101.7 (1350), 8192 x 8192 x 8192 838 / 780 (1410).  Of that, as the mean over 60 shapes: reads between the
-// products 256 x 256 6 %, 256 x 192 4 %, else 2 %; requests over the whole step, with three stages and more, 4 to 5 %; the
-// barrier in front of a half's last products 1 to 3 % where a CU has one workgroup.
+// us a launch, with LDS reads in one go, requests in half of a step and blocks of 64 x 128 to 256 x 256 in two or three
+// stages / as here, in turn on one machine: 8192 rows 768 -> 768 14.4 / 13.7, 768 -> 928 16.7 / 16.6, 768 -> 1536 23.2 / 23.1,
+// 768 -> 3072 42.4 / 41.8, 3072 -> 768 44.3 / 37.0; 2000 rows 768 -> 2304 13.5 / 12.4, 3072 -> 768 18.8 / 17.0; 2003 rows 3072 ->
+// 3072 45.9 / 37.2; 1200 rows 4096 -> 1024 23.3 / 20.4; 16384 rows 1024 -> 4096 126.3 / 119.8 (1150 TFLOP/s), 4096 -> 1024 108.6
+// / 103.4 (1330); 4096 x 4096 x 4096 108.6 / 103.4 (1330), 8192 x 8192 x 8192 897 / 753 (1460).
+// In the same blocks, as the mean over 60 shapes: reads between the products 256 x 256 6 %, else 2 %; requests over the
+// whole step, with three stages and more, 4 to 5 %; the barrier in front of a half's last products 1 to 3 % where a CU has
+// one workgroup.
 template <bool GELU, int WM, int WN, int TM, int TN, int ST>
 __global__ void __launch_bounds__(WM *WN * 64) dense_gemm_kernel(
     // (what the first requests need arrives in registers with the wave)
@@ -341,6 +342,10 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 // within 2 %).  8192 x 8192 x 8192 931 -> 863 us (64 x 128 blocks 2370 -> 1240, 128 x 192 1190 -> 930), 2003 rows 3072 -> 3072
 // 46.4 -> 44.6, 16384 rows 1024 -> 4096 128.8 -> 126.7.  Not where all blocks are at work at once: 2000 rows 768 -> 2304 (192
 // blocks) took 12.5 us instead of 12.0.
+// Where a group saves few tiles it is a trade: whole unpruned layers 512 wide, whose Q/K/V launch takes in 16 tiles a step
+// instead of 17, without groups / with them, us: on operands that change from pass to pass 33 x 337 rows 144.4 / 146.1, 21 x 600
+// 174.6 / 169.5, 24 x 512 163.4 / 160.8, 26 x 512 172.8 / 168.2; on the same ones at every pass 137.5 / 139.0, 157.8 / 159.3,
+// 143.4 / 143.5, 153.0 / 155.1.
 static int dg_group(int outer, int inner, int outer_rows, int inner_rows, int per_cu) {
     const int cus = std::max(et_device_cu_count(), 8), at_once = cus / 8 * per_cu;
     if ((long)outer * inner <= (long)cus * per_cu)
