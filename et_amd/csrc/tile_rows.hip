@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(TR_WAVES * 64) tile_rows_kernel(
     const unsigned lane_w2 = (unsigned)(hi * 256 + c16 * 16 + khalf8) * 2, hi4 = hi * 4;
     const QuotRem of = quot_rem(vid, a.div, a.div_magic);
     const int panel = a.by_group ? of.r : of.q;
-    const QuotRem rest = quot_rem_small(a.by_group ? of.q : of.r, a.ncg, a.ncg_magic); // (at most four linears)
+    const QuotRem rest = quot_rem(a.by_group ? of.q : of.r, a.ncg, a.ncg_magic);
     const int lin = rest.q, cg = rest.r;
     const int m0 = panel * TR_BM;
     // the panel: wave w fetches row w, DMA
