@@ -502,11 +502,13 @@ __device__ __forceinline__ void tl_flush_acc(f32x4 (&acc)[NB][MS], int j, const 
 // registers).  A row of 768 is one and a half pieces for 64 lanes and three for
 // 32, and two rows share the sums' exchanges: 140 vector instructions a wave and
 // LayerNorm fewer than row after row, and the layer tail keeps its registers out of
-// memory.  Whole layers of 16 x 512 rows 77.2 -> 75.0 us, with pruned values 79.1 ->
-// 77.1, the stack of 64 ragged sequences 2216 -> 2152.  The operands that come from
-// global memory (the skip rows, gamma, beta) are requested by tl_ln_fetch, which a wave
-// calls BEFORE the barrier that ends the staging writes, so that their latency runs
-// under the wait for the other waves.
+// memory.  Whole layers of 16 x 512 rows 82.4 -> 79.7 us, with pruned values 83.8 ->
+// 82.2, the stack of 64 ragged sequences 2287 -> 2226 (inputs that change from pass to
+// pass).  The sums are those of skip_layernorm.hip to the bit; those of a row over 64
+// lanes differed from them in the last bit of a variance.
+// The operands that come from global memory (the skip rows, gamma, beta) are requested
+// by tl_ln_fetch, which a wave calls BEFORE the barrier that ends the staging writes, so
+// that their latency runs under the wait for the other waves.
 template <int NB, int NW, int NLW>
 struct TlLnOperands {
     static constexpr int LPR = NW * NB > 64 ? 64 : 32;                         // lanes per row
