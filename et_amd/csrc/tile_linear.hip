@@ -2497,9 +2497,8 @@ int dense_from_plan(f16 *W, const f16 *data, const int *cptr, int K, int KC, int
 // rows on (many outputs) or some thousand (few).  The tile kernels stream W once per 32 or 64 rows and walk it tile by
 // tile.  3.0 of the 3.5 us stand for the launch, which dense_gemm_estimate leaves out.  On 252 full plans (16 to 16384 rows,
 // random weights, launches of a graph) the choice is then 0.1 % behind the faster side in the mean and 8 % at most, on the
-// 80 of bench/linear_forms.py (two runs) 0.1 to 0.2 and 2 to 8 %; with 0.3 us less 0.3 to 0.4 and 16 %, with 0.3 more 1.1 to 1.3
-// and 14 %.  Those launches find
-// their operands in the caches; where input and result do not stay there the tile kernels, which read W more often, take
+// 80 of bench/linear_forms.py 0.1 to 0.2 % (four runs; 2 to 12 % at most), with 0.3 us less 0.3 to 0.4 %, with 0.3 more 1.1
+// to 1.3 %.  Those launches find their operands in the caches; where input and result do not stay there the tile kernels, which read W more often, take
 // longer than estimated: from 48 MB on they count a tenth more.  99 plans of 256 to 1024 inputs for which that tenth decides,
 // or would with a lower line, by stream, how much longer than the product the tile kernels take on the same operands / on
 // operands that change: 10 to 16 MB +1 / -4 %, 16 to 24 +2 / +1, 40 to 48 +4 / +4 (from -3 to +15), 48 to 64 +8 / +6, 64 to 110 +1
