@@ -378,7 +378,8 @@ template <bool GELU, int WM, int WN, int TM, int TN, int ST> static int dg_launc
     // (every L2 that has part of the work takes the operand that all of the work shares)
     a.by_column = tl_order(2.0 * a.M * a.K, 2.0 * a.K * n, a.tiles_m, a.tiles_n, 4.5e6);
     const int outer = a.by_column ? a.tiles_n : a.tiles_m, inner = a.by_column ? a.tiles_m : a.tiles_n;
-    a.walk = group_walk(outer, inner, dg_group(outer, inner, a.by_column ? BN : BM, a.by_column ? BM : BN, lds <= 80 * 1024 ? 2 : 1));
+    if (!group_walk(a.walk, outer, inner, dg_group(outer, inner, a.by_column ? BN : BM, a.by_column ? BM : BN, lds <= 80 * 1024 ? 2 : 1)))
+        return ROWS_TOO_MANY;
     a.per_xcd = (a.walk.total + 7) / 8;
     constexpr auto kern = &dense_gemm_kernel<GELU, WM, WN, TM, TN, ST>;
     launch_kernel<kern>(dim3(a.per_xcd * 8), dim3(WM * WN * 64), lds, st, a.X, a.W[0], a.M, a.K, a.N[0],
@@ -467,8 +468,8 @@ void set_dense_form(int v) { g_dense_form = v < DG_FORMS ? v : -1; }
 
 // nlin linears over the same X in one launch.  Returns ET_ERR_UNSUPPORTED where
 // the shapes do not fit this kernel (the caller then takes the tile path).
-int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, const void *const *biases,
-                      const int *Ns, int nlin, int M, int K, bool gelu, hipStream_t st) {
+static int dense_gemm_rows(void *const *Ys, const void *X, const void *const *Ws, const void *const *biases,
+                           const int *Ns, int nlin, int M, int K, bool gelu, hipStream_t st) {
     if (nlin < 1 || nlin > DG_MAX_LIN || K < 32 || K % 32 != 0 || M <= 0)
         return ET_ERR_UNSUPPORTED;
     DgArgs a;
@@ -507,6 +508,20 @@ int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, con
 #undef DG_CASE
     }
     return ET_ERR_UNSUPPORTED;
+}
+int dense_gemm_launch(void *const *Ys, const void *X, const void *const *Ws, const void *const *biases,
+                      const int *Ns, int nlin, int M, int K, bool gelu, hipStream_t st) {
+    int rc = dense_gemm_rows(Ys, X, Ws, biases, Ns, nlin, M, K, gelu, st);
+    if (rc != ROWS_TOO_MANY)
+        return rc;
+    const int first = M / 2 / 256 * 256; // (rows are independent)
+    ET_REQUIRE(first > 0, ET_ERR_UNSUPPORTED, "dense product: %d rows and so many outputs are too many blocks", M);
+    void *rest[DG_MAX_LIN];
+    for (int i = 0; i < nlin; i++)
+        rest[i] = static_cast<f16 *>(Ys[i]) + (size_t)first * Ns[i];
+    rc = dense_gemm_launch(Ys, X, Ws, biases, Ns, nlin, first, K, gelu, st);
+    return rc != ET_OK ? rc
+                       : dense_gemm_launch(rest, static_cast<const f16 *>(X) + (size_t)first * K, Ws, biases, Ns, nlin, M - first, K, gelu, st);
 }
 
 } // namespace et

@@ -170,7 +170,7 @@ __device__ __forceinline__ bool tl_place(const TlArgs &a, int &rp, int &lin, int
         return false;
     const QuotRem of = quot_rem(vid, a.div, a.div_magic);
     rp = a.by_group ? of.r : of.q;
-    const QuotRem rest = quot_rem_small((a.by_group ? of.q : of.r) * a.ipw, a.ncg, a.ncg_magic); // (at most four linears)
+    const QuotRem rest = quot_rem((a.by_group ? of.q : of.r) * a.ipw, a.ncg, a.ncg_magic);
     lin = rest.q;
     cg = rest.r;
     return true;
@@ -2159,8 +2159,8 @@ static int launch_resident64(const TlArgs &a, size_t lds, hipStream_t st) {
     return launch_status("tile_linear (64-row panels) launch");
 }
 
-static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, int K,
-                       int KC, int nchunk, bool gelu, int mode, hipStream_t st) {
+static int tile_launch_rows(const TlProblem *probs, int nlin, const f16 *X, int M, int K,
+                            int KC, int nchunk, bool gelu, int mode, hipStream_t st) {
     TlArgs a;
     memset(&a, 0, sizeof(a));
     int nbr_max = 0;
@@ -2213,7 +2213,7 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         }
         return tile_rows_launch(l, Ys, nlin, X, M, K, pairs, gelu, raw, st);
     }
-    auto place = [&](int bm, int order) { // order: by_group, or -1 to be worked out
+    auto place = [&](int bm, int order) { // order: by_group, or -1 to be worked out; false: too many workgroups
         const int panels = (M + bm - 1) / bm, per_rp = a.ncg * nlin;
         while (per_rp % a.ipw)
             a.ipw--; // (a tuning value: the items of a workgroup are one panel's)
@@ -2229,6 +2229,7 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         a.div = a.by_group ? panels : per_rp / a.ipw;
         a.div_magic = magic_of(a.div);
         a.ncg_magic = magic_of(a.ncg);
+        return quotients_fit((int64_t)panels * (per_rp / a.ipw), a.div) && quotients_fit(per_rp, a.ncg);
     };
     int nb = 0, order = -1;
     if (mode == TL_PLAN && nchunk == 1) { // (on whole rows: returned above)
@@ -2236,7 +2237,8 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         a.ncg = c.ncg;
         a.ipw = c.d;
         if (c.form->rows == TL_BM64) {
-            place(TL_BM64, c.by_group);
+            if (!place(TL_BM64, c.by_group))
+                return ROWS_TOO_MANY;
             if (c.form->waves == 12)
                 return gelu ? launch_resident64<2, true, 12>(a, c.lds, st) : launch_resident64<2, false, 12>(a, c.lds, st);
             if (c.form->nb == 3)
@@ -2253,7 +2255,8 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
             const int brs = tall_block_rows(which);
             a.ncg = (nbr_max + brs - 1) / brs;
             a.ipw = 1;
-            place(16 * TL_TALL, -1);
+            if (!place(16 * TL_TALL, -1))
+                return ROWS_TOO_MANY;
             switch (which) {
             case TL_BY_TALL: return gelu ? launch_tall<1, false, true>(a, st) : launch_tall<1, false, false>(a, st);
             case TL_BY_TALL_2: return gelu ? launch_tall<2, false, true>(a, st) : launch_tall<2, false, false>(a, st);
@@ -2265,7 +2268,8 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
             const int cnb = which;
             a.ncg = (nbr_max + TL_CWAVES * cnb - 1) / (TL_CWAVES * cnb);
             a.ipw = 1;
-            place(TL_BM, -1);
+            if (!place(TL_BM, -1))
+                return ROWS_TOO_MANY;
             const size_t lds = 2 * (size_t)TL_BM * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16) +
                                (size_t)TL_CWAVES * TL_BM * (16 * cnb + 8) * sizeof(f16);
             switch (cnb) {
@@ -2279,7 +2283,8 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
         a.ncg = (nbr_max + TL_WAVES * nb - 1) / (TL_WAVES * nb);
         a.ipw = 1;
     }
-    place(TL_BM, order);
+    if (!place(TL_BM, order))
+        return ROWS_TOO_MANY;
     const size_t lds_x = (size_t)TL_BM * (KC + ((KC & 31) ? 0 : TL_PAD)) * sizeof(f16);
     const size_t lds_y = (size_t)TL_BM * (TL_WAVES * nb * 16 + TL_PAD) * sizeof(f16);
     // plan kernel: panel + one private staging tile per wave; generic kernel:
@@ -2294,6 +2299,22 @@ static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, in
     if (mode == TL_FILTER)
         return gelu ? launch_nb<true, TL_FILTER>(nb, a, lds, st) : launch_nb<false, TL_FILTER>(nb, a, lds, st);
     return gelu ? launch_nb<true, TL_DENSE>(nb, a, lds, st) : launch_nb<false, TL_DENSE>(nb, a, lds, st);
+}
+
+static int tile_launch(const TlProblem *probs, int nlin, const f16 *X, int M, int K, int KC, int nchunk, bool gelu, int mode,
+                       hipStream_t st) {
+    int rc = tile_launch_rows(probs, nlin, X, M, K, KC, nchunk, gelu, mode, st);
+    if (rc != ROWS_TOO_MANY)
+        return rc;
+    const int first = M / 2 / 64 * 64; // (rows are independent)
+    ET_REQUIRE(first > 0, ET_ERR_UNSUPPORTED, "tile_linear: %d rows and so many outputs are too many workgroups", M);
+    TlProblem rest[TL_MAX_LIN];
+    for (int i = 0; i < nlin; i++) {
+        rest[i] = probs[i];
+        rest[i].Y += (size_t)first * probs[i].N;
+    }
+    rc = tile_launch(probs, nlin, X, first, K, KC, nchunk, gelu, mode, st);
+    return rc != ET_OK ? rc : tile_launch(rest, nlin, X + (size_t)first * K, M - first, K, KC, nchunk, gelu, mode, st);
 }
 
 static void chunking(int K, int *KC, int *nchunk, int panel = TL_MAX_PANEL) {

@@ -297,10 +297,12 @@ int tile_rows_launch(const LfLinear *lins, f16 *const *Ys, int nlin, const f16 *
     const int per = (TR_WAVES >> a.ls) * a.nb;
     a.ncg = (nbr_max + per - 1) / per;
     const int panels = (M + TR_BM - 1) / TR_BM;
-    a.total = panels * a.ncg * nlin;
-    a.per_xcd = (a.total + 7) / 8;
     a.by_group = tl_order(2.0 * M * K, 1024.0 * pairs * nbr_max * nlin, panels, a.ncg * nlin, 2.5e6);
     a.div = a.by_group ? panels : a.ncg * nlin;
+    if (!quotients_fit((int64_t)panels * a.ncg * nlin, a.div) || !quotients_fit((int64_t)a.ncg * nlin, a.ncg))
+        return ROWS_TOO_MANY;
+    a.total = panels * a.ncg * nlin;
+    a.per_xcd = (a.total + 7) / 8;
     a.div_magic = magic_of(a.div);
     a.ncg_magic = magic_of(a.ncg);
     const size_t lds = tile_rows_lds(K);

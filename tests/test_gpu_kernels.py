@@ -1443,6 +1443,54 @@ def test_dense_product_walks_groups_of_tiles(K, M, N):
     assert np.abs(got.astype(np.float64) - want).max() <= 2.0 ** -11 * max(8.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("M,N", [
+    (65536, 32016),     # groups of sixteen row tiles would be beyond the quotient's 32 bits: eight
+    (65536, 131072),    # single tiles are: the rows in two launches
+])
+def test_dense_product_of_many_blocks(K, M, N):
+    """so many blocks of 32 x 64 that their places need smaller groups, or two launches, against torch"""
+    from et_amd import lib
+    g = torch.Generator(device="cuda").manual_seed(92)
+    X, W, b = (torch.randn(s, generator=g, device="cuda").to(torch.float16) for s in ((M, 32), (N, 32), (N,)))
+    try:
+        lib().et_tuning_set(b"dense_form", 8)
+        got = K.row_spmm_add_bias(X, W, b)
+    finally:
+        lib().et_tuning_set(b"dense_form", -1)
+    for m in range(0, M, 2048):
+        want = X[m:m + 2048].float() @ W.float().t() + b.float()
+        # 32 fp16 products summed in fp32, one rounding to half: half a unit in the last place of up to 64
+        assert (got[m:m + 2048].float() - want).abs().max().item() <= 2.0 ** -11 * 64, m
+
+
+@pytest.mark.parametrize("form", ["planned", "raw"])
+def test_tile_linear_of_many_workgroups(K, form):
+    """so many panels and column groups that their places need two launches: the bits of fewer rows at a time"""
+    from et_amd import lib
+    from et_amd.encoder import Linear_tile
+    M, N = 2049, 1 << 20
+    r = rng(93)
+    lin = make_tile_linear(r, N, 16, 0.0, seed=3, std=0.3, bias_std=0.2)
+    X = dev(randn_h(r, (M, 16)))
+    if form == "planned":
+        lt = Linear_tile(16, N, M, lin["row_offset"].size, lin["data"], lin["row_ptr"], lin["row_offset"], lin["bias"])
+        run = lambda x: lt.run(x)
+    else:
+        args = [dev(lin[k]) for k in ("row_ptr", "row_offset", "data", "bias")]
+        run = lambda x: K.tile_spmm_add_bias(x, *args, N)
+    # 32 rows x 8 block-rows a workgroup, the panels slowest: 65 x 8192 workgroups, places divided by 8192
+    keys = (("tile_form", 0, -1), ("tile_ipw", 1, 0)) if form == "planned" else (("tile_nb", 1, 0),)
+    try:
+        for key, value, _ in keys + (("tile_order", 0, 1),):
+            assert lib().et_tuning_set(key.encode(), value) == 0
+        got = run(X)
+        for m in range(0, M, 500):
+            assert torch.equal(got[m:m + 500], run(X[m:m + 500].contiguous())), m
+    finally:
+        for key, _, value in keys + (("tile_order", 0, 1),):
+            lib().et_tuning_set(key.encode(), value)
+
+
 @pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("M,Ns,Kd,gelu", [
     (1, (16,), 32, False),               # half a step of 64 columns, one piece of a block
